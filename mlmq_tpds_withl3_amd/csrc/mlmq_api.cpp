@@ -20,6 +20,7 @@
 
 #include "device_common.h"
 #include "hop_block.h"
+#include "region_solver.h"
 #include "solver_internal.h"
 
 struct mlmq_ctx {
@@ -68,6 +69,15 @@ struct mlmq_ctx {
     bool b_solved = false;
     hipGraphExec_t b_graph = nullptr;
     std::vector<uint64_t> b_graph_key;
+    // region solver: the graph's cut (regions.regions == 0: not cut) and the
+    // per-query state of up to r_queries queries
+    mlmq::RegionGraph regions;
+    uint32_t *r_inbox = nullptr, *r_act = nullptr;
+    uint32_t r_queries = 0;
+    uint64_t *r_ring = nullptr;
+    uint64_t r_ring_slots = 0;
+    bool r_ring_dirty = true;
+    uint32_t *h_ctl = nullptr;   // pinned: control block as copied out
     // this device's copy of the static workspace (mlmq_solve_noalloc)
     uint8_t *scratch = nullptr;
     std::string err;
@@ -147,8 +157,20 @@ void free_batch(mlmq_ctx *c) {
     c->b_slots_dirty = true;
 }
 
+void free_regions(mlmq_ctx *c) {
+    mlmq::region_free(&c->regions);
+    for (void *p : {(void *)c->r_inbox, (void *)c->r_act, (void *)c->r_ring})
+        if (p) (void)hipFree(p);
+    c->r_inbox = c->r_act = nullptr;
+    c->r_ring = nullptr;
+    c->r_queries = 0;
+    c->r_ring_slots = 0;
+    c->r_ring_dirty = true;
+}
+
 void free_graph(mlmq_ctx *c) {
     free_batch(c);
+    free_regions(c);
     if (c->owns_graph) {
         (void)hipFree(c->row);
         (void)hipFree(c->col);
@@ -224,11 +246,39 @@ int validate_csr(mlmq_ctx *c, int32_t n, int64_t m, const int64_t *row, const in
     return MLMQ_OK;
 }
 
+// The cut into regions (region_graph.h), where the graph has one.  A packed
+// edge holds weights below 2^(32 - kWeightShift).  `col`: the destinations
+// on the host, or null to copy them from the device.
+int build_regions(mlmq_ctx *c, const std::vector<uint32_t> &row, const uint32_t *col) {
+    const uint32_t n = (uint32_t)c->n;
+    if ((double)c->info.max_weight >= (double)(1u << (32 - mlmq::kWeightShift)) || c->m > 8ll * c->n ||
+        (uint32_t)c->info.max_nnz > mlmq::kRegionMaxDegree)
+        return MLMQ_OK;
+    std::vector<uint32_t> copy;
+    if (!col) {
+        copy.resize((size_t)c->m);
+        if (c->m)
+            HIP_TRY(c, hipMemcpy(copy.data(), c->col, sizeof(uint32_t) * (size_t)c->m, hipMemcpyDeviceToHost));
+        col = copy.data();
+    }
+    mlmq::RegionPlan plan;
+    if (!mlmq::region_plan(n, row.data(), col, &plan)) return MLMQ_OK;
+    const hipError_t e = mlmq::region_build(plan, n, (uint64_t)c->m, c->row, c->col, c->wgt,
+                                            (double)c->info.avg_weight, c->stream, &c->regions);
+    // past a limit, or no memory for the cut: the vertex queue serves the graph
+    if (e == hipErrorInvalidValue || e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        return MLMQ_OK;
+    }
+    HIP_TRY(c, e);
+    return MLMQ_OK;
+}
+
 // Device-side hop blocks (64 B per vertex) from the device CSR, and the hub
 // table: vertices with more than kSplitDeg out-edges, highest degree first,
 // at most kMaxHubs of them, each with a chunk size that keeps its chunk count
 // below 2^kChunkBits.
-int build_blocks(mlmq_ctx *c) {
+int build_blocks(mlmq_ctx *c, const uint32_t *host_col) {
     HIP_TRY(c, hipMalloc(&c->blocks, 64 * (size_t)c->n));
     // Back-edge slots fit when vertex ids and weights stay below 2^kBackShift
     // (the weight statistic is a float: rounding can only refuse a graph
@@ -265,7 +315,7 @@ int build_blocks(mlmq_ctx *c) {
         HIP_TRY(c, mlmq::launch_patch_hubs(c->hubs, c->nhubs, c->blocks, c->stream));
         HIP_TRY(c, hipStreamSynchronize(c->stream));
     }
-    return MLMQ_OK;
+    return build_regions(c, row, host_col);
 }
 
 int upload(mlmq_ctx *c, int32_t n, int64_t m, const int64_t *row, const int32_t *col,
@@ -326,7 +376,7 @@ int upload(mlmq_ctx *c, int32_t n, int64_t m, const int64_t *row, const int32_t 
     c->m = m;
     compute_info(&c->info, n, m, row, nullptr, w);
     c->sorted = true;
-    return build_blocks(c);
+    return build_blocks(c, reinterpret_cast<const uint32_t *>(col));
 }
 
 // Light-edge counts in the hop blocks for `delta` (light/heavy split).
@@ -557,6 +607,64 @@ struct QueryClock {
     clk::time_point q0, q1, s0, s1;
 };
 
+// The region solver answers the default queue mode on a cut graph.  Settings
+// that ask for a part of the vertex queue (its kernel variants, its profile,
+// a ring capacity) get the vertex queue.
+bool wants_regions(const mlmq_ctx *c, const mlmq_params &p) {
+    return c->regions.regions != 0 && p.queue_mode == MLMQ_QUEUE_L1SLF_L2DQ && !p.profile && !p.l1_blocks &&
+           !p.hub_split && !p.light_split && !p.defer_heavy && !p.strict_window && p.l1_donate == 0 &&
+           p.bucket_capacity == 0;
+}
+
+// Per-query state and ring of the region solver for nq queries on a grid of
+// at most `grid` workgroups.
+int ensure_region_space(mlmq_ctx *c, uint32_t nq, uint32_t grid) {
+    const mlmq::RegionGraph &g = c->regions;
+    if (c->r_queries < nq) {
+        for (void *p : {(void *)c->r_inbox, (void *)c->r_act})
+            if (p) (void)hipFree(p);
+        c->r_inbox = c->r_act = nullptr;
+        c->r_queries = 0;
+        HIP_TRY(c, hipMalloc(&c->r_inbox, sizeof(uint32_t) * ((size_t)nq * g.inbox_slots + 1)));
+        HIP_TRY(c, hipMalloc(&c->r_act, sizeof(uint32_t) * (size_t)nq * g.regions));
+        c->r_queries = nq;
+    }
+    // Each region of a query is in the ring at most once and each workgroup
+    // waits on one ticket; twice that, so that a slot is long read when the
+    // ring comes round to it (a writer that finds it full waits, bounded).
+    uint64_t need = 1024;
+    while (need < 2 * ((uint64_t)nq * g.regions + grid)) need *= 2;
+    if (c->r_ring_slots < need) {
+        if (c->r_ring) (void)hipFree(c->r_ring);
+        c->r_ring = nullptr;
+        c->r_ring_slots = 0;
+        HIP_TRY(c, hipMalloc(&c->r_ring, sizeof(uint64_t) * need));
+        c->r_ring_slots = need;
+        c->r_ring_dirty = true;
+    }
+    if (c->r_ring_dirty) {
+        HIP_TRY(c, mlmq::launch_fill_u64(c->r_ring, c->r_ring_slots, mlmq::kEmpty, c->stream));
+        c->r_ring_dirty = false;
+    }
+    if (!c->ctl) {
+        HIP_TRY(c, hipMalloc(&c->ctl, sizeof(uint32_t) * mlmq::kCtlWords));
+        c->ctl_host.assign(mlmq::kCtlWords, 0);
+    }
+    if (!c->h_ctl)
+        HIP_TRY(c, hipHostMalloc((void **)&c->h_ctl, sizeof(uint32_t) * mlmq::kCtlWords, hipHostMallocDefault));
+    return MLMQ_OK;
+}
+
+// Grid of a region solve: one workgroup per region task, at least
+// `at_least`, at most what the device holds.
+int region_grid(mlmq_ctx *c, uint64_t tasks, uint64_t at_least, uint32_t *grid) {
+    int occ = 0;
+    HIP_TRY(c, mlmq::region_occupancy(&occ));
+    if (occ < 1) return fail(c, MLMQ_E_HIP, "region solver cannot be resident");
+    *grid = (uint32_t)std::min<uint64_t>((uint64_t)occ * c->cus, std::max(tasks, at_least));
+    return MLMQ_OK;
+}
+
 // Reset and persistent launch of one query, on the context's stream; the
 // control block after the solve is copied into h (kCtlWords words).
 // fill_slots > 0 first fills that many ring slots with empty records.
@@ -630,6 +738,117 @@ void fill_timing(mlmq_ctx *c, const uint32_t *h, const QueryClock &t, int blocks
     timing->detail_cycles[4] = 0;
     timing->donated = st[mlmq::kStatDonated];
     timing->hub_chunks = st[mlmq::kStatChunks];
+}
+
+// nq queries by the region solver: from `src`, or from the device array
+// `sources`; distances into `dist`, one row of n after another.  On success
+// the control block is in ctl_host.
+int run_regions(mlmq_ctx *c, uint32_t nq, int32_t src, const uint32_t *sources, uint32_t *dist, uint64_t *qtime,
+                const mlmq_params &p, uint32_t grid, QueryClock *t) {
+    const mlmq::RegionGraph &g = c->regions;
+    mlmq::RegionLaunch L{};
+    L.space = {dist, c->r_inbox, c->r_act, (uint64_t)g.n, g.inbox_slots, g.regions};
+    L.ring = c->r_ring;
+    L.ring_mask = (uint32_t)(c->r_ring_slots - 1);
+    L.ctl = c->ctl;
+    L.qtime = qtime;
+    L.timeout_ticks = (uint64_t)((p.timeout_s > 0 ? p.timeout_s : 60.0) * (double)c->wall_khz * 1000.0);
+    L.nq = nq;
+    L.grid = grid;
+    t->q0 = clk::now();
+    HIP_TRY(c, hipEventRecord(c->ev_reset, c->stream));
+    HIP_TRY(c, mlmq::launch_region_reset(g, L, sources, (uint32_t)src, c->stream));
+    HIP_TRY(c, hipEventRecord(c->ev_start, c->stream));
+    c->r_ring_dirty = true;   // until the solve has left it clean
+    HIP_TRY(c, mlmq::launch_region_solver(g, L, c->stream));
+    HIP_TRY(c, hipEventRecord(c->ev_stop, c->stream));
+    HIP_TRY(c, hipMemcpyAsync(c->h_ctl, c->ctl, sizeof(uint32_t) * mlmq::kCtlWords, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    t->s1 = clk::now();
+    // one wait for both kernels: the reset's share of it from its events
+    float reset_ms = 0;
+    (void)hipEventElapsedTime(&reset_ms, c->ev_reset, c->ev_start);
+    t->q1 = t->s0 = std::min(t->s1, t->q0 + std::chrono::duration_cast<clk::duration>(
+                                              std::chrono::duration<double, std::milli>(reset_ms)));
+    std::copy(c->h_ctl, c->h_ctl + mlmq::kCtlWords, c->ctl_host.begin());
+    const int rc = query_status(c, c->ctl_host.data(), 1);
+    if (rc == MLMQ_OK) c->r_ring_dirty = false;
+    return rc;
+}
+
+// One query, distances into the context's row.
+int solve_regions(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *timing) {
+    uint32_t grid = 0;
+    int rc = region_grid(c, c->regions.regions, (uint64_t)p.work_blocks, &grid);
+    if (rc == MLMQ_OK) rc = ensure_region_space(c, 1, grid);
+    if (rc) return rc;
+    QueryClock t;
+    rc = run_regions(c, 1, src, nullptr, c->dist, nullptr, p, grid, &t);
+    if (rc) return rc;
+    c->solved = true;
+    c->last_buckets = (uint32_t)p.buckets;
+    c->last_window = (uint32_t)p.bucket_window;
+    c->last_cap_log2 = ceil_log2(c->r_ring_slots);
+    if (timing) {
+        fill_timing(c, c->ctl_host.data(), t, (int)grid, c->last_cap_log2, 0, timing);
+        timing->waves = mlmq::kRegionWaves * (int32_t)grid;
+    }
+    return MLMQ_OK;
+}
+
+// Statistics of a batch from its device counters and the queries' clock ticks.
+void fill_batch_timing(mlmq_ctx *c, const uint32_t *h, const std::vector<uint64_t> &qt, int32_t nq, double solve_ms,
+                       const mlmq_params &p, mlmq_batch_timing *timing) {
+    std::memset(timing, 0, sizeof(*timing));
+    float dev_ms = 0;
+    (void)hipEventElapsedTime(&dev_ms, c->ev_start, c->ev_stop);
+    timing->solve_ms = solve_ms;
+    timing->device_ms = dev_ms;
+    std::vector<double> lat((size_t)nq);
+    double sum = 0;
+    for (int32_t i = 0; i < nq; ++i) {
+        lat[i] = (double)(qt[2 * i + 1] - qt[2 * i]) / (double)c->wall_khz;
+        sum += lat[i];
+    }
+    std::sort(lat.begin(), lat.end());
+    timing->query_ms_p50 = lat[(size_t)(0.50 * (nq - 1))];
+    timing->query_ms_p99 = lat[(size_t)(0.99 * (nq - 1))];
+    timing->query_ms_max = lat.back();
+    timing->query_ms_mean = sum / nq;
+    timing->queries = nq;
+    timing->waves_per_query = p.batch_waves;
+    const uint64_t *st = reinterpret_cast<const uint64_t *>(h + mlmq::kStatsOff);
+    timing->relaxations = st[mlmq::kStatRelax];
+    timing->improvements = st[mlmq::kStatImprove];
+    timing->l2_pushes = st[mlmq::kStatL2Push] + (uint64_t)nq;
+    timing->stale = st[mlmq::kStatStale];
+    timing->batches = st[mlmq::kStatBatches];
+    timing->idle_polls = st[mlmq::kStatIdle];
+}
+
+// A batch by the region solver: every query of it in flight at once.
+int batch_regions(mlmq_ctx *c, int32_t nq, const mlmq_params &p, mlmq_batch_timing *timing) {
+    uint32_t grid = 0;
+    int rc = region_grid(c, (uint64_t)nq * c->regions.regions, 0, &grid);
+    if (rc == MLMQ_OK) rc = ensure_region_space(c, (uint32_t)nq, grid);
+    if (rc) return rc;
+    QueryClock t;
+    rc = run_regions(c, (uint32_t)nq, 0, c->b_sources, c->b_dist, c->b_qtime, p, grid, &t);
+    if (rc) return rc;
+    c->b_nq = nq;
+    c->b_solved = true;
+    if (!timing) return MLMQ_OK;
+    std::vector<uint64_t> qt(2 * (size_t)nq);
+    HIP_TRY(c, hipMemcpy(qt.data(), c->b_qtime, sizeof(uint64_t) * qt.size(), hipMemcpyDeviceToHost));
+    fill_batch_timing(c, c->ctl_host.data(), qt, nq, ms_since(t.q0, t.s1), p, timing);
+    float reset_ms = 0;   // the launch counts its row reset, as the vertex queue's does
+    (void)hipEventElapsedTime(&reset_ms, c->ev_reset, c->ev_start);
+    timing->device_ms += reset_ms;
+    timing->work_blocks = nq;
+    timing->bucket_capacity = (int64_t)c->r_ring_slots;
+    if (!p.batch_stats)
+        timing->relaxations = timing->improvements = timing->stale = timing->batches = timing->idle_polls = 0;
+    return MLMQ_OK;
 }
 
 }  // namespace
@@ -714,6 +933,7 @@ int mlmq_destroy(mlmq_ctx *c) {
     if (c->dist) (void)hipFree(c->dist);
     if (c->ctl) (void)hipFree(c->ctl);
     if (c->slots) (void)hipFree(c->slots);
+    if (c->h_ctl) (void)hipHostFree(c->h_ctl);
     free_batch(c);
     if (c->ev_reset) (void)hipEventDestroy(c->ev_reset);
     if (c->ev_start) (void)hipEventDestroy(c->ev_start);
@@ -805,7 +1025,7 @@ int mlmq_attach_device_csr(mlmq_ctx *c, int32_t n, int64_t m, const int32_t *row
     c->n = n;
     c->m = m;
     compute_info(&c->info, n, m, nullptr, row.data(), w.data());
-    return build_blocks(c);
+    return build_blocks(c, nullptr);
 }
 
 int mlmq_graph_stats(mlmq_ctx *c, mlmq_graph_info *info) {
@@ -843,6 +1063,10 @@ int mlmq_solve(mlmq_ctx *c, int32_t src, const mlmq_params *params, mlmq_timing 
     // The reset below overwrites the last solve's distances: until this solve
     // succeeds there is no result to copy out.
     c->solved = false;
+    if (wants_regions(c, q.p)) {
+        rc = solve_regions(c, src, q.p, timing);
+        if (rc != MLMQ_E_QUEUE_OVERFLOW) return rc;
+    }
 
     const uint32_t nb = (uint32_t)q.p.buckets;
     uint32_t cap_log2 = q.cap_log2;
@@ -978,6 +1202,13 @@ int mlmq_solve_batch(mlmq_ctx *c, const int32_t *sources, int32_t nq, const mlmq
     }
     if (!c->b_gctl) HIP_TRY(c, hipMalloc(&c->b_gctl, sizeof(uint32_t) * mlmq::kCtlWords));
     HIP_TRY(c, hipMemcpy(c->b_sources, sources, sizeof(int32_t) * nq, hipMemcpyHostToDevice));
+
+    // A chosen number of workgroups, one query each, is the vertex queue's.
+    // (kRegionQueries: a record's query field.)
+    if (wants_regions(c, p) && p.work_blocks == 0 && nq <= (int32_t)mlmq::kRegionQueries) {
+        const int rrc = batch_regions(c, nq, p, timing);
+        if (rrc != MLMQ_E_QUEUE_OVERFLOW && rrc != MLMQ_E_NOMEM) return rrc;
+    }
 
     const double timeout_s = p.timeout_s > 0 ? p.timeout_s : 60.0;
     uint64_t retries = 0;
@@ -1122,34 +1353,10 @@ int mlmq_solve_batch(mlmq_ctx *c, const int32_t *sources, int32_t nq, const mlmq
         c->b_nq = nq;
         c->b_solved = true;
         if (timing) {
-            std::memset(timing, 0, sizeof(*timing));
-            float dev_ms = 0;
-            (void)hipEventElapsedTime(&dev_ms, c->ev_start, c->ev_stop);
-            timing->solve_ms = ms_since(s0, s1);
-            timing->device_ms = dev_ms;
-            std::vector<double> lat((size_t)nq);
-            double sum = 0;
-            for (int32_t i = 0; i < nq; ++i) {
-                lat[i] = (double)(qt[2 * i + 1] - qt[2 * i]) / (double)c->wall_khz;
-                sum += lat[i];
-            }
-            std::sort(lat.begin(), lat.end());
-            timing->query_ms_p50 = lat[(size_t)(0.50 * (nq - 1))];
-            timing->query_ms_p99 = lat[(size_t)(0.99 * (nq - 1))];
-            timing->query_ms_max = lat.back();
-            timing->query_ms_mean = sum / nq;
-            timing->queries = nq;
+            fill_batch_timing(c, g.data(), qt, nq, ms_since(s0, s1), p, timing);
             timing->work_blocks = blocks;
-            timing->waves_per_query = p.batch_waves;
             timing->graph_replay = use_graph ? 1 : 0;
             timing->bucket_capacity = (int64_t)1 << cap_log2;
-            const uint64_t *st = reinterpret_cast<const uint64_t *>(g.data() + mlmq::kStatsOff);
-            timing->relaxations = st[mlmq::kStatRelax];
-            timing->improvements = st[mlmq::kStatImprove];
-            timing->l2_pushes = st[mlmq::kStatL2Push] + (uint64_t)nq;
-            timing->stale = st[mlmq::kStatStale];
-            timing->batches = st[mlmq::kStatBatches];
-            timing->idle_polls = st[mlmq::kStatIdle];
             timing->retries = retries;
         }
         return MLMQ_OK;

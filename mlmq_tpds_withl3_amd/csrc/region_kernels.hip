@@ -1,0 +1,811 @@
+// Region solver: shortest paths on a graph cut into regions that fit LDS.
+//
+// The vertex queue of sssp_kernels.hip pays one batch of dependent round
+// trips to memory per hop of the longest shortest path (about 2.3 us), and a
+// road graph has thousands of hops.  Here a hop inside a region costs a few
+// LDS round trips (about 0.3 us); only the 3-4 % of edges that leave a region
+// go through memory.
+//
+// A workgroup serves one region at a time.  Its waves share LDS words only and
+// never meet at a barrier while the region is served:
+//   * the relaxers own the region's vertices, four per lane, and hold their
+//     edges in registers.  A relaxer reads its vertices' distances (one 16-byte
+//     LDS read per lane), and a lane whose vertex is lower than it last
+//     expanded it lowers the heads by one LDS atomicMin per edge.  There is no
+//     queue: the comparison is the queue.  A lone wave issues one instruction
+//     per 8 cycles and an LDS round trip takes 64, so the hop costs what its
+//     instructions cost, and these are few;
+//   * the sender holds the exits.  When an exit's tail fell it lowers the
+//     target region's inbox slot with an agent-scope atomicMin, then marks that
+//     region active;
+//   * the poller reads its own region's inbox and activity word over and
+//     over, applies what improves, and adopts, settles and leaves regions.
+// Neighbouring served regions thus exchange distances at the latency of one
+// atomic and one poll.
+//
+// Quiet: LDS word `version` is raised by a relaxer after the atomicMins of an
+// expansion and by the poller after it applied news.  A relaxer or sender that
+// finds nothing to do publishes the version it read before it looked
+// (`checked`).  When every wave has checked the current version nothing is
+// left: whoever had work to do has not checked a version as new as the one
+// its cause raised, and a cause that has not raised the version yet is itself
+// such a wave.
+//
+// Activity word of a region, per query:
+//   kNew     never served
+//   kLeft    served and left: its distances are in the row
+//   kActive  has work: one credit is outstanding for it
+//   kIdle    served by a workgroup that polls it, no work known
+//   kOver    the solve is over
+// A sender completes its inbox write, then exchanges kActive into the word.
+// Reading kNew or kLeft it takes a credit and publishes a record in the ring;
+// reading kIdle it takes a credit only, the poller will see the word.  A
+// poller that finds its region quiet exchanges kIdle for kActive and then
+// reads the inbox once more: whatever was written by a sender that read
+// kActive is seen now, and the poller goes back to kActive with the credit it
+// still holds.  Otherwise it returns the credit.  Leaving writes the
+// distances back and then swaps kIdle for kLeft, which fails if a sender came
+// first.
+//
+// Ring: a workgroup without a region takes the next ticket (kHeadOff) and
+// polls that slot alone; a sender takes the next position (kRingTailOff) and
+// publishes there.  When every region has a workgroup, workgroup i starts on
+// region i without a record and leaves only after a long idle time, so that
+// records of regions whose workgroup is not resident are served all the same:
+// no workgroup ever waits for another one to become resident.
+//
+// Termination: credits taken are counted in kTailOff, returned ones in
+// kDoneOff.  Work in a region is covered by its own credit, or by the credit
+// of the sender whose message caused it and which has not yet marked it
+// active; a region returns its credit only when it is quiet and everything it
+// sent is marked.  So the return that makes both counts equal proves that no
+// work is left; its workgroup marks every region kOver and publishes one exit
+// record per workgroup of the grid, for the ticket each of them takes last.
+#include "device_common.h"
+#include "region_solver.h"
+#include "solver_internal.h"
+
+namespace mlmq {
+
+namespace {
+
+constexpr uint32_t kRingTailOff = kHungryOff;   // ring positions taken
+constexpr uint32_t kNew = 0, kActive = 1, kOver = 2, kIdle = 3, kLeft = 4;
+// Quiet polls before an active region returns its credit.
+constexpr uint32_t kSettle = 2;
+// Record: low word region | flags, high word query | seed's local id << 20.
+constexpr uint32_t kSeedFlag = 0x80000000u;
+constexpr uint32_t kVisitFlag = 0x40000000u;    // the region's distances are in the row
+constexpr uint32_t kQueryBits = 20;
+static_assert(kRegionQueries == 1u << kQueryBits && kQueryBits + kRegionIdBits <= 32, "record");
+
+constexpr uint32_t kThreads = kRegionWaves * kWave;
+constexpr uint32_t kPollerWave = kRelaxers, kSenderWave = kRelaxers + 1;
+
+struct RegionArgs {
+    const RegionHdr *hdr;
+    const uint32_t *image;
+    const uint32_t *verts;
+    RegionQuerySpace space;
+    uint64_t *ring;
+    uint32_t ring_mask;
+    uint32_t *ctl;
+    uint64_t *qtime;
+    uint64_t timeout_ticks;
+    uint32_t regions;
+    uint32_t tasks;          // regions x queries
+    uint32_t width;          // window of a wave's expansions
+    uint32_t preadopt;       // workgroup i starts on task i
+    uint32_t linger;         // idle polls before a region is left
+};
+
+struct RegionLds {
+    alignas(16) uint32_t dist[kRegionVerts];
+    uint32_t version;
+    uint32_t over;                     // the region is left: a wave without work returns
+    uint32_t checked[kRelaxers + 1];   // relaxers, sender
+    uint32_t rec[2];                   // adopted record
+    uint32_t state0;                   // activity word as adopted
+};
+
+__device__ __forceinline__ uint32_t sh_ld(uint32_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void sh_st(uint32_t *p, uint32_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ uint32_t sh_min(uint32_t *p, uint32_t v) {
+    return __hip_atomic_fetch_min(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void sh_add(uint32_t *p, uint32_t v) {
+    (void)__hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ uint32_t xchg32(uint32_t *p, uint32_t v) {
+    return __hip_atomic_exchange(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Rank of this lane among the set lanes of `m`.
+__device__ __forceinline__ uint32_t rank_of(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+// This lane's id, computed anew: keeps one wave's address arithmetic out of the
+// other waves' registers.
+__device__ __forceinline__ uint32_t fresh_lane() {
+    uint32_t lane = lane_id();
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
+// Every outstanding load, store and atomic of this wave is complete.
+__device__ __forceinline__ void wait_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// LDS accesses of a wave execute in order; this keeps the compiler's order too.
+__device__ __forceinline__ void lds_order() { asm volatile("" ::: "memory"); }
+__device__ __forceinline__ uint32_t *at_offset(uint32_t *base, uint32_t bytes) {
+    return reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(base) + bytes);
+}
+
+// ---- a relaxer ----
+
+struct RelaxStats {
+    uint32_t relax, improve, sweeps;
+};
+
+typedef uint32_t Quad __attribute__((ext_vector_type(4)));
+
+// Waits for a version other than `checked`.  A wave that has waited a while
+// naps longer: it leaves the issue slots to the waves of active regions.
+__device__ __forceinline__ void wait_version(RegionLds &S, uint32_t checked) {
+    for (uint32_t turn = 0; uniform(sh_ld(&S.version)) == checked; ++turn) {
+        if (turn < 32) __builtin_amdgcn_s_sleep(1);
+        else __builtin_amdgcn_s_sleep(8);
+    }
+}
+
+// Least value of the wave.
+__device__ __forceinline__ uint32_t wave_least(uint32_t x) {
+    // as a maximum of the complements: lanes outside a row keep the identity 0
+    return ~read_lane(wave_incl_max(~x), kWave - 1);
+}
+
+// More lowered vertices than this in a wave are expanded in order.
+constexpr uint32_t kWindowCount = 16;
+
+// Lower the heads of edges kFrom .. kTo - 1 of this lane's vertex at distance d.
+template <uint32_t kFrom, uint32_t kTo>
+__device__ __forceinline__ void lower_heads(RegionLds &S, const uint32_t (&edge)[kLaneEdges], uint32_t mask,
+                                            uint32_t shift, uint32_t d) {
+#pragma unroll
+    for (uint32_t k = kFrom; k < kTo; ++k) (void)sh_min(at_offset(S.dist, edge[k] & mask), d + (edge[k] >> shift));
+}
+
+__device__ __forceinline__ void run_relaxer(RegionLds &S, const RegionHdr &h, const uint32_t *image, uint32_t w,
+                                            uint32_t width, RelaxStats &st) {
+    const uint32_t lane = fresh_lane();
+    const uint32_t thread = w * kWave + lane;
+    uint32_t edge[kLaneVerts][kLaneEdges], last[kLaneVerts], most[kLaneVerts];
+    uint32_t degrees = 0;   // edges of each vertex, 8 bits each
+#pragma unroll
+    for (uint32_t i = 0; i < kLaneVerts; ++i) {
+        most[i] = image[kImageMost + w * kLaneVerts + i];
+        // a vertex is expanded below `last`; past the end: never
+        last[i] = i * kRegionThreads + thread < h.nv ? kUnreached : 0u;
+#pragma unroll
+        for (uint32_t k = 0; k < kLaneEdges; ++k) {
+            edge[i][k] = image[(i * kLaneEdges + k) * kRegionThreads + thread];
+            if (edge[i][k] >> kWeightShift != ~0u >> kWeightShift) degrees += 1u << 8 * i;
+        }
+    }
+    const Quad *own = reinterpret_cast<const Quad *>(S.dist + thread * kLaneVerts);
+    uint32_t checked = 0, expanded = 0, sweeps = 0;
+    for (;;) {
+        // the version before the distances
+        const uint32_t seen = sh_ld(&S.version);
+        lds_order();
+        const Quad now = *own;
+        lds_order();
+        const uint32_t cur[kLaneVerts] = {now[0], now[1], now[2], now[3]};
+        // edges are decoded as they are used: kept decoded, they would not fit
+        // the registers (the compiler must not see the constants)
+        uint32_t mask = kOffsetMask, shift = kWeightShift;
+        asm volatile("" : "+s"(mask), "+s"(shift));
+        uint64_t low[kLaneVerts], any = 0;
+        uint32_t count = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < kLaneVerts; ++i) {
+            low[i] = ballot(cur[i] < last[i]);
+            any |= low[i];
+            count += popc(low[i]);
+        }
+        if (any == 0) {
+            checked = uniform(seen);
+            if (uniform(sh_ld(&S.over))) break;
+            if (lane == 0) sh_st(&S.checked[w], checked);
+            wait_version(S, checked);
+            continue;
+        }
+        // Many at once: only those within `width` of the least (the others
+        // stay lower than last expanded, and come up again)
+        uint32_t limit = kUnreached;
+        if (count > kWindowCount) {
+            uint32_t least = kUnreached;
+#pragma unroll
+            for (uint32_t i = 0; i < kLaneVerts; ++i) least = min(least, cur[i] < last[i] ? cur[i] : kUnreached);
+            limit = wave_least(least) + width;
+#pragma unroll
+            for (uint32_t i = 0; i < kLaneVerts; ++i) low[i] = ballot(cur[i] < last[i] && cur[i] <= limit);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < kLaneVerts; ++i) {
+            if (low[i] == 0) continue;
+            expanded += popc(low[i]);
+            if (cur[i] < last[i] && cur[i] <= limit) {
+                last[i] = cur[i];
+                st.relax += (degrees >> 8 * i) & 0xFFu;   // per lane
+                lower_heads<0, kLaneEdges / 2>(S, edge[i], mask, shift, cur[i]);
+                if (most[i] > kLaneEdges / 2) lower_heads<kLaneEdges / 2, kLaneEdges>(S, edge[i], mask, shift, cur[i]);
+            }
+        }
+        sweeps += 1;
+        lds_order();
+        if (lane == 0) sh_add(&S.version, 1u);
+    }
+    st.improve += expanded;
+    st.sweeps += sweeps;
+}
+
+// ---- the sender and the poller ----
+
+struct MessageStats {
+    uint32_t credits, activations, messages, polls;
+};
+
+__device__ __forceinline__ void region_raise(const RegionArgs &a, uint32_t code) {
+    if (lane_id() == 0) {
+        cas32(a.ctl + kErrOff, kErrNone, code);
+        st_relaxed(a.ctl + kExitOff, 1u);
+    }
+}
+
+// Publish the records of the lanes with `valid` set.
+__device__ __forceinline__ void ring_push(const RegionArgs &a, bool valid, uint64_t rec) {
+    const uint64_t m = ballot(valid);
+    if (m == 0) return;
+    uint32_t pos0 = 0;
+    if (lane_id() == 0) pos0 = fetch_add(a.ctl + kRingTailOff, popc(m));
+    const uint32_t pos = read_lane(pos0, 0) + rank_of(m);
+    bool ok = true;
+    if (valid) {
+        uint64_t *slot = a.ring + (pos & a.ring_mask);
+        uint32_t spins = 0;
+        while (!cas64(slot, kEmpty, rec)) {
+            if (++spins > kSpinLimit) {
+                ok = false;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(2);
+        }
+    }
+    if (ballot(!ok)) region_raise(a, kErrOverflow);
+}
+
+template <int kG>
+__device__ __forceinline__ void run_sender(const RegionArgs &a, RegionLds &S, const RegionHdr &h,
+                                           const uint32_t *image, uint32_t query, uint32_t *inbox_all, uint32_t *act,
+                                           MessageStats &st) {
+    const uint32_t lane = fresh_lane();
+    const uint32_t *exits = image + kImageExits;
+    uint32_t edge[kG], slot[kG], reg[kG], last[kG];   // last: least distance sent
+#pragma unroll
+    for (int g = 0; g < kG; ++g) {
+        const uint32_t x = g * kWave + lane;
+        edge[g] = x < h.nx ? exits[x] : 0u;
+        slot[g] = x < h.nx ? exits[h.nx + x] : 0u;
+        reg[g] = x < h.nx ? exits[2 * h.nx + x] : 0u;
+        last[g] = x < h.nx ? kUnreached : 0u;         // 0: never sends
+    }
+    for (;;) {
+        const uint32_t version = uniform(sh_ld(&S.version));
+        if (uniform(sh_ld(&S.over))) break;
+        lds_order();
+        uint32_t d[kG], was[kG], state[kG];
+#pragma unroll
+        for (int g = 0; g < kG; ++g) d[g] = sh_ld(at_offset(S.dist, edge[g] & kOffsetMask));
+        bool send = false;
+#pragma unroll
+        for (int g = 0; g < kG; ++g) {
+            d[g] += edge[g] >> kWeightShift;
+            send = send || d[g] < last[g];
+        }
+        if (ballot(send) == 0) {
+            if (lane == 0) sh_st(&S.checked[kRelaxers], version);
+            wait_version(S, version);
+            continue;
+        }
+#pragma unroll
+        for (int g = 0; g < kG; ++g) {
+            was[g] = 0;
+            if (d[g] < last[g]) {
+                was[g] = fetch_min(inbox_all + slot[g], d[g]);
+                last[g] = d[g];
+                st.messages += 1;   // per lane
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < kG; ++g) asm volatile("" : "+v"(was[g])::"memory");   // complete before the marks
+#pragma unroll
+        for (int g = 0; g < kG; ++g) {
+            state[g] = kActive;
+            if (was[g] > d[g]) state[g] = xchg32(act + reg[g], kActive);
+        }
+#pragma unroll
+        for (int g = 0; g < kG; ++g) asm volatile("" : "+v"(state[g])::"memory");
+        uint32_t woken = 0;
+#pragma unroll
+        for (int g = 0; g < kG; ++g) woken += popc(ballot(state[g] != kActive));
+        if (woken) {
+            st.activations += lane == 0 ? woken : 0u;
+            uint32_t t = 0;
+            if (lane == 0) t = fetch_add(a.ctl + kTailOff, woken);
+            asm volatile("" : "+v"(t)::"memory");
+#pragma unroll
+            for (int g = 0; g < kG; ++g)
+                ring_push(a, state[g] == kNew || state[g] == kLeft,
+                          (uint64_t)query << 32 | reg[g] | (state[g] == kLeft ? kVisitFlag : 0u));
+            wait_memory();
+        }
+    }
+}
+
+// Return a credit; the last one ends the solve.
+__device__ __forceinline__ void return_credit(const RegionArgs &a, uint32_t query, MessageStats &st) {
+    const uint32_t lane = fresh_lane();
+    st.credits += lane == 0 ? 1u : 0u;
+    if (a.qtime && lane == 0)
+        __hip_atomic_fetch_max(a.qtime + 2 * query + 1, (uint64_t)wall_clock64(), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    uint32_t done = 0;
+    if (lane == 0) done = fetch_add(a.ctl + kDoneOff, 1u) + 1u;
+    asm volatile("" : "+v"(done)::"memory");
+    done = read_lane(done, 0);
+    const uint32_t tail = uniform(ld_relaxed(a.ctl + kTailOff));
+    if (done != tail) return;
+    const uint32_t ring_tail = uniform(ld_relaxed(a.ctl + kRingTailOff));
+    for (uint32_t i = lane; i < gridDim.x; i += kWave) {
+        uint64_t *slot = a.ring + ((ring_tail + i) & a.ring_mask);
+        __hip_atomic_store(slot, kRegionExit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    for (uint32_t i = lane; i < a.tasks; i += kWave) {
+        const uint32_t q = i / a.regions;
+        st_relaxed(a.space.act + q * a.space.act_stride + (i - q * a.regions), kOver);
+    }
+    wait_memory();
+    if (lane == 0) st_relaxed(a.ctl + kExitOff, 1u);
+}
+
+// Serves the adopted region until it is left or the solve is over.
+template <int kG>
+__device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, const RegionHdr &h,
+                                           const uint32_t *image, uint32_t region, uint32_t query, uint32_t *dist,
+                                           uint32_t *inbox, uint32_t *act, uint32_t seed, uint32_t state0,
+                                           uint64_t deadline, MessageStats &st) {
+    const uint32_t lane = fresh_lane();
+    uint32_t to[kG], seen[kG], val[kG];
+#pragma unroll
+    for (int g = 0; g < kG; ++g) {
+        const uint32_t x = g * kWave + lane;
+        to[g] = x < h.nin ? image[image_inbox(h) + x] : 0u;
+        seen[g] = x < h.nin ? kUnreached : 0u;   // 0: never news
+    }
+    // slots past the end repeat the last one (a region without any reads the
+    // spare word behind the inboxes or its neighbour's, and ignores it)
+    uint32_t at[kG];
+#pragma unroll
+    for (int g = 0; g < kG; ++g) at[g] = min(g * kWave + lane, h.nin ? h.nin - 1u : 0u);
+    uint32_t quiet = 0;
+    bool dirty = false, idle = state0 == kIdle;
+    // the waves look once at the adopted distances in any case: a version they
+    // have not checked
+    if (lane == 0) {
+        if (seed) sh_st(S.dist + (seed - 1u), 0u);
+        lds_order();
+        sh_add(&S.version, 1u);
+    }
+    dirty = seed != 0;
+    for (uint32_t turn = 0;; ++turn) {
+        if ((turn & 31u) == 0) {
+            if (uniform(ld_relaxed(a.ctl + kErrOff))) return;
+            if (wall_clock64() > deadline) {
+                region_raise(a, kErrTimeout);
+                return;
+            }
+        }
+        st.polls += lane == 0 ? 1u : 0u;
+        if (idle) {
+            // a sender marks the region after its message: the mark is enough
+            const uint32_t state = uniform(ld_relaxed(act + region));
+            if (state == kOver) break;
+            if (state == kIdle) {
+                __builtin_amdgcn_s_sleep(4);
+                if (++quiet < a.linger) continue;
+                quiet = 0;
+                if (dirty) {
+                    for (uint32_t i = lane; i < h.nv; i += kWave) {
+                        const uint32_t x = sh_ld(S.dist + local_id(i));
+                        if (x < kUnreached) st_relaxed(dist + a.verts[h.first + i], x);
+                    }
+                    dirty = false;
+                }
+                wait_memory();
+                uint32_t left = 0;
+                if (lane == 0) left = cas32(act + region, kIdle, kLeft) ? 1u : 0u;
+                if (read_lane(left, 0)) return;
+                continue;
+            }
+            idle = false;
+            quiet = 0;
+        }
+#pragma unroll
+        for (int g = 0; g < kG; ++g) val[g] = ld_relaxed(inbox + at[g]);
+        bool news = false, lower = false;
+#pragma unroll
+        for (int g = 0; g < kG; ++g) {
+            if (val[g] < seen[g]) {
+                news = true;
+                seen[g] = val[g];
+                lower = sh_min(at_offset(S.dist, to[g]), val[g]) > val[g] || lower;
+            }
+        }
+        if (ballot(lower)) {
+            lds_order();
+            if (lane == 0) sh_add(&S.version, 1u);
+        }
+        if (ballot(news)) {
+            dirty = true;
+            quiet = 0;
+            continue;
+        }
+        // the checks before the version: it only grows
+        const uint32_t done = sh_ld(&S.checked[min(lane, kRelaxers)]);
+        lds_order();
+        if (ballot(done != uniform(sh_ld(&S.version)))) {
+            quiet = 0;
+            continue;
+        }
+        if (++quiet < kSettle) continue;
+        quiet = 0;
+        uint32_t was = 0;
+        if (lane == 0) was = xchg32(act + region, kIdle);
+        asm volatile("" : "+v"(was)::"memory");
+        bool more = false;
+#pragma unroll
+        for (int g = 0; g < kG; ++g) val[g] = ld_relaxed(inbox + at[g]);
+#pragma unroll
+        for (int g = 0; g < kG; ++g) more = more || val[g] < seen[g];
+        if (ballot(more) == 0) {
+            idle = true;
+            return_credit(a, query, st);
+            continue;
+        }
+        if (lane == 0) was = xchg32(act + region, kActive);
+        asm volatile("" : "+v"(was)::"memory");
+        // a sender took another credit for this region meanwhile: one is enough
+        if (read_lane(was, 0) == kActive) return_credit(a, query, st);
+    }
+    // the solve is over
+    if (dirty)
+        for (uint32_t i = lane; i < h.nv; i += kWave) {
+            const uint32_t x = sh_ld(S.dist + local_id(i));
+            if (x < kUnreached) dist[a.verts[h.first + i]] = x;
+        }
+}
+
+__global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a) {
+    __shared__ RegionLds S;
+    const uint32_t wave = uniform(threadIdx.x / kWave);
+    const uint32_t lane = lane_id();
+    const uint64_t deadline = wall_clock64() + a.timeout_ticks;
+    RelaxStats rs{};
+    MessageStats ms{};
+    bool first = a.preadopt != 0;
+    for (;;) {
+        // adopt: this workgroup's own region first, then the next ticket's record
+        if (wave == kPollerWave && lane == 0) {
+            uint64_t rec = kEmpty;
+            bool rec_own = false;
+            if (first && blockIdx.x < a.tasks) {
+                const uint32_t q = blockIdx.x / a.regions, r = blockIdx.x - q * a.regions;
+                rec_own = cas32(a.space.act + q * a.space.act_stride + r, kNew, kIdle);
+                if (rec_own) rec = (uint64_t)q << 32 | r;
+            }
+            if (rec == kEmpty) {
+                uint64_t *slot = a.ring + (fetch_add(a.ctl + kHeadOff, 1u) & a.ring_mask);
+                for (uint32_t turn = 1;; ++turn) {
+                    rec = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (rec != kEmpty) {
+                        xchg64(slot, kEmpty);
+                        break;
+                    }
+                    // after an error no record will come; a finished solve
+                    // has put this ticket's exit record in place
+                    if ((turn & 15u) == 0 && (ld_relaxed(a.ctl + kErrOff) || wall_clock64() > deadline)) {
+                        rec = kRegionExit;
+                        break;
+                    }
+                    __builtin_amdgcn_s_sleep(4);
+                }
+            }
+            // adopted idle, or through a record: active
+            S.state0 = rec_own ? kIdle : kActive;
+            S.rec[0] = (uint32_t)rec;
+            S.rec[1] = (uint32_t)(rec >> 32);
+            S.version = S.over = 0;
+            for (uint32_t i = 0; i <= kRelaxers; ++i) S.checked[i] = 0;
+        }
+        first = false;
+        __syncthreads();
+        const uint32_t rec_lo = uniform(S.rec[0]), rec_hi = uniform(S.rec[1]);
+        if (((uint64_t)rec_hi << 32 | rec_lo) == kRegionExit) break;
+        const uint32_t region = rec_lo & ~(kSeedFlag | kVisitFlag);
+        const uint32_t query = rec_hi & ((1u << kQueryBits) - 1u);
+        const uint32_t seed = rec_lo & kSeedFlag ? (rec_hi >> kQueryBits) + 1u : 0u;
+        uint32_t *dist = a.space.dist + query * a.space.dist_stride;
+        uint32_t *inbox = a.space.inbox + query * a.space.inbox_stride;
+        uint32_t *act = a.space.act + query * a.space.act_stride;
+        const RegionHdr h = a.hdr[region];
+        const uint32_t *image = a.image + h.image;
+        for (uint32_t i = threadIdx.x; i < kRegionVerts; i += kThreads)
+            S.dist[local_id(i)] = (rec_lo & kVisitFlag) && i < h.nv ? ld_relaxed(dist + a.verts[h.first + i]) : kUnreached;
+        __syncthreads();
+        if (wave < kRelaxers) {
+            run_relaxer(S, h, image, wave, a.width, rs);
+        } else if (wave == kPollerWave) {
+            uint32_t *in = inbox + h.inbox;
+            const uint32_t state0 = uniform(S.state0);
+            if (h.nin <= 2 * kWave) run_poller<2>(a, S, h, image, region, query, dist, in, act, seed, state0, deadline, ms);
+            else if (h.nin <= 4 * kWave) run_poller<4>(a, S, h, image, region, query, dist, in, act, seed, state0, deadline, ms);
+            else run_poller<6>(a, S, h, image, region, query, dist, in, act, seed, state0, deadline, ms);
+            if (lane == 0) {
+                sh_st(&S.over, 1u);
+                lds_order();
+                sh_add(&S.version, 1u);   // wakes the waiting waves
+            }
+        } else if (wave == kSenderWave) {
+            if (h.nx <= 2 * kWave) run_sender<2>(a, S, h, image, query, inbox, act, ms);
+            else if (h.nx <= 4 * kWave) run_sender<4>(a, S, h, image, query, inbox, act, ms);
+            else run_sender<6>(a, S, h, image, query, inbox, act, ms);
+        }
+        __syncthreads();
+    }
+    uint64_t *stats = reinterpret_cast<uint64_t *>(a.ctl + kStatsOff);
+    if (wave < kRelaxers) {
+        const uint32_t relax = wave_sum(rs.relax);
+        if (lane == 0) {
+            add64(stats + kStatRelax, relax);
+            add64(stats + kStatImprove, rs.improve);
+            add64(stats + kStatBatches, rs.sweeps);
+        }
+    } else {
+        const uint32_t messages = wave_sum(ms.messages);
+        if (lane == 0) {
+            if (ms.credits) {
+                fetch_add(a.ctl + kTakenOff, ms.credits);
+                add64(stats + kStatL2Pop, ms.credits);
+            }
+            if (ms.activations) add64(stats + kStatL2Push, ms.activations);
+            if (messages) {
+                add64(stats + kStatAtomic, messages);
+                add64(stats + kStatRelax, messages);
+            }
+            if (ms.polls) add64(stats + kStatIdle, ms.polls);
+        }
+    }
+}
+
+// ---- reset ----
+
+__global__ __launch_bounds__(256) void region_reset_kernel(RegionQuerySpace sp, uint32_t n, uint32_t slots,
+                                                           uint32_t regions, uint32_t nq, const uint32_t *sources,
+                                                           uint32_t src, const uint32_t *where, uint32_t *ctl,
+                                                           uint64_t *ring, uint64_t *qtime) {
+    const uint32_t stride = gridDim.x * blockDim.x;
+    const uint32_t t0 = blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint32_t q = blockIdx.y; q < nq; q += gridDim.y) {
+        const uint32_t s = sources ? sources[q] : src;
+        uint32_t *dist = sp.dist + q * sp.dist_stride;
+        uint32_t *inbox = sp.inbox + q * sp.inbox_stride;
+        uint32_t *act = sp.act + q * sp.act_stride;
+        for (uint32_t i = t0; i < n; i += stride) dist[i] = i == s ? 0u : kUnreached;
+        for (uint32_t i = t0; i < slots; i += stride) inbox[i] = kUnreached;
+        const uint32_t at = where[s];
+        for (uint32_t i = t0; i < regions; i += stride) act[i] = i == at >> kRegionIdBits ? kActive : kNew;
+        if (t0 == 0) {
+            ring[q] = (uint64_t)((at & (kRegionVerts - 1u)) << kQueryBits | q) << 32 | kSeedFlag | at >> kRegionIdBits;
+            if (qtime) {
+                qtime[2 * q] = wall_clock64();
+                qtime[2 * q + 1] = 0;
+            }
+        }
+    }
+    if (blockIdx.y == 0)
+        for (uint32_t i = t0; i < kCtlWords; i += stride) ctl[i] = i == kTailOff || i == kRingTailOff ? nq : 0u;
+}
+
+// ---- building ----
+
+__global__ __launch_bounds__(256) void region_where_kernel(const uint32_t *verts, const uint32_t *first,
+                                                           uint32_t *where) {
+    const uint32_t r = blockIdx.x, lo = first[r], hi = first[r + 1];
+    for (uint32_t i = lo + threadIdx.x; i < hi; i += blockDim.x)
+        where[verts[i]] = r << kRegionIdBits | local_id(i - lo);
+}
+
+// Per region: exits.  Each takes an inbox slot of the region it enters:
+// tmp[e] = its number there.
+__global__ __launch_bounds__(256) void region_count_kernel(const uint32_t *row, const uint32_t *col,
+                                                           const uint32_t *verts, const uint32_t *where,
+                                                           RegionHdr *hdr, uint32_t *tmp) {
+    __shared__ uint32_t nx;
+    RegionHdr &h = hdr[blockIdx.x];
+    if (threadIdx.x == 0) nx = 0;
+    __syncthreads();
+    uint32_t mx = 0;
+    for (uint32_t i = threadIdx.x; i < h.nv; i += blockDim.x) {
+        const uint32_t u = verts[h.first + i], lo = row[u], hi = row[u + 1];
+        uint32_t inside = 0;
+        for (uint32_t e = lo; e < hi; ++e) {
+            const uint32_t r = where[col[e]] >> kRegionIdBits;
+            if (r == blockIdx.x && inside++ < kLaneEdges) continue;
+            ++mx;
+            tmp[e] = atomicAdd(&hdr[r].nin, 1u);
+        }
+    }
+    atomicAdd(&nx, mx);
+    __syncthreads();
+    if (threadIdx.x == 0) h.nx = nx;
+}
+
+__global__ __launch_bounds__(kRegionThreads) void region_image_kernel(const uint32_t *row, const uint32_t *col,
+                                                                      const uint32_t *wgt, const uint32_t *verts,
+                                                                      const uint32_t *where, const RegionHdr *hdr,
+                                                                      const uint32_t *tmp, uint32_t *image) {
+    __shared__ uint32_t most[kRelaxers * kLaneVerts], exits;
+    const RegionHdr h = hdr[blockIdx.x];
+    uint32_t *img = image + h.image;
+    if (threadIdx.x < kRelaxers * kLaneVerts) most[threadIdx.x] = 0;
+    if (threadIdx.x == 0) exits = 0;
+    __syncthreads();
+    uint32_t *xedge = img + kImageExits, *xslot = xedge + h.nx, *xreg = xslot + h.nx;
+    for (uint32_t i = 0; i < kLaneVerts; ++i) {
+        const uint32_t p = i * kRegionThreads + threadIdx.x;
+        const uint32_t own = 4 * local_id(p);
+        uint32_t inside = 0;
+        if (p < h.nv) {
+            const uint32_t u = verts[h.first + p], lo = row[u], hi = row[u + 1];
+            for (uint32_t e = lo; e < hi; ++e) {
+                const uint32_t to = where[col[e]], r = to >> kRegionIdBits, head = 4 * (to & (kRegionVerts - 1u));
+                if (r == blockIdx.x && inside < kLaneEdges) {
+                    img[(i * kLaneEdges + inside) * kRegionThreads + threadIdx.x] = head | wgt[e] << kWeightShift;
+                    ++inside;
+                    continue;
+                }
+                const RegionHdr &t = hdr[r];
+                const uint32_t x = atomicAdd(&exits, 1u);
+                xedge[x] = own | wgt[e] << kWeightShift;
+                xslot[x] = t.inbox + tmp[e];
+                xreg[x] = r;
+                image[t.image + image_inbox(t) + tmp[e]] = head;
+            }
+        }
+        atomicMax(&most[threadIdx.x / kWave * kLaneVerts + i], inside);
+        // absent edges: to the vertex itself, which they cannot lower
+        for (uint32_t k = inside; k < kLaneEdges; ++k)
+            img[(i * kLaneEdges + k) * kRegionThreads + threadIdx.x] = own | ~0u << kWeightShift;
+    }
+    __syncthreads();
+    if (threadIdx.x < kRelaxers * kLaneVerts) img[kImageMost + threadIdx.x] = most[threadIdx.x];
+}
+
+RegionArgs make_region_args(const RegionGraph &g, const RegionLaunch &L) {
+    RegionArgs a;
+    a.hdr = g.hdr;
+    a.image = g.image;
+    a.verts = g.verts;
+    a.space = L.space;
+    a.ring = L.ring;
+    a.ring_mask = L.ring_mask;
+    a.ctl = L.ctl;
+    a.qtime = L.qtime;
+    a.timeout_ticks = L.timeout_ticks;
+    a.regions = g.regions;
+    a.tasks = g.regions * L.nq;
+    a.width = g.width;
+    a.preadopt = L.grid >= a.tasks ? 1u : 0u;
+    // A region that keeps its workgroup is left only if some other may need
+    // it: after about 2 ms (polls of about 0.7 us).
+    a.linger = a.preadopt ? 3000u : 6u;
+    return a;
+}
+
+}  // namespace
+
+hipError_t region_occupancy(int *blocks_per_cu) {
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        blocks_per_cu, reinterpret_cast<const void *>(&region_solver_kernel), kThreads, 0);
+}
+
+void region_free(RegionGraph *g) {
+    for (void *p : {(void *)g->hdr, (void *)g->image, (void *)g->verts, (void *)g->where})
+        if (p) (void)hipFree(p);
+    *g = RegionGraph{};
+}
+
+hipError_t region_build(const RegionPlan &plan, uint32_t n, uint64_t m, const uint32_t *row, const uint32_t *col,
+                        const uint32_t *wgt, double mean_weight, hipStream_t s, RegionGraph *g) {
+    *g = RegionGraph{};
+    const uint32_t nr = (uint32_t)plan.first.size() - 1;
+    if (nr > (1u << (32 - kRegionIdBits))) return hipErrorInvalidValue;
+    std::vector<RegionHdr> hdr(nr);
+    for (uint32_t r = 0; r < nr; ++r) hdr[r] = RegionHdr{plan.first[r], plan.first[r + 1] - plan.first[r], 0, 0, 0, 0, {0, 0}};
+    uint32_t *tmp = nullptr, *first = nullptr;
+    hipError_t e = hipMalloc(&g->hdr, sizeof(RegionHdr) * nr);
+    if (e == hipSuccess) e = hipMalloc(&g->verts, sizeof(uint32_t) * (size_t)n);
+    if (e == hipSuccess) e = hipMalloc(&g->where, sizeof(uint32_t) * (size_t)n);
+    if (e == hipSuccess) e = hipMalloc(&tmp, sizeof(uint32_t) * (size_t)(m ? m : 1));
+    if (e == hipSuccess) e = hipMalloc(&first, sizeof(uint32_t) * ((size_t)nr + 1));
+    if (e == hipSuccess) e = hipMemcpy(g->hdr, hdr.data(), sizeof(RegionHdr) * nr, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(g->verts, plan.order.data(), sizeof(uint32_t) * (size_t)n, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(first, plan.first.data(), sizeof(uint32_t) * ((size_t)nr + 1), hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(region_where_kernel, dim3(nr), dim3(256), 0, s, g->verts, first, g->where);
+        hipLaunchKernelGGL(region_count_kernel, dim3(nr), dim3(256), 0, s, row, col, g->verts, g->where, g->hdr, tmp);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(hdr.data(), g->hdr, sizeof(RegionHdr) * nr, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    uint64_t slots = 0, words = 0;
+    if (e == hipSuccess) {
+        for (RegionHdr &h : hdr) {
+            if (h.nx > kRegionExits || h.nin > kRegionInbox) e = hipErrorInvalidValue;
+            h.inbox = (uint32_t)slots;
+            h.image = (uint32_t)words;
+            slots += h.nin;
+            words += image_words(h);
+        }
+        g->n = n;
+        g->regions = nr;
+        g->inbox_slots = (uint32_t)slots;
+        // eight mean edge weights
+        g->width = (uint32_t)std::min(1e9, std::max(1.0, 8.0 * mean_weight));
+        if (words > 0xFFFFFFF0ull) e = hipErrorInvalidValue;
+    }
+    if (e == hipSuccess) e = hipMalloc(&g->image, sizeof(uint32_t) * words);
+    if (e == hipSuccess) e = hipMemcpy(g->hdr, hdr.data(), sizeof(RegionHdr) * nr, hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(region_image_kernel, dim3(nr), dim3(kRegionThreads), 0, s, row, col, wgt, g->verts, g->where, g->hdr,
+                           tmp, g->image);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (tmp) (void)hipFree(tmp);
+    if (first) (void)hipFree(first);
+    if (e != hipSuccess) region_free(g);
+    return e;
+}
+
+hipError_t launch_region_reset(const RegionGraph &g, const RegionLaunch &L, const uint32_t *sources, uint32_t src,
+                               hipStream_t s) {
+    uint32_t longest = g.n > g.inbox_slots ? g.n : g.inbox_slots;
+    if (longest < kCtlWords) longest = kCtlWords;
+    uint32_t x = (longest + 1023) / 1024;
+    if (x > 2048) x = 2048;
+    const uint32_t y = L.nq < 1024 ? L.nq : 1024;
+    hipLaunchKernelGGL(region_reset_kernel, dim3(x, y), dim3(256), 0, s, L.space, g.n, g.inbox_slots, g.regions, L.nq,
+                       sources, src, g.where, L.ctl, L.ring, L.qtime);
+    return hipGetLastError();
+}
+
+hipError_t launch_region_solver(const RegionGraph &g, const RegionLaunch &L, hipStream_t s) {
+    hipLaunchKernelGGL(region_solver_kernel, dim3(L.grid), dim3(kThreads), 0, s,
+                       make_region_args(g, L));
+    return hipGetLastError();
+}
+
+}  // namespace mlmq

@@ -1,0 +1,61 @@
+// Internal interface of the region solver (region_kernels.hip): shortest
+// paths on a graph cut into regions (region_graph.h).  Not part of the ABI.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "region_graph.h"
+
+namespace mlmq {
+
+constexpr int kRegionWaves = kRelaxers + 2;   // waves of a workgroup
+
+constexpr uint32_t kRegionQueries = 1u << 20;   // queries of one launch
+
+// A cut graph on the device.
+struct RegionGraph {
+    uint32_t n = 0;
+    uint32_t regions = 0;
+    uint32_t inbox_slots = 0;
+    uint32_t width = 0;          // threshold step inside a region
+    RegionHdr *hdr = nullptr;    // per region
+    uint32_t *image = nullptr;
+    uint32_t *verts = nullptr;   // region-ordered vertex list
+    uint32_t *where = nullptr;   // vertex -> region << kRegionIdBits | local id
+};
+
+constexpr uint64_t kRegionExit = ~1ull;   // slot value that ends a workgroup
+
+struct RegionQuerySpace {        // per-query state; query q at the strides below
+    uint32_t *dist;
+    uint32_t *inbox;
+    uint32_t *act;
+    uint64_t dist_stride, inbox_stride, act_stride;
+};
+
+struct RegionLaunch {
+    RegionQuerySpace space;
+    uint64_t *ring;
+    uint32_t ring_mask;
+    uint32_t *ctl;               // control block (device_common.h)
+    uint64_t *qtime;             // optional: per query, wall-clock ticks of its start and end
+    uint64_t timeout_ticks;
+    uint32_t nq;
+    uint32_t grid;
+};
+
+hipError_t region_occupancy(int *blocks_per_cu);
+// Builds the device side of a cut (temporary device memory: 4 bytes per edge).
+// Returns hipErrorInvalidValue when some region exceeds the limits.
+hipError_t region_build(const RegionPlan &plan, uint32_t n, uint64_t m, const uint32_t *row, const uint32_t *col,
+                        const uint32_t *wgt, double mean_weight, hipStream_t s, RegionGraph *g);
+void region_free(RegionGraph *g);
+// Per-query reset (distances, inboxes, activity), the control block and the
+// seed records, then the solver.  `sources` is a device array of nq vertices,
+// or null: one query from `src`.
+hipError_t launch_region_reset(const RegionGraph &g, const RegionLaunch &L, const uint32_t *sources, uint32_t src,
+                               hipStream_t s);
+hipError_t launch_region_solver(const RegionGraph &g, const RegionLaunch &L, hipStream_t s);
+
+}  // namespace mlmq
