@@ -20,6 +20,7 @@
 
 #include "device_common.h"
 #include "hop_block.h"
+#include "pushpull_solver.h"
 #include "region_solver.h"
 #include "solver_internal.h"
 
@@ -78,6 +79,10 @@ struct mlmq_ctx {
     uint64_t r_ring_slots = 0;
     bool r_ring_dirty = true;
     uint32_t *h_ctl = nullptr;   // pinned: control block as copied out
+    // push-pull solver: the graph's push bound (0: not for this graph), and
+    // the per-query marks, vertex lists, counters
+    uint32_t pp_bound = 0;
+    uint32_t *pp_mark = nullptr, *pp_front = nullptr, *pp_count = nullptr;
     // this device's copy of the static workspace (mlmq_solve_noalloc)
     uint8_t *scratch = nullptr;
     std::string err;
@@ -168,9 +173,17 @@ void free_regions(mlmq_ctx *c) {
     c->r_ring_dirty = true;
 }
 
+void free_pushpull(mlmq_ctx *c) {
+    for (void *p : {(void *)c->pp_mark, (void *)c->pp_front, (void *)c->pp_count})
+        if (p) (void)hipFree(p);
+    c->pp_mark = c->pp_front = c->pp_count = nullptr;
+    c->pp_bound = 0;
+}
+
 void free_graph(mlmq_ctx *c) {
     free_batch(c);
     free_regions(c);
+    free_pushpull(c);
     if (c->owns_graph) {
         (void)hipFree(c->row);
         (void)hipFree(c->col);
@@ -271,6 +284,37 @@ int build_regions(mlmq_ctx *c, const std::vector<uint32_t> &row, const uint32_t 
         return MLMQ_OK;
     }
     HIP_TRY(c, e);
+    return MLMQ_OK;
+}
+
+// The push-pull solver's preparation, for undirected graphs of strongly varying
+// degree: a standard deviation of at least twice the mean (an RMAT graph has
+// 4 to 10 times, a road graph or grid under half, a few hubs in a large sparse
+// graph under one), with enough edges that pushing all of them costs more than
+// its twenty launches.  `w`: the weights on the host.
+int build_pushpull(mlmq_ctx *c, const int32_t *w) {
+    const mlmq_graph_info &gi = c->info;
+    if (!c->sorted || c->regions.regions || c->m < 4ll * c->n || gi.dev_nnz < 2.0f * gi.avg_nnz) return MLMQ_OK;
+    uint32_t *flag = nullptr, bad = 0;
+    HIP_TRY(c, hipMalloc(&flag, sizeof(uint32_t)));
+    hipError_t e = mlmq::launch_fill_u32(flag, 1, 0u, c->stream);
+    if (e == hipSuccess)
+        e = mlmq::launch_symmetry_check(c->row, c->col, c->wgt, (uint32_t)c->n, flag, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(&bad, flag, sizeof(bad), hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    (void)hipFree(flag);
+    HIP_TRY(c, e);
+    if (bad) return MLMQ_OK;
+    // The bound: the weight that 5 % of the edges do not exceed.  On RMAT-22
+    // the pushes up to it examine 9 % of the edges and the pull 7 %; half of it
+    // 3 and 15 %, twice 24 and 4 %.
+    std::vector<int32_t> sample;
+    const int64_t step = std::max<int64_t>(1, c->m / 65536);
+    for (int64_t i = step / 2; i < c->m; i += step) sample.push_back(w[i]);
+    std::nth_element(sample.begin(), sample.begin() + sample.size() / 20, sample.end());
+    c->pp_bound = (uint32_t)std::max(1, sample[sample.size() / 20]);
+    HIP_TRY(c, mlmq::launch_bound_counts(c->row, c->wgt, (uint32_t)c->n, c->pp_bound, c->blocks, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
     return MLMQ_OK;
 }
 
@@ -376,7 +420,8 @@ int upload(mlmq_ctx *c, int32_t n, int64_t m, const int64_t *row, const int32_t 
     c->m = m;
     compute_info(&c->info, n, m, row, nullptr, w);
     c->sorted = true;
-    return build_blocks(c, reinterpret_cast<const uint32_t *>(col));
+    rc = build_blocks(c, reinterpret_cast<const uint32_t *>(col));
+    return rc ? rc : build_pushpull(c, w);
 }
 
 // Light-edge counts in the hop blocks for `delta` (light/heavy split).
@@ -405,11 +450,20 @@ int ensure_dist(mlmq_ctx *c) {
     return MLMQ_OK;
 }
 
-int ensure_queue(mlmq_ctx *c, uint32_t nbuckets, uint32_t cap_log2) {
+// The control block and its host copies.
+int ensure_ctl(mlmq_ctx *c) {
     if (!c->ctl) {
         HIP_TRY(c, hipMalloc(&c->ctl, sizeof(uint32_t) * mlmq::kCtlWords));
         c->ctl_host.assign(mlmq::kCtlWords, 0);
     }
+    if (!c->h_ctl)
+        HIP_TRY(c, hipHostMalloc((void **)&c->h_ctl, sizeof(uint32_t) * mlmq::kCtlWords, hipHostMallocDefault));
+    return MLMQ_OK;
+}
+
+int ensure_queue(mlmq_ctx *c, uint32_t nbuckets, uint32_t cap_log2) {
+    const int crc = ensure_ctl(c);
+    if (crc) return crc;
     const uint64_t need = (uint64_t)nbuckets << cap_log2;
     if (c->slots && c->slots_count < need) {
         (void)hipFree(c->slots);
@@ -616,6 +670,13 @@ bool wants_regions(const mlmq_ctx *c, const mlmq_params &p) {
            p.bucket_capacity == 0;
 }
 
+// The push-pull solver answers the same calls on the graphs it is for; the
+// light/heavy edge split is one of its own.
+bool wants_pushpull(const mlmq_ctx *c, const mlmq_params &p) {
+    return c->pp_bound != 0 && p.queue_mode == MLMQ_QUEUE_L1SLF_L2DQ && !p.profile && !p.l1_blocks && !p.hub_split &&
+           !p.defer_heavy && !p.strict_window && p.l1_donate == 0 && p.bucket_capacity == 0;
+}
+
 // Per-query state and ring of the region solver for nq queries on a grid of
 // at most `grid` workgroups.
 int ensure_region_space(mlmq_ctx *c, uint32_t nq, uint32_t grid) {
@@ -646,13 +707,7 @@ int ensure_region_space(mlmq_ctx *c, uint32_t nq, uint32_t grid) {
         HIP_TRY(c, mlmq::launch_fill_u64(c->r_ring, c->r_ring_slots, mlmq::kEmpty, c->stream));
         c->r_ring_dirty = false;
     }
-    if (!c->ctl) {
-        HIP_TRY(c, hipMalloc(&c->ctl, sizeof(uint32_t) * mlmq::kCtlWords));
-        c->ctl_host.assign(mlmq::kCtlWords, 0);
-    }
-    if (!c->h_ctl)
-        HIP_TRY(c, hipHostMalloc((void **)&c->h_ctl, sizeof(uint32_t) * mlmq::kCtlWords, hipHostMallocDefault));
-    return MLMQ_OK;
+    return ensure_ctl(c);
 }
 
 // Grid of a region solve: one workgroup per region task, at least
@@ -792,6 +847,81 @@ int solve_regions(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *t
     if (timing) {
         fill_timing(c, c->ctl_host.data(), t, (int)grid, c->last_cap_log2, 0, timing);
         timing->waves = mlmq::kRegionWaves * (int32_t)grid;
+    }
+    return MLMQ_OK;
+}
+
+// One query by the push-pull solver, distances into the context's row.
+// MLMQ_E_QUEUE_OVERFLOW: more rounds than it is meant for.
+int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *timing) {
+    const size_t n = (size_t)c->n;
+    int rc = ensure_ctl(c);
+    if (rc) return rc;
+    if (!c->pp_mark) HIP_TRY(c, hipMalloc(&c->pp_mark, sizeof(uint32_t) * n));
+    if (!c->pp_front) HIP_TRY(c, hipMalloc(&c->pp_front, sizeof(uint32_t) * 2 * n));
+    constexpr size_t kCountWords = mlmq::kMaxRounds + 2;   // 8-byte aligned end, then the work counters
+    static_assert(kCountWords % 2 == 0 && kCountWords + 4 <= mlmq::kCtlWords, "copied through the control block's buffer");
+    if (!c->pp_count) HIP_TRY(c, hipMalloc(&c->pp_count, sizeof(uint32_t) * (kCountWords + 4)));
+    mlmq::PushPullLaunch L{};
+    L.col = c->col;
+    L.wgt = c->wgt;
+    L.blocks = c->blocks;
+    L.id_mask = c->packed ? (1u << mlmq::kBackShift) - 1u : 0xFFFFFFFFu;
+    L.dist = c->dist;
+    L.mark = c->pp_mark;
+    L.front[0] = c->pp_front;
+    L.front[1] = c->pp_front + n;
+    L.count = c->pp_count;
+    L.work = reinterpret_cast<uint64_t *>(c->pp_count + kCountWords);
+    L.n = (uint32_t)n;
+    L.bound = c->pp_bound;
+    const double timeout_ms = (p.timeout_s > 0 ? p.timeout_s : 60.0) * 1e3;
+    QueryClock t;
+    t.q0 = clk::now();
+    HIP_TRY(c, hipEventRecord(c->ev_reset, c->stream));
+    HIP_TRY(c, mlmq::launch_pushpull_reset(L, (uint32_t)src, c->stream));
+    HIP_TRY(c, hipEventRecord(c->ev_start, c->stream));
+    uint32_t round = 0;
+    for (; round < mlmq::kBoundedRounds; ++round) HIP_TRY(c, mlmq::launch_push(L, round, true, c->stream));
+    HIP_TRY(c, mlmq::launch_pull(L, round, c->stream));
+    const uint32_t *h = c->h_ctl;
+    for (uint32_t more = mlmq::kFullRounds;; more = 8) {
+        for (uint32_t k = 0; k < more; ++k, ++round) HIP_TRY(c, mlmq::launch_push(L, round, false, c->stream));
+        HIP_TRY(c, hipEventRecord(c->ev_stop, c->stream));
+        HIP_TRY(c, hipMemcpyAsync(c->h_ctl, c->pp_count, sizeof(uint32_t) * (kCountWords + 4), hipMemcpyDeviceToHost,
+                                  c->stream));
+        HIP_TRY(c, hipStreamSynchronize(c->stream));
+        t.s1 = clk::now();
+        if (ms_since(t.q0, t.s1) > timeout_ms) return fail(c, MLMQ_E_TIMEOUT, "watchdog expired");
+        if (h[round] == 0) break;
+        if (round + 8 > mlmq::kMaxRounds)
+            return fail(c, MLMQ_E_QUEUE_OVERFLOW, "push-pull solver: too many rounds");
+    }
+    float reset_ms = 0;
+    (void)hipEventElapsedTime(&reset_ms, c->ev_reset, c->ev_start);
+    t.q1 = t.s0 = std::min(t.s1, t.q0 + std::chrono::duration_cast<clk::duration>(
+                                            std::chrono::duration<double, std::milli>(reset_ms)));
+    // queue counts: every vertex queued in some round, all in the first bucket
+    uint64_t queued = 0;
+    for (uint32_t r = 0; r < round; ++r) queued += h[r];
+    const uint64_t *work = reinterpret_cast<const uint64_t *>(h + kCountWords);
+    std::vector<uint32_t> &ctl = c->ctl_host;
+    std::fill(ctl.begin(), ctl.end(), 0u);
+    ctl[mlmq::kTailOff] = ctl[mlmq::kTakenOff] = ctl[mlmq::kDoneOff] = (uint32_t)queued;
+    ctl[mlmq::kExitOff] = 1;
+    uint64_t *st = reinterpret_cast<uint64_t *>(ctl.data() + mlmq::kStatsOff);
+    st[mlmq::kStatL2Push] = queued - 1;   // without the source, as the kernels count
+    st[mlmq::kStatL2Pop] = queued;
+    st[mlmq::kStatRelax] = st[mlmq::kStatAtomic] = work[0];
+    st[mlmq::kStatImprove] = work[1];
+    st[mlmq::kStatBatches] = round;
+    c->solved = true;
+    c->last_buckets = (uint32_t)p.buckets;
+    c->last_window = (uint32_t)p.bucket_window;
+    c->last_cap_log2 = ceil_log2(n);
+    if (timing) {
+        fill_timing(c, ctl.data(), t, (int)mlmq::push_groups(L.n), c->last_cap_log2, 0, timing);
+        timing->waves = mlmq::kPushWaves * timing->work_blocks;
     }
     return MLMQ_OK;
 }
@@ -1065,6 +1195,9 @@ int mlmq_solve(mlmq_ctx *c, int32_t src, const mlmq_params *params, mlmq_timing 
     c->solved = false;
     if (wants_regions(c, q.p)) {
         rc = solve_regions(c, src, q.p, timing);
+        if (rc != MLMQ_E_QUEUE_OVERFLOW) return rc;
+    } else if (wants_pushpull(c, q.p)) {
+        rc = solve_pushpull(c, src, q.p, timing);
         if (rc != MLMQ_E_QUEUE_OVERFLOW) return rc;
     }
 

@@ -1,0 +1,351 @@
+// Push-pull solver: shortest paths on undirected power-law graphs.
+//
+// Most of such a graph's edges are heavy edges of hubs, and they lower nothing:
+// on RMAT-22 (weights 1..1000) every vertex of degree 30 is reached at a
+// distance of 10-100, so a hub's edges of weight 100-1000 only matter to the
+// few vertices that have no lighter way in.  The vertex queue still relaxes
+// each of the 128 M edges once.  Here
+//   1. rounds of pushes lower vertices up to a bound B only: a vertex at
+//      distance d reads its edges of weight <= B - d, a prefix of its sorted
+//      adjacency whose length comes from its hop block;
+//   2. one pull: every vertex beyond B looks at its own few edges, lightest
+//      first, until the weight alone exceeds the best sum;
+//   3. rounds of full pushes from the pulled vertices, and from what phase 1
+//      may have left, finish the rest.
+// Edges examined on RMAT-22: about 25 % of the graph (B = the 5 % quantile of
+// the weights), against 105 % before.  Any B gives the same distances: a
+// vertex's last improvement is always followed by a push of all its edges,
+// or found by the pull of the edge's other end.  The graph must be undirected
+// (checked edge by edge when it is loaded): the pull reads out-edges as
+// in-edges.
+//
+// Every round is one launch, and no workgroup waits for another.  A round that
+// finds nothing costs its launch.
+#include "device_common.h"
+#include "hop_block.h"
+#include "pushpull_solver.h"
+
+namespace mlmq {
+
+namespace {
+
+constexpr uint32_t kGroup = 256;        // threads of a workgroup
+constexpr uint32_t kBuffer = 2048;      // queued vertices a workgroup gathers
+constexpr uint32_t kUnroll = 4;
+
+struct OutBuffer {
+    uint32_t n;
+    uint32_t base;
+    uint32_t v[kBuffer];
+};
+
+__device__ __forceinline__ void queue_vertex(OutBuffer &B, uint32_t *out, uint32_t *count, uint32_t v) {
+    const uint32_t p = atomicAdd(&B.n, 1u);
+    if (p < kBuffer) B.v[p] = v;
+    else out[fetch_add(count, 1u)] = v;
+}
+
+// All threads of the workgroup.
+__device__ __forceinline__ void flush_buffer(OutBuffer &B, uint32_t *out, uint32_t *count) {
+    __syncthreads();
+    const uint32_t have = min(B.n, kBuffer);
+    if (threadIdx.x == 0 && have) B.base = fetch_add(count, have);
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < have; i += kGroup) out[B.base + i] = B.v[i];
+    __syncthreads();
+}
+
+// Lower v to nd; queue it once a round when that succeeds.
+__device__ __forceinline__ bool lower(const PushPullLaunch &L, OutBuffer &B, uint32_t *out, uint32_t *count,
+                                      uint32_t round, uint32_t v, uint32_t nd) {
+    if (fetch_min(L.dist + v, nd) <= nd) return false;
+    if (__hip_atomic_exchange(L.mark + v, round + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != round + 1u)
+        queue_vertex(B, out, count, v);
+    return true;
+}
+
+// A workgroup takes its share of the round's vertices, at most one per thread:
+// few vertices of many edges are spread over all workgroups.  Inline vertices
+// are pushed by their thread; the others' edges are numbered through and
+// dealt out to all threads.
+template <bool kBounded>
+__global__ __launch_bounds__(kGroup) void push_kernel(PushPullLaunch L, uint32_t round) {
+    __shared__ OutBuffer B;
+    __shared__ uint32_t s_first[kGroup + 1], s_start[kGroup], s_dist[kGroup], s_wave[kGroup / kWave];
+    __shared__ uint32_t s_work[2];
+    const uint32_t count = L.count[round];
+    if (count == 0) return;
+    const uint32_t *in = L.front[round & 1u];
+    uint32_t *out = L.front[(round + 1u) & 1u], *out_count = L.count + round + 1;
+    const uint32_t share = min(kGroup, (count + gridDim.x - 1) / gridDim.x);
+    if (threadIdx.x == 0) {
+        B.n = 0;
+        s_work[0] = s_work[1] = 0;
+    }
+    uint32_t edges = 0, improved = 0;
+    for (uint32_t b = blockIdx.x * share; b < count; b += gridDim.x * share) {
+        const bool have = threadIdx.x < share && b + threadIdx.x < count;
+        uint32_t len = 0, start = 0, d = 0;
+        __syncthreads();
+        if (have) {
+            const uint32_t v = in[b + threadIdx.x];
+            const uint4 *p = L.blocks + 4ull * v;
+            const uint4 q0 = p[0], q1 = p[1], q2 = p[2], q3 = p[3];
+            d = L.dist[v];
+            const uint32_t limit = kBounded ? L.bound : kUnreached - 1u;
+            if (q0.x <= kInlineEdges) {
+                const uint32_t word[14] = {q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x,
+                                           q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
+                uint32_t was[kInlineEdges];
+#pragma unroll
+                for (uint32_t k = 0; k < kInlineEdges; ++k)
+                    was[k] = k < q0.x ? L.dist[word[2 * k] & L.id_mask] : 0u;
+#pragma unroll
+                for (uint32_t k = 0; k < kInlineEdges; ++k) {
+                    const uint32_t nd = d + word[2 * k + 1];
+                    if (nd < was[k] && nd <= limit)
+                        improved += lower(L, B, out, out_count, round, word[2 * k] & L.id_mask, nd) ? 1u : 0u;
+                }
+                edges += q0.x;
+            } else {
+                start = q0.y;
+                len = q0.x;
+                if (kBounded) {
+                    // the least step that covers every weight up to bound - d
+                    const uint32_t room = L.bound - min(d, L.bound);
+                    const uint32_t step = L.bound / kBoundSteps + 1u;
+                    const uint32_t j = min(room / step, kBoundSteps - 1u);
+                    const uint32_t word[8] = {q2.x, q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
+#pragma unroll
+                    for (uint32_t k = 0; k < kBoundSteps; ++k)
+                        if (k == j) len = word[k];
+                }
+            }
+        }
+        // number the edges
+        const uint32_t incl = wave_incl_add(len);
+        const uint32_t wave = threadIdx.x / kWave;
+        if (lane_id() == kWave - 1) s_wave[wave] = incl;
+        s_start[threadIdx.x] = start;
+        s_dist[threadIdx.x] = d;
+        __syncthreads();
+        uint32_t before = 0, total = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kGroup / kWave; ++k) {
+            before += k < wave ? s_wave[k] : 0u;
+            total += s_wave[k];
+        }
+        s_first[threadIdx.x] = before + incl - len;
+        if (threadIdx.x == 0) s_first[kGroup] = total;
+        __syncthreads();
+        edges += threadIdx.x == 0 ? total : 0u;
+        for (uint32_t e0 = threadIdx.x; e0 < total; e0 += kUnroll * kGroup) {
+            uint32_t c[kUnroll], nd[kUnroll], was[kUnroll];
+#pragma unroll
+            for (uint32_t j = 0; j < kUnroll; ++j) {
+                const uint32_t e = e0 + j * kGroup;
+                // the last vertex whose first edge is <= e
+                uint32_t lo = 0;
+#pragma unroll
+                for (uint32_t k = kGroup / 2; k; k /= 2)
+                    if (s_first[lo + k] <= e) lo += k;
+                const uint32_t at = e < total ? s_start[lo] + (e - s_first[lo]) : s_start[lo];
+                c[j] = L.col[at];
+                nd[j] = e < total ? s_dist[lo] + L.wgt[at] : kUnreached;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < kUnroll; ++j) was[j] = L.dist[c[j]];
+#pragma unroll
+            for (uint32_t j = 0; j < kUnroll; ++j)
+                if (nd[j] < was[j] && (!kBounded || nd[j] <= L.bound))
+                    improved += lower(L, B, out, out_count, round, c[j], nd[j]) ? 1u : 0u;
+        }
+    }
+    flush_buffer(B, out, out_count);
+    edges = wave_sum(edges);
+    improved = wave_sum(improved);
+    if (lane_id() == 0) {
+        atomicAdd(&s_work[0], edges);
+        atomicAdd(&s_work[1], improved);
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 && s_work[threadIdx.x]) add64(L.work + threadIdx.x, s_work[threadIdx.x]);
+}
+
+// Every vertex beyond the bound takes the best distance over its edges.
+__global__ __launch_bounds__(kGroup) void pull_kernel(PushPullLaunch L, uint32_t round) {
+    __shared__ OutBuffer B;
+    __shared__ uint32_t s_work[2];
+    uint32_t *out = L.front[round & 1u], *out_count = L.count + round;
+    if (threadIdx.x == 0) {
+        B.n = 0;
+        s_work[0] = s_work[1] = 0;
+    }
+    __syncthreads();
+    uint32_t edges = 0, improved = 0;
+    for (uint32_t base = blockIdx.x * kGroup; base < L.n; base += gridDim.x * kGroup) {
+        const uint32_t v = base + threadIdx.x;
+        const uint32_t d = v < L.n ? L.dist[v] : 0u;
+        uint32_t best = d, deg = 0, start = 0;
+        if (d > L.bound) {
+            const uint4 *p = L.blocks + 4ull * v;
+            const uint4 q0 = p[0];
+            if (q0.x > kInlineEdges) {
+                deg = q0.x;
+                start = q0.y;
+            } else if (q0.x) {
+                const uint4 q1 = p[1], q2 = p[2], q3 = p[3];
+                const uint32_t word[14] = {q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x,
+                                           q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
+                uint32_t from[kInlineEdges];
+#pragma unroll
+                for (uint32_t k = 0; k < kInlineEdges; ++k)
+                    from[k] = k < q0.x ? L.dist[word[2 * k] & L.id_mask] : kUnreached;
+#pragma unroll
+                for (uint32_t k = 0; k < kInlineEdges; ++k)
+                    if (from[k] < kUnreached) best = min(best, from[k] + word[2 * k + 1]);
+                edges += q0.x;
+            }
+        }
+        // the others one after another, 64 edges at a time, lightest first
+        for (uint64_t rest = ballot(deg != 0); rest; rest &= rest - 1) {
+            const uint32_t l = (uint32_t)__builtin_ctzll(rest);
+            const uint32_t s = read_lane(start, l), n = read_lane(deg, l);
+            uint32_t b = read_lane(best, l);
+            for (uint32_t at = 0; at < n; at += kWave) {
+                const bool in = at + lane_id() < n;
+                const uint32_t e = s + (in ? at + lane_id() : n - 1u);
+                const uint32_t c = L.col[e], w = L.wgt[e];
+                const uint32_t from = L.dist[c];
+                uint32_t x = in && from < kUnreached ? from + w : ~0u;
+                x = ~read_lane(wave_incl_max(~x), kWave - 1);
+                b = min(b, x);
+                edges += in ? 1u : 0u;
+                if (read_lane(w, kWave - 1) >= b) break;
+            }
+            if (lane_id() == l) best = b;
+        }
+        if (best < d) {
+            // (only this thread lowers v in this launch, and no vertex beyond
+            // the bound is in the list yet; the mark belongs to the pushes)
+            L.dist[v] = best;
+            ++improved;
+            queue_vertex(B, out, out_count, v);
+        }
+    }
+    flush_buffer(B, out, out_count);
+    edges = wave_sum(edges);
+    improved = wave_sum(improved);
+    if (lane_id() == 0) {
+        atomicAdd(&s_work[0], edges);
+        atomicAdd(&s_work[1], improved);
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 && s_work[threadIdx.x]) add64(L.work + threadIdx.x, s_work[threadIdx.x]);
+}
+
+__global__ __launch_bounds__(256) void pushpull_reset_kernel(PushPullLaunch L, uint32_t src) {
+    const uint32_t stride = gridDim.x * blockDim.x, t = blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint32_t i = t; i < L.n; i += stride) {
+        L.dist[i] = i == src ? 0u : kUnreached;
+        L.mark[i] = 0;
+    }
+    for (uint32_t i = t; i <= kMaxRounds; i += stride) L.count[i] = i == 0 ? 1u : 0u;
+    if (t == 0) {
+        L.front[0][0] = src;
+        L.work[0] = L.work[1] = 0;
+    }
+}
+
+__global__ __launch_bounds__(256) void symmetry_kernel(const uint32_t *row, const uint32_t *col, const uint32_t *wgt,
+                                                       uint32_t n, uint32_t *asymmetric) {
+    // a wave per vertex, an edge per lane
+    const uint32_t waves = gridDim.x * blockDim.x / kWave;
+    for (uint32_t u = (blockIdx.x * blockDim.x + threadIdx.x) / kWave; u < n; u += waves) {
+        const uint32_t lo = row[u], hi = row[u + 1];
+        bool bad = false;
+        for (uint32_t e = lo + lane_id(); e < hi; e += kWave) {
+            const uint32_t v = col[e], w = wgt[e];
+            uint32_t a = row[v], b = row[v + 1];
+            bool found = false;
+            if (b - a > kInlineEdges) {
+                while (a < b) {   // first entry >= (w, u)
+                    const uint32_t m = a + (b - a) / 2, mw = wgt[m];
+                    if (mw < w || (mw == w && col[m] < u)) a = m + 1;
+                    else b = m;
+                }
+                found = a < row[v + 1] && wgt[a] == w && col[a] == u;
+            } else {
+                for (; a < b; ++a) found = found || (wgt[a] == w && col[a] == u);
+            }
+            bad = bad || !found;
+        }
+        if (ballot(bad) && lane_id() == 0) *asymmetric = 1;
+    }
+}
+
+__global__ __launch_bounds__(256) void bound_count_kernel(const uint32_t *row, const uint32_t *wgt, uint32_t n,
+                                                          uint32_t bound, uint4 *blocks) {
+    const uint32_t stride = gridDim.x * blockDim.x;
+    const uint32_t step = bound / kBoundSteps + 1u;
+    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride) {
+        const uint32_t s = row[v], e = row[v + 1];
+        if (e - s <= kInlineEdges) continue;
+        uint32_t at = s;
+        for (uint32_t j = 0; j < kBoundSteps; ++j) {
+            // edges of weight < step * (j + 1); the last step covers the bound
+            const uint32_t top = step * (j + 1);
+            uint32_t lo = at, hi = e;
+            while (lo < hi) {
+                const uint32_t mid = lo + (hi - lo) / 2;
+                if (wgt[mid] < top) lo = mid + 1;
+                else hi = mid;
+            }
+            at = lo;
+            reinterpret_cast<uint32_t *>(blocks + 4ull * v)[8 + j] = at - s;
+        }
+    }
+}
+
+uint32_t groups_for(uint64_t items, uint32_t most) {
+    const uint64_t g = (items + kGroup - 1) / kGroup;
+    return (uint32_t)(g < 1 ? 1 : g > most ? most : g);
+}
+
+}  // namespace
+
+hipError_t launch_symmetry_check(const uint32_t *row, const uint32_t *col, const uint32_t *wgt, uint32_t n,
+                                 uint32_t *asymmetric, hipStream_t s) {
+    hipLaunchKernelGGL(symmetry_kernel, dim3(groups_for((uint64_t)n * kWave, 16384)), dim3(256), 0, s, row, col, wgt,
+                       n, asymmetric);
+    return hipGetLastError();
+}
+
+hipError_t launch_bound_counts(const uint32_t *row, const uint32_t *wgt, uint32_t n, uint32_t bound, uint4 *blocks,
+                               hipStream_t s) {
+    hipLaunchKernelGGL(bound_count_kernel, dim3(groups_for(n, 16384)), dim3(256), 0, s, row, wgt, n, bound, blocks);
+    return hipGetLastError();
+}
+
+hipError_t launch_pushpull_reset(const PushPullLaunch &L, uint32_t src, hipStream_t s) {
+    hipLaunchKernelGGL(pushpull_reset_kernel, dim3(groups_for(L.n, 4096)), dim3(256), 0, s, L, src);
+    return hipGetLastError();
+}
+
+// Eight workgroups per CU hold their out buffers in LDS at once; a graph of
+// few vertices never fills them.
+uint32_t push_groups(uint32_t n) { return groups_for((uint64_t)n * 8, 2048); }
+
+hipError_t launch_push(const PushPullLaunch &L, uint32_t round, bool bounded, hipStream_t s) {
+    const dim3 grid(push_groups(L.n)), group(kGroup);
+    if (bounded) hipLaunchKernelGGL(push_kernel<true>, grid, group, 0, s, L, round);
+    else hipLaunchKernelGGL(push_kernel<false>, grid, group, 0, s, L, round);
+    return hipGetLastError();
+}
+
+hipError_t launch_pull(const PushPullLaunch &L, uint32_t round, hipStream_t s) {
+    hipLaunchKernelGGL(pull_kernel, dim3(groups_for(L.n, 4096)), dim3(kGroup), 0, s, L, round);
+    return hipGetLastError();
+}
+
+}  // namespace mlmq

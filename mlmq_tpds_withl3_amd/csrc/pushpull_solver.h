@@ -1,0 +1,48 @@
+// Internal interface of the push-pull solver (pushpull_kernels.hip): shortest
+// paths on undirected power-law graphs.  Not part of the ABI.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace mlmq {
+
+// Per graph: the push bound, and words 8..15 of every hop block with more than
+// kInlineEdges edges = its edges of weight <= bound * (j + 1) / 8, j = 0..7.
+constexpr uint32_t kBoundSteps = 8;
+// Rounds of pushes up to the bound before the pull, and of full pushes after
+// it, that are launched before the host looks.
+constexpr uint32_t kBoundedRounds = 12;
+constexpr uint32_t kFullRounds = 5;
+constexpr uint32_t kMaxRounds = 1024;   // counters per query
+
+struct PushPullLaunch {
+    const uint32_t *col;
+    const uint32_t *wgt;
+    const uint4 *blocks;
+    uint32_t id_mask;        // vertex bits of an inline edge's destination word
+    uint32_t *dist;          // n
+    uint32_t *mark;          // n: last round that queued the vertex
+    uint32_t *front[2];      // n each: the rounds' vertices, by parity
+    uint32_t *count;         // kMaxRounds + 1: vertices of each round
+    uint64_t *work;          // edges examined, improvements
+    uint32_t n;
+    uint32_t bound;
+};
+
+// *asymmetric = 1 if some edge (u, v, w) has no edge (v, u, w).  Rows of more
+// than kInlineEdges edges are sorted by (weight, destination).
+hipError_t launch_symmetry_check(const uint32_t *row, const uint32_t *col, const uint32_t *wgt, uint32_t n,
+                                 uint32_t *asymmetric, hipStream_t s);
+hipError_t launch_bound_counts(const uint32_t *row, const uint32_t *wgt, uint32_t n, uint32_t bound, uint4 *blocks,
+                               hipStream_t s);
+hipError_t launch_pushpull_reset(const PushPullLaunch &L, uint32_t src, hipStream_t s);
+// Workgroups of a push launch, and waves of each.
+uint32_t push_groups(uint32_t n);
+constexpr int kPushWaves = 4;
+// Round r expands the vertices of count[r] into those of count[r + 1].
+hipError_t launch_push(const PushPullLaunch &L, uint32_t round, bool bounded, hipStream_t s);
+// Adds the pulled vertices to those of count[round].
+hipError_t launch_pull(const PushPullLaunch &L, uint32_t round, hipStream_t s);
+
+}  // namespace mlmq
