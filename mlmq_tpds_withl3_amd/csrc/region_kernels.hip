@@ -31,21 +31,20 @@
 // its cause raised, and a cause that has not raised the version yet is itself
 // such a wave.
 //
-// Activity word of a region, per query:
-//   kNew     never served
-//   kLeft    served and left: its distances are in the row
-//   kActive  has work: one credit is outstanding for it
-//   kIdle    served by a workgroup that polls it, no work known
-//   kOver    the solve is over
-// A sender completes its inbox write, then exchanges kActive into the word.
-// Reading kNew or kLeft it takes a credit and publishes a record in the ring;
-// reading kIdle it takes a credit only, the poller will see the word.  A
-// poller that finds its region quiet exchanges kIdle for kActive and then
-// reads the inbox once more: whatever was written by a sender that read
-// kActive is seen now, and the poller goes back to kActive with the credit it
-// still holds.  Otherwise it returns the credit.  Leaving writes the
-// distances back and then swaps kIdle for kLeft, which fails if a sender came
-// first.
+// Activity word of a region, per query, in bits:
+//   kWork     has work: one credit is or will be outstanding for it
+//   kCounted  that credit has been counted
+//   kServed   a workgroup serves the region and polls this word
+//   kVisited  its distances are in the row
+//   kOver     the solve is over
+// A sender completes its inbox write, then sets kWork.  If it was clear, the
+// sender counts a credit, only then sets kCounted, and publishes a record in
+// the ring unless the region is served.  A poller that finds its region quiet
+// and counted clears both bits and then reads the inbox once more: whatever was
+// written by a sender that found kWork set is seen now, and the poller sets
+// kWork again and keeps its credit, unless a sender did first.  Otherwise it
+// returns the credit.  Leaving writes the distances back and then clears
+// kServed, which fails if kWork came first.
 //
 // Ring: a workgroup without a region takes the next ticket (kHeadOff) and
 // polls that slot alone; a sender takes the next position (kRingTailOff) and
@@ -54,10 +53,10 @@
 // records of regions whose workgroup is not resident are served all the same:
 // no workgroup ever waits for another one to become resident.
 //
-// Termination: credits taken are counted in kTailOff, returned ones in
-// kDoneOff.  Work in a region is covered by its own credit, or by the credit
-// of the sender whose message caused it and which has not yet marked it
-// active; a region returns its credit only when it is quiet and everything it
+// Termination: credits are counted in kTailOff before they can be returned, and
+// returned ones in kDoneOff.  Work in a region is covered by its own credit, or
+// by that of the sender whose message caused it and which has not finished
+// marking; a region returns its credit only when it is quiet and everything it
 // sent is marked.  So the return that makes both counts equal proves that no
 // work is left; its workgroup marks every region kOver and publishes one exit
 // record per workgroup of the grid, for the ticket each of them takes last.
@@ -70,7 +69,7 @@ namespace mlmq {
 namespace {
 
 constexpr uint32_t kRingTailOff = kHungryOff;   // ring positions taken
-constexpr uint32_t kNew = 0, kActive = 1, kOver = 2, kIdle = 3, kLeft = 4;
+constexpr uint32_t kWork = 1, kCounted = 2, kServed = 4, kVisited = 8, kOver = 16;
 // Quiet polls before an active region returns its credit.
 constexpr uint32_t kSettle = 2;
 // Record: low word region | flags, high word query | seed's local id << 20.
@@ -105,7 +104,7 @@ struct RegionLds {
     uint32_t over;                     // the region is left: a wave without work returns
     uint32_t checked[kRelaxers + 1];   // relaxers, sender
     uint32_t rec[2];                   // adopted record
-    uint32_t state0;                   // activity word as adopted
+    uint32_t own;                      // adopted without a record: no work yet
 };
 
 __device__ __forceinline__ uint32_t sh_ld(uint32_t *p) {
@@ -120,8 +119,8 @@ __device__ __forceinline__ uint32_t sh_min(uint32_t *p, uint32_t v) {
 __device__ __forceinline__ void sh_add(uint32_t *p, uint32_t v) {
     (void)__hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-__device__ __forceinline__ uint32_t xchg32(uint32_t *p, uint32_t v) {
-    return __hip_atomic_exchange(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ uint32_t fetch_or(uint32_t *p, uint32_t v) {
+    return __hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // Rank of this lane among the set lanes of `m`.
 __device__ __forceinline__ uint32_t rank_of(uint64_t m) {
@@ -332,23 +331,28 @@ __device__ __forceinline__ void run_sender(const RegionArgs &a, RegionLds &S, co
         for (int g = 0; g < kG; ++g) asm volatile("" : "+v"(was[g])::"memory");   // complete before the marks
 #pragma unroll
         for (int g = 0; g < kG; ++g) {
-            state[g] = kActive;
-            if (was[g] > d[g]) state[g] = xchg32(act + reg[g], kActive);
+            state[g] = kWork;
+            if (was[g] > d[g]) state[g] = fetch_or(act + reg[g], kWork);
         }
 #pragma unroll
         for (int g = 0; g < kG; ++g) asm volatile("" : "+v"(state[g])::"memory");
         uint32_t woken = 0;
 #pragma unroll
-        for (int g = 0; g < kG; ++g) woken += popc(ballot(state[g] != kActive));
+        for (int g = 0; g < kG; ++g) woken += popc(ballot(!(state[g] & kWork)));
         if (woken) {
             st.activations += lane == 0 ? woken : 0u;
             uint32_t t = 0;
             if (lane == 0) t = fetch_add(a.ctl + kTailOff, woken);
-            asm volatile("" : "+v"(t)::"memory");
+            asm volatile("" : "+v"(t)::"memory");   // counted before it can be returned
+#pragma unroll
+            for (int g = 0; g < kG; ++g) {
+                const bool wake = !(state[g] & kWork);
+                if (wake) (void)fetch_or(act + reg[g], kCounted);
+            }
 #pragma unroll
             for (int g = 0; g < kG; ++g)
-                ring_push(a, state[g] == kNew || state[g] == kLeft,
-                          (uint64_t)query << 32 | reg[g] | (state[g] == kLeft ? kVisitFlag : 0u));
+                ring_push(a, !(state[g] & (kWork | kServed)),
+                          (uint64_t)query << 32 | reg[g] | (state[g] & kVisited ? kVisitFlag : 0u));
             wait_memory();
         }
     }
@@ -384,7 +388,7 @@ __device__ __forceinline__ void return_credit(const RegionArgs &a, uint32_t quer
 template <int kG>
 __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, const RegionHdr &h,
                                            const uint32_t *image, uint32_t region, uint32_t query, uint32_t *dist,
-                                           uint32_t *inbox, uint32_t *act, uint32_t seed, uint32_t state0,
+                                           uint32_t *inbox, uint32_t *act, uint32_t seed, uint32_t base, bool idle,
                                            uint64_t deadline, MessageStats &st) {
     const uint32_t lane = fresh_lane();
     uint32_t to[kG], seen[kG], val[kG];
@@ -400,7 +404,7 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
 #pragma unroll
     for (int g = 0; g < kG; ++g) at[g] = min(g * kWave + lane, h.nin ? h.nin - 1u : 0u);
     uint32_t quiet = 0;
-    bool dirty = false, idle = state0 == kIdle;
+    bool dirty = false;
     // the waves look once at the adopted distances in any case: a version they
     // have not checked
     if (lane == 0) {
@@ -421,8 +425,8 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
         if (idle) {
             // a sender marks the region after its message: the mark is enough
             const uint32_t state = uniform(ld_relaxed(act + region));
-            if (state == kOver) break;
-            if (state == kIdle) {
+            if (state & kOver) break;
+            if (!(state & kWork)) {
                 __builtin_amdgcn_s_sleep(4);
                 if (++quiet < a.linger) continue;
                 quiet = 0;
@@ -435,7 +439,7 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
                 }
                 wait_memory();
                 uint32_t left = 0;
-                if (lane == 0) left = cas32(act + region, kIdle, kLeft) ? 1u : 0u;
+                if (lane == 0) left = cas32(act + region, base, kVisited) ? 1u : 0u;
                 if (read_lane(left, 0)) return;
                 continue;
             }
@@ -471,9 +475,10 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
         }
         if (++quiet < kSettle) continue;
         quiet = 0;
-        uint32_t was = 0;
-        if (lane == 0) was = xchg32(act + region, kIdle);
-        asm volatile("" : "+v"(was)::"memory");
+        uint32_t cleared = 0;
+        if (lane == 0) cleared = cas32(act + region, base | kWork | kCounted, base) ? 1u : 0u;
+        asm volatile("" : "+v"(cleared)::"memory");
+        if (!read_lane(cleared, 0)) continue;   // its sender is about to count the credit
         bool more = false;
 #pragma unroll
         for (int g = 0; g < kG; ++g) val[g] = ld_relaxed(inbox + at[g]);
@@ -484,10 +489,11 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
             return_credit(a, query, st);
             continue;
         }
-        if (lane == 0) was = xchg32(act + region, kActive);
+        uint32_t was = 0;
+        if (lane == 0) was = fetch_or(act + region, kWork);
         asm volatile("" : "+v"(was)::"memory");
-        // a sender took another credit for this region meanwhile: one is enough
-        if (read_lane(was, 0) == kActive) return_credit(a, query, st);
+        if (read_lane(was, 0) & kWork) return_credit(a, query, st);   // a sender's credit covers the news
+        else if (lane == 0) (void)fetch_or(act + region, kCounted);
     }
     // the solve is over
     if (dirty)
@@ -512,7 +518,7 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
             bool rec_own = false;
             if (first && blockIdx.x < a.tasks) {
                 const uint32_t q = blockIdx.x / a.regions, r = blockIdx.x - q * a.regions;
-                rec_own = cas32(a.space.act + q * a.space.act_stride + r, kNew, kIdle);
+                rec_own = cas32(a.space.act + q * a.space.act_stride + r, 0u, kServed);
                 if (rec_own) rec = (uint64_t)q << 32 | r;
             }
             if (rec == kEmpty) {
@@ -532,8 +538,13 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
                     __builtin_amdgcn_s_sleep(4);
                 }
             }
-            // adopted idle, or through a record: active
-            S.state0 = rec_own ? kIdle : kActive;
+            if (!rec_own && rec != kRegionExit) {
+                // (its word: kWork, kCounted and perhaps kVisited)
+                const uint32_t q = (uint32_t)(rec >> 32) & (kRegionQueries - 1u);
+                const uint32_t r = (uint32_t)rec & ~(kSeedFlag | kVisitFlag);
+                (void)fetch_or(a.space.act + q * a.space.act_stride + r, kServed);
+            }
+            S.own = rec_own ? 1u : 0u;
             S.rec[0] = (uint32_t)rec;
             S.rec[1] = (uint32_t)(rec >> 32);
             S.version = S.over = 0;
@@ -558,10 +569,11 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
             run_relaxer(S, h, image, wave, a.width, rs);
         } else if (wave == kPollerWave) {
             uint32_t *in = inbox + h.inbox;
-            const uint32_t state0 = uniform(S.state0);
-            if (h.nin <= 2 * kWave) run_poller<2>(a, S, h, image, region, query, dist, in, act, seed, state0, deadline, ms);
-            else if (h.nin <= 4 * kWave) run_poller<4>(a, S, h, image, region, query, dist, in, act, seed, state0, deadline, ms);
-            else run_poller<6>(a, S, h, image, region, query, dist, in, act, seed, state0, deadline, ms);
+            const bool idle = uniform(S.own) != 0;
+            const uint32_t held = kServed | (rec_lo & kVisitFlag ? kVisited : 0u);
+            if (h.nin <= 2 * kWave) run_poller<2>(a, S, h, image, region, query, dist, in, act, seed, held, idle, deadline, ms);
+            else if (h.nin <= 4 * kWave) run_poller<4>(a, S, h, image, region, query, dist, in, act, seed, held, idle, deadline, ms);
+            else run_poller<6>(a, S, h, image, region, query, dist, in, act, seed, held, idle, deadline, ms);
             if (lane == 0) {
                 sh_st(&S.over, 1u);
                 lds_order();
@@ -615,7 +627,7 @@ __global__ __launch_bounds__(256) void region_reset_kernel(RegionQuerySpace sp, 
         for (uint32_t i = t0; i < n; i += stride) dist[i] = i == s ? 0u : kUnreached;
         for (uint32_t i = t0; i < slots; i += stride) inbox[i] = kUnreached;
         const uint32_t at = where[s];
-        for (uint32_t i = t0; i < regions; i += stride) act[i] = i == at >> kRegionIdBits ? kActive : kNew;
+        for (uint32_t i = t0; i < regions; i += stride) act[i] = i == at >> kRegionIdBits ? kWork | kCounted : 0u;
         if (t0 == 0) {
             ring[q] = (uint64_t)((at & (kRegionVerts - 1u)) << kQueryBits | q) << 32 | kSeedFlag | at >> kRegionIdBits;
             if (qtime) {
