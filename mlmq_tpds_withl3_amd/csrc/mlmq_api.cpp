@@ -79,9 +79,10 @@ struct mlmq_ctx {
     uint64_t r_ring_slots = 0;
     bool r_ring_dirty = true;
     uint32_t *h_ctl = nullptr;   // pinned: control block as copied out
-    // push-pull solver: the graph's push bound (0: not for this graph), and
+    // push-pull solver: the graph's reach and hub degree (reach 0: not for
+    // this graph), and
     // the per-query marks, vertex lists, counters
-    uint32_t pp_bound = 0;
+    uint32_t pp_reach = 0, pp_hub = 0;
     uint32_t *pp_mark = nullptr, *pp_front = nullptr, *pp_count = nullptr;
     // this device's copy of the static workspace (mlmq_solve_noalloc)
     uint8_t *scratch = nullptr;
@@ -177,7 +178,7 @@ void free_pushpull(mlmq_ctx *c) {
     for (void *p : {(void *)c->pp_mark, (void *)c->pp_front, (void *)c->pp_count})
         if (p) (void)hipFree(p);
     c->pp_mark = c->pp_front = c->pp_count = nullptr;
-    c->pp_bound = 0;
+    c->pp_reach = 0;
 }
 
 void free_graph(mlmq_ctx *c) {
@@ -305,15 +306,17 @@ int build_pushpull(mlmq_ctx *c, const int32_t *w) {
     (void)hipFree(flag);
     HIP_TRY(c, e);
     if (bad) return MLMQ_OK;
-    // The bound: the weight that 5 % of the edges do not exceed.  On RMAT-22
+    // The reach: the weight that 5 % of the edges do not exceed.  On RMAT-22
     // the pushes up to it examine 9 % of the edges and the pull 7 %; half of it
     // 3 and 15 %, twice 24 and 4 %.
     std::vector<int32_t> sample;
     const int64_t step = std::max<int64_t>(1, c->m / 65536);
     for (int64_t i = step / 2; i < c->m; i += step) sample.push_back(w[i]);
     std::nth_element(sample.begin(), sample.begin() + sample.size() / 20, sample.end());
-    c->pp_bound = (uint32_t)std::max(1, sample[sample.size() / 20]);
-    HIP_TRY(c, mlmq::launch_bound_counts(c->row, c->wgt, (uint32_t)c->n, c->pp_bound, c->blocks, c->stream));
+    c->pp_reach = (uint32_t)std::max(1, sample[sample.size() / 20]);
+    // hubs: every shortest path of some length runs through their neighbourhood
+    c->pp_hub = (uint32_t)std::min(32.0 * gi.avg_nnz, 0.5 * gi.max_nnz);
+    HIP_TRY(c, mlmq::launch_bound_counts(c->row, c->wgt, (uint32_t)c->n, c->pp_reach, c->blocks, c->stream));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     return MLMQ_OK;
 }
@@ -673,7 +676,7 @@ bool wants_regions(const mlmq_ctx *c, const mlmq_params &p) {
 // The push-pull solver answers the same calls on the graphs it is for; the
 // light/heavy edge split is one of its own.
 bool wants_pushpull(const mlmq_ctx *c, const mlmq_params &p) {
-    return c->pp_bound != 0 && p.queue_mode == MLMQ_QUEUE_L1SLF_L2DQ && !p.profile && !p.l1_blocks && !p.hub_split &&
+    return c->pp_reach != 0 && p.queue_mode == MLMQ_QUEUE_L1SLF_L2DQ && !p.profile && !p.l1_blocks && !p.hub_split &&
            !p.defer_heavy && !p.strict_window && p.l1_donate == 0 && p.bucket_capacity == 0;
 }
 
@@ -874,7 +877,9 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
     L.count = c->pp_count;
     L.work = reinterpret_cast<uint64_t *>(c->pp_count + kCountWords);
     L.n = (uint32_t)n;
-    L.bound = c->pp_bound;
+    L.bound = c->pp_count + mlmq::kMaxRounds + 1;
+    L.reach = c->pp_reach;
+    L.hub_degree = c->pp_hub;
     const double timeout_ms = (p.timeout_s > 0 ? p.timeout_s : 60.0) * 1e3;
     QueryClock t;
     t.q0 = clk::now();
@@ -885,7 +890,7 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
     for (; round < mlmq::kBoundedRounds; ++round) HIP_TRY(c, mlmq::launch_push(L, round, true, c->stream));
     HIP_TRY(c, mlmq::launch_pull(L, round, c->stream));
     const uint32_t *h = c->h_ctl;
-    for (uint32_t more = mlmq::kFullRounds;; more = 8) {
+    for (uint32_t more = mlmq::kFullRounds;; more = 4) {
         for (uint32_t k = 0; k < more; ++k, ++round) HIP_TRY(c, mlmq::launch_push(L, round, false, c->stream));
         HIP_TRY(c, hipEventRecord(c->ev_stop, c->stream));
         HIP_TRY(c, hipMemcpyAsync(c->h_ctl, c->pp_count, sizeof(uint32_t) * (kCountWords + 4), hipMemcpyDeviceToHost,
@@ -894,7 +899,7 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
         t.s1 = clk::now();
         if (ms_since(t.q0, t.s1) > timeout_ms) return fail(c, MLMQ_E_TIMEOUT, "watchdog expired");
         if (h[round] == 0) break;
-        if (round + 8 > mlmq::kMaxRounds)
+        if (round + 4 > mlmq::kMaxRounds)
             return fail(c, MLMQ_E_QUEUE_OVERFLOW, "push-pull solver: too many rounds");
     }
     float reset_ms = 0;

@@ -5,19 +5,22 @@
 // distance of 10-100, so a hub's edges of weight 100-1000 only matter to the
 // few vertices that have no lighter way in.  The vertex queue still relaxes
 // each of the 128 M edges once.  Here
-//   1. rounds of pushes lower vertices up to a bound B only: a vertex at
+//   1. rounds of pushes settle vertices up to a bound B only: a vertex at
 //      distance d reads its edges of weight <= B - d, a prefix of its sorted
-//      adjacency whose length comes from its hop block;
+//      adjacency whose length comes from its hop block.  B is the distance of
+//      the nearest hub pushed so far plus the graph's `reach` (until a hub is
+//      met there is no bound: a source at the rim first finds its way in);
 //   2. one pull: every vertex beyond B looks at its own few edges, lightest
 //      first, until the weight alone exceeds the best sum;
-//   3. rounds of full pushes from the pulled vertices, and from what phase 1
+//   3. rounds of full pushes from the vertices beyond B, and from what phase 1
 //      may have left, finish the rest.
-// Edges examined on RMAT-22: about 25 % of the graph (B = the 5 % quantile of
-// the weights), against 105 % before.  Any B gives the same distances: a
-// vertex's last improvement is always followed by a push of all its edges,
-// or found by the pull of the edge's other end.  The graph must be undirected
-// (checked edge by edge when it is loaded): the pull reads out-edges as
-// in-edges.
+// Edges examined on RMAT-22: about 25 % of the graph (reach = the 5 % quantile
+// of the weights), against 105 % before.  Any B gives the same distances, also
+// one that falls while phase 1 runs: a vertex lowered to at most B is pushed
+// to everything it can bring to at most B, what it could bring further is
+// pulled from the other end, and a vertex beyond B is pushed in phase 3.  The
+// graph must be undirected (checked edge by edge when it is loaded): the pull
+// reads out-edges as in-edges.
 //
 // Every round is one launch, and no workgroup waits for another.  A round that
 // finds nothing costs its launch.
@@ -75,6 +78,7 @@ __global__ __launch_bounds__(kGroup) void push_kernel(PushPullLaunch L, uint32_t
     __shared__ uint32_t s_work[2];
     const uint32_t count = L.count[round];
     if (count == 0) return;
+    const uint32_t bound = kBounded ? *L.bound : kUnreached - 1u;
     const uint32_t *in = L.front[round & 1u];
     uint32_t *out = L.front[(round + 1u) & 1u], *out_count = L.count + round + 1;
     const uint32_t share = min(kGroup, (count + gridDim.x - 1) / gridDim.x);
@@ -92,8 +96,9 @@ __global__ __launch_bounds__(kGroup) void push_kernel(PushPullLaunch L, uint32_t
             const uint4 *p = L.blocks + 4ull * v;
             const uint4 q0 = p[0], q1 = p[1], q2 = p[2], q3 = p[3];
             d = L.dist[v];
-            const uint32_t limit = kBounded ? L.bound : kUnreached - 1u;
-            if (q0.x <= kInlineEdges) {
+            if (d > bound) {
+                // beyond the bound by now: phase 3 pushes it
+            } else if (q0.x <= kInlineEdges) {
                 const uint32_t word[14] = {q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x,
                                            q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
                 uint32_t was[kInlineEdges];
@@ -103,7 +108,7 @@ __global__ __launch_bounds__(kGroup) void push_kernel(PushPullLaunch L, uint32_t
 #pragma unroll
                 for (uint32_t k = 0; k < kInlineEdges; ++k) {
                     const uint32_t nd = d + word[2 * k + 1];
-                    if (nd < was[k] && nd <= limit)
+                    if (nd < was[k] && nd <= bound)
                         improved += lower(L, B, out, out_count, round, word[2 * k] & L.id_mask, nd) ? 1u : 0u;
                 }
                 edges += q0.x;
@@ -111,10 +116,15 @@ __global__ __launch_bounds__(kGroup) void push_kernel(PushPullLaunch L, uint32_t
                 start = q0.y;
                 len = q0.x;
                 if (kBounded) {
-                    // the least step that covers every weight up to bound - d
-                    const uint32_t room = L.bound - min(d, L.bound);
-                    const uint32_t step = L.bound / kBoundSteps + 1u;
-                    const uint32_t j = min(room / step, kBoundSteps - 1u);
+                    uint32_t limit = bound;
+                    if (q0.x >= L.hub_degree && d + L.reach < limit) {
+                        limit = d + L.reach;
+                        (void)fetch_min(L.bound, limit);
+                    }
+                    // the least step that covers every weight up to limit - d
+                    const uint32_t room = limit - d;
+                    const uint32_t step = L.reach / kBoundSteps + 1u;
+                    const uint32_t j = room / step;
                     const uint32_t word[8] = {q2.x, q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
 #pragma unroll
                     for (uint32_t k = 0; k < kBoundSteps; ++k)
@@ -157,7 +167,7 @@ __global__ __launch_bounds__(kGroup) void push_kernel(PushPullLaunch L, uint32_t
             for (uint32_t j = 0; j < kUnroll; ++j) was[j] = L.dist[c[j]];
 #pragma unroll
             for (uint32_t j = 0; j < kUnroll; ++j)
-                if (nd[j] < was[j] && (!kBounded || nd[j] <= L.bound))
+                if (nd[j] < was[j] && nd[j] <= bound)
                     improved += lower(L, B, out, out_count, round, c[j], nd[j]) ? 1u : 0u;
         }
     }
@@ -183,11 +193,12 @@ __global__ __launch_bounds__(kGroup) void pull_kernel(PushPullLaunch L, uint32_t
     }
     __syncthreads();
     uint32_t edges = 0, improved = 0;
+    const uint32_t bound = *L.bound;
     for (uint32_t base = blockIdx.x * kGroup; base < L.n; base += gridDim.x * kGroup) {
         const uint32_t v = base + threadIdx.x;
         const uint32_t d = v < L.n ? L.dist[v] : 0u;
         uint32_t best = d, deg = 0, start = 0;
-        if (d > L.bound) {
+        if (d > bound) {
             const uint4 *p = L.blocks + 4ull * v;
             const uint4 q0 = p[0];
             if (q0.x > kInlineEdges) {
@@ -225,12 +236,14 @@ __global__ __launch_bounds__(kGroup) void pull_kernel(PushPullLaunch L, uint32_t
             }
             if (lane_id() == l) best = b;
         }
-        if (best < d) {
-            // (only this thread lowers v in this launch, and no vertex beyond
-            // the bound is in the list yet; the mark belongs to the pushes)
-            L.dist[v] = best;
-            ++improved;
-            queue_vertex(B, out, out_count, v);
+        if (v < L.n && d > bound && best < kUnreached) {
+            // (only this thread lowers v in this launch)
+            if (best < d) {
+                L.dist[v] = best;
+                ++improved;
+            }
+            // phase 1 may have left it in the list
+            if (L.mark[v] != round) queue_vertex(B, out, out_count, v);
         }
     }
     flush_buffer(B, out, out_count);
@@ -254,6 +267,7 @@ __global__ __launch_bounds__(256) void pushpull_reset_kernel(PushPullLaunch L, u
     if (t == 0) {
         L.front[0][0] = src;
         L.work[0] = L.work[1] = 0;
+        *L.bound = kUnreached - 1u;
     }
 }
 
@@ -285,15 +299,15 @@ __global__ __launch_bounds__(256) void symmetry_kernel(const uint32_t *row, cons
 }
 
 __global__ __launch_bounds__(256) void bound_count_kernel(const uint32_t *row, const uint32_t *wgt, uint32_t n,
-                                                          uint32_t bound, uint4 *blocks) {
+                                                          uint32_t reach, uint4 *blocks) {
     const uint32_t stride = gridDim.x * blockDim.x;
-    const uint32_t step = bound / kBoundSteps + 1u;
+    const uint32_t step = reach / kBoundSteps + 1u;
     for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride) {
         const uint32_t s = row[v], e = row[v + 1];
         if (e - s <= kInlineEdges) continue;
         uint32_t at = s;
         for (uint32_t j = 0; j < kBoundSteps; ++j) {
-            // edges of weight < step * (j + 1); the last step covers the bound
+            // edges of weight < step * (j + 1); the last step covers the reach
             const uint32_t top = step * (j + 1);
             uint32_t lo = at, hi = e;
             while (lo < hi) {
@@ -321,9 +335,9 @@ hipError_t launch_symmetry_check(const uint32_t *row, const uint32_t *col, const
     return hipGetLastError();
 }
 
-hipError_t launch_bound_counts(const uint32_t *row, const uint32_t *wgt, uint32_t n, uint32_t bound, uint4 *blocks,
+hipError_t launch_bound_counts(const uint32_t *row, const uint32_t *wgt, uint32_t n, uint32_t reach, uint4 *blocks,
                                hipStream_t s) {
-    hipLaunchKernelGGL(bound_count_kernel, dim3(groups_for(n, 16384)), dim3(256), 0, s, row, wgt, n, bound, blocks);
+    hipLaunchKernelGGL(bound_count_kernel, dim3(groups_for(n, 16384)), dim3(256), 0, s, row, wgt, n, reach, blocks);
     return hipGetLastError();
 }
 

@@ -7,8 +7,8 @@
 
 namespace mlmq {
 
-// Per graph: the push bound, and words 8..15 of every hop block with more than
-// kInlineEdges edges = its edges of weight <= bound * (j + 1) / 8, j = 0..7.
+// Per graph: the reach of phase 1, and words 8..15 of every hop block with more
+// than kInlineEdges edges = its edges of weight < (reach / 8 + 1) * (j + 1).
 constexpr uint32_t kBoundSteps = 8;
 // Rounds of pushes up to the bound before the pull, and of full pushes after
 // it, that are launched before the host looks.
@@ -26,15 +26,17 @@ struct PushPullLaunch {
     uint32_t *front[2];      // n each: the rounds' vertices, by parity
     uint32_t *count;         // kMaxRounds + 1: vertices of each round
     uint64_t *work;          // edges examined, improvements
+    uint32_t *bound;         // distance up to which phase 1 settles
     uint32_t n;
-    uint32_t bound;
+    uint32_t reach;          // the bound lies this far beyond the nearest hub
+    uint32_t hub_degree;
 };
 
 // *asymmetric = 1 if some edge (u, v, w) has no edge (v, u, w).  Rows of more
 // than kInlineEdges edges are sorted by (weight, destination).
 hipError_t launch_symmetry_check(const uint32_t *row, const uint32_t *col, const uint32_t *wgt, uint32_t n,
                                  uint32_t *asymmetric, hipStream_t s);
-hipError_t launch_bound_counts(const uint32_t *row, const uint32_t *wgt, uint32_t n, uint32_t bound, uint4 *blocks,
+hipError_t launch_bound_counts(const uint32_t *row, const uint32_t *wgt, uint32_t n, uint32_t reach, uint4 *blocks,
                                hipStream_t s);
 hipError_t launch_pushpull_reset(const PushPullLaunch &L, uint32_t src, hipStream_t s);
 // Workgroups of a push launch, and waves of each.
