@@ -555,6 +555,9 @@ int mlmq::ctx_graph_view(const mlmq_ctx *c, DeviceGraphView *v) {
     v->device = c->device;
     v->cus = c->cus;
     v->wall_khz = c->wall_khz;
+    v->regions = c->regions;
+    v->pp_reach = c->pp_reach;
+    v->pp_hub = c->pp_hub;
     return MLMQ_OK;
 }
 
@@ -812,6 +815,8 @@ int run_regions(mlmq_ctx *c, uint32_t nq, int32_t src, const uint32_t *sources, 
     L.qtime = qtime;
     L.timeout_ticks = (uint64_t)((p.timeout_s > 0 ? p.timeout_s : 60.0) * (double)c->wall_khz * 1000.0);
     L.nq = nq;
+    L.tasks = nq * g.regions;
+    L.longest = std::max(g.n, g.inbox_slots);
     L.grid = grid;
     t->q0 = clk::now();
     HIP_TRY(c, hipEventRecord(c->ev_reset, c->stream));
@@ -865,7 +870,11 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
     constexpr size_t kCountWords = mlmq::kMaxRounds + 2;   // 8-byte aligned end, then the work counters
     static_assert(kCountWords % 2 == 0 && kCountWords + 4 <= mlmq::kCtlWords, "copied through the control block's buffer");
     if (!c->pp_count) HIP_TRY(c, hipMalloc(&c->pp_count, sizeof(uint32_t) * (kCountWords + 4)));
-    mlmq::PushPullLaunch L{};
+    mlmq::PushPullQueries Q{};
+    Q.nq = 1;
+    Q.max_n = (uint32_t)n;
+    mlmq::PushPullLaunch &L = Q.one;
+    L.src = (uint32_t)src;
     L.col = c->col;
     L.wgt = c->wgt;
     L.blocks = c->blocks;
@@ -884,14 +893,14 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
     QueryClock t;
     t.q0 = clk::now();
     HIP_TRY(c, hipEventRecord(c->ev_reset, c->stream));
-    HIP_TRY(c, mlmq::launch_pushpull_reset(L, (uint32_t)src, c->stream));
+    HIP_TRY(c, mlmq::launch_pushpull_reset(Q, c->stream));
     HIP_TRY(c, hipEventRecord(c->ev_start, c->stream));
     uint32_t round = 0;
-    for (; round < mlmq::kBoundedRounds; ++round) HIP_TRY(c, mlmq::launch_push(L, round, true, c->stream));
-    HIP_TRY(c, mlmq::launch_pull(L, round, c->stream));
+    for (; round < mlmq::kBoundedRounds; ++round) HIP_TRY(c, mlmq::launch_push(Q, round, true, c->stream));
+    HIP_TRY(c, mlmq::launch_pull(Q, round, c->stream));
     const uint32_t *h = c->h_ctl;
     for (uint32_t more = mlmq::kFullRounds;; more = 4) {
-        for (uint32_t k = 0; k < more; ++k, ++round) HIP_TRY(c, mlmq::launch_push(L, round, false, c->stream));
+        for (uint32_t k = 0; k < more; ++k, ++round) HIP_TRY(c, mlmq::launch_push(Q, round, false, c->stream));
         HIP_TRY(c, hipEventRecord(c->ev_stop, c->stream));
         HIP_TRY(c, hipMemcpyAsync(c->h_ctl, c->pp_count, sizeof(uint32_t) * (kCountWords + 4), hipMemcpyDeviceToHost,
                                   c->stream));

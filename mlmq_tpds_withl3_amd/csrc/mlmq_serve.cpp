@@ -19,6 +19,8 @@
 
 #include "arena.h"
 #include "device_common.h"
+#include "hop_block.h"
+#include "pushpull_solver.h"
 #include "solver_internal.h"
 
 namespace {
@@ -50,6 +52,16 @@ struct GraphEntry {
     std::unordered_map<int32_t, uint32_t *> expected;
 };
 
+// Solver of a request in a launch lane.
+enum class Engine : uint8_t { kQueue, kRegions, kPushPull };
+
+// Most ring slots of a lane's region solver (8 MiB); requests that would need
+// more of them in one launch go to the vertex queue.
+constexpr uint64_t kLaneRing = 1u << 20;
+// Full rounds of the push-pull solver in a lane, which nobody watches: most
+// graphs need 5 to 9, an empty round costs about 2 us.
+constexpr uint32_t kLaneRounds = 16;
+
 struct Lane {
     hipStream_t s = nullptr;
     hipEvent_t ev_solve = nullptr, ev_done = nullptr;
@@ -60,7 +72,19 @@ struct Lane {
     std::vector<int32_t> ids;
     std::vector<Slot> slots;
     std::vector<uint32_t> caps;   // ring capacity (log2) each request ran with
+    std::vector<Engine> engines;
+    // of the region and push-pull solvers: their query tables and the outcomes
+    // (h_tab: pinned), control block and query times, ring
+    uint8_t *h_tab = nullptr, *d_tab = nullptr;
+    uint32_t *ctl = nullptr;
+    uint64_t *times = nullptr;
+    uint64_t *ring = nullptr;
+    uint64_t ring_slots = 0;
+    bool ring_dirty = true;
 };
+
+constexpr size_t kTabBytes = sizeof(mlmq::RegionQuery) + sizeof(mlmq::PushPullLaunch) + sizeof(mlmq::ServeOutcome);
+static_assert(sizeof(mlmq::RegionQuery) % 8 == 0 && sizeof(mlmq::PushPullLaunch) % 8 == 0, "packed one after another");
 
 // ---- live serving state ----
 constexpr uint32_t kLiveEntries = 4096;     // request table entries
@@ -315,6 +339,63 @@ int add_graph_ctx(mlmq_server *s, mlmq_ctx *ctx, const mlmq_serve_graph_params *
     s->graphs.push_back(std::move(g));
     if (graph_id) *graph_id = (int32_t)s->graphs.size() - 1;
     return MLMQ_OK;
+}
+
+// Which solver serves a request of g whose slot is `slot_bytes` long: as for
+// single queries, and the solver's state must fit the queue partition of the
+// slot, which it takes the place of.  A burst of 17 road-264k, 8 road-1M and 7
+// RMAT-18 requests in one launch: device 43 ms all by the vertex queue, 7.2 ms
+// this way (of it 0.7 ms push-pull, all of a launch's queries in the same
+// rounds, and 6.4 ms regions, all of its queries in the same ring).
+Engine engine_of(const GraphEntry &g, uint64_t slot_bytes) {
+    if (g.p.hub_split || g.p.bucket_capacity) return Engine::kQueue;
+    const uint64_t room = slot_bytes - g.row_bytes - g.ctl_bytes;
+    if (g.v.regions.regions) {
+        const uint64_t words = (uint64_t)g.v.regions.inbox_slots + 1 + g.v.regions.regions;
+        return !g.p.light_split && sizeof(uint32_t) * words <= room ? Engine::kRegions : Engine::kQueue;
+    }
+    const uint64_t words = 3ull * (uint64_t)g.v.n + mlmq::kMaxRounds + 2 + 4;
+    return g.v.pp_reach && sizeof(uint32_t) * words <= room ? Engine::kPushPull : Engine::kQueue;
+}
+
+// A push-pull query whose state lies in `part`.
+mlmq::PushPullLaunch pushpull_query(const GraphEntry &g, uint32_t src, uint32_t *dist, uint8_t *part, uint64_t *time) {
+    constexpr uint32_t kCountWords = mlmq::kMaxRounds + 2;
+    static_assert(kCountWords % 2 == 0, "the work counters behind the counts are 64-bit");
+    mlmq::PushPullLaunch L{};
+    L.col = g.v.col;
+    L.wgt = g.v.wgt;
+    L.blocks = g.v.blocks;
+    L.id_mask = g.v.packed ? (1u << mlmq::kBackShift) - 1u : 0xFFFFFFFFu;
+    L.n = (uint32_t)g.v.n;
+    L.dist = dist;
+    L.count = (uint32_t *)part;
+    L.bound = L.count + mlmq::kMaxRounds + 1;
+    L.work = (uint64_t *)(L.count + kCountWords);
+    L.mark = L.count + kCountWords + 4;
+    L.front[0] = L.mark + L.n;
+    L.front[1] = L.front[0] + L.n;
+    L.reach = g.v.pp_reach;
+    L.hub_degree = g.v.pp_hub;
+    L.src = src;
+    L.time = time;
+    return L;
+}
+
+// A clean ring of at least `tasks` + `grid` records, twice over.
+hipError_t lane_ring(Lane &l, uint64_t tasks, uint32_t grid) {
+    uint64_t need = 1024;
+    while (need < 2 * (tasks + grid)) need *= 2;
+    if (l.ring_slots < need) {
+        if (l.ring) (void)hipFree(l.ring);
+        l.ring = nullptr;
+        l.ring_slots = 0;
+        l.ring_dirty = true;
+        const hipError_t e = hipMalloc((void **)&l.ring, sizeof(uint64_t) * need);
+        if (e != hipSuccess) return e;
+        l.ring_slots = need;
+    }
+    return l.ring_dirty ? mlmq::launch_fill_u64(l.ring, l.ring_slots, mlmq::kEmpty, l.s) : hipSuccess;
 }
 
 double live_now(const Live &L) {
@@ -852,6 +933,11 @@ int mlmq_server_create(int device, const mlmq_server_config *cfg, mlmq_server **
         const size_t tb = mlmq::serve_request_bytes() * (size_t)c.max_batch;
         if (e == hipSuccess) e = hipHostMalloc((void **)&l.h_reqs, tb, hipHostMallocDefault);
         if (e == hipSuccess) e = hipMalloc((void **)&l.d_reqs, tb);
+        const size_t side = kTabBytes * (size_t)c.max_batch;
+        if (e == hipSuccess) e = hipHostMalloc((void **)&l.h_tab, side, hipHostMallocDefault);
+        if (e == hipSuccess) e = hipMalloc((void **)&l.d_tab, side);
+        if (e == hipSuccess) e = hipMalloc((void **)&l.ctl, sizeof(uint32_t) * mlmq::kCtlWords);
+        if (e == hipSuccess) e = hipMalloc((void **)&l.times, 2 * sizeof(uint64_t) * (size_t)c.max_batch);
     }
     if (e != hipSuccess) {
         const int rc = e == hipErrorOutOfMemory ? MLMQ_E_NOMEM : MLMQ_E_HIP;
@@ -876,7 +962,9 @@ int mlmq_server_destroy(mlmq_server *s) {
         if (l.ev_solve) (void)hipEventDestroy(l.ev_solve);
         if (l.ev_done) (void)hipEventDestroy(l.ev_done);
         if (l.h_reqs) (void)hipHostFree(l.h_reqs);
-        if (l.d_reqs) (void)hipFree(l.d_reqs);
+        if (l.h_tab) (void)hipHostFree(l.h_tab);
+        for (void *p : {(void *)l.d_reqs, (void *)l.d_tab, (void *)l.ctl, (void *)l.times, (void *)l.ring})
+            if (p) (void)hipFree(p);
         if (l.s) (void)hipStreamDestroy(l.s);
     }
     for (GraphEntry &g : s->graphs) {
@@ -1014,6 +1102,7 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
 
     const uint64_t timeout_ticks = (uint64_t)(s->cfg.timeout_s * (double)s->wall_khz * 1000.0);
     std::vector<int32_t> retries(nreq, 0);
+    std::vector<char> queue_only(nreq, 0);   // another solver has given the request up
     int32_t next = 0, finished = 0, launches = 0, pending = 0;
     uint64_t inflight = 0, peak_inflight = 0, batch_sum = 0;
     const uint64_t peak_before = s->arena.used;
@@ -1021,6 +1110,9 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
     double wall_ms = 0.0;
     int rc = MLMQ_OK;
     const size_t rb = mlmq::serve_request_bytes();
+    int occ = 0;
+    HIP_TRY(s, mlmq::region_occupancy(&occ));
+    const uint32_t region_groups = (uint32_t)(std::max(occ, 1) * s->cus);
 
     HIP_TRY(s, hipEventRecord(s->ev_ref, s->lanes[0].s));
     HIP_TRY(s, hipEventSynchronize(s->ev_ref));
@@ -1064,23 +1156,56 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
             return 1;
         }
         const uint32_t nb = (uint32_t)l.ids.size();
-        // Few requests in the launch: spread each over more waves, up to
-        // spread_waves for the whole launch, as one-wave workgroups (they go
-        // to distinct CUs, as in the single-query solver).
+        // The solver of each request.
+        uint64_t tasks = 0;
+        uint32_t nqueue = 0, nregion = 0, npush = 0;
+        l.engines.resize(nb);
+        for (uint32_t i = 0; i < nb; ++i) {
+            const GraphEntry &g = s->graphs[reqs[l.ids[i]].graph];
+            Engine &e = l.engines[i];
+            e = queue_only[l.ids[i]] ? Engine::kQueue : engine_of(g, l.slots[i].bytes);
+            if (e == Engine::kRegions) {
+                const uint64_t more = tasks + g.v.regions.regions;
+                if (2 * (more + region_groups) > kLaneRing) e = Engine::kQueue;
+                else tasks = more;
+            }
+            nregion += e == Engine::kRegions;
+            npush += e == Engine::kPushPull;
+            nqueue += e == Engine::kQueue;
+        }
+        const uint32_t region_grid = (uint32_t)std::min<uint64_t>(region_groups, tasks);
+        if (nregion && lane_ring(l, tasks, region_grid) != hipSuccess) {
+            (void)hipGetLastError();
+            for (Engine &e : l.engines)
+                if (e == Engine::kRegions) e = Engine::kQueue;
+            nqueue += nregion;
+            nregion = 0;
+        }
+        // Few requests for the vertex queue: spread each over more waves, up
+        // to spread_waves for the whole launch, as one-wave workgroups (they
+        // go to distinct CUs, as in the single-query solver).
         uint32_t widest = 0;
         for (int32_t id : l.ids) {
             const GraphEntry &g = s->graphs[reqs[id].graph];
             widest = std::max(widest, (uint32_t)g.p.workgroups * (uint32_t)width);
         }
         uint32_t fill = 0;
-        if (s->cfg.spread_waves > 0) {
-            fill = std::min<uint32_t>((uint32_t)s->cfg.spread_waves / nb, kMaxSpread);
+        if (s->cfg.spread_waves > 0 && nqueue > 0) {
+            fill = std::min<uint32_t>((uint32_t)s->cfg.spread_waves / nqueue, kMaxSpread);
             if (fill <= widest) fill = 0;
         }
         mlmq::ServeLaunch S{};
         S.reqs = l.d_reqs;
         S.nreq = nb;
         S.waves = fill ? 1 : width;
+        mlmq::RegionLaunch R{};
+        mlmq::PushPullQueries P{};
+        const mlmq::RegionGraph *region_graph = nullptr;
+        auto *h_region = (mlmq::RegionQuery *)l.h_tab;
+        auto *h_push = (mlmq::PushPullLaunch *)(h_region + nregion);
+        auto *h_out = (mlmq::ServeOutcome *)(h_push + npush);
+        auto *d_push = (mlmq::PushPullLaunch *)(l.d_tab + ((uint8_t *)h_push - l.h_tab));
+        auto *d_out = (mlmq::ServeOutcome *)(l.d_tab + ((uint8_t *)h_out - l.h_tab));
         bool any_expect = false;
         uint32_t wg_first = 0;
         for (uint32_t i = 0; i < nb; ++i) {
@@ -1092,24 +1217,72 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
             L.cap_log2 = l.caps[i];
             L.dist = (uint32_t *)b;
             L.ctl = (uint32_t *)(b + g.row_bytes);
-            L.slots = (uint64_t *)(b + g.row_bytes + g.ctl_bytes);
+            uint8_t *part = b + g.row_bytes + g.ctl_bytes;
+            L.slots = (uint64_t *)part;
             const uint32_t *expect = nullptr;
             if (s->cfg.verify) {
                 auto it = g.expected.find(reqs[id].src);
                 if (it != g.expected.end()) expect = it->second;
             }
             any_expect |= expect != nullptr;
-            const uint32_t wg = fill ? fill : (uint32_t)g.p.workgroups;
+            S.max_n = std::max(S.max_n, L.n);
+            h_out[i] = mlmq::ServeOutcome{};
+            uint32_t wg = 0;
+            if (l.engines[i] == Engine::kQueue) {
+                wg = fill ? fill : (uint32_t)g.p.workgroups;
+                S.max_part_slots = std::max(S.max_part_slots, (uint64_t)L.nbuckets << L.cap_log2);
+                S.ext = S.ext || L.light_split || L.defer_heavy || L.strict_window;
+            } else if (l.engines[i] == Engine::kRegions) {
+                region_graph = &g.v.regions;
+                uint32_t *inbox = (uint32_t *)part;
+                h_region[R.nq] = mlmq::region_query(*region_graph, L.dist, inbox, inbox + region_graph->inbox_slots + 1,
+                                                    (uint32_t)reqs[id].src);
+                h_out[i] = {l.ctl, nullptr, l.times + 2 * R.nq};
+                R.longest = std::max({R.longest, region_graph->n, region_graph->inbox_slots});
+                ++R.nq;
+            } else {
+                uint64_t *time = l.times + 2 * (nregion + P.nq);
+                const mlmq::PushPullLaunch q = pushpull_query(g, (uint32_t)reqs[id].src, L.dist, part, time);
+                h_push[P.nq++] = q;
+                h_out[i] = {nullptr, q.count + mlmq::kBoundedRounds + kLaneRounds, time};
+                P.max_n = std::max(P.max_n, L.n);
+            }
             mlmq::serve_request_write(l.h_reqs, i, L, (uint32_t)reqs[id].src, sl.fresh, expect, wg_first, wg);
             wg_first += wg;
-            S.max_n = std::max(S.max_n, L.n);
-            S.max_part_slots = std::max(S.max_part_slots, (uint64_t)L.nbuckets << L.cap_log2);
-            S.ext = S.ext || L.light_split || L.defer_heavy || L.strict_window;
         }
         S.grid = wg_first;
         const size_t tb = rb * nb;
         HIP_TRY(s, hipMemcpyAsync(l.d_reqs, l.h_reqs, tb, hipMemcpyHostToDevice, l.s));
+        if (nregion + npush) {
+            const size_t used = (size_t)((uint8_t *)(h_out + nb) - l.h_tab);
+            HIP_TRY(s, hipMemcpyAsync(l.d_tab, l.h_tab, used, hipMemcpyHostToDevice, l.s));
+        }
         HIP_TRY(s, mlmq::launch_serve(S, l.s));
+        if (npush) {
+            P.table = d_push;
+            HIP_TRY(s, mlmq::launch_pushpull_reset(P, l.s));
+            uint32_t round = 0;
+            for (; round < mlmq::kBoundedRounds; ++round) HIP_TRY(s, mlmq::launch_push(P, round, true, l.s));
+            HIP_TRY(s, mlmq::launch_pull(P, round, l.s));
+            for (uint32_t k = 0; k < kLaneRounds; ++k, ++round) HIP_TRY(s, mlmq::launch_push(P, round, false, l.s));
+        }
+        if (nregion) {
+            R.tasks = (uint32_t)tasks;
+            R.grid = region_grid;
+            R.ring = l.ring;
+            R.ring_mask = (uint32_t)(l.ring_slots - 1);
+            R.ctl = l.ctl;
+            R.qtime = l.times;
+            R.timeout_ticks = timeout_ticks;
+            R.shared = inflight > 0;
+            // (a lone query starts a workgroup on each region)
+            if (nregion > 1) R.table = (const mlmq::RegionQuery *)l.d_tab;
+            else R.space = {h_region[0].dist, h_region[0].inbox, h_region[0].act, 0, 0, 0};
+            l.ring_dirty = true;   // until the solve has left it clean
+            HIP_TRY(s, mlmq::launch_region_reset(*region_graph, R, nullptr, h_region[0].src, l.s));
+            HIP_TRY(s, mlmq::launch_region_solver(*region_graph, R, l.s));
+        }
+        if (nregion + npush) HIP_TRY(s, mlmq::launch_serve_outcome(S, d_out, l.s));
         HIP_TRY(s, hipEventRecord(l.ev_solve, l.s));
         if (any_expect) HIP_TRY(s, mlmq::launch_serve_verify(S, l.s));
         HIP_TRY(s, hipMemcpyAsync(l.h_reqs, l.d_reqs, tb, hipMemcpyDeviceToHost, l.s));
@@ -1132,6 +1305,7 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
         float done_ms = 0.0f;
         HIP_TRY(s, hipEventElapsedTime(&done_ms, s->ev_ref, l.ev_solve));
         std::vector<int32_t> rerun;   // overflowed requests, in launch order
+        bool ring_used = false, ring_clean = true;
         for (size_t i = 0; i < l.ids.size(); ++i) {
             const int32_t id = l.ids[i];
             const int32_t gi = reqs[id].graph;
@@ -1142,9 +1316,17 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
             Slot sl = l.slots[i];
             mlmq_serve_result &r = results[id];
             const int st = device_status(status);
-            if (st == MLMQ_E_QUEUE_OVERFLOW && g.cap_log2 < 30) {
-                // Grow the graph's partitions once per launch and run again.
-                if (g.cap_log2 == l.caps[i]) {
+            const bool queue = l.engines[i] == Engine::kQueue;
+            if (l.engines[i] == Engine::kRegions) {
+                ring_used = true;
+                ring_clean &= st == MLMQ_OK;
+            }
+            if (st == MLMQ_E_QUEUE_OVERFLOW && (!queue || g.cap_log2 < 30)) {
+                // Run again: by the vertex queue, or with larger partitions
+                // (the graph's grow once per launch).
+                if (!queue) {
+                    queue_only[id] = 1;
+                } else if (g.cap_log2 == l.caps[i]) {
                     drop_free_slots(s, g);
                     ++g.cap_log2;
                     size_slots(g);
@@ -1166,11 +1348,13 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
                                           sizeof(int32_t) * (size_t)g.v.n, hipMemcpyDeviceToHost, l.s));
                 HIP_TRY(s, hipStreamSynchronize(l.s));
             }
-            // A failed solve leaves records in its partition: refill before reuse.
-            sl.fresh = st != MLMQ_OK;
+            // A failed solve leaves records in its partition, another solver
+            // its own state: refill before reuse.
+            sl.fresh = st != MLMQ_OK || !queue;
             give_back(s, gi, sl);
             ++finished;
         }
+        if (ring_used && ring_clean) l.ring_dirty = false;
         for (auto it = rerun.rbegin(); it != rerun.rend(); ++it) {
             s->pending.push_front(*it);
             ++pending;

@@ -67,20 +67,28 @@ __device__ __forceinline__ bool lower(const PushPullLaunch &L, OutBuffer &B, uin
     return true;
 }
 
+// This workgroup's query.
+template <bool kTable>
+__device__ __forceinline__ PushPullLaunch query_of(const PushPullLaunch &one, const PushPullLaunch *table) {
+    if constexpr (kTable) return table[blockIdx.y];
+    else return one;
+}
+
 // A workgroup takes its share of the round's vertices, at most one per thread:
 // few vertices of many edges are spread over all workgroups.  Inline vertices
 // are pushed by their thread; the others' edges are numbered through and
 // dealt out to all threads.
-template <bool kBounded>
-__global__ __launch_bounds__(kGroup) void push_kernel(PushPullLaunch L, uint32_t round) {
+template <bool kTable, bool kBounded>
+__global__ __launch_bounds__(kGroup) void push_kernel(PushPullLaunch one, const PushPullLaunch *table, uint32_t round) {
+    const PushPullLaunch L = query_of<kTable>(one, table);
     __shared__ OutBuffer B;
     __shared__ uint32_t s_first[kGroup + 1], s_start[kGroup], s_dist[kGroup], s_wave[kGroup / kWave];
     __shared__ uint32_t s_work[2];
     const uint32_t count = L.count[round];
     if (count == 0) return;
     const uint32_t bound = kBounded ? *L.bound : kUnreached - 1u;
-    const uint32_t *in = L.front[round & 1u];
-    uint32_t *out = L.front[(round + 1u) & 1u], *out_count = L.count + round + 1;
+    const uint32_t *in = (round & 1u ? L.front[1] : L.front[0]);
+    uint32_t *out = (round & 1u ? L.front[0] : L.front[1]), *out_count = L.count + round + 1;
     const uint32_t share = min(kGroup, (count + gridDim.x - 1) / gridDim.x);
     if (threadIdx.x == 0) {
         B.n = 0;
@@ -180,13 +188,17 @@ __global__ __launch_bounds__(kGroup) void push_kernel(PushPullLaunch L, uint32_t
     }
     __syncthreads();
     if (threadIdx.x < 2 && s_work[threadIdx.x]) add64(L.work + threadIdx.x, s_work[threadIdx.x]);
+    // (its last round's other workgroups end at about the same time)
+    if (kTable && blockIdx.x == 0 && threadIdx.x == 0) L.time[1] = wall_clock64();
 }
 
 // Every vertex beyond the bound takes the best distance over its edges.
-__global__ __launch_bounds__(kGroup) void pull_kernel(PushPullLaunch L, uint32_t round) {
+template <bool kTable>
+__global__ __launch_bounds__(kGroup) void pull_kernel(PushPullLaunch one, const PushPullLaunch *table, uint32_t round) {
+    const PushPullLaunch L = query_of<kTable>(one, table);
     __shared__ OutBuffer B;
     __shared__ uint32_t s_work[2];
-    uint32_t *out = L.front[round & 1u], *out_count = L.count + round;
+    uint32_t *out = (round & 1u ? L.front[1] : L.front[0]), *out_count = L.count + round;
     if (threadIdx.x == 0) {
         B.n = 0;
         s_work[0] = s_work[1] = 0;
@@ -257,7 +269,10 @@ __global__ __launch_bounds__(kGroup) void pull_kernel(PushPullLaunch L, uint32_t
     if (threadIdx.x < 2 && s_work[threadIdx.x]) add64(L.work + threadIdx.x, s_work[threadIdx.x]);
 }
 
-__global__ __launch_bounds__(256) void pushpull_reset_kernel(PushPullLaunch L, uint32_t src) {
+template <bool kTable>
+__global__ __launch_bounds__(256) void pushpull_reset_kernel(PushPullLaunch one, const PushPullLaunch *table) {
+    const PushPullLaunch L = query_of<kTable>(one, table);
+    const uint32_t src = L.src;
     const uint32_t stride = gridDim.x * blockDim.x, t = blockIdx.x * blockDim.x + threadIdx.x;
     for (uint32_t i = t; i < L.n; i += stride) {
         L.dist[i] = i == src ? 0u : kUnreached;
@@ -268,6 +283,7 @@ __global__ __launch_bounds__(256) void pushpull_reset_kernel(PushPullLaunch L, u
         L.front[0][0] = src;
         L.work[0] = L.work[1] = 0;
         *L.bound = kUnreached - 1u;
+        if (kTable) L.time[0] = L.time[1] = wall_clock64();
     }
 }
 
@@ -341,8 +357,10 @@ hipError_t launch_bound_counts(const uint32_t *row, const uint32_t *wgt, uint32_
     return hipGetLastError();
 }
 
-hipError_t launch_pushpull_reset(const PushPullLaunch &L, uint32_t src, hipStream_t s) {
-    hipLaunchKernelGGL(pushpull_reset_kernel, dim3(groups_for(L.n, 4096)), dim3(256), 0, s, L, src);
+hipError_t launch_pushpull_reset(const PushPullQueries &Q, hipStream_t s) {
+    const dim3 grid(groups_for(Q.max_n, 4096), Q.nq);
+    if (Q.table) hipLaunchKernelGGL(pushpull_reset_kernel<true>, grid, dim3(256), 0, s, Q.one, Q.table);
+    else hipLaunchKernelGGL(pushpull_reset_kernel<false>, grid, dim3(256), 0, s, Q.one, Q.table);
     return hipGetLastError();
 }
 
@@ -350,15 +368,22 @@ hipError_t launch_pushpull_reset(const PushPullLaunch &L, uint32_t src, hipStrea
 // few vertices never fills them.
 uint32_t push_groups(uint32_t n) { return groups_for((uint64_t)n * 8, 2048); }
 
-hipError_t launch_push(const PushPullLaunch &L, uint32_t round, bool bounded, hipStream_t s) {
-    const dim3 grid(push_groups(L.n)), group(kGroup);
-    if (bounded) hipLaunchKernelGGL(push_kernel<true>, grid, group, 0, s, L, round);
-    else hipLaunchKernelGGL(push_kernel<false>, grid, group, 0, s, L, round);
+hipError_t launch_push(const PushPullQueries &Q, uint32_t round, bool bounded, hipStream_t s) {
+    // several queries share the device, but a round of one may be most of the work
+    const uint32_t share = 2048 / Q.nq > 256 ? 2048 / Q.nq : 256;
+    const uint32_t x = push_groups(Q.max_n);
+    const dim3 grid(x < share ? x : share, Q.nq), group(kGroup);
+    if (Q.table && bounded) hipLaunchKernelGGL((push_kernel<true, true>), grid, group, 0, s, Q.one, Q.table, round);
+    else if (Q.table) hipLaunchKernelGGL((push_kernel<true, false>), grid, group, 0, s, Q.one, Q.table, round);
+    else if (bounded) hipLaunchKernelGGL((push_kernel<false, true>), grid, group, 0, s, Q.one, Q.table, round);
+    else hipLaunchKernelGGL((push_kernel<false, false>), grid, group, 0, s, Q.one, Q.table, round);
     return hipGetLastError();
 }
 
-hipError_t launch_pull(const PushPullLaunch &L, uint32_t round, hipStream_t s) {
-    hipLaunchKernelGGL(pull_kernel, dim3(groups_for(L.n, 4096)), dim3(kGroup), 0, s, L, round);
+hipError_t launch_pull(const PushPullQueries &Q, uint32_t round, hipStream_t s) {
+    const dim3 grid(groups_for(Q.max_n, 4096), Q.nq), group(kGroup);
+    if (Q.table) hipLaunchKernelGGL(pull_kernel<true>, grid, group, 0, s, Q.one, Q.table, round);
+    else hipLaunchKernelGGL(pull_kernel<false>, grid, group, 0, s, Q.one, Q.table, round);
     return hipGetLastError();
 }
 

@@ -30,6 +30,16 @@ struct PushPullLaunch {
     uint32_t n;
     uint32_t reach;          // the bound lies this far beyond the nearest hub
     uint32_t hub_degree;
+    uint32_t src;
+    uint64_t *time;          // table launches: ticks of the query's start and end
+};
+
+// Queries of one sequence of launches: one, or a table of them.
+struct PushPullQueries {
+    PushPullLaunch one;
+    const PushPullLaunch *table;   // nq entries in device memory (null: `one`)
+    uint32_t nq;
+    uint32_t max_n;                // most vertices of a query
 };
 
 // *asymmetric = 1 if some edge (u, v, w) has no edge (v, u, w).  Rows of more
@@ -38,13 +48,13 @@ hipError_t launch_symmetry_check(const uint32_t *row, const uint32_t *col, const
                                  uint32_t *asymmetric, hipStream_t s);
 hipError_t launch_bound_counts(const uint32_t *row, const uint32_t *wgt, uint32_t n, uint32_t reach, uint4 *blocks,
                                hipStream_t s);
-hipError_t launch_pushpull_reset(const PushPullLaunch &L, uint32_t src, hipStream_t s);
-// Workgroups of a push launch, and waves of each.
+hipError_t launch_pushpull_reset(const PushPullQueries &Q, hipStream_t s);
+// Workgroups of a push launch of one query, and waves of each.
 uint32_t push_groups(uint32_t n);
 constexpr int kPushWaves = 4;
 // Round r expands the vertices of count[r] into those of count[r + 1].
-hipError_t launch_push(const PushPullLaunch &L, uint32_t round, bool bounded, hipStream_t s);
+hipError_t launch_push(const PushPullQueries &Q, uint32_t round, bool bounded, hipStream_t s);
 // Adds the pulled vertices to those of count[round].
-hipError_t launch_pull(const PushPullLaunch &L, uint32_t round, hipStream_t s);
+hipError_t launch_pull(const PushPullQueries &Q, uint32_t round, hipStream_t s);
 
 }  // namespace mlmq

@@ -82,10 +82,12 @@ constexpr uint32_t kThreads = kRegionWaves * kWave;
 constexpr uint32_t kPollerWave = kRelaxers, kSenderWave = kRelaxers + 1;
 
 struct RegionArgs {
-    const RegionHdr *hdr;
+    const RegionHdr *hdr;        // nq queries on one graph ...
     const uint32_t *image;
     const uint32_t *verts;
     RegionQuerySpace space;
+    const RegionQuery *table;    // ... or each on its own
+    uint32_t nq;
     uint64_t *ring;
     uint32_t ring_mask;
     uint32_t *ctl;
@@ -359,6 +361,7 @@ __device__ __forceinline__ void run_sender(const RegionArgs &a, RegionLds &S, co
 }
 
 // Return a credit; the last one ends the solve.
+template <bool kTable>
 __device__ __forceinline__ void return_credit(const RegionArgs &a, uint32_t query, MessageStats &st) {
     const uint32_t lane = fresh_lane();
     st.credits += lane == 0 ? 1u : 0u;
@@ -376,20 +379,29 @@ __device__ __forceinline__ void return_credit(const RegionArgs &a, uint32_t quer
         uint64_t *slot = a.ring + ((ring_tail + i) & a.ring_mask);
         __hip_atomic_store(slot, kRegionExit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    for (uint32_t i = lane; i < a.tasks; i += kWave) {
-        const uint32_t q = i / a.regions;
-        st_relaxed(a.space.act + q * a.space.act_stride + (i - q * a.regions), kOver);
+    if constexpr (kTable) {
+        for (uint32_t q = 0; q < a.nq; ++q) {
+            uint32_t *act = a.table[q].act;
+            const uint32_t regions = a.table[q].regions;
+            for (uint32_t i = lane; i < regions; i += kWave) st_relaxed(act + i, kOver);
+        }
+    } else {
+        for (uint32_t i = lane; i < a.tasks; i += kWave) {
+            const uint32_t q = i / a.regions;
+            st_relaxed(a.space.act + q * a.space.act_stride + (i - q * a.regions), kOver);
+        }
     }
     wait_memory();
     if (lane == 0) st_relaxed(a.ctl + kExitOff, 1u);
 }
 
 // Serves the adopted region until it is left or the solve is over.
-template <int kG>
+template <bool kTable, int kG>
 __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, const RegionHdr &h,
-                                           const uint32_t *image, uint32_t region, uint32_t query, uint32_t *dist,
-                                           uint32_t *inbox, uint32_t *act, uint32_t seed, uint32_t base, bool idle,
-                                           uint64_t deadline, MessageStats &st) {
+                                           const uint32_t *image, const uint32_t *verts, uint32_t region,
+                                           uint32_t query, uint32_t *dist, uint32_t *inbox, uint32_t *act,
+                                           uint32_t seed, uint32_t base, bool idle, uint64_t deadline,
+                                           MessageStats &st) {
     const uint32_t lane = fresh_lane();
     uint32_t to[kG], seen[kG], val[kG];
 #pragma unroll
@@ -433,7 +445,7 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
                 if (dirty) {
                     for (uint32_t i = lane; i < h.nv; i += kWave) {
                         const uint32_t x = sh_ld(S.dist + local_id(i));
-                        if (x < kUnreached) st_relaxed(dist + a.verts[h.first + i], x);
+                        if (x < kUnreached) st_relaxed(dist + verts[i], x);
                     }
                     dirty = false;
                 }
@@ -486,23 +498,24 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
         for (int g = 0; g < kG; ++g) more = more || val[g] < seen[g];
         if (ballot(more) == 0) {
             idle = true;
-            return_credit(a, query, st);
+            return_credit<kTable>(a, query, st);
             continue;
         }
         uint32_t was = 0;
         if (lane == 0) was = fetch_or(act + region, kWork);
         asm volatile("" : "+v"(was)::"memory");
-        if (read_lane(was, 0) & kWork) return_credit(a, query, st);   // a sender's credit covers the news
+        if (read_lane(was, 0) & kWork) return_credit<kTable>(a, query, st);   // a sender's credit covers the news
         else if (lane == 0) (void)fetch_or(act + region, kCounted);
     }
     // the solve is over
     if (dirty)
         for (uint32_t i = lane; i < h.nv; i += kWave) {
             const uint32_t x = sh_ld(S.dist + local_id(i));
-            if (x < kUnreached) dist[a.verts[h.first + i]] = x;
+            if (x < kUnreached) dist[verts[i]] = x;
         }
 }
 
+template <bool kTable>
 __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a) {
     __shared__ RegionLds S;
     const uint32_t wave = uniform(threadIdx.x / kWave);
@@ -510,7 +523,7 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
     const uint64_t deadline = wall_clock64() + a.timeout_ticks;
     RelaxStats rs{};
     MessageStats ms{};
-    bool first = a.preadopt != 0;
+    bool first = !kTable && a.preadopt != 0;
     for (;;) {
         // adopt: this workgroup's own region first, then the next ticket's record
         if (wave == kPollerWave && lane == 0) {
@@ -542,7 +555,7 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
                 // (its word: kWork, kCounted and perhaps kVisited)
                 const uint32_t q = (uint32_t)(rec >> 32) & (kRegionQueries - 1u);
                 const uint32_t r = (uint32_t)rec & ~(kSeedFlag | kVisitFlag);
-                (void)fetch_or(a.space.act + q * a.space.act_stride + r, kServed);
+                (void)fetch_or((kTable ? a.table[q].act : a.space.act + q * a.space.act_stride) + r, kServed);
             }
             S.own = rec_own ? 1u : 0u;
             S.rec[0] = (uint32_t)rec;
@@ -557,23 +570,26 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
         const uint32_t region = rec_lo & ~(kSeedFlag | kVisitFlag);
         const uint32_t query = rec_hi & ((1u << kQueryBits) - 1u);
         const uint32_t seed = rec_lo & kSeedFlag ? (rec_hi >> kQueryBits) + 1u : 0u;
-        uint32_t *dist = a.space.dist + query * a.space.dist_stride;
-        uint32_t *inbox = a.space.inbox + query * a.space.inbox_stride;
-        uint32_t *act = a.space.act + query * a.space.act_stride;
-        const RegionHdr h = a.hdr[region];
-        const uint32_t *image = a.image + h.image;
+        const RegionQuery *of = kTable ? a.table + query : nullptr;
+        uint32_t *dist = kTable ? of->dist : a.space.dist + query * a.space.dist_stride;
+        uint32_t *inbox = kTable ? of->inbox : a.space.inbox + query * a.space.inbox_stride;
+        uint32_t *act = kTable ? of->act : a.space.act + query * a.space.act_stride;
+        const RegionHdr h = (kTable ? of->hdr : a.hdr)[region];
+        const uint32_t *image = (kTable ? of->image : a.image) + h.image;
+        const uint32_t *verts = (kTable ? of->verts : a.verts) + h.first;
+        const uint32_t width = kTable ? of->width : a.width;
         for (uint32_t i = threadIdx.x; i < kRegionVerts; i += kThreads)
-            S.dist[local_id(i)] = (rec_lo & kVisitFlag) && i < h.nv ? ld_relaxed(dist + a.verts[h.first + i]) : kUnreached;
+            S.dist[local_id(i)] = (rec_lo & kVisitFlag) && i < h.nv ? ld_relaxed(dist + verts[i]) : kUnreached;
         __syncthreads();
         if (wave < kRelaxers) {
-            run_relaxer(S, h, image, wave, a.width, rs);
+            run_relaxer(S, h, image, wave, width, rs);
         } else if (wave == kPollerWave) {
             uint32_t *in = inbox + h.inbox;
             const bool idle = uniform(S.own) != 0;
             const uint32_t held = kServed | (rec_lo & kVisitFlag ? kVisited : 0u);
-            if (h.nin <= 2 * kWave) run_poller<2>(a, S, h, image, region, query, dist, in, act, seed, held, idle, deadline, ms);
-            else if (h.nin <= 4 * kWave) run_poller<4>(a, S, h, image, region, query, dist, in, act, seed, held, idle, deadline, ms);
-            else run_poller<6>(a, S, h, image, region, query, dist, in, act, seed, held, idle, deadline, ms);
+            if (h.nin <= 2 * kWave) run_poller<kTable, 2>(a, S, h, image, verts, region, query, dist, in, act, seed, held, idle, deadline, ms);
+            else if (h.nin <= 4 * kWave) run_poller<kTable, 4>(a, S, h, image, verts, region, query, dist, in, act, seed, held, idle, deadline, ms);
+            else run_poller<kTable, 6>(a, S, h, image, verts, region, query, dist, in, act, seed, held, idle, deadline, ms);
             if (lane == 0) {
                 sh_st(&S.over, 1u);
                 lds_order();
@@ -613,31 +629,44 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
 
 // ---- reset ----
 
-__global__ __launch_bounds__(256) void region_reset_kernel(RegionQuerySpace sp, uint32_t n, uint32_t slots,
-                                                           uint32_t regions, uint32_t nq, const uint32_t *sources,
-                                                           uint32_t src, const uint32_t *where, uint32_t *ctl,
-                                                           uint64_t *ring, uint64_t *qtime) {
+template <bool kTable>
+__global__ __launch_bounds__(256) void region_reset_kernel(RegionArgs a, uint32_t n, uint32_t slots,
+                                                           const uint32_t *sources, uint32_t src,
+                                                           const uint32_t *where) {
     const uint32_t stride = gridDim.x * blockDim.x;
     const uint32_t t0 = blockIdx.x * blockDim.x + threadIdx.x;
-    for (uint32_t q = blockIdx.y; q < nq; q += gridDim.y) {
-        const uint32_t s = sources ? sources[q] : src;
-        uint32_t *dist = sp.dist + q * sp.dist_stride;
-        uint32_t *inbox = sp.inbox + q * sp.inbox_stride;
-        uint32_t *act = sp.act + q * sp.act_stride;
+    for (uint32_t q = blockIdx.y; q < a.nq; q += gridDim.y) {
+        uint32_t s, *dist, *inbox, *act, at, regions = a.regions;
+        if constexpr (kTable) {
+            const RegionQuery &of = a.table[q];
+            s = of.src;
+            dist = of.dist;
+            inbox = of.inbox;
+            act = of.act;
+            at = of.where[s];
+            n = of.n;
+            slots = of.slots;
+            regions = of.regions;
+        } else {
+            s = sources ? sources[q] : src;
+            dist = a.space.dist + q * a.space.dist_stride;
+            inbox = a.space.inbox + q * a.space.inbox_stride;
+            act = a.space.act + q * a.space.act_stride;
+            at = where[s];
+        }
         for (uint32_t i = t0; i < n; i += stride) dist[i] = i == s ? 0u : kUnreached;
         for (uint32_t i = t0; i < slots; i += stride) inbox[i] = kUnreached;
-        const uint32_t at = where[s];
         for (uint32_t i = t0; i < regions; i += stride) act[i] = i == at >> kRegionIdBits ? kWork | kCounted : 0u;
         if (t0 == 0) {
-            ring[q] = (uint64_t)((at & (kRegionVerts - 1u)) << kQueryBits | q) << 32 | kSeedFlag | at >> kRegionIdBits;
-            if (qtime) {
-                qtime[2 * q] = wall_clock64();
-                qtime[2 * q + 1] = 0;
+            a.ring[q] = (uint64_t)((at & (kRegionVerts - 1u)) << kQueryBits | q) << 32 | kSeedFlag | at >> kRegionIdBits;
+            if (a.qtime) {
+                a.qtime[2 * q] = wall_clock64();
+                a.qtime[2 * q + 1] = 0;
             }
         }
     }
     if (blockIdx.y == 0)
-        for (uint32_t i = t0; i < kCtlWords; i += stride) ctl[i] = i == kTailOff || i == kRingTailOff ? nq : 0u;
+        for (uint32_t i = t0; i < kCtlWords; i += stride) a.ctl[i] = i == kTailOff || i == kRingTailOff ? a.nq : 0u;
 }
 
 // ---- building ----
@@ -721,26 +750,34 @@ RegionArgs make_region_args(const RegionGraph &g, const RegionLaunch &L) {
     a.image = g.image;
     a.verts = g.verts;
     a.space = L.space;
+    a.table = L.table;
+    a.nq = L.nq;
     a.ring = L.ring;
     a.ring_mask = L.ring_mask;
     a.ctl = L.ctl;
     a.qtime = L.qtime;
     a.timeout_ticks = L.timeout_ticks;
     a.regions = g.regions;
-    a.tasks = g.regions * L.nq;
+    a.tasks = L.tasks;
     a.width = g.width;
-    a.preadopt = L.grid >= a.tasks ? 1u : 0u;
+    a.preadopt = L.grid >= L.tasks ? 1u : 0u;
     // A region that keeps its workgroup is left only if some other may need
-    // it: after about 2 ms (polls of about 0.7 us).
-    a.linger = a.preadopt ? 3000u : 6u;
+    // it: after about 2 ms (polls of about 0.7 us), or 0.1 ms beside other
+    // launches, whose workgroups may keep some of this one's from starting.
+    a.linger = !a.preadopt ? 6u : L.shared ? 150u : 3000u;
     return a;
 }
 
 }  // namespace
 
+// (both instantiations of the kernel need the same)
 hipError_t region_occupancy(int *blocks_per_cu) {
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        blocks_per_cu, reinterpret_cast<const void *>(&region_solver_kernel), kThreads, 0);
+        blocks_per_cu, reinterpret_cast<const void *>(&region_solver_kernel<true>), kThreads, 0);
+}
+
+RegionQuery region_query(const RegionGraph &g, uint32_t *dist, uint32_t *inbox, uint32_t *act, uint32_t src) {
+    return {g.hdr, g.image, g.verts, g.where, dist, inbox, act, g.n, g.inbox_slots, g.regions, g.width, src};
 }
 
 void region_free(RegionGraph *g) {
@@ -804,19 +841,23 @@ hipError_t region_build(const RegionPlan &plan, uint32_t n, uint64_t m, const ui
 
 hipError_t launch_region_reset(const RegionGraph &g, const RegionLaunch &L, const uint32_t *sources, uint32_t src,
                                hipStream_t s) {
-    uint32_t longest = g.n > g.inbox_slots ? g.n : g.inbox_slots;
-    if (longest < kCtlWords) longest = kCtlWords;
+    const uint32_t longest = L.longest > kCtlWords ? L.longest : kCtlWords;
     uint32_t x = (longest + 1023) / 1024;
     if (x > 2048) x = 2048;
-    const uint32_t y = L.nq < 1024 ? L.nq : 1024;
-    hipLaunchKernelGGL(region_reset_kernel, dim3(x, y), dim3(256), 0, s, L.space, g.n, g.inbox_slots, g.regions, L.nq,
-                       sources, src, g.where, L.ctl, L.ring, L.qtime);
+    const dim3 grid(x, L.nq < 1024 ? L.nq : 1024);
+    const RegionArgs a = make_region_args(g, L);
+    if (L.table)
+        hipLaunchKernelGGL(region_reset_kernel<true>, grid, dim3(256), 0, s, a, 0u, 0u, nullptr, 0u, nullptr);
+    else
+        hipLaunchKernelGGL(region_reset_kernel<false>, grid, dim3(256), 0, s, a, g.n, g.inbox_slots, sources, src,
+                           g.where);
     return hipGetLastError();
 }
 
 hipError_t launch_region_solver(const RegionGraph &g, const RegionLaunch &L, hipStream_t s) {
-    hipLaunchKernelGGL(region_solver_kernel, dim3(L.grid), dim3(kThreads), 0, s,
-                       make_region_args(g, L));
+    const RegionArgs a = make_region_args(g, L);
+    if (L.table) hipLaunchKernelGGL(region_solver_kernel<true>, dim3(L.grid), dim3(kThreads), 0, s, a);
+    else hipLaunchKernelGGL(region_solver_kernel<false>, dim3(L.grid), dim3(kThreads), 0, s, a);
     return hipGetLastError();
 }
 

@@ -34,8 +34,20 @@ struct RegionQuerySpace {        // per-query state; query q at the strides belo
     uint64_t dist_stride, inbox_stride, act_stride;
 };
 
+// A query of a launch over several graphs, each with its own space.
+struct RegionQuery {
+    const RegionHdr *hdr;
+    const uint32_t *image, *verts, *where;
+    uint32_t *dist, *inbox, *act;   // n, inbox_slots, regions words
+    uint32_t n, slots, regions, width, src;
+};
+
 struct RegionLaunch {
-    RegionQuerySpace space;
+    RegionQuerySpace space;      // nq queries on one graph, or
+    const RegionQuery *table;    // nq entries in device memory (null: `space`)
+    uint32_t tasks;              // regions of all queries
+    uint32_t longest;            // most vertices, inbox slots or regions of a query
+    bool shared;                 // other launches may hold part of the device
     uint64_t *ring;
     uint32_t ring_mask;
     uint32_t *ctl;               // control block (device_common.h)
@@ -46,6 +58,7 @@ struct RegionLaunch {
 };
 
 hipError_t region_occupancy(int *blocks_per_cu);
+RegionQuery region_query(const RegionGraph &g, uint32_t *dist, uint32_t *inbox, uint32_t *act, uint32_t src);
 // Builds the device side of a cut (temporary device memory: 4 bytes per edge).
 // Returns hipErrorInvalidValue when some region exceeds the limits.
 hipError_t region_build(const RegionPlan &plan, uint32_t n, uint64_t m, const uint32_t *row, const uint32_t *col,
@@ -53,7 +66,8 @@ hipError_t region_build(const RegionPlan &plan, uint32_t n, uint64_t m, const ui
 void region_free(RegionGraph *g);
 // Per-query reset (distances, inboxes, activity), the control block and the
 // seed records, then the solver.  `sources` is a device array of nq vertices,
-// or null: one query from `src`.
+// or null: one query from `src`.  With a table, the graph and the sources are
+// ignored.
 hipError_t launch_region_reset(const RegionGraph &g, const RegionLaunch &L, const uint32_t *sources, uint32_t src,
                                hipStream_t s);
 hipError_t launch_region_solver(const RegionGraph &g, const RegionLaunch &L, hipStream_t s);

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "region_solver.h"
+
 struct mlmq_ctx;
 
 namespace mlmq {
@@ -23,6 +25,8 @@ struct DeviceGraphView {
     int device;
     int cus;
     int wall_khz;
+    RegionGraph regions;              // the graph's regions (none: not cut)
+    uint32_t pp_reach, pp_hub;        // of the push-pull solver (reach 0: not for it)
 };
 int ctx_graph_view(const mlmq_ctx *c, DeviceGraphView *v);
 // Light-edge counts of the context's hop blocks for `delta` (light/heavy split).
@@ -97,7 +101,7 @@ struct BatchLaunch {
 size_t serve_request_bytes();
 // Request i of a host-side table: L names the graph, the slot (L.dist,
 // L.ctl, L.slots) and the settings; workgroups [wg_first, wg_first +
-// wg_count) of the launch serve it.
+// wg_count) of the launch serve it (none: another solver does).
 void serve_request_write(void *table, uint32_t i, const SolverLaunch &L, uint32_t src, bool fresh,
                          const uint32_t *expect, uint32_t wg_first, uint32_t wg_count);
 void serve_request_read(const void *table, uint32_t i, uint32_t *status, uint32_t *mismatches,
@@ -138,6 +142,14 @@ struct StreamLaunch {
 hipError_t stream_occupancy(int *blocks_per_cu);
 hipError_t launch_stream(const StreamLaunch &S, hipStream_t s);
 hipError_t launch_serve(const ServeLaunch &S, hipStream_t s);
+// Outcome of a request that another solver ran (all null: the vertex queue did).
+struct ServeOutcome {
+    const uint32_t *ctl;      // region solver: control block of its launch
+    const uint32_t *rest;     // push-pull solver: vertices its last round left
+    const uint64_t *time;     // start and end ticks
+};
+// Fills in status and times of those requests.
+hipError_t launch_serve_outcome(const ServeLaunch &S, const ServeOutcome *out, hipStream_t s);
 hipError_t launch_serve_verify(const ServeLaunch &S, hipStream_t s);
 hipError_t batch_occupancy(int waves, int l1_cap, bool ext, bool stats, bool pair, int *blocks_per_cu);
 hipError_t launch_batch_reset(uint32_t *dist_all, uint32_t n, uint32_t nq, const uint32_t *sources,

@@ -881,6 +881,7 @@ struct ServeRequest {
 // grid (x: row chunks, y: requests)
 __global__ __launch_bounds__(256) void serve_reset_kernel(ServeRequest *reqs) {
     const ServeRequest &r = reqs[blockIdx.y];
+    if (r.wg_count == 0) return;
     const uint32_t n = r.a.n;
     const uint64_t part_slots = (uint64_t)r.a.q.nbuckets << r.a.q.cap_log2;
     const uint32_t src = r.src;
@@ -948,6 +949,26 @@ __global__ __launch_bounds__(kWaves * 64) void sssp_serve_kernel(ServeRequest *r
         __hip_atomic_fetch_max(&r->t_end, (uint64_t)wall_clock64(), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
     }
+}
+
+// A region solve is sound when every credit was returned and taken; a
+// push-pull query is done when its last round left nothing.
+__global__ __launch_bounds__(256) void serve_outcome_kernel(ServeRequest *reqs, uint32_t nreq, const ServeOutcome *out) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nreq) return;
+    const ServeOutcome o = out[i];
+    if (!o.time) return;
+    uint32_t e = kErrNone;
+    if (o.rest) {
+        if (*o.rest) e = kErrOverflow;
+    } else {
+        e = o.ctl[kErrOff];
+        const uint32_t tail = o.ctl[kTailOff];
+        if (e == kErrNone && (o.ctl[kExitOff] != 1u || tail != o.ctl[kTakenOff] || tail != o.ctl[kDoneOff])) e = kErrInternal;
+    }
+    reqs[i].status = e;
+    reqs[i].t_start = o.time[0];
+    reqs[i].t_end = o.time[1];
 }
 
 // grid (x: row chunks, y: requests)
@@ -1551,6 +1572,7 @@ hipError_t launch_serve(const ServeLaunch &S, hipStream_t s) {
     const uint64_t longest = S.max_part_slots > S.max_n ? S.max_part_slots : (uint64_t)S.max_n;
     uint32_t chunks = (uint32_t)((longest + 256 * 64 - 1) / (256 * 64));
     if (chunks > 512) chunks = 512;
+    if (S.grid == 0) return hipSuccess;
     hipLaunchKernelGGL(serve_reset_kernel, dim3(chunks, S.nreq), dim3(256), 0, s, reqs);
     const dim3 grid(S.grid);
     const uint32_t nr = S.nreq;
@@ -1570,6 +1592,12 @@ hipError_t launch_serve(const ServeLaunch &S, hipStream_t s) {
         hipLaunchKernelGGL((sssp_serve_kernel<1, true>), grid, dim3(kWave), 0, s, reqs, nr);
     else
         hipLaunchKernelGGL((sssp_serve_kernel<1>), grid, dim3(kWave), 0, s, reqs, nr);
+    return hipGetLastError();
+}
+
+hipError_t launch_serve_outcome(const ServeLaunch &S, const ServeOutcome *out, hipStream_t s) {
+    hipLaunchKernelGGL(serve_outcome_kernel, dim3((S.nreq + 255) / 256), dim3(256), 0, s,
+                       static_cast<ServeRequest *>(S.reqs), S.nreq, out);
     return hipGetLastError();
 }
 
