@@ -22,6 +22,7 @@
 #include "hop_block.h"
 #include "pushpull_solver.h"
 #include "region_solver.h"
+#include "row_copy.h"
 #include "solver_internal.h"
 
 struct mlmq_ctx {
@@ -79,6 +80,7 @@ struct mlmq_ctx {
     uint64_t r_ring_slots = 0;
     bool r_ring_dirty = true;
     uint32_t *h_ctl = nullptr;   // pinned: control block as copied out
+    mlmq::RowStage stage;        // rows on their way to the host
     // push-pull solver: the graph's reach and hub degree (reach 0: not for
     // this graph), and
     // the per-query marks, vertex lists, counters
@@ -362,6 +364,7 @@ int build_blocks(mlmq_ctx *c, const uint32_t *host_col) {
         HIP_TRY(c, mlmq::launch_patch_hubs(c->hubs, c->nhubs, c->blocks, c->stream));
         HIP_TRY(c, hipStreamSynchronize(c->stream));
     }
+    if (c->stage.reserve(sizeof(int32_t) * (size_t)c->n) != hipSuccess) (void)hipGetLastError();
     return build_regions(c, row, host_col);
 }
 
@@ -801,6 +804,14 @@ void fill_timing(mlmq_ctx *c, const uint32_t *h, const QueryClock &t, int blocks
     timing->hub_chunks = st[mlmq::kStatChunks];
 }
 
+// A distance row to host memory.
+int row_to_host(mlmq_ctx *c, int32_t *host_out, const uint32_t *row) {
+    const mlmq::RowCopy r{host_out, row, sizeof(int32_t) * (size_t)c->n};
+    if (c->stage.reserve(r.bytes) != hipSuccess) (void)hipGetLastError();
+    HIP_TRY(c, c->stage.copy(&r, 1, c->stream));
+    return MLMQ_OK;
+}
+
 // nq queries by the region solver: from `src`, or from the device array
 // `sources`; distances into `dist`, one row of n after another.  On success
 // the control block is in ctl_host.
@@ -1078,6 +1089,7 @@ int mlmq_destroy(mlmq_ctx *c) {
     if (c->ctl) (void)hipFree(c->ctl);
     if (c->slots) (void)hipFree(c->slots);
     if (c->h_ctl) (void)hipHostFree(c->h_ctl);
+    c->stage.release();
     free_batch(c);
     if (c->ev_reset) (void)hipEventDestroy(c->ev_reset);
     if (c->ev_start) (void)hipEventDestroy(c->ev_start);
@@ -1515,9 +1527,7 @@ int mlmq_copy_batch_dist(mlmq_ctx *c, int32_t query, int32_t *host_out) {
     if (!c->b_solved) return fail(c, MLMQ_E_NOGRAPH, "no completed batch");
     if (query < 0 || query >= c->b_nq) return fail(c, MLMQ_E_INVALID, "query index out of range");
     HIP_TRY(c, hipSetDevice(c->device));
-    HIP_TRY(c, hipMemcpy(host_out, c->b_dist + (uint64_t)query * (uint64_t)c->n,
-                         sizeof(int32_t) * (size_t)c->n, hipMemcpyDeviceToHost));
-    return MLMQ_OK;
+    return row_to_host(c, host_out, c->b_dist + (uint64_t)query * (uint64_t)c->n);
 }
 
 int mlmq_last_queue_counts(const mlmq_ctx *c, mlmq_queue_counts *out) {
@@ -1542,8 +1552,7 @@ int mlmq_copy_dist(mlmq_ctx *c, int32_t *host_out) {
     if (!c || !host_out) return MLMQ_E_INVALID;
     if (!c->solved) return fail(c, MLMQ_E_NOGRAPH, "no completed solve");
     HIP_TRY(c, hipSetDevice(c->device));
-    HIP_TRY(c, hipMemcpy(host_out, c->dist, sizeof(int32_t) * (size_t)c->n, hipMemcpyDeviceToHost));
-    return MLMQ_OK;
+    return row_to_host(c, host_out, c->dist);
 }
 
 int mlmq_dist_device_ptr(mlmq_ctx *c, const int32_t **out) {

@@ -21,6 +21,7 @@
 #include "device_common.h"
 #include "hop_block.h"
 #include "pushpull_solver.h"
+#include "row_copy.h"
 #include "solver_internal.h"
 
 namespace {
@@ -147,6 +148,7 @@ struct mlmq_server {
     std::deque<int32_t> pending;   // waiting request ids, in arrival order
     hipEvent_t ev_ref = nullptr;
     Live live;
+    mlmq::RowStage stage;          // rows on their way to the host
     std::string err;
 };
 
@@ -512,9 +514,8 @@ int live_finish(mlmq_server *s, int32_t e, uint32_t status, uint32_t mism, uint6
         return MLMQ_OK;
     }
     if (st == MLMQ_OK && r.dist_out) {
-        HIP_TRY(s, hipMemcpyAsync(r.dist_out, s->arena.base + sl.off, sizeof(int32_t) * (size_t)g.v.n,
-                                  hipMemcpyDeviceToHost, L.side));
-        HIP_TRY(s, hipStreamSynchronize(L.side));
+        const mlmq::RowCopy row{r.dist_out, s->arena.base + sl.off, sizeof(int32_t) * (size_t)g.v.n};
+        HIP_TRY(s, s->stage.copy(&row, 1, L.side));
     }
     r.res.status = st;
     r.res.retries = r.retries;
@@ -925,6 +926,8 @@ int mlmq_server_create(int device, const mlmq_server_config *cfg, mlmq_server **
     if (e == hipSuccess) e = hipMalloc(&arena, c.hbm_budget);
     if (e == hipSuccess) s->arena.reset((uint8_t *)arena, c.hbm_budget);
     if (e == hipSuccess) e = hipEventCreate(&s->ev_ref);
+    // (whole from the start: it can't grow under a running live launch)
+    if (e == hipSuccess && s->stage.reserve(2 * mlmq::RowStage::kPiece) != hipSuccess) (void)hipGetLastError();
     s->lanes.resize(c.streams);
     for (Lane &l : s->lanes) {
         if (e == hipSuccess) e = hipStreamCreateWithFlags(&l.s, hipStreamNonBlocking);
@@ -972,6 +975,7 @@ int mlmq_server_destroy(mlmq_server *s) {
         mlmq_destroy(g.ctx);
     }
     if (s->arena.base) (void)hipFree(s->arena.base);
+    s->stage.release();
     if (s->ev_ref) (void)hipEventDestroy(s->ev_ref);
     delete s;
     return MLMQ_OK;
@@ -1305,6 +1309,7 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
         float done_ms = 0.0f;
         HIP_TRY(s, hipEventElapsedTime(&done_ms, s->ev_ref, l.ev_solve));
         std::vector<int32_t> rerun;   // overflowed requests, in launch order
+        std::vector<mlmq::RowCopy> rows;
         bool ring_used = false, ring_clean = true;
         for (size_t i = 0; i < l.ids.size(); ++i) {
             const int32_t id = l.ids[i];
@@ -1343,11 +1348,8 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
             r.device_ms = te > ts ? (double)(te - ts) / (double)s->wall_khz : 0.0;
             const bool verified = s->cfg.verify && g.expected.count(reqs[id].src) != 0;
             r.mismatches = verified ? (int32_t)mism : -1;
-            if (st == MLMQ_OK && reqs[id].dist_out) {
-                HIP_TRY(s, hipMemcpyAsync(reqs[id].dist_out, s->arena.base + sl.off,
-                                          sizeof(int32_t) * (size_t)g.v.n, hipMemcpyDeviceToHost, l.s));
-                HIP_TRY(s, hipStreamSynchronize(l.s));
-            }
+            if (st == MLMQ_OK && reqs[id].dist_out)
+                rows.push_back({reqs[id].dist_out, s->arena.base + sl.off, sizeof(int32_t) * (size_t)g.v.n});
             // A failed solve leaves records in its partition, another solver
             // its own state: refill before reuse.
             sl.fresh = st != MLMQ_OK || !queue;
@@ -1355,6 +1357,8 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
             ++finished;
         }
         if (ring_used && ring_clean) l.ring_dirty = false;
+        // (no slot is handed out again before the next launch)
+        const hipError_t copied = s->stage.copy(rows.data(), rows.size(), l.s);
         for (auto it = rerun.rbegin(); it != rerun.rend(); ++it) {
             s->pending.push_front(*it);
             ++pending;
@@ -1365,6 +1369,7 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
         l.slots.clear();
         l.caps.clear();
         wall_ms = std::max(wall_ms, (double)done_ms);
+        if (copied != hipSuccess) return hip_fail(s, copied, "copy of the rows");
         return MLMQ_OK;
     };
 
