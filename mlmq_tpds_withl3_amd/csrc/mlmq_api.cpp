@@ -75,6 +75,7 @@ struct mlmq_ctx {
     // per-query state of up to r_queries queries
     mlmq::RegionGraph regions;
     uint32_t *r_inbox = nullptr, *r_act = nullptr;
+    mlmq::RegionProgress *r_progress = nullptr;
     uint32_t r_queries = 0;
     uint64_t *r_ring = nullptr;
     uint64_t r_ring_slots = 0;
@@ -167,9 +168,10 @@ void free_batch(mlmq_ctx *c) {
 
 void free_regions(mlmq_ctx *c) {
     mlmq::region_free(&c->regions);
-    for (void *p : {(void *)c->r_inbox, (void *)c->r_act, (void *)c->r_ring})
+    for (void *p : {(void *)c->r_inbox, (void *)c->r_act, (void *)c->r_progress, (void *)c->r_ring})
         if (p) (void)hipFree(p);
     c->r_inbox = c->r_act = nullptr;
+    c->r_progress = nullptr;
     c->r_ring = nullptr;
     c->r_queries = 0;
     c->r_ring_slots = 0;
@@ -691,12 +693,14 @@ bool wants_pushpull(const mlmq_ctx *c, const mlmq_params &p) {
 int ensure_region_space(mlmq_ctx *c, uint32_t nq, uint32_t grid) {
     const mlmq::RegionGraph &g = c->regions;
     if (c->r_queries < nq) {
-        for (void *p : {(void *)c->r_inbox, (void *)c->r_act})
+        for (void *p : {(void *)c->r_inbox, (void *)c->r_act, (void *)c->r_progress})
             if (p) (void)hipFree(p);
         c->r_inbox = c->r_act = nullptr;
+        c->r_progress = nullptr;
         c->r_queries = 0;
         HIP_TRY(c, hipMalloc(&c->r_inbox, sizeof(uint32_t) * ((size_t)nq * g.inbox_slots + 1)));
         HIP_TRY(c, hipMalloc(&c->r_act, sizeof(uint32_t) * (size_t)nq * g.regions));
+        HIP_TRY(c, hipMalloc(&c->r_progress, sizeof(mlmq::RegionProgress) * (size_t)nq));
         c->r_queries = nq;
     }
     // Each region of a query is in the ring at most once and each workgroup
@@ -828,6 +832,8 @@ int run_regions(mlmq_ctx *c, uint32_t nq, int32_t src, const uint32_t *sources, 
     L.nq = nq;
     L.tasks = nq * g.regions;
     L.longest = std::max(g.n, g.inbox_slots);
+    L.progress = c->r_progress;
+    L.admit = mlmq::region_admit(g.regions, nq, grid);
     L.grid = grid;
     t->q0 = clk::now();
     HIP_TRY(c, hipEventRecord(c->ev_reset, c->stream));

@@ -79,6 +79,7 @@ struct Lane {
     uint8_t *h_tab = nullptr, *d_tab = nullptr;
     uint32_t *ctl = nullptr;
     uint64_t *times = nullptr;
+    mlmq::RegionProgress *progress = nullptr;
     uint64_t *ring = nullptr;
     uint64_t ring_slots = 0;
     bool ring_dirty = true;
@@ -940,6 +941,7 @@ int mlmq_server_create(int device, const mlmq_server_config *cfg, mlmq_server **
         if (e == hipSuccess) e = hipHostMalloc((void **)&l.h_tab, side, hipHostMallocDefault);
         if (e == hipSuccess) e = hipMalloc((void **)&l.d_tab, side);
         if (e == hipSuccess) e = hipMalloc((void **)&l.ctl, sizeof(uint32_t) * mlmq::kCtlWords);
+        if (e == hipSuccess) e = hipMalloc((void **)&l.progress, sizeof(mlmq::RegionProgress) * (size_t)c.max_batch);
         if (e == hipSuccess) e = hipMalloc((void **)&l.times, 2 * sizeof(uint64_t) * (size_t)c.max_batch);
     }
     if (e != hipSuccess) {
@@ -966,7 +968,8 @@ int mlmq_server_destroy(mlmq_server *s) {
         if (l.ev_done) (void)hipEventDestroy(l.ev_done);
         if (l.h_reqs) (void)hipHostFree(l.h_reqs);
         if (l.h_tab) (void)hipHostFree(l.h_tab);
-        for (void *p : {(void *)l.d_reqs, (void *)l.d_tab, (void *)l.ctl, (void *)l.times, (void *)l.ring})
+        for (void *p : {(void *)l.d_reqs, (void *)l.d_tab, (void *)l.ctl, (void *)l.times,
+                        (void *)l.progress, (void *)l.ring})
             if (p) (void)hipFree(p);
         if (l.s) (void)hipStreamDestroy(l.s);
     }
@@ -1272,6 +1275,8 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
         }
         if (nregion) {
             R.tasks = (uint32_t)tasks;
+            R.progress = l.progress;
+            R.admit = mlmq::region_admit(tasks / nregion, nregion, region_grid);
             R.grid = region_grid;
             R.ring = l.ring;
             R.ring_mask = (uint32_t)(l.ring_slots - 1);

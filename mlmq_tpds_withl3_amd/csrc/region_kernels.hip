@@ -53,13 +53,16 @@
 // records of regions whose workgroup is not resident are served all the same:
 // no workgroup ever waits for another one to become resident.
 //
-// Termination: credits are counted in kTailOff before they can be returned, and
-// returned ones in kDoneOff.  Work in a region is covered by its own credit, or
-// by that of the sender whose message caused it and which has not finished
-// marking; a region returns its credit only when it is quiet and everything it
-// sent is marked.  So the return that makes both counts equal proves that no
-// work is left; its workgroup marks every region kOver and publishes one exit
-// record per workgroup of the grid, for the ticket each of them takes last.
+// Termination: a query's credits are counted before they can be returned.  Work
+// in a region is covered by its own credit, or by that of the sender whose
+// message caused it and which has not finished marking; a region returns its
+// credit only when it is quiet and everything it sent is marked.  So the return
+// that leaves none proves that the query is over; its workgroup publishes the
+// seed of the next query that waits, and marks every region of this one kOver.
+// Whoever ends the last query publishes one exit record per workgroup of the
+// grid, for the ticket each of them takes last.
+#include <algorithm>
+#include <cmath>
 #include "device_common.h"
 #include "region_solver.h"
 #include "solver_internal.h"
@@ -69,6 +72,8 @@ namespace mlmq {
 namespace {
 
 constexpr uint32_t kRingTailOff = kHungryOff;   // ring positions taken
+constexpr uint32_t kNextOff = kHeadOff + kStride;           // queries admitted
+constexpr uint32_t kFinishedOff = kHeadOff + 2 * kStride;   // queries over
 constexpr uint32_t kWork = 1, kCounted = 2, kServed = 4, kVisited = 8, kOver = 16;
 // Quiet polls before an active region returns its credit.
 constexpr uint32_t kSettle = 2;
@@ -87,7 +92,8 @@ struct RegionArgs {
     const uint32_t *verts;
     RegionQuerySpace space;
     const RegionQuery *table;    // ... or each on its own
-    uint32_t nq;
+    RegionProgress *progress;    // per query
+    uint32_t nq, admit;
     uint64_t *ring;
     uint32_t ring_mask;
     uint32_t *ctl;
@@ -344,7 +350,7 @@ __device__ __forceinline__ void run_sender(const RegionArgs &a, RegionLds &S, co
         if (woken) {
             st.activations += lane == 0 ? woken : 0u;
             uint32_t t = 0;
-            if (lane == 0) t = fetch_add(a.ctl + kTailOff, woken);
+            if (lane == 0) t = fetch_add(&a.progress[query].credits, woken);
             asm volatile("" : "+v"(t)::"memory");   // counted before it can be returned
 #pragma unroll
             for (int g = 0; g < kG; ++g) {
@@ -360,48 +366,47 @@ __device__ __forceinline__ void run_sender(const RegionArgs &a, RegionLds &S, co
     }
 }
 
-// Return a credit; the last one ends the solve.
-template <bool kTable>
-__device__ __forceinline__ void return_credit(const RegionArgs &a, uint32_t query, MessageStats &st) {
+// Return a credit.  The query's last one ends it: the next query is admitted,
+// and the last query ends the solve.
+__device__ __forceinline__ void return_credit(const RegionArgs &a, uint32_t query, uint32_t *act, uint32_t regions,
+                                              MessageStats &st) {
     const uint32_t lane = fresh_lane();
     st.credits += lane == 0 ? 1u : 0u;
-    if (a.qtime && lane == 0)
-        __hip_atomic_fetch_max(a.qtime + 2 * query + 1, (uint64_t)wall_clock64(), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t done = 0;
-    if (lane == 0) done = fetch_add(a.ctl + kDoneOff, 1u) + 1u;
-    asm volatile("" : "+v"(done)::"memory");
-    done = read_lane(done, 0);
-    const uint32_t tail = uniform(ld_relaxed(a.ctl + kTailOff));
-    if (done != tail) return;
+    uint32_t held = 0;
+    if (lane == 0) held = fetch_add(&a.progress[query].credits, ~0u);
+    asm volatile("" : "+v"(held)::"memory");
+    if (read_lane(held, 0) != 1u) return;
+    if (a.qtime && lane == 0) a.qtime[2 * query + 1] = wall_clock64();
+    uint32_t next = ~0u;
+    if (a.admit < a.nq) {
+        if (lane == 0) next = fetch_add(a.ctl + kNextOff, 1u);
+        next = read_lane(next, 0);
+        if (next < a.nq) {
+            if (a.qtime && lane == 0) a.qtime[2 * next] = wall_clock64();
+            ring_push(a, lane == 0, a.progress[next].seed);
+        }
+    }
+    for (uint32_t i = lane; i < regions; i += kWave) st_relaxed(act + i, kOver);
+    wait_memory();
+    uint32_t over = 0;
+    if (lane == 0) over = fetch_add(a.ctl + kFinishedOff, 1u) + 1u;
+    if (read_lane(over, 0) != a.nq) return;
     const uint32_t ring_tail = uniform(ld_relaxed(a.ctl + kRingTailOff));
     for (uint32_t i = lane; i < gridDim.x; i += kWave) {
         uint64_t *slot = a.ring + ((ring_tail + i) & a.ring_mask);
         __hip_atomic_store(slot, kRegionExit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if constexpr (kTable) {
-        for (uint32_t q = 0; q < a.nq; ++q) {
-            uint32_t *act = a.table[q].act;
-            const uint32_t regions = a.table[q].regions;
-            for (uint32_t i = lane; i < regions; i += kWave) st_relaxed(act + i, kOver);
-        }
-    } else {
-        for (uint32_t i = lane; i < a.tasks; i += kWave) {
-            const uint32_t q = i / a.regions;
-            st_relaxed(a.space.act + q * a.space.act_stride + (i - q * a.regions), kOver);
-        }
     }
     wait_memory();
     if (lane == 0) st_relaxed(a.ctl + kExitOff, 1u);
 }
 
 // Serves the adopted region until it is left or the solve is over.
-template <bool kTable, int kG>
+template <int kG>
 __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, const RegionHdr &h,
                                            const uint32_t *image, const uint32_t *verts, uint32_t region,
                                            uint32_t query, uint32_t *dist, uint32_t *inbox, uint32_t *act,
-                                           uint32_t seed, uint32_t base, bool idle, uint64_t deadline,
-                                           MessageStats &st) {
+                                           uint32_t regions, uint32_t seed, uint32_t base, bool idle,
+                                           uint64_t deadline, MessageStats &st) {
     const uint32_t lane = fresh_lane();
     uint32_t to[kG], seen[kG], val[kG];
 #pragma unroll
@@ -498,13 +503,13 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
         for (int g = 0; g < kG; ++g) more = more || val[g] < seen[g];
         if (ballot(more) == 0) {
             idle = true;
-            return_credit<kTable>(a, query, st);
+            return_credit(a, query, act, regions, st);
             continue;
         }
         uint32_t was = 0;
         if (lane == 0) was = fetch_or(act + region, kWork);
         asm volatile("" : "+v"(was)::"memory");
-        if (read_lane(was, 0) & kWork) return_credit<kTable>(a, query, st);   // a sender's credit covers the news
+        if (read_lane(was, 0) & kWork) return_credit(a, query, act, regions, st);   // a sender's credit covers the news
         else if (lane == 0) (void)fetch_or(act + region, kCounted);
     }
     // the solve is over
@@ -578,6 +583,7 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
         const uint32_t *image = (kTable ? of->image : a.image) + h.image;
         const uint32_t *verts = (kTable ? of->verts : a.verts) + h.first;
         const uint32_t width = kTable ? of->width : a.width;
+        const uint32_t regions = kTable ? of->regions : a.regions;
         for (uint32_t i = threadIdx.x; i < kRegionVerts; i += kThreads)
             S.dist[local_id(i)] = (rec_lo & kVisitFlag) && i < h.nv ? ld_relaxed(dist + verts[i]) : kUnreached;
         __syncthreads();
@@ -587,9 +593,9 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
             uint32_t *in = inbox + h.inbox;
             const bool idle = uniform(S.own) != 0;
             const uint32_t held = kServed | (rec_lo & kVisitFlag ? kVisited : 0u);
-            if (h.nin <= 2 * kWave) run_poller<kTable, 2>(a, S, h, image, verts, region, query, dist, in, act, seed, held, idle, deadline, ms);
-            else if (h.nin <= 4 * kWave) run_poller<kTable, 4>(a, S, h, image, verts, region, query, dist, in, act, seed, held, idle, deadline, ms);
-            else run_poller<kTable, 6>(a, S, h, image, verts, region, query, dist, in, act, seed, held, idle, deadline, ms);
+            if (h.nin <= 2 * kWave) run_poller<2>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, held, idle, deadline, ms);
+            else if (h.nin <= 4 * kWave) run_poller<4>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, held, idle, deadline, ms);
+            else run_poller<6>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, held, idle, deadline, ms);
             if (lane == 0) {
                 sh_st(&S.over, 1u);
                 lds_order();
@@ -615,9 +621,13 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
         if (lane == 0) {
             if (ms.credits) {
                 fetch_add(a.ctl + kTakenOff, ms.credits);
+                fetch_add(a.ctl + kDoneOff, ms.credits);
                 add64(stats + kStatL2Pop, ms.credits);
             }
-            if (ms.activations) add64(stats + kStatL2Push, ms.activations);
+            if (ms.activations) {
+                fetch_add(a.ctl + kTailOff, ms.activations);
+                add64(stats + kStatL2Push, ms.activations);
+            }
             if (messages) {
                 add64(stats + kStatAtomic, messages);
                 add64(stats + kStatRelax, messages);
@@ -658,7 +668,9 @@ __global__ __launch_bounds__(256) void region_reset_kernel(RegionArgs a, uint32_
         for (uint32_t i = t0; i < slots; i += stride) inbox[i] = kUnreached;
         for (uint32_t i = t0; i < regions; i += stride) act[i] = i == at >> kRegionIdBits ? kWork | kCounted : 0u;
         if (t0 == 0) {
-            a.ring[q] = (uint64_t)((at & (kRegionVerts - 1u)) << kQueryBits | q) << 32 | kSeedFlag | at >> kRegionIdBits;
+            const uint64_t seed = (uint64_t)((at & (kRegionVerts - 1u)) << kQueryBits | q) << 32 | kSeedFlag | at >> kRegionIdBits;
+            a.progress[q] = {seed, 1u, 0u};
+            if (q < a.admit) a.ring[q] = seed;
             if (a.qtime) {
                 a.qtime[2 * q] = wall_clock64();
                 a.qtime[2 * q + 1] = 0;
@@ -666,7 +678,7 @@ __global__ __launch_bounds__(256) void region_reset_kernel(RegionArgs a, uint32_
         }
     }
     if (blockIdx.y == 0)
-        for (uint32_t i = t0; i < kCtlWords; i += stride) a.ctl[i] = i == kTailOff || i == kRingTailOff ? a.nq : 0u;
+        for (uint32_t i = t0; i < kCtlWords; i += stride) a.ctl[i] = i == kTailOff ? a.nq : i == kRingTailOff || i == kNextOff ? a.admit : 0u;
 }
 
 // ---- building ----
@@ -751,7 +763,9 @@ RegionArgs make_region_args(const RegionGraph &g, const RegionLaunch &L) {
     a.verts = g.verts;
     a.space = L.space;
     a.table = L.table;
+    a.progress = L.progress;
     a.nq = L.nq;
+    a.admit = L.admit;
     a.ring = L.ring;
     a.ring_mask = L.ring_mask;
     a.ctl = L.ctl;
@@ -774,6 +788,21 @@ RegionArgs make_region_args(const RegionGraph &g, const RegionLaunch &L) {
 hipError_t region_occupancy(int *blocks_per_cu) {
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(
         blocks_per_cu, reinterpret_cast<const void *>(&region_solver_kernel<true>), kThreads, 0);
+}
+
+// A query's wavefront has work in about as many regions at once as the square
+// root of their number.  With more queries in flight than workgroups can follow
+// a region waits in the ring, is expanded from distances that are far from
+// final, and again when they fall: 64 queries on road 264k all at once expand
+// each vertex 7.4 times, a few at a time 2.2 times, as a lone query does.
+// Batch on 264k / 1.06M (24 queries), ms, at kAdmit = 0.15, 0.2, 0.25, 0.3,
+// 0.4, all at once: 4.2, 3.5, 3.0, 2.9, 3.8, 5.9 / 7.0, 4.9, 4.6, 4.1, 5.7,
+// 11.9.  Graphs of few regions: enough of them for every workgroup.
+uint32_t region_admit(uint64_t regions, uint32_t nq, uint32_t grid) {
+    constexpr double kAdmit = 0.27, kAdmitTasks = 1.5;
+    const double r = regions ? (double)regions : 1.0;
+    const uint64_t k = (uint64_t)(grid * std::max(kAdmitTasks / r, kAdmit / std::sqrt(r)));
+    return (uint32_t)(k < 1 ? 1 : k < nq ? k : nq);
 }
 
 RegionQuery region_query(const RegionGraph &g, uint32_t *dist, uint32_t *inbox, uint32_t *act, uint32_t src) {

@@ -42,22 +42,33 @@ struct RegionQuery {
     uint32_t n, slots, regions, width, src;
 };
 
+// Progress of a query: its seed record, and the regions with work (credits).
+struct RegionProgress {
+    uint64_t seed;
+    uint32_t credits;
+    uint32_t pad;
+};
+
 struct RegionLaunch {
     RegionQuerySpace space;      // nq queries on one graph, or
     const RegionQuery *table;    // nq entries in device memory (null: `space`)
     uint32_t tasks;              // regions of all queries
     uint32_t longest;            // most vertices, inbox slots or regions of a query
     bool shared;                 // other launches may hold part of the device
+    RegionProgress *progress;    // nq entries
     uint64_t *ring;
     uint32_t ring_mask;
     uint32_t *ctl;               // control block (device_common.h)
     uint64_t *qtime;             // optional: per query, wall-clock ticks of its start and end
     uint64_t timeout_ticks;
     uint32_t nq;
+    uint32_t admit;              // queries in flight at once
     uint32_t grid;
 };
 
 hipError_t region_occupancy(int *blocks_per_cu);
+// Queries of `regions` regions each to have in flight on `grid` workgroups.
+uint32_t region_admit(uint64_t regions, uint32_t nq, uint32_t grid);
 RegionQuery region_query(const RegionGraph &g, uint32_t *dist, uint32_t *inbox, uint32_t *act, uint32_t src);
 // Builds the device side of a cut (temporary device memory: 4 bytes per edge).
 // Returns hipErrorInvalidValue when some region exceeds the limits.
