@@ -830,7 +830,6 @@ int run_regions(mlmq_ctx *c, uint32_t nq, int32_t src, const uint32_t *sources, 
     L.qtime = qtime;
     L.timeout_ticks = (uint64_t)((p.timeout_s > 0 ? p.timeout_s : 60.0) * (double)c->wall_khz * 1000.0);
     L.nq = nq;
-    L.tasks = nq * g.regions;
     L.longest = std::max(g.n, g.inbox_slots);
     L.progress = c->r_progress;
     L.admit = mlmq::region_admit(g.regions, nq, grid);

@@ -1274,7 +1274,6 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
             for (uint32_t k = 0; k < kLaneRounds; ++k, ++round) HIP_TRY(s, mlmq::launch_push(P, round, false, l.s));
         }
         if (nregion) {
-            R.tasks = (uint32_t)tasks;
             R.progress = l.progress;
             R.admit = mlmq::region_admit(tasks / nregion, nregion, region_grid);
             R.grid = region_grid;
@@ -1283,8 +1282,6 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
             R.ctl = l.ctl;
             R.qtime = l.times;
             R.timeout_ticks = timeout_ticks;
-            R.shared = inflight > 0;
-            // (a lone query starts a workgroup on each region)
             if (nregion > 1) R.table = (const mlmq::RegionQuery *)l.d_tab;
             else R.space = {h_region[0].dist, h_region[0].inbox, h_region[0].act, 0, 0, 0};
             l.ring_dirty = true;   // until the solve has left it clean

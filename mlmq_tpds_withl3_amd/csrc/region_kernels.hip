@@ -48,10 +48,12 @@
 //
 // Ring: a workgroup without a region takes the next ticket (kHeadOff) and
 // polls that slot alone; a sender takes the next position (kRingTailOff) and
-// publishes there.  When every region has a workgroup, workgroup i starts on
-// region i without a record and leaves only after a long idle time, so that
-// records of regions whose workgroup is not resident are served all the same:
-// no workgroup ever waits for another one to become resident.
+// publishes there.  A region is left as soon as it has returned its credit.
+// (Regions that keep a workgroup were tried where every region has one: to
+// poll an idle region's word is faster than a record, a ticket and the region's
+// edges from L2 anew, but the pollers slow everyone: road 264k 631 against
+// 595 us, 4-NN 700k 1335 against 965 us.)  No workgroup ever waits for another
+// one to become resident.
 //
 // Termination: a query's credits are counted before they can be returned.  Work
 // in a region is covered by its own credit, or by that of the sender whose
@@ -100,10 +102,7 @@ struct RegionArgs {
     uint64_t *qtime;
     uint64_t timeout_ticks;
     uint32_t regions;
-    uint32_t tasks;          // regions x queries
     uint32_t width;          // window of a wave's expansions
-    uint32_t preadopt;       // workgroup i starts on task i
-    uint32_t linger;         // idle polls before a region is left
 };
 
 struct RegionLds {
@@ -112,7 +111,6 @@ struct RegionLds {
     uint32_t over;                     // the region is left: a wave without work returns
     uint32_t checked[kRelaxers + 1];   // relaxers, sender
     uint32_t rec[2];                   // adopted record
-    uint32_t own;                      // adopted without a record: no work yet
 };
 
 __device__ __forceinline__ uint32_t sh_ld(uint32_t *p) {
@@ -183,24 +181,46 @@ __device__ __forceinline__ void lower_heads(RegionLds &S, const uint32_t (&edge)
     for (uint32_t k = kFrom; k < kTo; ++k) (void)sh_min(at_offset(S.dist, edge[k] & mask), d + (edge[k] >> shift));
 }
 
-__device__ __forceinline__ void run_relaxer(RegionLds &S, const RegionHdr &h, const uint32_t *image, uint32_t w,
+__device__ __forceinline__ void run_relaxer(RegionLds &S, const RegionHdr &h, const uint32_t *image,
+                                            const uint32_t *verts, uint32_t *dist, bool visited, uint32_t w,
                                             uint32_t width, RelaxStats &st) {
     const uint32_t lane = fresh_lane();
     const uint32_t thread = w * kWave + lane;
     uint32_t edge[kLaneVerts][kLaneEdges], last[kLaneVerts], most[kLaneVerts];
     uint32_t degrees = 0;   // edges of each vertex, 8 bits each
+    // the distances, by way of the vertex list, beside the edges
+    Quad start = {kUnreached, kUnreached, kUnreached, kUnreached};
+    uint32_t vert[kLaneVerts];
+    if (visited) {
+#pragma unroll
+        for (uint32_t i = 0; i < kLaneVerts; ++i) vert[i] = verts[min(i * kRegionThreads + thread, h.nv - 1u)];
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kLaneVerts; ++i)
+#pragma unroll
+        for (uint32_t k = 0; k < kLaneEdges; ++k) edge[i][k] = image[(i * kLaneEdges + k) * kRegionThreads + thread];
+    if (visited) {
+#pragma unroll
+        for (uint32_t i = 0; i < kLaneVerts; ++i) {
+            const uint32_t x = ld_relaxed(dist + vert[i]);
+            start[i] = i * kRegionThreads + thread < h.nv ? x : kUnreached;
+        }
+    }
+    Quad *own = reinterpret_cast<Quad *>(S.dist + thread * kLaneVerts);
+    *own = start;
 #pragma unroll
     for (uint32_t i = 0; i < kLaneVerts; ++i) {
         most[i] = image[kImageMost + w * kLaneVerts + i];
-        // a vertex is expanded below `last`; past the end: never
-        last[i] = i * kRegionThreads + thread < h.nv ? kUnreached : 0u;
+        // a vertex is expanded below `last` (a region that was left is expanded
+        // as far as it has distances); past the end: never
+        last[i] = i * kRegionThreads + thread < h.nv ? start[i] : 0u;
 #pragma unroll
         for (uint32_t k = 0; k < kLaneEdges; ++k) {
-            edge[i][k] = image[(i * kLaneEdges + k) * kRegionThreads + thread];
             if (edge[i][k] >> kWeightShift != ~0u >> kWeightShift) degrees += 1u << 8 * i;
         }
     }
-    const Quad *own = reinterpret_cast<const Quad *>(S.dist + thread * kLaneVerts);
+    __syncthreads();
+    if (visited) __syncthreads();   // until the sender has read them
     uint32_t checked = 0, expanded = 0, sweeps = 0;
     for (;;) {
         // the version before the distances
@@ -295,8 +315,8 @@ __device__ __forceinline__ void ring_push(const RegionArgs &a, bool valid, uint6
 
 template <int kG>
 __device__ __forceinline__ void run_sender(const RegionArgs &a, RegionLds &S, const RegionHdr &h,
-                                           const uint32_t *image, uint32_t query, uint32_t *inbox_all, uint32_t *act,
-                                           MessageStats &st) {
+                                           const uint32_t *image, bool visited, uint32_t query, uint32_t *inbox_all,
+                                           uint32_t *act, MessageStats &st) {
     const uint32_t lane = fresh_lane();
     const uint32_t *exits = image + kImageExits;
     uint32_t edge[kG], slot[kG], reg[kG], last[kG];   // last: least distance sent
@@ -307,6 +327,13 @@ __device__ __forceinline__ void run_sender(const RegionArgs &a, RegionLds &S, co
         slot[g] = x < h.nx ? exits[h.nx + x] : 0u;
         reg[g] = x < h.nx ? exits[2 * h.nx + x] : 0u;
         last[g] = x < h.nx ? kUnreached : 0u;         // 0: never sends
+    }
+    __syncthreads();
+    if (visited) {   // what the adopted distances give was sent before
+#pragma unroll
+        for (int g = 0; g < kG; ++g)
+            last[g] = min(last[g], sh_ld(at_offset(S.dist, edge[g] & kOffsetMask)) + (edge[g] >> kWeightShift));
+        __syncthreads();
     }
     for (;;) {
         const uint32_t version = uniform(sh_ld(&S.version));
@@ -405,8 +432,8 @@ template <int kG>
 __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, const RegionHdr &h,
                                            const uint32_t *image, const uint32_t *verts, uint32_t region,
                                            uint32_t query, uint32_t *dist, uint32_t *inbox, uint32_t *act,
-                                           uint32_t regions, uint32_t seed, uint32_t base, bool idle,
-                                           uint64_t deadline, MessageStats &st) {
+                                           uint32_t regions, uint32_t seed, bool visited, uint64_t deadline,
+                                           MessageStats &st) {
     const uint32_t lane = fresh_lane();
     uint32_t to[kG], seen[kG], val[kG];
 #pragma unroll
@@ -421,7 +448,10 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
 #pragma unroll
     for (int g = 0; g < kG; ++g) at[g] = min(g * kWave + lane, h.nin ? h.nin - 1u : 0u);
     uint32_t quiet = 0;
-    bool dirty = false;
+    bool dirty = false, idle = false;
+    const uint32_t base = kServed | (visited ? kVisited : 0u);
+    __syncthreads();
+    if (visited) __syncthreads();
     // the waves look once at the adopted distances in any case: a version they
     // have not checked
     if (lane == 0) {
@@ -440,13 +470,9 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
         }
         st.polls += lane == 0 ? 1u : 0u;
         if (idle) {
-            // a sender marks the region after its message: the mark is enough
             const uint32_t state = uniform(ld_relaxed(act + region));
             if (state & kOver) break;
             if (!(state & kWork)) {
-                __builtin_amdgcn_s_sleep(4);
-                if (++quiet < a.linger) continue;
-                quiet = 0;
                 if (dirty) {
                     for (uint32_t i = lane; i < h.nv; i += kWave) {
                         const uint32_t x = sh_ld(S.dist + local_id(i));
@@ -460,8 +486,8 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
                 if (read_lane(left, 0)) return;
                 continue;
             }
+            // (a sender marks the region after its message)
             idle = false;
-            quiet = 0;
         }
 #pragma unroll
         for (int g = 0; g < kG; ++g) val[g] = ld_relaxed(inbox + at[g]);
@@ -528,47 +554,36 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
     const uint64_t deadline = wall_clock64() + a.timeout_ticks;
     RelaxStats rs{};
     MessageStats ms{};
-    bool first = !kTable && a.preadopt != 0;
     for (;;) {
-        // adopt: this workgroup's own region first, then the next ticket's record
+        // adopt the next ticket's region
         if (wave == kPollerWave && lane == 0) {
-            uint64_t rec = kEmpty;
-            bool rec_own = false;
-            if (first && blockIdx.x < a.tasks) {
-                const uint32_t q = blockIdx.x / a.regions, r = blockIdx.x - q * a.regions;
-                rec_own = cas32(a.space.act + q * a.space.act_stride + r, 0u, kServed);
-                if (rec_own) rec = (uint64_t)q << 32 | r;
-            }
-            if (rec == kEmpty) {
-                uint64_t *slot = a.ring + (fetch_add(a.ctl + kHeadOff, 1u) & a.ring_mask);
-                for (uint32_t turn = 1;; ++turn) {
-                    rec = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    if (rec != kEmpty) {
-                        xchg64(slot, kEmpty);
-                        break;
-                    }
-                    // after an error no record will come; a finished solve
-                    // has put this ticket's exit record in place
-                    if ((turn & 15u) == 0 && (ld_relaxed(a.ctl + kErrOff) || wall_clock64() > deadline)) {
-                        rec = kRegionExit;
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(4);
+            uint64_t *slot = a.ring + (fetch_add(a.ctl + kHeadOff, 1u) & a.ring_mask);
+            uint64_t rec;
+            for (uint32_t turn = 1;; ++turn) {
+                rec = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (rec != kEmpty) {
+                    xchg64(slot, kEmpty);
+                    break;
                 }
+                // after an error no record will come; a finished solve has put
+                // this ticket's exit record in place
+                if ((turn & 15u) == 0 && (ld_relaxed(a.ctl + kErrOff) || wall_clock64() > deadline)) {
+                    rec = kRegionExit;
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(4);
             }
-            if (!rec_own && rec != kRegionExit) {
+            if (rec != kRegionExit) {
                 // (its word: kWork, kCounted and perhaps kVisited)
                 const uint32_t q = (uint32_t)(rec >> 32) & (kRegionQueries - 1u);
                 const uint32_t r = (uint32_t)rec & ~(kSeedFlag | kVisitFlag);
                 (void)fetch_or((kTable ? a.table[q].act : a.space.act + q * a.space.act_stride) + r, kServed);
             }
-            S.own = rec_own ? 1u : 0u;
             S.rec[0] = (uint32_t)rec;
             S.rec[1] = (uint32_t)(rec >> 32);
             S.version = S.over = 0;
             for (uint32_t i = 0; i <= kRelaxers; ++i) S.checked[i] = 0;
         }
-        first = false;
         __syncthreads();
         const uint32_t rec_lo = uniform(S.rec[0]), rec_hi = uniform(S.rec[1]);
         if (((uint64_t)rec_hi << 32 | rec_lo) == kRegionExit) break;
@@ -584,27 +599,24 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
         const uint32_t *verts = (kTable ? of->verts : a.verts) + h.first;
         const uint32_t width = kTable ? of->width : a.width;
         const uint32_t regions = kTable ? of->regions : a.regions;
-        for (uint32_t i = threadIdx.x; i < kRegionVerts; i += kThreads)
-            S.dist[local_id(i)] = (rec_lo & kVisitFlag) && i < h.nv ? ld_relaxed(dist + verts[i]) : kUnreached;
-        __syncthreads();
+        const bool visited = (rec_lo & kVisitFlag) != 0;
+        // (each role loads what it holds, then meets the others once)
         if (wave < kRelaxers) {
-            run_relaxer(S, h, image, wave, width, rs);
+            run_relaxer(S, h, image, verts, dist, visited, wave, width, rs);
         } else if (wave == kPollerWave) {
             uint32_t *in = inbox + h.inbox;
-            const bool idle = uniform(S.own) != 0;
-            const uint32_t held = kServed | (rec_lo & kVisitFlag ? kVisited : 0u);
-            if (h.nin <= 2 * kWave) run_poller<2>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, held, idle, deadline, ms);
-            else if (h.nin <= 4 * kWave) run_poller<4>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, held, idle, deadline, ms);
-            else run_poller<6>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, held, idle, deadline, ms);
+            if (h.nin <= 2 * kWave) run_poller<2>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
+            else if (h.nin <= 4 * kWave) run_poller<4>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
+            else run_poller<6>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
             if (lane == 0) {
                 sh_st(&S.over, 1u);
                 lds_order();
                 sh_add(&S.version, 1u);   // wakes the waiting waves
             }
         } else if (wave == kSenderWave) {
-            if (h.nx <= 2 * kWave) run_sender<2>(a, S, h, image, query, inbox, act, ms);
-            else if (h.nx <= 4 * kWave) run_sender<4>(a, S, h, image, query, inbox, act, ms);
-            else run_sender<6>(a, S, h, image, query, inbox, act, ms);
+            if (h.nx <= 2 * kWave) run_sender<2>(a, S, h, image, visited, query, inbox, act, ms);
+            else if (h.nx <= 4 * kWave) run_sender<4>(a, S, h, image, visited, query, inbox, act, ms);
+            else run_sender<6>(a, S, h, image, visited, query, inbox, act, ms);
         }
         __syncthreads();
     }
@@ -772,13 +784,7 @@ RegionArgs make_region_args(const RegionGraph &g, const RegionLaunch &L) {
     a.qtime = L.qtime;
     a.timeout_ticks = L.timeout_ticks;
     a.regions = g.regions;
-    a.tasks = L.tasks;
     a.width = g.width;
-    a.preadopt = L.grid >= L.tasks ? 1u : 0u;
-    // A region that keeps its workgroup is left only if some other may need
-    // it: after about 2 ms (polls of about 0.7 us), or 0.1 ms beside other
-    // launches, whose workgroups may keep some of this one's from starting.
-    a.linger = !a.preadopt ? 6u : L.shared ? 150u : 3000u;
     return a;
 }
 

@@ -52,9 +52,7 @@ struct RegionProgress {
 struct RegionLaunch {
     RegionQuerySpace space;      // nq queries on one graph, or
     const RegionQuery *table;    // nq entries in device memory (null: `space`)
-    uint32_t tasks;              // regions of all queries
     uint32_t longest;            // most vertices, inbox slots or regions of a query
-    bool shared;                 // other launches may hold part of the device
     RegionProgress *progress;    // nq entries
     uint64_t *ring;
     uint32_t ring_mask;
