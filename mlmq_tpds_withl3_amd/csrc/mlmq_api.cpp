@@ -723,11 +723,13 @@ int ensure_region_space(mlmq_ctx *c, uint32_t nq, uint32_t grid) {
     return ensure_ctl(c);
 }
 
-// Grid of a region solve: one workgroup per region task, at least
-// `at_least`, at most what the device holds.
-int region_grid(mlmq_ctx *c, uint64_t tasks, uint64_t at_least, uint32_t *grid) {
+// Workgroups of a region solve of nq queries: one per region and query, at
+// least `at_least`, at most what the device holds.
+int region_grid(mlmq_ctx *c, uint32_t nq, uint64_t at_least, uint32_t *relaxers, uint32_t *grid) {
     int occ = 0;
-    HIP_TRY(c, mlmq::region_occupancy(&occ));
+    const uint64_t tasks = (uint64_t)nq * c->regions.regions;
+    *relaxers = mlmq::region_relaxers(c->regions.regions, nq, (uint32_t)c->cus);
+    HIP_TRY(c, mlmq::region_occupancy(*relaxers, &occ));
     if (occ < 1) return fail(c, MLMQ_E_HIP, "region solver cannot be resident");
     *grid = (uint32_t)std::min<uint64_t>((uint64_t)occ * c->cus, std::max(tasks, at_least));
     return MLMQ_OK;
@@ -820,7 +822,7 @@ int row_to_host(mlmq_ctx *c, int32_t *host_out, const uint32_t *row) {
 // `sources`; distances into `dist`, one row of n after another.  On success
 // the control block is in ctl_host.
 int run_regions(mlmq_ctx *c, uint32_t nq, int32_t src, const uint32_t *sources, uint32_t *dist, uint64_t *qtime,
-                const mlmq_params &p, uint32_t grid, QueryClock *t) {
+                const mlmq_params &p, uint32_t relaxers, uint32_t grid, QueryClock *t) {
     const mlmq::RegionGraph &g = c->regions;
     mlmq::RegionLaunch L{};
     L.space = {dist, c->r_inbox, c->r_act, (uint64_t)g.n, g.inbox_slots, g.regions};
@@ -833,6 +835,7 @@ int run_regions(mlmq_ctx *c, uint32_t nq, int32_t src, const uint32_t *sources, 
     L.longest = std::max(g.n, g.inbox_slots);
     L.progress = c->r_progress;
     L.admit = mlmq::region_admit(g.regions, nq, grid);
+    L.relaxers = relaxers;
     L.grid = grid;
     t->q0 = clk::now();
     HIP_TRY(c, hipEventRecord(c->ev_reset, c->stream));
@@ -857,12 +860,12 @@ int run_regions(mlmq_ctx *c, uint32_t nq, int32_t src, const uint32_t *sources, 
 
 // One query, distances into the context's row.
 int solve_regions(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *timing) {
-    uint32_t grid = 0;
-    int rc = region_grid(c, c->regions.regions, (uint64_t)p.work_blocks, &grid);
+    uint32_t relaxers = 0, grid = 0;
+    int rc = region_grid(c, 1, (uint64_t)p.work_blocks, &relaxers, &grid);
     if (rc == MLMQ_OK) rc = ensure_region_space(c, 1, grid);
     if (rc) return rc;
     QueryClock t;
-    rc = run_regions(c, 1, src, nullptr, c->dist, nullptr, p, grid, &t);
+    rc = run_regions(c, 1, src, nullptr, c->dist, nullptr, p, relaxers, grid, &t);
     if (rc) return rc;
     c->solved = true;
     c->last_buckets = (uint32_t)p.buckets;
@@ -870,7 +873,7 @@ int solve_regions(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *t
     c->last_cap_log2 = ceil_log2(c->r_ring_slots);
     if (timing) {
         fill_timing(c, c->ctl_host.data(), t, (int)grid, c->last_cap_log2, 0, timing);
-        timing->waves = mlmq::kRegionWaves * (int32_t)grid;
+        timing->waves = mlmq::region_waves(relaxers) * (int32_t)grid;
     }
     return MLMQ_OK;
 }
@@ -988,12 +991,12 @@ void fill_batch_timing(mlmq_ctx *c, const uint32_t *h, const std::vector<uint64_
 
 // A batch by the region solver: every query of it in flight at once.
 int batch_regions(mlmq_ctx *c, int32_t nq, const mlmq_params &p, mlmq_batch_timing *timing) {
-    uint32_t grid = 0;
-    int rc = region_grid(c, (uint64_t)nq * c->regions.regions, 0, &grid);
+    uint32_t relaxers = 0, grid = 0;
+    int rc = region_grid(c, (uint32_t)nq, 0, &relaxers, &grid);
     if (rc == MLMQ_OK) rc = ensure_region_space(c, (uint32_t)nq, grid);
     if (rc) return rc;
     QueryClock t;
-    rc = run_regions(c, (uint32_t)nq, 0, c->b_sources, c->b_dist, c->b_qtime, p, grid, &t);
+    rc = run_regions(c, (uint32_t)nq, 0, c->b_sources, c->b_dist, c->b_qtime, p, relaxers, grid, &t);
     if (rc) return rc;
     c->b_nq = nq;
     c->b_solved = true;

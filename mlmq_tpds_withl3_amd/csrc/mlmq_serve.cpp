@@ -1117,9 +1117,10 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
     double wall_ms = 0.0;
     int rc = MLMQ_OK;
     const size_t rb = mlmq::serve_request_bytes();
-    int occ = 0;
-    HIP_TRY(s, mlmq::region_occupancy(&occ));
-    const uint32_t region_groups = (uint32_t)(std::max(occ, 1) * s->cus);
+    int few = 0, many = 0;
+    HIP_TRY(s, mlmq::region_occupancy(mlmq::kFew, &few));
+    HIP_TRY(s, mlmq::region_occupancy(mlmq::kMany, &many));
+    const uint32_t region_groups = (uint32_t)(std::max({few, many, 1}) * s->cus);
 
     HIP_TRY(s, hipEventRecord(s->ev_ref, s->lanes[0].s));
     HIP_TRY(s, hipEventSynchronize(s->ev_ref));
@@ -1180,7 +1181,9 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
             npush += e == Engine::kPushPull;
             nqueue += e == Engine::kQueue;
         }
-        const uint32_t region_grid = (uint32_t)std::min<uint64_t>(region_groups, tasks);
+        const uint32_t relaxers = mlmq::region_relaxers(nregion ? tasks / nregion : 0, nregion, (uint32_t)s->cus);
+        const uint32_t region_grid =
+            (uint32_t)std::min<uint64_t>(std::max(relaxers == mlmq::kMany ? many : few, 1) * s->cus, tasks);
         if (nregion && lane_ring(l, tasks, region_grid) != hipSuccess) {
             (void)hipGetLastError();
             for (Engine &e : l.engines)
@@ -1276,6 +1279,7 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
         if (nregion) {
             R.progress = l.progress;
             R.admit = mlmq::region_admit(tasks / nregion, nregion, region_grid);
+            R.relaxers = relaxers;
             R.grid = region_grid;
             R.ring = l.ring;
             R.ring_mask = (uint32_t)(l.ring_slots - 1);

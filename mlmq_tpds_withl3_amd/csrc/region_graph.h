@@ -1,18 +1,18 @@
 // Regions: a road-like graph cut into pieces whose edges fit the registers of
 // one workgroup and whose distances fit its LDS.
 //
-// Every vertex belongs to one region of at most kRegionVerts vertices.  Thread
-// t of a region's kRegionThreads relaxing threads owns the vertices with local
-// ids t * kLaneVerts + i, and holds up to kLaneEdges out-edges of each.
-// Vertices are laid out by falling degree, position p at thread
-// p % kRegionThreads, i = p / kRegionThreads, so that the vertices a wave
-// handles at once have about as many edges.  Any further edge of a vertex is
-// treated like an edge between regions, from the region to itself.
+// Every vertex belongs to one region of at most kRegionVerts vertices.  The
+// region's vertex list goes by falling degree, so that the 64 vertices of a
+// block, which a wave handles at once, have about as many edges.  The vertices
+// at positions p and p + kRegionVerts / 2, which the same thread handles, have
+// adjacent local ids.  A thread of the solver holds up to kLaneEdges out-edges
+// of each of its vertices.  Any further edge of a vertex is treated like an edge
+// between regions, from the region to itself.
 //
 // A region's image, in 32-bit words:
 //
-//   kLaneVerts x kLaneEdges x kRegionThreads   edge k of every thread's vertex i
-//   kRelaxers x kLaneVerts                     most edges of a wave's vertices i
+//   kLaneEdges x kRegionVerts   edge k of every vertex, by position
+//   kBlocks                     most edges of a block's vertices
 //   nx x 3      exits: edge word of the tail, inbox slot of the edge in its
 //               target region, target region
 //   nin         inbox: the entered vertex, per slot
@@ -34,13 +34,10 @@
 
 namespace mlmq {
 
-constexpr uint32_t kRelaxers = 4;          // relaxing waves of a workgroup
-constexpr uint32_t kRegionThreads = 64 * kRelaxers;
-constexpr uint32_t kLaneVerts = 4;
 constexpr uint32_t kLaneEdges = 8;
 constexpr uint32_t kRegionIdBits = 10;
-constexpr uint32_t kRegionVerts = kRegionThreads * kLaneVerts;
-static_assert(kRegionVerts == 1u << kRegionIdBits, "local ids");
+constexpr uint32_t kRegionVerts = 1u << kRegionIdBits;
+constexpr uint32_t kBlocks = kRegionVerts / 64;
 constexpr uint32_t kWeightShift = 2 + kRegionIdBits;
 constexpr uint32_t kOffsetMask = (1u << kWeightShift) - 4u;
 constexpr uint32_t kRegionExits = 384;     // exits and inbox slots of a region:
@@ -61,10 +58,10 @@ struct RegionHdr {
 #define MLMQ_HD
 #endif
 // Local id of position p of a region's vertex list.
-MLMQ_HD inline uint32_t local_id(uint32_t p) { return p % kRegionThreads * kLaneVerts + p / kRegionThreads; }
+MLMQ_HD inline uint32_t local_id(uint32_t p) { return p % (kRegionVerts / 2) * 2 + p / (kRegionVerts / 2); }
 // Word offsets of the image's parts.
-constexpr uint32_t kImageMost = kLaneVerts * kLaneEdges * kRegionThreads;
-constexpr uint32_t kImageExits = kImageMost + kRelaxers * kLaneVerts;
+constexpr uint32_t kImageMost = kLaneEdges * kRegionVerts;
+constexpr uint32_t kImageExits = kImageMost + kBlocks;
 MLMQ_HD inline uint32_t image_inbox(const RegionHdr &h) { return kImageExits + 3 * h.nx; }
 MLMQ_HD inline uint32_t image_words(const RegionHdr &h) { return image_inbox(h) + h.nin; }
 

@@ -8,9 +8,9 @@
 //
 // A workgroup serves one region at a time.  Its waves share LDS words only and
 // never meet at a barrier while the region is served:
-//   * the relaxers own the region's vertices, four per lane, and hold their
-//     edges in registers.  A relaxer reads its vertices' distances (one 16-byte
-//     LDS read per lane), and a lane whose vertex is lower than it last
+//   * the relaxers own the region's vertices, two or four per lane, and hold
+//     their edges in registers.  A relaxer reads its vertices' distances (8-byte
+//     LDS reads), and a lane whose vertex is lower than it last
 //     expanded it lowers the heads by one LDS atomicMin per edge.  There is no
 //     queue: the comparison is the queue.  A lone wave issues one instruction
 //     per 8 cycles and an LDS round trip takes 64, so the hop costs what its
@@ -85,8 +85,9 @@ constexpr uint32_t kVisitFlag = 0x40000000u;    // the region's distances are in
 constexpr uint32_t kQueryBits = 20;
 static_assert(kRegionQueries == 1u << kQueryBits && kQueryBits + kRegionIdBits <= 32, "record");
 
-constexpr uint32_t kThreads = kRegionWaves * kWave;
-constexpr uint32_t kPollerWave = kRelaxers, kSenderWave = kRelaxers + 1;
+// Threads of a workgroup with kR relaxing waves and its waves resident per SIMD.
+template <uint32_t kR> constexpr uint32_t kThreads = (kR + 2) * kWave;
+template <uint32_t kR> constexpr uint32_t kPerSimd = kR == kFew ? 6 : 5;
 
 struct RegionArgs {
     const RegionHdr *hdr;        // nq queries on one graph ...
@@ -109,7 +110,7 @@ struct RegionLds {
     alignas(16) uint32_t dist[kRegionVerts];
     uint32_t version;
     uint32_t over;                     // the region is left: a wave without work returns
-    uint32_t checked[kRelaxers + 1];   // relaxers, sender
+    uint32_t checked[kMany + 1];       // relaxers, sender
     uint32_t rec[2];                   // adopted record
 };
 
@@ -153,7 +154,7 @@ struct RelaxStats {
     uint32_t relax, improve, sweeps;
 };
 
-typedef uint32_t Quad __attribute__((ext_vector_type(4)));
+typedef uint32_t Pair __attribute__((ext_vector_type(2)));
 
 // Waits for a version other than `checked`.  A wave that has waited a while
 // naps longer: it leaves the issue slots to the waves of active regions.
@@ -181,39 +182,46 @@ __device__ __forceinline__ void lower_heads(RegionLds &S, const uint32_t (&edge)
     for (uint32_t k = kFrom; k < kTo; ++k) (void)sh_min(at_offset(S.dist, edge[k] & mask), d + (edge[k] >> shift));
 }
 
+template <uint32_t kR>
 __device__ __forceinline__ void run_relaxer(RegionLds &S, const RegionHdr &h, const uint32_t *image,
                                             const uint32_t *verts, uint32_t *dist, bool visited, uint32_t w,
                                             uint32_t width, RelaxStats &st) {
     const uint32_t lane = fresh_lane();
+    constexpr uint32_t kLaneVerts = kRegionVerts / (kR * kWave);
+    constexpr uint32_t kStep = kR * kWave;   // from one of a lane's vertices to the next
     const uint32_t thread = w * kWave + lane;
     uint32_t edge[kLaneVerts][kLaneEdges], last[kLaneVerts], most[kLaneVerts];
     uint32_t degrees = 0;   // edges of each vertex, 8 bits each
     // the distances, by way of the vertex list, beside the edges
-    Quad start = {kUnreached, kUnreached, kUnreached, kUnreached};
-    uint32_t vert[kLaneVerts];
+    uint32_t start[kLaneVerts], vert[kLaneVerts];
+#pragma unroll
+    for (uint32_t i = 0; i < kLaneVerts; ++i) start[i] = kUnreached;
     if (visited) {
 #pragma unroll
-        for (uint32_t i = 0; i < kLaneVerts; ++i) vert[i] = verts[min(i * kRegionThreads + thread, h.nv - 1u)];
+        for (uint32_t i = 0; i < kLaneVerts; ++i) vert[i] = verts[min(i * kStep + thread, h.nv - 1u)];
     }
 #pragma unroll
     for (uint32_t i = 0; i < kLaneVerts; ++i)
 #pragma unroll
-        for (uint32_t k = 0; k < kLaneEdges; ++k) edge[i][k] = image[(i * kLaneEdges + k) * kRegionThreads + thread];
+        for (uint32_t k = 0; k < kLaneEdges; ++k) edge[i][k] = image[k * kRegionVerts + i * kStep + thread];
     if (visited) {
 #pragma unroll
         for (uint32_t i = 0; i < kLaneVerts; ++i) {
             const uint32_t x = ld_relaxed(dist + vert[i]);
-            start[i] = i * kRegionThreads + thread < h.nv ? x : kUnreached;
+            start[i] = i * kStep + thread < h.nv ? x : kUnreached;
         }
     }
-    Quad *own = reinterpret_cast<Quad *>(S.dist + thread * kLaneVerts);
-    *own = start;
+    // pair j: this lane's vertices j and j + kPairs
+    constexpr uint32_t kPairs = kLaneVerts / 2;
+    Pair *own = reinterpret_cast<Pair *>(S.dist) + thread;
+#pragma unroll
+    for (uint32_t j = 0; j < kPairs; ++j) own[j * kStep] = Pair{start[j], start[j + kPairs]};
 #pragma unroll
     for (uint32_t i = 0; i < kLaneVerts; ++i) {
-        most[i] = image[kImageMost + w * kLaneVerts + i];
+        most[i] = image[kImageMost + i * kR + w];
         // a vertex is expanded below `last` (a region that was left is expanded
         // as far as it has distances); past the end: never
-        last[i] = i * kRegionThreads + thread < h.nv ? start[i] : 0u;
+        last[i] = i * kStep + thread < h.nv ? start[i] : 0u;
 #pragma unroll
         for (uint32_t k = 0; k < kLaneEdges; ++k) {
             if (edge[i][k] >> kWeightShift != ~0u >> kWeightShift) degrees += 1u << 8 * i;
@@ -226,9 +234,14 @@ __device__ __forceinline__ void run_relaxer(RegionLds &S, const RegionHdr &h, co
         // the version before the distances
         const uint32_t seen = sh_ld(&S.version);
         lds_order();
-        const Quad now = *own;
+        uint32_t cur[kLaneVerts];
+#pragma unroll
+        for (uint32_t j = 0; j < kPairs; ++j) {
+            const Pair now = own[j * kStep];
+            cur[j] = now[0];
+            cur[j + kPairs] = now[1];
+        }
         lds_order();
-        const uint32_t cur[kLaneVerts] = {now[0], now[1], now[2], now[3]};
         // edges are decoded as they are used: kept decoded, they would not fit
         // the registers (the compiler must not see the constants)
         uint32_t mask = kOffsetMask, shift = kWeightShift;
@@ -313,7 +326,7 @@ __device__ __forceinline__ void ring_push(const RegionArgs &a, bool valid, uint6
     if (ballot(!ok)) region_raise(a, kErrOverflow);
 }
 
-template <int kG>
+template <uint32_t kR, int kG>
 __device__ __forceinline__ void run_sender(const RegionArgs &a, RegionLds &S, const RegionHdr &h,
                                            const uint32_t *image, bool visited, uint32_t query, uint32_t *inbox_all,
                                            uint32_t *act, MessageStats &st) {
@@ -349,7 +362,7 @@ __device__ __forceinline__ void run_sender(const RegionArgs &a, RegionLds &S, co
             send = send || d[g] < last[g];
         }
         if (ballot(send) == 0) {
-            if (lane == 0) sh_st(&S.checked[kRelaxers], version);
+            if (lane == 0) sh_st(&S.checked[kR], version);
             wait_version(S, version);
             continue;
         }
@@ -428,7 +441,7 @@ __device__ __forceinline__ void return_credit(const RegionArgs &a, uint32_t quer
 }
 
 // Serves the adopted region until it is left or the solve is over.
-template <int kG>
+template <uint32_t kR, int kG>
 __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, const RegionHdr &h,
                                            const uint32_t *image, const uint32_t *verts, uint32_t region,
                                            uint32_t query, uint32_t *dist, uint32_t *inbox, uint32_t *act,
@@ -510,7 +523,7 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
             continue;
         }
         // the checks before the version: it only grows
-        const uint32_t done = sh_ld(&S.checked[min(lane, kRelaxers)]);
+        const uint32_t done = sh_ld(&S.checked[min(lane, kR)]);
         lds_order();
         if (ballot(done != uniform(sh_ld(&S.version)))) {
             quiet = 0;
@@ -546,8 +559,8 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
         }
 }
 
-template <bool kTable>
-__global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a) {
+template <bool kTable, uint32_t kR>
+__global__ __launch_bounds__(kThreads<kR>, kPerSimd<kR>) void region_solver_kernel(RegionArgs a) {
     __shared__ RegionLds S;
     const uint32_t wave = uniform(threadIdx.x / kWave);
     const uint32_t lane = lane_id();
@@ -556,7 +569,7 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
     MessageStats ms{};
     for (;;) {
         // adopt the next ticket's region
-        if (wave == kPollerWave && lane == 0) {
+        if (wave == kR && lane == 0) {
             uint64_t *slot = a.ring + (fetch_add(a.ctl + kHeadOff, 1u) & a.ring_mask);
             uint64_t rec;
             for (uint32_t turn = 1;; ++turn) {
@@ -582,7 +595,7 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
             S.rec[0] = (uint32_t)rec;
             S.rec[1] = (uint32_t)(rec >> 32);
             S.version = S.over = 0;
-            for (uint32_t i = 0; i <= kRelaxers; ++i) S.checked[i] = 0;
+            for (uint32_t i = 0; i <= kR; ++i) S.checked[i] = 0;
         }
         __syncthreads();
         const uint32_t rec_lo = uniform(S.rec[0]), rec_hi = uniform(S.rec[1]);
@@ -601,27 +614,27 @@ __global__ __launch_bounds__(kThreads, 6) void region_solver_kernel(RegionArgs a
         const uint32_t regions = kTable ? of->regions : a.regions;
         const bool visited = (rec_lo & kVisitFlag) != 0;
         // (each role loads what it holds, then meets the others once)
-        if (wave < kRelaxers) {
-            run_relaxer(S, h, image, verts, dist, visited, wave, width, rs);
-        } else if (wave == kPollerWave) {
+        if (wave < kR) {
+            run_relaxer<kR>(S, h, image, verts, dist, visited, wave, width, rs);
+        } else if (wave == kR) {
             uint32_t *in = inbox + h.inbox;
-            if (h.nin <= 2 * kWave) run_poller<2>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
-            else if (h.nin <= 4 * kWave) run_poller<4>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
-            else run_poller<6>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
+            if (h.nin <= 2 * kWave) run_poller<kR, 2>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
+            else if (h.nin <= 4 * kWave) run_poller<kR, 4>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
+            else run_poller<kR, 6>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
             if (lane == 0) {
                 sh_st(&S.over, 1u);
                 lds_order();
                 sh_add(&S.version, 1u);   // wakes the waiting waves
             }
-        } else if (wave == kSenderWave) {
-            if (h.nx <= 2 * kWave) run_sender<2>(a, S, h, image, visited, query, inbox, act, ms);
-            else if (h.nx <= 4 * kWave) run_sender<4>(a, S, h, image, visited, query, inbox, act, ms);
-            else run_sender<6>(a, S, h, image, visited, query, inbox, act, ms);
+        } else if (wave == kR + 1) {
+            if (h.nx <= 2 * kWave) run_sender<kR, 2>(a, S, h, image, visited, query, inbox, act, ms);
+            else if (h.nx <= 4 * kWave) run_sender<kR, 4>(a, S, h, image, visited, query, inbox, act, ms);
+            else run_sender<kR, 6>(a, S, h, image, visited, query, inbox, act, ms);
         }
         __syncthreads();
     }
     uint64_t *stats = reinterpret_cast<uint64_t *>(a.ctl + kStatsOff);
-    if (wave < kRelaxers) {
+    if (wave < kR) {
         const uint32_t relax = wave_sum(rs.relax);
         if (lane == 0) {
             add64(stats + kStatRelax, relax);
@@ -727,19 +740,18 @@ __global__ __launch_bounds__(256) void region_count_kernel(const uint32_t *row, 
     if (threadIdx.x == 0) h.nx = nx;
 }
 
-__global__ __launch_bounds__(kRegionThreads) void region_image_kernel(const uint32_t *row, const uint32_t *col,
+__global__ __launch_bounds__(256) void region_image_kernel(const uint32_t *row, const uint32_t *col,
                                                                       const uint32_t *wgt, const uint32_t *verts,
                                                                       const uint32_t *where, const RegionHdr *hdr,
                                                                       const uint32_t *tmp, uint32_t *image) {
-    __shared__ uint32_t most[kRelaxers * kLaneVerts], exits;
+    __shared__ uint32_t most[kBlocks], exits;
     const RegionHdr h = hdr[blockIdx.x];
     uint32_t *img = image + h.image;
-    if (threadIdx.x < kRelaxers * kLaneVerts) most[threadIdx.x] = 0;
+    if (threadIdx.x < kBlocks) most[threadIdx.x] = 0;
     if (threadIdx.x == 0) exits = 0;
     __syncthreads();
     uint32_t *xedge = img + kImageExits, *xslot = xedge + h.nx, *xreg = xslot + h.nx;
-    for (uint32_t i = 0; i < kLaneVerts; ++i) {
-        const uint32_t p = i * kRegionThreads + threadIdx.x;
+    for (uint32_t p = threadIdx.x; p < kRegionVerts; p += blockDim.x) {
         const uint32_t own = 4 * local_id(p);
         uint32_t inside = 0;
         if (p < h.nv) {
@@ -747,7 +759,7 @@ __global__ __launch_bounds__(kRegionThreads) void region_image_kernel(const uint
             for (uint32_t e = lo; e < hi; ++e) {
                 const uint32_t to = where[col[e]], r = to >> kRegionIdBits, head = 4 * (to & (kRegionVerts - 1u));
                 if (r == blockIdx.x && inside < kLaneEdges) {
-                    img[(i * kLaneEdges + inside) * kRegionThreads + threadIdx.x] = head | wgt[e] << kWeightShift;
+                    img[inside * kRegionVerts + p] = head | wgt[e] << kWeightShift;
                     ++inside;
                     continue;
                 }
@@ -759,13 +771,13 @@ __global__ __launch_bounds__(kRegionThreads) void region_image_kernel(const uint
                 image[t.image + image_inbox(t) + tmp[e]] = head;
             }
         }
-        atomicMax(&most[threadIdx.x / kWave * kLaneVerts + i], inside);
+        atomicMax(&most[p / kWave], inside);
         // absent edges: to the vertex itself, which they cannot lower
         for (uint32_t k = inside; k < kLaneEdges; ++k)
-            img[(i * kLaneEdges + k) * kRegionThreads + threadIdx.x] = own | ~0u << kWeightShift;
+            img[k * kRegionVerts + p] = own | ~0u << kWeightShift;
     }
     __syncthreads();
-    if (threadIdx.x < kRelaxers * kLaneVerts) img[kImageMost + threadIdx.x] = most[threadIdx.x];
+    if (threadIdx.x < kBlocks) img[kImageMost + threadIdx.x] = most[threadIdx.x];
 }
 
 RegionArgs make_region_args(const RegionGraph &g, const RegionLaunch &L) {
@@ -790,14 +802,29 @@ RegionArgs make_region_args(const RegionGraph &g, const RegionLaunch &L) {
 
 }  // namespace
 
-// (both instantiations of the kernel need the same)
-hipError_t region_occupancy(int *blocks_per_cu) {
+hipError_t region_occupancy(uint32_t relaxers, int *blocks_per_cu) {
+    // (with and without a table the kernels need the same)
+    const void *k = relaxers == kMany ? reinterpret_cast<const void *>(&region_solver_kernel<true, kMany>)
+                                      : reinterpret_cast<const void *>(&region_solver_kernel<true, kFew>);
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        blocks_per_cu, reinterpret_cast<const void *>(&region_solver_kernel<true>), kThreads, 0);
+        blocks_per_cu, k, (int)(relaxers == kMany ? kThreads<kMany> : kThreads<kFew>), 0);
 }
 
-// A query's wavefront has work in about as many regions at once as the square
-// root of their number.  With more queries in flight than workgroups can follow
+// A hop is shorter where eight waves with two vertices per lane do what four
+// waves with four do (their loop has half the instructions, and a lone wave
+// issues one per 8 cycles), but only two such workgroups fit a CU, not four.
+// So few relaxers once the wavefronts of all queries (see region_admit) may
+// fill those, also from the middle of the graph.  us at 4 / 8 relaxers, by
+// nq sqrt(regions): a query on 2k 57 / 41 (1.4), 50k 250 / 186 (7), 264k from
+// its middle 414 / 372 (16), 1.06M 908 / 787 (32), 2.5M 1303 / 1183 (49), 4M
+// 1604 / 1814 (62), 6.26M 1987 / 3263 (78); 3 queries on 264k 842 / 673 (48),
+// 20 on 50k 493 / 626 (140), 64 on 20k 417 / 553 (286).
+uint32_t region_relaxers(uint64_t regions, uint32_t nq, uint32_t cus) {
+    return nq * std::sqrt((double)regions) <= 0.21 * cus ? kMany : kFew;
+}
+
+// A query's wavefront has work in about as many regions at once as a few times
+// the square root of their number.  With more queries in flight than workgroups can follow
 // a region waits in the ring, is expanded from distances that are far from
 // final, and again when they fall: 64 queries on road 264k all at once expand
 // each vertex 7.4 times, a few at a time 2.2 times, as a lone query does.
@@ -863,7 +890,7 @@ hipError_t region_build(const RegionPlan &plan, uint32_t n, uint64_t m, const ui
     if (e == hipSuccess) e = hipMalloc(&g->image, sizeof(uint32_t) * words);
     if (e == hipSuccess) e = hipMemcpy(g->hdr, hdr.data(), sizeof(RegionHdr) * nr, hipMemcpyHostToDevice);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(region_image_kernel, dim3(nr), dim3(kRegionThreads), 0, s, row, col, wgt, g->verts, g->where, g->hdr,
+        hipLaunchKernelGGL(region_image_kernel, dim3(nr), dim3(256), 0, s, row, col, wgt, g->verts, g->where, g->hdr,
                            tmp, g->image);
         e = hipGetLastError();
     }
@@ -891,8 +918,14 @@ hipError_t launch_region_reset(const RegionGraph &g, const RegionLaunch &L, cons
 
 hipError_t launch_region_solver(const RegionGraph &g, const RegionLaunch &L, hipStream_t s) {
     const RegionArgs a = make_region_args(g, L);
-    if (L.table) hipLaunchKernelGGL(region_solver_kernel<true>, dim3(L.grid), dim3(kThreads), 0, s, a);
-    else hipLaunchKernelGGL(region_solver_kernel<false>, dim3(L.grid), dim3(kThreads), 0, s, a);
+    if (L.table && L.relaxers == kMany)
+        hipLaunchKernelGGL((region_solver_kernel<true, kMany>), dim3(L.grid), dim3(kThreads<kMany>), 0, s, a);
+    else if (L.table)
+        hipLaunchKernelGGL((region_solver_kernel<true, kFew>), dim3(L.grid), dim3(kThreads<kFew>), 0, s, a);
+    else if (L.relaxers == kMany)
+        hipLaunchKernelGGL((region_solver_kernel<false, kMany>), dim3(L.grid), dim3(kThreads<kMany>), 0, s, a);
+    else
+        hipLaunchKernelGGL((region_solver_kernel<false, kFew>), dim3(L.grid), dim3(kThreads<kFew>), 0, s, a);
     return hipGetLastError();
 }
 

@@ -9,8 +9,6 @@
 
 namespace mlmq {
 
-constexpr int kRegionWaves = kRelaxers + 2;   // waves of a workgroup
-
 constexpr uint32_t kRegionQueries = 1u << 20;   // queries of one launch
 
 // A cut graph on the device.
@@ -61,10 +59,17 @@ struct RegionLaunch {
     uint64_t timeout_ticks;
     uint32_t nq;
     uint32_t admit;              // queries in flight at once
+    uint32_t relaxers;           // kFew or kMany
     uint32_t grid;
 };
 
-hipError_t region_occupancy(int *blocks_per_cu);
+// Workgroups come in two sizes: with kFew relaxers many are resident, with
+// kMany a hop is shorter.
+constexpr uint32_t kFew = 4, kMany = 8;
+hipError_t region_occupancy(uint32_t relaxers, int *blocks_per_cu);
+// Relaxers of a workgroup for nq queries of `regions` regions each.
+uint32_t region_relaxers(uint64_t regions, uint32_t nq, uint32_t cus);
+inline int region_waves(uint32_t relaxers) { return (int)relaxers + 2; }
 // Queries of `regions` regions each to have in flight on `grid` workgroups.
 uint32_t region_admit(uint64_t regions, uint32_t nq, uint32_t grid);
 RegionQuery region_query(const RegionGraph &g, uint32_t *dist, uint32_t *inbox, uint32_t *act, uint32_t src);

@@ -3,7 +3,7 @@ against the oracle, bit for bit, at the sizes where it can go wrong: region
 sizes around 1024, more than eight edges per vertex, weights at the packed
 limit, one-way and zero-weight edges, separate components, and batches with
 more regions than the device serves at once (regions are left and adopted
-again).  The timing tells which solver ran: the region solver reports six
+again).  The timing tells which solver ran: the region solver reports six or ten
 waves per workgroup.  Tolerance: none, distances are whole numbers."""
 import sys
 
@@ -60,7 +60,7 @@ def check(solver, graph, sources, regions, **params):
         ref, work, _ = O.dijkstra(row, col, w, int(src))
         bad = np.flatnonzero(solver.dist() != ref)
         assert bad.size == 0, f"source {src}: {bad.size} mismatches, first v={bad[0]}"
-        assert (t["waves"] == 6 * t["work_blocks"]) == regions
+        assert (t["waves"] in (6 * t["work_blocks"], 10 * t["work_blocks"])) == regions
         assert t["relaxations"] >= work
         q = solver.queue_counts()
         assert q["writes"] == q["reads"] and sum(q["writes"]) == q["completed"] == t["l2_pushes"]
@@ -129,7 +129,7 @@ def test_distances_near_the_end_of_range(solver):
     solver.load_csr(row, col, w)
     t = solver.solve(0, timeout_s=TIMEOUT)
     d = np.arange(n, dtype=np.int64) * ((1 << 20) - 2)
-    assert t["waves"] == 6 * t["work_blocks"]
+    assert t["waves"] == 10 * t["work_blocks"]
     assert np.array_equal(solver.dist(), np.where(d < 0x7FFFFFFF, d, 0x7FFFFFFF).astype(np.int32))
 
 
