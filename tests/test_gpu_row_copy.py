@@ -3,12 +3,14 @@
 ordinary memory at odd addresses, into pinned memory, and several rows of a
 serving launch at once.  Every word is compared; the words beside the row keep
 their values."""
+import contextlib
+import ctypes
 import sys
 
 import numpy as np
 import pytest
-import torch
 
+from hip_rt import hip
 from mlmq_tpds_withl3_amd import Solver
 from mlmq_tpds_withl3_amd._lib import check
 from mlmq_tpds_withl3_amd.serve import Server
@@ -21,6 +23,17 @@ PIECE = (4 << 20) // 4
 def say(msg):
     print(f"[gpu-row-copy] {msg}", flush=True)
     sys.stdout.flush()
+
+
+@contextlib.contextmanager
+def pinned(n):
+    """n words of pinned memory, each -7."""
+    p = ctypes.c_void_p()
+    assert hip().hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(4 * n), ctypes.c_uint(0)) == 0
+    row = np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_int32)), shape=(n,))
+    row[:] = -7
+    yield row
+    assert hip().hipHostFree(p) == 0
 
 
 def stars(n):
@@ -47,10 +60,10 @@ def test_sizes(n):
     check(s._L.mlmq_copy_dist(s._h, around[33:].ctypes.data), s._h)
     assert np.array_equal(around[33:33 + n], expect)
     assert (around[:33] == -7).all() and (around[33 + n:] == -7).all()
-    pinned = torch.full((n + 2,), -7, dtype=torch.int32, pin_memory=True)
-    check(s._L.mlmq_copy_dist(s._h, pinned.data_ptr() + 4), s._h)
-    assert np.array_equal(pinned.numpy()[1:-1], expect)
-    assert pinned[0] == -7 and pinned[-1] == -7
+    with pinned(n + 2) as row:
+        check(s._L.mlmq_copy_dist(s._h, row[1:].ctypes.data), s._h)
+        assert np.array_equal(row[1:-1], expect)
+        assert row[0] == -7 and row[-1] == -7
     s.close()
 
 
@@ -62,10 +75,9 @@ def test_rows_of_a_launch():
         s.add_graph(g[:3])
     which = np.array([2, 0, 1, 0, 2, 1, 1], dtype=np.int32)
     rows = [np.full(len(graphs[g][3]), -1, dtype=np.int32) for g in which]
-    keep = torch.full((len(rows[3]),), -1, dtype=torch.int32, pin_memory=True)
-    rows[3] = keep.numpy()
-    res, _ = s.run(np.zeros(len(which)), which, np.zeros(len(which), dtype=np.int32), dist_out=rows)
-    assert (res["status"] == 0).all()
-    for g, row in zip(which, rows):
-        assert np.array_equal(row, graphs[g][3])
+    with pinned(len(rows[3])) as rows[3]:
+        res, _ = s.run(np.zeros(len(which)), which, np.zeros(len(which), dtype=np.int32), dist_out=rows)
+        assert (res["status"] == 0).all()
+        for g, row in zip(which, rows):
+            assert np.array_equal(row, graphs[g][3])
     s.close()
