@@ -76,6 +76,7 @@ struct mlmq_ctx {
     mlmq::RegionGraph regions;
     uint32_t *r_inbox = nullptr, *r_act = nullptr;
     mlmq::RegionProgress *r_progress = nullptr;
+    mlmq::RegionCounts *r_counts = nullptr;
     uint32_t r_queries = 0;
     uint64_t *r_ring = nullptr;
     uint64_t r_ring_slots = 0;
@@ -168,10 +169,11 @@ void free_batch(mlmq_ctx *c) {
 
 void free_regions(mlmq_ctx *c) {
     mlmq::region_free(&c->regions);
-    for (void *p : {(void *)c->r_inbox, (void *)c->r_act, (void *)c->r_progress, (void *)c->r_ring})
+    for (void *p : {(void *)c->r_inbox, (void *)c->r_act, (void *)c->r_progress, (void *)c->r_counts, (void *)c->r_ring})
         if (p) (void)hipFree(p);
     c->r_inbox = c->r_act = nullptr;
     c->r_progress = nullptr;
+    c->r_counts = nullptr;
     c->r_ring = nullptr;
     c->r_queries = 0;
     c->r_ring_slots = 0;
@@ -670,6 +672,12 @@ mlmq::SolverLaunch query_launch(const mlmq_ctx *c, const QueryPlan &q, uint32_t 
 
 struct QueryClock {
     clk::time_point q0, q1, s0, s1;
+    double device_ms = -1;   // of the solve, where its kernels took the time (else: by events)
+    // The reset took reset_ms of the one wait for both.
+    void split(double reset_ms) {
+        q1 = s0 = std::min(s1, q0 + std::chrono::duration_cast<clk::duration>(
+                                        std::chrono::duration<double, std::milli>(reset_ms)));
+    }
 };
 
 // The region solver answers the default queue mode on a cut graph.  Settings
@@ -703,6 +711,7 @@ int ensure_region_space(mlmq_ctx *c, uint32_t nq, uint32_t grid) {
         HIP_TRY(c, hipMalloc(&c->r_progress, sizeof(mlmq::RegionProgress) * (size_t)nq));
         c->r_queries = nq;
     }
+    if (!c->r_counts) HIP_TRY(c, hipMalloc(&c->r_counts, sizeof(mlmq::RegionCounts) * mlmq::kRegionGroups));
     // Each region of a query is in the ring at most once and each workgroup
     // waits on one ticket; twice that, so that a slot is long read when the
     // ring comes round to it (a writer that finds it full waits, bounded).
@@ -731,7 +740,8 @@ int region_grid(mlmq_ctx *c, uint32_t nq, uint64_t at_least, uint32_t *relaxers,
     *relaxers = mlmq::region_relaxers(c->regions.regions, nq, (uint32_t)c->cus);
     HIP_TRY(c, mlmq::region_occupancy(*relaxers, &occ));
     if (occ < 1) return fail(c, MLMQ_E_HIP, "region solver cannot be resident");
-    *grid = (uint32_t)std::min<uint64_t>((uint64_t)occ * c->cus, std::max(tasks, at_least));
+    const uint64_t most = std::min<uint64_t>((uint64_t)occ * c->cus, mlmq::kRegionGroups);
+    *grid = (uint32_t)std::min(most, std::max(tasks, at_least));
     return MLMQ_OK;
 }
 
@@ -785,9 +795,9 @@ void fill_timing(mlmq_ctx *c, const uint32_t *h, const QueryClock &t, int blocks
                  uint64_t retries, mlmq_timing *timing) {
     std::memset(timing, 0, sizeof(*timing));
     float dev_ms = 0;
-    (void)hipEventElapsedTime(&dev_ms, c->ev_start, c->ev_stop);
+    if (t.device_ms < 0) (void)hipEventElapsedTime(&dev_ms, c->ev_start, c->ev_stop);
     timing->solve_ms = ms_since(t.s0, t.s1);
-    timing->device_ms = dev_ms;
+    timing->device_ms = t.device_ms < 0 ? dev_ms : t.device_ms;
     timing->reset_ms = ms_since(t.q0, t.q1);
     timing->query_wall_ms = ms_since(t.q0, t.s1);
     timing->work_blocks = blocks;
@@ -820,7 +830,7 @@ int row_to_host(mlmq_ctx *c, int32_t *host_out, const uint32_t *row) {
 
 // nq queries by the region solver: from `src`, or from the device array
 // `sources`; distances into `dist`, one row of n after another.  On success
-// the control block is in ctl_host.
+// ctl_host says what happened, in a control block's places.
 int run_regions(mlmq_ctx *c, uint32_t nq, int32_t src, const uint32_t *sources, uint32_t *dist, uint64_t *qtime,
                 const mlmq_params &p, uint32_t relaxers, uint32_t grid, QueryClock *t) {
     const mlmq::RegionGraph &g = c->regions;
@@ -837,23 +847,33 @@ int run_regions(mlmq_ctx *c, uint32_t nq, int32_t src, const uint32_t *sources, 
     L.admit = mlmq::region_admit(g.regions, nq, grid);
     L.relaxers = relaxers;
     L.grid = grid;
+    auto *sum = reinterpret_cast<mlmq::RegionSummary *>(c->h_ctl);
+    sum->error = mlmq::kErrInternal;
+    L.counts = c->r_counts;
+    L.summary = sum;
     t->q0 = clk::now();
-    HIP_TRY(c, hipEventRecord(c->ev_reset, c->stream));
     HIP_TRY(c, mlmq::launch_region_reset(g, L, sources, (uint32_t)src, c->stream));
-    HIP_TRY(c, hipEventRecord(c->ev_start, c->stream));
     c->r_ring_dirty = true;   // until the solve has left it clean
     HIP_TRY(c, mlmq::launch_region_solver(g, L, c->stream));
-    HIP_TRY(c, hipEventRecord(c->ev_stop, c->stream));
-    HIP_TRY(c, hipMemcpyAsync(c->h_ctl, c->ctl, sizeof(uint32_t) * mlmq::kCtlWords, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     t->s1 = clk::now();
-    // one wait for both kernels: the reset's share of it from its events
-    float reset_ms = 0;
-    (void)hipEventElapsedTime(&reset_ms, c->ev_reset, c->ev_start);
-    t->q1 = t->s0 = std::min(t->s1, t->q0 + std::chrono::duration_cast<clk::duration>(
-                                              std::chrono::duration<double, std::milli>(reset_ms)));
-    std::copy(c->h_ctl, c->h_ctl + mlmq::kCtlWords, c->ctl_host.begin());
-    const int rc = query_status(c, c->ctl_host.data(), 1);
+    t->split((double)(sum->start - sum->reset) / c->wall_khz);
+    t->device_ms = (double)(sum->end - sum->start) / c->wall_khz;
+    std::vector<uint32_t> &ctl = c->ctl_host;
+    std::fill(ctl.begin(), ctl.end(), 0u);
+    ctl[mlmq::kTailOff] = nq + (uint32_t)sum->all.activations;
+    ctl[mlmq::kTakenOff] = ctl[mlmq::kDoneOff] = (uint32_t)sum->all.credits;
+    ctl[mlmq::kErrOff] = sum->error;
+    ctl[mlmq::kExitOff] = sum->over;
+    uint64_t *st = reinterpret_cast<uint64_t *>(ctl.data() + mlmq::kStatsOff);
+    st[mlmq::kStatL2Push] = sum->all.activations;
+    st[mlmq::kStatL2Pop] = sum->all.credits;
+    st[mlmq::kStatRelax] = sum->all.relaxations + sum->all.messages;
+    st[mlmq::kStatAtomic] = sum->all.messages;
+    st[mlmq::kStatImprove] = sum->all.expansions;
+    st[mlmq::kStatBatches] = sum->all.sweeps;
+    st[mlmq::kStatIdle] = sum->all.polls;
+    const int rc = query_status(c, ctl.data(), 1);
     if (rc == MLMQ_OK) c->r_ring_dirty = false;
     return rc;
 }
@@ -886,9 +906,9 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
     if (rc) return rc;
     if (!c->pp_mark) HIP_TRY(c, hipMalloc(&c->pp_mark, sizeof(uint32_t) * n));
     if (!c->pp_front) HIP_TRY(c, hipMalloc(&c->pp_front, sizeof(uint32_t) * 2 * n));
-    constexpr size_t kCountWords = mlmq::kMaxRounds + 2;   // 8-byte aligned end, then the work counters
-    static_assert(kCountWords % 2 == 0 && kCountWords + 4 <= mlmq::kCtlWords, "copied through the control block's buffer");
-    if (!c->pp_count) HIP_TRY(c, hipMalloc(&c->pp_count, sizeof(uint32_t) * (kCountWords + 4)));
+    constexpr size_t kCountWords = mlmq::kMaxRounds + 2;   // 8-byte aligned end, then the work counters and times
+    static_assert(sizeof(mlmq::PushPullSummary) <= sizeof(uint32_t) * mlmq::kCtlWords, "fits the control block's buffer");
+    if (!c->pp_count) HIP_TRY(c, hipMalloc(&c->pp_count, sizeof(uint32_t) * (kCountWords + 8)));
     mlmq::PushPullQueries Q{};
     Q.nq = 1;
     Q.max_n = (uint32_t)n;
@@ -904,40 +924,35 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
     L.front[1] = c->pp_front + n;
     L.count = c->pp_count;
     L.work = reinterpret_cast<uint64_t *>(c->pp_count + kCountWords);
+    L.time = L.work + 2;
     L.n = (uint32_t)n;
     L.bound = c->pp_count + mlmq::kMaxRounds + 1;
     L.reach = c->pp_reach;
     L.hub_degree = c->pp_hub;
     const double timeout_ms = (p.timeout_s > 0 ? p.timeout_s : 60.0) * 1e3;
     QueryClock t;
+    auto *h = reinterpret_cast<mlmq::PushPullSummary *>(c->h_ctl);
     t.q0 = clk::now();
-    HIP_TRY(c, hipEventRecord(c->ev_reset, c->stream));
     HIP_TRY(c, mlmq::launch_pushpull_reset(Q, c->stream));
-    HIP_TRY(c, hipEventRecord(c->ev_start, c->stream));
     uint32_t round = 0;
     for (; round < mlmq::kBoundedRounds; ++round) HIP_TRY(c, mlmq::launch_push(Q, round, true, c->stream));
     HIP_TRY(c, mlmq::launch_pull(Q, round, c->stream));
-    const uint32_t *h = c->h_ctl;
     for (uint32_t more = mlmq::kFullRounds;; more = 4) {
         for (uint32_t k = 0; k < more; ++k, ++round) HIP_TRY(c, mlmq::launch_push(Q, round, false, c->stream));
-        HIP_TRY(c, hipEventRecord(c->ev_stop, c->stream));
-        HIP_TRY(c, hipMemcpyAsync(c->h_ctl, c->pp_count, sizeof(uint32_t) * (kCountWords + 4), hipMemcpyDeviceToHost,
-                                  c->stream));
+        HIP_TRY(c, mlmq::launch_pushpull_summary(L, round, h, c->stream));
         HIP_TRY(c, hipStreamSynchronize(c->stream));
         t.s1 = clk::now();
         if (ms_since(t.q0, t.s1) > timeout_ms) return fail(c, MLMQ_E_TIMEOUT, "watchdog expired");
-        if (h[round] == 0) break;
+        if (h->count[round] == 0) break;
         if (round + 4 > mlmq::kMaxRounds)
             return fail(c, MLMQ_E_QUEUE_OVERFLOW, "push-pull solver: too many rounds");
     }
-    float reset_ms = 0;
-    (void)hipEventElapsedTime(&reset_ms, c->ev_reset, c->ev_start);
-    t.q1 = t.s0 = std::min(t.s1, t.q0 + std::chrono::duration_cast<clk::duration>(
-                                            std::chrono::duration<double, std::milli>(reset_ms)));
+    t.split((double)(h->time[1] - h->time[0]) / c->wall_khz);
+    t.device_ms = (double)(h->time[2] - h->time[1]) / c->wall_khz;
     // queue counts: every vertex queued in some round, all in the first bucket
     uint64_t queued = 0;
-    for (uint32_t r = 0; r < round; ++r) queued += h[r];
-    const uint64_t *work = reinterpret_cast<const uint64_t *>(h + kCountWords);
+    for (uint32_t r = 0; r < round; ++r) queued += h->count[r];
+    const uint64_t *work = h->work;
     std::vector<uint32_t> &ctl = c->ctl_host;
     std::fill(ctl.begin(), ctl.end(), 0u);
     ctl[mlmq::kTailOff] = ctl[mlmq::kTakenOff] = ctl[mlmq::kDoneOff] = (uint32_t)queued;
@@ -961,12 +976,10 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
 
 // Statistics of a batch from its device counters and the queries' clock ticks.
 void fill_batch_timing(mlmq_ctx *c, const uint32_t *h, const std::vector<uint64_t> &qt, int32_t nq, double solve_ms,
-                       const mlmq_params &p, mlmq_batch_timing *timing) {
+                       double device_ms, const mlmq_params &p, mlmq_batch_timing *timing) {
     std::memset(timing, 0, sizeof(*timing));
-    float dev_ms = 0;
-    (void)hipEventElapsedTime(&dev_ms, c->ev_start, c->ev_stop);
     timing->solve_ms = solve_ms;
-    timing->device_ms = dev_ms;
+    timing->device_ms = device_ms;
     std::vector<double> lat((size_t)nq);
     double sum = 0;
     for (int32_t i = 0; i < nq; ++i) {
@@ -1003,10 +1016,8 @@ int batch_regions(mlmq_ctx *c, int32_t nq, const mlmq_params &p, mlmq_batch_timi
     if (!timing) return MLMQ_OK;
     std::vector<uint64_t> qt(2 * (size_t)nq);
     HIP_TRY(c, hipMemcpy(qt.data(), c->b_qtime, sizeof(uint64_t) * qt.size(), hipMemcpyDeviceToHost));
-    fill_batch_timing(c, c->ctl_host.data(), qt, nq, ms_since(t.q0, t.s1), p, timing);
-    float reset_ms = 0;   // the launch counts its row reset, as the vertex queue's does
-    (void)hipEventElapsedTime(&reset_ms, c->ev_reset, c->ev_start);
-    timing->device_ms += reset_ms;
+    // (the launch counts its row reset, as the vertex queue's does)
+    fill_batch_timing(c, c->ctl_host.data(), qt, nq, ms_since(t.q0, t.s1), t.device_ms + ms_since(t.q0, t.q1), p, timing);
     timing->work_blocks = nq;
     timing->bucket_capacity = (int64_t)c->r_ring_slots;
     if (!p.batch_stats)
@@ -1520,7 +1531,9 @@ int mlmq_solve_batch(mlmq_ctx *c, const int32_t *sources, int32_t nq, const mlmq
         c->b_nq = nq;
         c->b_solved = true;
         if (timing) {
-            fill_batch_timing(c, g.data(), qt, nq, ms_since(s0, s1), p, timing);
+            float dev_ms = 0;
+            (void)hipEventElapsedTime(&dev_ms, c->ev_start, c->ev_stop);
+            fill_batch_timing(c, g.data(), qt, nq, ms_since(s0, s1), dev_ms, p, timing);
             timing->work_blocks = blocks;
             timing->graph_replay = use_graph ? 1 : 0;
             timing->bucket_capacity = (int64_t)1 << cap_log2;

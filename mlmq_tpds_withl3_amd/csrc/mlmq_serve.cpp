@@ -80,6 +80,7 @@ struct Lane {
     uint32_t *ctl = nullptr;
     uint64_t *times = nullptr;
     mlmq::RegionProgress *progress = nullptr;
+    mlmq::RegionCounts *counts = nullptr;
     uint64_t *ring = nullptr;
     uint64_t ring_slots = 0;
     bool ring_dirty = true;
@@ -942,6 +943,7 @@ int mlmq_server_create(int device, const mlmq_server_config *cfg, mlmq_server **
         if (e == hipSuccess) e = hipMalloc((void **)&l.d_tab, side);
         if (e == hipSuccess) e = hipMalloc((void **)&l.ctl, sizeof(uint32_t) * mlmq::kCtlWords);
         if (e == hipSuccess) e = hipMalloc((void **)&l.progress, sizeof(mlmq::RegionProgress) * (size_t)c.max_batch);
+        if (e == hipSuccess) e = hipMalloc((void **)&l.counts, sizeof(mlmq::RegionCounts) * mlmq::kRegionGroups);
         if (e == hipSuccess) e = hipMalloc((void **)&l.times, 2 * sizeof(uint64_t) * (size_t)c.max_batch);
     }
     if (e != hipSuccess) {
@@ -969,7 +971,7 @@ int mlmq_server_destroy(mlmq_server *s) {
         if (l.h_reqs) (void)hipHostFree(l.h_reqs);
         if (l.h_tab) (void)hipHostFree(l.h_tab);
         for (void *p : {(void *)l.d_reqs, (void *)l.d_tab, (void *)l.ctl, (void *)l.times,
-                        (void *)l.progress, (void *)l.ring})
+                        (void *)l.progress, (void *)l.counts, (void *)l.ring})
             if (p) (void)hipFree(p);
         if (l.s) (void)hipStreamDestroy(l.s);
     }
@@ -1120,7 +1122,7 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
     int few = 0, many = 0;
     HIP_TRY(s, mlmq::region_occupancy(mlmq::kFew, &few));
     HIP_TRY(s, mlmq::region_occupancy(mlmq::kMany, &many));
-    const uint32_t region_groups = (uint32_t)(std::max({few, many, 1}) * s->cus);
+    const uint32_t region_groups = std::min<uint32_t>((uint32_t)(std::max({few, many, 1}) * s->cus), mlmq::kRegionGroups);
 
     HIP_TRY(s, hipEventRecord(s->ev_ref, s->lanes[0].s));
     HIP_TRY(s, hipEventSynchronize(s->ev_ref));
@@ -1183,7 +1185,7 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
         }
         const uint32_t relaxers = mlmq::region_relaxers(nregion ? tasks / nregion : 0, nregion, (uint32_t)s->cus);
         const uint32_t region_grid =
-            (uint32_t)std::min<uint64_t>(std::max(relaxers == mlmq::kMany ? many : few, 1) * s->cus, tasks);
+            (uint32_t)std::min<uint64_t>({(uint64_t)std::max(relaxers == mlmq::kMany ? many : few, 1) * s->cus, region_groups, tasks});
         if (nregion && lane_ring(l, tasks, region_grid) != hipSuccess) {
             (void)hipGetLastError();
             for (Engine &e : l.engines)
@@ -1278,6 +1280,7 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
         }
         if (nregion) {
             R.progress = l.progress;
+            R.counts = l.counts;
             R.admit = mlmq::region_admit(tasks / nregion, nregion, region_grid);
             R.relaxers = relaxers;
             R.grid = region_grid;

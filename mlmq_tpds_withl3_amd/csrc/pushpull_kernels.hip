@@ -86,6 +86,7 @@ __global__ __launch_bounds__(kGroup) void push_kernel(PushPullLaunch one, const 
     __shared__ uint32_t s_work[2];
     const uint32_t count = L.count[round];
     if (count == 0) return;
+    if (!kTable && round == 0 && blockIdx.x == 0 && threadIdx.x == 0) L.time[1] = wall_clock64();
     const uint32_t bound = kBounded ? *L.bound : kUnreached - 1u;
     const uint32_t *in = (round & 1u ? L.front[1] : L.front[0]);
     uint32_t *out = (round & 1u ? L.front[0] : L.front[1]), *out_count = L.count + round + 1;
@@ -283,8 +284,17 @@ __global__ __launch_bounds__(256) void pushpull_reset_kernel(PushPullLaunch one,
         L.front[0][0] = src;
         L.work[0] = L.work[1] = 0;
         *L.bound = kUnreached - 1u;
-        if (kTable) L.time[0] = L.time[1] = wall_clock64();
+        L.time[0] = L.time[1] = wall_clock64();
     }
+}
+
+__global__ __launch_bounds__(256) void pushpull_summary_kernel(PushPullLaunch L, uint32_t rounds, PushPullSummary *out) {
+    for (uint32_t i = threadIdx.x; i <= rounds; i += blockDim.x) out->count[i] = L.count[i];
+    if (threadIdx.x < 2) {
+        out->work[threadIdx.x] = L.work[threadIdx.x];
+        out->time[threadIdx.x] = L.time[threadIdx.x];
+    }
+    if (threadIdx.x == 0) out->time[2] = wall_clock64();
 }
 
 __global__ __launch_bounds__(256) void symmetry_kernel(const uint32_t *row, const uint32_t *col, const uint32_t *wgt,
@@ -377,6 +387,11 @@ hipError_t launch_push(const PushPullQueries &Q, uint32_t round, bool bounded, h
     else if (Q.table) hipLaunchKernelGGL((push_kernel<true, false>), grid, group, 0, s, Q.one, Q.table, round);
     else if (bounded) hipLaunchKernelGGL((push_kernel<false, true>), grid, group, 0, s, Q.one, Q.table, round);
     else hipLaunchKernelGGL((push_kernel<false, false>), grid, group, 0, s, Q.one, Q.table, round);
+    return hipGetLastError();
+}
+
+hipError_t launch_pushpull_summary(const PushPullLaunch &L, uint32_t rounds, PushPullSummary *out, hipStream_t s) {
+    hipLaunchKernelGGL(pushpull_summary_kernel, dim3(1), dim3(256), 0, s, L, rounds, out);
     return hipGetLastError();
 }
 

@@ -31,7 +31,7 @@ struct PushPullLaunch {
     uint32_t reach;          // the bound lies this far beyond the nearest hub
     uint32_t hub_degree;
     uint32_t src;
-    uint64_t *time;          // table launches: ticks of the query's start and end
+    uint64_t *time;          // ticks: reset, and start of the first round or (tables) the end
 };
 
 // Queries of one sequence of launches: one, or a table of them.
@@ -40,6 +40,13 @@ struct PushPullQueries {
     const PushPullLaunch *table;   // nq entries in device memory (null: `one`)
     uint32_t nq;
     uint32_t max_n;                // most vertices of a query
+};
+
+// Outcome of a query, written to host memory.
+struct PushPullSummary {
+    uint64_t work[2];
+    uint64_t time[3];               // ticks: reset, first round, now
+    uint32_t count[kMaxRounds + 1];
 };
 
 // *asymmetric = 1 if some edge (u, v, w) has no edge (v, u, w).  Rows of more
@@ -54,6 +61,8 @@ uint32_t push_groups(uint32_t n);
 constexpr int kPushWaves = 4;
 // Round r expands the vertices of count[r] into those of count[r + 1].
 hipError_t launch_push(const PushPullQueries &Q, uint32_t round, bool bounded, hipStream_t s);
+// count[0 .. rounds], work and times of a single query.
+hipError_t launch_pushpull_summary(const PushPullLaunch &L, uint32_t rounds, PushPullSummary *out, hipStream_t s);
 // Adds the pulled vertices to those of count[round].
 hipError_t launch_pull(const PushPullQueries &Q, uint32_t round, hipStream_t s);
 

@@ -76,6 +76,9 @@ namespace {
 constexpr uint32_t kRingTailOff = kHungryOff;   // ring positions taken
 constexpr uint32_t kNextOff = kHeadOff + kStride;           // queries admitted
 constexpr uint32_t kFinishedOff = kHeadOff + 2 * kStride;   // queries over
+constexpr uint32_t kLeftOff = kHeadOff + 3 * kStride;       // workgroups that are done
+constexpr uint32_t kResetOff = kHeadOff + 4 * kStride;      // ticks of the reset and the
+constexpr uint32_t kStartOff = kHeadOff + 5 * kStride;      // solver's start (64 bits)
 constexpr uint32_t kWork = 1, kCounted = 2, kServed = 4, kVisited = 8, kOver = 16;
 // Quiet polls before an active region returns its credit.
 constexpr uint32_t kSettle = 2;
@@ -99,12 +102,16 @@ struct RegionArgs {
     uint32_t nq, admit;
     uint64_t *ring;
     uint32_t ring_mask;
+    RegionCounts *counts;
     uint32_t *ctl;
+    RegionSummary *summary;
     uint64_t *qtime;
     uint64_t timeout_ticks;
     uint32_t regions;
     uint32_t width;          // window of a wave's expansions
 };
+
+constexpr uint32_t kCounters = sizeof(RegionCounts) / sizeof(uint64_t);
 
 struct RegionLds {
     alignas(16) uint32_t dist[kRegionVerts];
@@ -112,6 +119,8 @@ struct RegionLds {
     uint32_t over;                     // the region is left: a wave without work returns
     uint32_t checked[kMany + 1];       // relaxers, sender
     uint32_t rec[2];                   // adopted record
+    uint32_t last;                     // this workgroup is the last one
+    unsigned long long total[kCounters];
 };
 
 __device__ __forceinline__ uint32_t sh_ld(uint32_t *p) {
@@ -300,7 +309,6 @@ struct MessageStats {
 __device__ __forceinline__ void region_raise(const RegionArgs &a, uint32_t code) {
     if (lane_id() == 0) {
         cas32(a.ctl + kErrOff, kErrNone, code);
-        st_relaxed(a.ctl + kExitOff, 1u);
     }
 }
 
@@ -436,8 +444,6 @@ __device__ __forceinline__ void return_credit(const RegionArgs &a, uint32_t quer
         uint64_t *slot = a.ring + ((ring_tail + i) & a.ring_mask);
         __hip_atomic_store(slot, kRegionExit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    wait_memory();
-    if (lane == 0) st_relaxed(a.ctl + kExitOff, 1u);
 }
 
 // Serves the adopted region until it is left or the solve is over.
@@ -567,6 +573,9 @@ __global__ __launch_bounds__(kThreads<kR>, kPerSimd<kR>) void region_solver_kern
     const uint64_t deadline = wall_clock64() + a.timeout_ticks;
     RelaxStats rs{};
     MessageStats ms{};
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        __hip_atomic_store(reinterpret_cast<uint64_t *>(a.ctl + kStartOff), (uint64_t)wall_clock64(), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
     for (;;) {
         // adopt the next ticket's region
         if (wave == kR && lane == 0) {
@@ -633,33 +642,48 @@ __global__ __launch_bounds__(kThreads<kR>, kPerSimd<kR>) void region_solver_kern
         }
         __syncthreads();
     }
-    uint64_t *stats = reinterpret_cast<uint64_t *>(a.ctl + kStatsOff);
-    if (wave < kR) {
-        const uint32_t relax = wave_sum(rs.relax);
-        if (lane == 0) {
-            add64(stats + kStatRelax, relax);
-            add64(stats + kStatImprove, rs.improve);
-            add64(stats + kStatBatches, rs.sweeps);
-        }
-    } else {
-        const uint32_t messages = wave_sum(ms.messages);
-        if (lane == 0) {
-            if (ms.credits) {
-                fetch_add(a.ctl + kTakenOff, ms.credits);
-                fetch_add(a.ctl + kDoneOff, ms.credits);
-                add64(stats + kStatL2Pop, ms.credits);
-            }
-            if (ms.activations) {
-                fetch_add(a.ctl + kTailOff, ms.activations);
-                add64(stats + kStatL2Push, ms.activations);
-            }
-            if (messages) {
-                add64(stats + kStatAtomic, messages);
-                add64(stats + kStatRelax, messages);
-            }
-            if (ms.polls) add64(stats + kStatIdle, ms.polls);
-        }
+    // What the workgroup did goes to its own entry; whoever is last adds them up
+    // (a thousand workgroups that add to the same words take tens of us).
+    if (threadIdx.x < kCounters) S.total[threadIdx.x] = 0;
+    __syncthreads();
+    const uint32_t mine[kCounters] = {ms.credits, ms.activations, ms.messages, ms.polls, rs.relax, 0, 0, 0};
+#pragma unroll
+    for (uint32_t k = 0; k < kCounters; ++k)
+        if (mine[k]) atomicAdd(&S.total[k], (unsigned long long)mine[k]);
+    if (wave < kR && lane == 0) {
+        atomicAdd(&S.total[5], (unsigned long long)rs.improve);
+        atomicAdd(&S.total[6], (unsigned long long)rs.sweeps);
     }
+    __syncthreads();
+    auto *entry = reinterpret_cast<uint64_t *>(a.counts + blockIdx.x);
+    if (wave == 0) {
+        if (lane < kCounters)
+            __hip_atomic_store(entry + lane, (uint64_t)S.total[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        wait_memory();
+        if (lane == 0) S.last = fetch_add(a.ctl + kLeftOff, 1u) == gridDim.x - 1 ? 1u : 0u;
+        if (lane < kCounters) S.total[lane] = 0;
+    }
+    __syncthreads();
+    if (!S.last) return;
+    for (uint32_t i = threadIdx.x; i < gridDim.x * kCounters; i += kThreads<kR>) {
+        const uint64_t x = __hip_atomic_load(reinterpret_cast<uint64_t *>(a.counts) + i, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+        if (x) atomicAdd(&S.total[i % kCounters], (unsigned long long)x);
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    RegionSummary out;
+    out.all = {S.total[0], S.total[1], S.total[2], S.total[3], S.total[4], S.total[5], S.total[6], 0};
+    out.reset = *reinterpret_cast<uint64_t *>(a.ctl + kResetOff);
+    out.start = __hip_atomic_load(reinterpret_cast<uint64_t *>(a.ctl + kStartOff), __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+    out.error = ld_relaxed(a.ctl + kErrOff);
+    out.over = ld_relaxed(a.ctl + kFinishedOff) == a.nq ? 1u : 0u;
+    a.ctl[kTailOff] = a.nq + (uint32_t)out.all.activations;
+    a.ctl[kTakenOff] = a.ctl[kDoneOff] = (uint32_t)out.all.credits;
+    a.ctl[kExitOff] = out.over;
+    out.end = wall_clock64();
+    if (a.summary) *a.summary = out;
 }
 
 // ---- reset ----
@@ -703,7 +727,10 @@ __global__ __launch_bounds__(256) void region_reset_kernel(RegionArgs a, uint32_
         }
     }
     if (blockIdx.y == 0)
-        for (uint32_t i = t0; i < kCtlWords; i += stride) a.ctl[i] = i == kTailOff ? a.nq : i == kRingTailOff || i == kNextOff ? a.admit : 0u;
+        for (uint32_t i = t0; i < kCtlWords; i += stride) {
+            if (i == kResetOff) *reinterpret_cast<uint64_t *>(a.ctl + i) = wall_clock64();
+            else if (i != kResetOff + 1) a.ctl[i] = i == kRingTailOff || i == kNextOff ? a.admit : 0u;
+        }
 }
 
 // ---- building ----
@@ -792,7 +819,9 @@ RegionArgs make_region_args(const RegionGraph &g, const RegionLaunch &L) {
     a.admit = L.admit;
     a.ring = L.ring;
     a.ring_mask = L.ring_mask;
+    a.counts = L.counts;
     a.ctl = L.ctl;
+    a.summary = L.summary;
     a.qtime = L.qtime;
     a.timeout_ticks = L.timeout_ticks;
     a.regions = g.regions;

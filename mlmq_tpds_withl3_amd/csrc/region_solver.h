@@ -47,6 +47,19 @@ struct RegionProgress {
     uint32_t pad;
 };
 
+// What a workgroup did; after a solve, what all did.
+struct RegionCounts {
+    uint64_t credits, activations, messages, polls, relaxations, expansions, sweeps, pad;
+};
+constexpr uint32_t kRegionGroups = 4096;   // most workgroups of a launch
+
+// Outcome of a solve, written by its last workgroup.
+struct RegionSummary {
+    RegionCounts all;
+    uint64_t reset, start, end;   // wall-clock ticks
+    uint32_t error, over;         // device error; 1: every query is over
+};
+
 struct RegionLaunch {
     RegionQuerySpace space;      // nq queries on one graph, or
     const RegionQuery *table;    // nq entries in device memory (null: `space`)
@@ -54,7 +67,9 @@ struct RegionLaunch {
     RegionProgress *progress;    // nq entries
     uint64_t *ring;
     uint32_t ring_mask;
+    RegionCounts *counts;        // grid entries
     uint32_t *ctl;               // control block (device_common.h)
+    RegionSummary *summary;      // optional, may be host memory
     uint64_t *qtime;             // optional: per query, wall-clock ticks of its start and end
     uint64_t timeout_ticks;
     uint32_t nq;
