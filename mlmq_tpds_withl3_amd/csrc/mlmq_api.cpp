@@ -906,9 +906,10 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
     if (rc) return rc;
     if (!c->pp_mark) HIP_TRY(c, hipMalloc(&c->pp_mark, sizeof(uint32_t) * n));
     if (!c->pp_front) HIP_TRY(c, hipMalloc(&c->pp_front, sizeof(uint32_t) * 2 * n));
-    constexpr size_t kCountWords = mlmq::kMaxRounds + 2;   // 8-byte aligned end, then the work counters and times
+    constexpr size_t kCountWords = mlmq::kMaxRounds + 2;   // 8-byte aligned end, then the times and the work
     static_assert(sizeof(mlmq::PushPullSummary) <= sizeof(uint32_t) * mlmq::kCtlWords, "fits the control block's buffer");
-    if (!c->pp_count) HIP_TRY(c, hipMalloc(&c->pp_count, sizeof(uint32_t) * (kCountWords + 8)));
+    if (!c->pp_count)
+        HIP_TRY(c, hipMalloc(&c->pp_count, sizeof(uint32_t) * (kCountWords + 4) + sizeof(mlmq::PushPullWork) * mlmq::kWorkEntries));
     mlmq::PushPullQueries Q{};
     Q.nq = 1;
     Q.max_n = (uint32_t)n;
@@ -923,8 +924,8 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
     L.front[0] = c->pp_front;
     L.front[1] = c->pp_front + n;
     L.count = c->pp_count;
-    L.work = reinterpret_cast<uint64_t *>(c->pp_count + kCountWords);
-    L.time = L.work + 2;
+    L.time = reinterpret_cast<uint64_t *>(c->pp_count + kCountWords);
+    L.work = reinterpret_cast<mlmq::PushPullWork *>(L.time + 2);
     L.n = (uint32_t)n;
     L.bound = c->pp_count + mlmq::kMaxRounds + 1;
     L.reach = c->pp_reach;
@@ -952,7 +953,6 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
     // queue counts: every vertex queued in some round, all in the first bucket
     uint64_t queued = 0;
     for (uint32_t r = 0; r < round; ++r) queued += h->count[r];
-    const uint64_t *work = h->work;
     std::vector<uint32_t> &ctl = c->ctl_host;
     std::fill(ctl.begin(), ctl.end(), 0u);
     ctl[mlmq::kTailOff] = ctl[mlmq::kTakenOff] = ctl[mlmq::kDoneOff] = (uint32_t)queued;
@@ -960,8 +960,8 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
     uint64_t *st = reinterpret_cast<uint64_t *>(ctl.data() + mlmq::kStatsOff);
     st[mlmq::kStatL2Push] = queued - 1;   // without the source, as the kernels count
     st[mlmq::kStatL2Pop] = queued;
-    st[mlmq::kStatRelax] = st[mlmq::kStatAtomic] = work[0];
-    st[mlmq::kStatImprove] = work[1];
+    st[mlmq::kStatRelax] = st[mlmq::kStatAtomic] = h->work.edges;
+    st[mlmq::kStatImprove] = h->work.improved;
     st[mlmq::kStatBatches] = round;
     c->solved = true;
     c->last_buckets = (uint32_t)p.buckets;

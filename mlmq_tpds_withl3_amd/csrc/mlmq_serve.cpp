@@ -358,14 +358,13 @@ Engine engine_of(const GraphEntry &g, uint64_t slot_bytes) {
         const uint64_t words = (uint64_t)g.v.regions.inbox_slots + 1 + g.v.regions.regions;
         return !g.p.light_split && sizeof(uint32_t) * words <= room ? Engine::kRegions : Engine::kQueue;
     }
-    const uint64_t words = 3ull * (uint64_t)g.v.n + mlmq::kMaxRounds + 2 + 4;
+    const uint64_t words = 3ull * (uint64_t)g.v.n + mlmq::kMaxRounds + 2;
     return g.v.pp_reach && sizeof(uint32_t) * words <= room ? Engine::kPushPull : Engine::kQueue;
 }
 
 // A push-pull query whose state lies in `part`.
 mlmq::PushPullLaunch pushpull_query(const GraphEntry &g, uint32_t src, uint32_t *dist, uint8_t *part, uint64_t *time) {
     constexpr uint32_t kCountWords = mlmq::kMaxRounds + 2;
-    static_assert(kCountWords % 2 == 0, "the work counters behind the counts are 64-bit");
     mlmq::PushPullLaunch L{};
     L.col = g.v.col;
     L.wgt = g.v.wgt;
@@ -375,8 +374,7 @@ mlmq::PushPullLaunch pushpull_query(const GraphEntry &g, uint32_t src, uint32_t 
     L.dist = dist;
     L.count = (uint32_t *)part;
     L.bound = L.count + mlmq::kMaxRounds + 1;
-    L.work = (uint64_t *)(L.count + kCountWords);
-    L.mark = L.count + kCountWords + 4;
+    L.mark = L.count + kCountWords;
     L.front[0] = L.mark + L.n;
     L.front[1] = L.front[0] + L.n;
     L.reach = g.v.pp_reach;

@@ -32,8 +32,8 @@ namespace mlmq {
 
 namespace {
 
-constexpr uint32_t kGroup = 256;        // threads of a workgroup
-constexpr uint32_t kBuffer = 2048;      // queued vertices a workgroup gathers
+constexpr uint32_t kGroup = 512;        // threads of a workgroup
+constexpr uint32_t kBuffer = 4096;      // queued vertices a workgroup gathers
 constexpr uint32_t kUnroll = 4;
 
 struct OutBuffer {
@@ -58,13 +58,52 @@ __device__ __forceinline__ void flush_buffer(OutBuffer &B, uint32_t *out, uint32
     __syncthreads();
 }
 
-// Lower v to nd; queue it once a round when that succeeds.
-__device__ __forceinline__ bool lower(const PushPullLaunch &L, OutBuffer &B, uint32_t *out, uint32_t *count,
-                                      uint32_t round, uint32_t v, uint32_t nd) {
-    if (fetch_min(L.dist + v, nd) <= nd) return false;
-    if (__hip_atomic_exchange(L.mark + v, round + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != round + 1u)
-        queue_vertex(B, out, count, v);
-    return true;
+// All threads of the workgroup: adds to its entry (thousands of workgroups that
+// add to the same two words take longer than most rounds' work).
+__device__ __forceinline__ void count_work(const PushPullLaunch &L, uint32_t *s_work, uint32_t edges, uint32_t improved) {
+    if (!L.work) return;
+    edges = wave_sum(edges);
+    improved = wave_sum(improved);
+    if (lane_id() == 0) {
+        atomicAdd(&s_work[0], edges);
+        atomicAdd(&s_work[1], improved);
+    }
+    __syncthreads();
+    if (threadIdx.x != 0 || s_work[0] == 0) return;
+    L.work[blockIdx.x].edges += s_work[0];
+    L.work[blockIdx.x].improved += s_work[1];
+}
+
+// Lower v[k] to nd[k] where it was above nd[k]; queue each vertex once a round
+// when that succeeds.  All k are under way at once: one after another (two
+// dependent atomics of about 1.5 us each) they were most of a round's time.
+// Returns how many fell.
+template <uint32_t kN>
+__device__ __forceinline__ uint32_t lower(const PushPullLaunch &L, OutBuffer &B, uint32_t *out, uint32_t *count,
+                                          uint32_t round, uint32_t bound, const uint32_t (&v)[kN],
+                                          const uint32_t (&nd)[kN], const uint32_t (&was)[kN]) {
+    uint32_t old[kN], seen[kN], fell = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kN; ++k) {
+        old[k] = 0;
+        if (nd[k] < was[k] && nd[k] <= bound) old[k] = fetch_min(L.dist + v[k], nd[k]);
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kN; ++k) asm volatile("" : "+v"(old[k]));
+#pragma unroll
+    for (uint32_t k = 0; k < kN; ++k) {
+        seen[k] = round + 1u;
+        if (old[k] > nd[k]) {
+            seen[k] = __hip_atomic_exchange(L.mark + v[k], round + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ++fell;
+        }
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kN; ++k) asm volatile("" : "+v"(seen[k]));
+#pragma unroll
+    for (uint32_t k = 0; k < kN; ++k)
+        if (seen[k] != round + 1u) queue_vertex(B, out, count, v[k]);
+    return fell;
 }
 
 // This workgroup's query.
@@ -91,6 +130,9 @@ __global__ __launch_bounds__(kGroup) void push_kernel(PushPullLaunch one, const 
     const uint32_t *in = (round & 1u ? L.front[1] : L.front[0]);
     uint32_t *out = (round & 1u ? L.front[0] : L.front[1]), *out_count = L.count + round + 1;
     const uint32_t share = min(kGroup, (count + gridDim.x - 1) / gridDim.x);
+    if (blockIdx.x * share >= count) return;
+    // half of the places that are searched for an edge's vertex
+    const uint32_t half = share > 1 ? 1u << (31 - __builtin_clz(share - 1)) : 0u;
     if (threadIdx.x == 0) {
         B.n = 0;
         s_work[0] = s_work[1] = 0;
@@ -100,26 +142,27 @@ __global__ __launch_bounds__(kGroup) void push_kernel(PushPullLaunch one, const 
         const bool have = threadIdx.x < share && b + threadIdx.x < count;
         uint32_t len = 0, start = 0, d = 0;
         __syncthreads();
+        // (loads without conditions: under one each they would wait for the last)
+        const uint32_t v = in[have ? b + threadIdx.x : b];
+        const uint4 *p = L.blocks + 4ull * v;
+        const uint4 q0 = p[0], q1 = p[1], q2 = p[2], q3 = p[3];
+        d = L.dist[v];
         if (have) {
-            const uint32_t v = in[b + threadIdx.x];
-            const uint4 *p = L.blocks + 4ull * v;
-            const uint4 q0 = p[0], q1 = p[1], q2 = p[2], q3 = p[3];
-            d = L.dist[v];
             if (d > bound) {
                 // beyond the bound by now: phase 3 pushes it
             } else if (q0.x <= kInlineEdges) {
                 const uint32_t word[14] = {q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x,
                                            q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
-                uint32_t was[kInlineEdges];
-#pragma unroll
-                for (uint32_t k = 0; k < kInlineEdges; ++k)
-                    was[k] = k < q0.x ? L.dist[word[2 * k] & L.id_mask] : 0u;
+                uint32_t to[kInlineEdges], nd[kInlineEdges], was[kInlineEdges];
 #pragma unroll
                 for (uint32_t k = 0; k < kInlineEdges; ++k) {
-                    const uint32_t nd = d + word[2 * k + 1];
-                    if (nd < was[k] && nd <= bound)
-                        improved += lower(L, B, out, out_count, round, word[2 * k] & L.id_mask, nd) ? 1u : 0u;
+                    to[k] = word[2 * k] & L.id_mask;
+                    nd[k] = d + word[2 * k + 1];
+                    was[k] = L.dist[k < q0.x ? to[k] : v];
                 }
+#pragma unroll
+                for (uint32_t k = 0; k < kInlineEdges; ++k) was[k] = k < q0.x ? was[k] : 0u;
+                improved += lower(L, B, out, out_count, round, bound, to, nd, was);
                 edges += q0.x;
             } else {
                 start = q0.y;
@@ -158,37 +201,33 @@ __global__ __launch_bounds__(kGroup) void push_kernel(PushPullLaunch one, const 
         if (threadIdx.x == 0) s_first[kGroup] = total;
         __syncthreads();
         edges += threadIdx.x == 0 ? total : 0u;
-        for (uint32_t e0 = threadIdx.x; e0 < total; e0 += kUnroll * kGroup) {
-            uint32_t c[kUnroll], nd[kUnroll], was[kUnroll];
+        for (uint32_t e0 = 0; e0 < total; e0 += kUnroll * kGroup) {
+            uint32_t at[kUnroll], c[kUnroll], nd[kUnroll], was[kUnroll];
 #pragma unroll
             for (uint32_t j = 0; j < kUnroll; ++j) {
-                const uint32_t e = e0 + j * kGroup;
+                at[j] = 0;
+                nd[j] = kUnreached;
+                if (e0 + j * kGroup >= total) continue;   // (uniform)
+                const uint32_t e = e0 + j * kGroup + threadIdx.x;
                 // the last vertex whose first edge is <= e
                 uint32_t lo = 0;
-#pragma unroll
-                for (uint32_t k = kGroup / 2; k; k /= 2)
+                for (uint32_t k = half; k; k /= 2)
                     if (s_first[lo + k] <= e) lo += k;
-                const uint32_t at = e < total ? s_start[lo] + (e - s_first[lo]) : s_start[lo];
-                c[j] = L.col[at];
-                nd[j] = e < total ? s_dist[lo] + L.wgt[at] : kUnreached;
+                at[j] = e < total ? s_start[lo] + (e - s_first[lo]) : s_start[lo];
+                nd[j] = e < total ? s_dist[lo] : kUnreached;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < kUnroll; ++j) {
+                c[j] = L.col[at[j]];
+                nd[j] = min(nd[j] + L.wgt[at[j]], kUnreached);   // (no edge: not below any distance)
             }
 #pragma unroll
             for (uint32_t j = 0; j < kUnroll; ++j) was[j] = L.dist[c[j]];
-#pragma unroll
-            for (uint32_t j = 0; j < kUnroll; ++j)
-                if (nd[j] < was[j] && nd[j] <= bound)
-                    improved += lower(L, B, out, out_count, round, c[j], nd[j]) ? 1u : 0u;
+            improved += lower(L, B, out, out_count, round, bound, c, nd, was);
         }
     }
     flush_buffer(B, out, out_count);
-    edges = wave_sum(edges);
-    improved = wave_sum(improved);
-    if (lane_id() == 0) {
-        atomicAdd(&s_work[0], edges);
-        atomicAdd(&s_work[1], improved);
-    }
-    __syncthreads();
-    if (threadIdx.x < 2 && s_work[threadIdx.x]) add64(L.work + threadIdx.x, s_work[threadIdx.x]);
+    count_work(L, s_work, edges, improved);
     // (its last round's other workgroups end at about the same time)
     if (kTable && blockIdx.x == 0 && threadIdx.x == 0) L.time[1] = wall_clock64();
 }
@@ -223,11 +262,10 @@ __global__ __launch_bounds__(kGroup) void pull_kernel(PushPullLaunch one, const 
                                            q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
                 uint32_t from[kInlineEdges];
 #pragma unroll
-                for (uint32_t k = 0; k < kInlineEdges; ++k)
-                    from[k] = k < q0.x ? L.dist[word[2 * k] & L.id_mask] : kUnreached;
+                for (uint32_t k = 0; k < kInlineEdges; ++k) from[k] = L.dist[k < q0.x ? word[2 * k] & L.id_mask : v];
 #pragma unroll
                 for (uint32_t k = 0; k < kInlineEdges; ++k)
-                    if (from[k] < kUnreached) best = min(best, from[k] + word[2 * k + 1]);
+                    if (k < q0.x && from[k] < kUnreached) best = min(best, from[k] + word[2 * k + 1]);
                 edges += q0.x;
             }
         }
@@ -260,14 +298,7 @@ __global__ __launch_bounds__(kGroup) void pull_kernel(PushPullLaunch one, const 
         }
     }
     flush_buffer(B, out, out_count);
-    edges = wave_sum(edges);
-    improved = wave_sum(improved);
-    if (lane_id() == 0) {
-        atomicAdd(&s_work[0], edges);
-        atomicAdd(&s_work[1], improved);
-    }
-    __syncthreads();
-    if (threadIdx.x < 2 && s_work[threadIdx.x]) add64(L.work + threadIdx.x, s_work[threadIdx.x]);
+    count_work(L, s_work, edges, improved);
 }
 
 template <bool kTable>
@@ -280,9 +311,10 @@ __global__ __launch_bounds__(256) void pushpull_reset_kernel(PushPullLaunch one,
         L.mark[i] = 0;
     }
     for (uint32_t i = t; i <= kMaxRounds; i += stride) L.count[i] = i == 0 ? 1u : 0u;
+    if (L.work)
+        for (uint32_t i = t; i < kWorkEntries; i += stride) L.work[i] = PushPullWork{0, 0};
     if (t == 0) {
         L.front[0][0] = src;
-        L.work[0] = L.work[1] = 0;
         *L.bound = kUnreached - 1u;
         L.time[0] = L.time[1] = wall_clock64();
     }
@@ -290,10 +322,19 @@ __global__ __launch_bounds__(256) void pushpull_reset_kernel(PushPullLaunch one,
 
 __global__ __launch_bounds__(256) void pushpull_summary_kernel(PushPullLaunch L, uint32_t rounds, PushPullSummary *out) {
     for (uint32_t i = threadIdx.x; i <= rounds; i += blockDim.x) out->count[i] = L.count[i];
-    if (threadIdx.x < 2) {
-        out->work[threadIdx.x] = L.work[threadIdx.x];
-        out->time[threadIdx.x] = L.time[threadIdx.x];
+    __shared__ unsigned long long s_edges, s_improved;
+    if (threadIdx.x == 0) s_edges = s_improved = 0;
+    __syncthreads();
+    uint64_t edges = 0, improved = 0;
+    for (uint32_t i = threadIdx.x; i < kWorkEntries; i += blockDim.x) {
+        edges += L.work[i].edges;
+        improved += L.work[i].improved;
     }
+    if (edges) atomicAdd(&s_edges, (unsigned long long)edges);
+    if (improved) atomicAdd(&s_improved, (unsigned long long)improved);
+    __syncthreads();
+    if (threadIdx.x < 2) out->time[threadIdx.x] = L.time[threadIdx.x];
+    if (threadIdx.x == 0) out->work = PushPullWork{s_edges, s_improved};
     if (threadIdx.x == 0) out->time[2] = wall_clock64();
 }
 
@@ -374,13 +415,21 @@ hipError_t launch_pushpull_reset(const PushPullQueries &Q, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Eight workgroups per CU hold their out buffers in LDS at once; a graph of
-// few vertices never fills them.
-uint32_t push_groups(uint32_t n) { return groups_for((uint64_t)n * 8, 2048); }
+// A workgroup reserves its places in the next round's list by one atomic, and
+// those of all workgroups, on the one word, take about 15 ns each: with 2048
+// workgroups of 256 threads some waited 30 us of a 35 us round of RMAT-18.  So
+// the workgroups are few and large; four per CU where a round has enough work
+// for them (us, RMAT-18 / 20 / 22: 2048 of 256 358 / 626 / 1119, 1024 of 512
+// 304 / 537 / 1089, 512 of 512 280 / 557 / 1114, 512 of 1024 314 / 559 / 1131).
+// A graph of few vertices never fills two per CU.
+uint32_t push_groups(uint32_t n) {
+    const uint32_t most = n / 1024 < 512 ? 512 : n / 1024 < 1024 ? n / 1024 : 1024;
+    return groups_for((uint64_t)n * 8, most);
+}
 
 hipError_t launch_push(const PushPullQueries &Q, uint32_t round, bool bounded, hipStream_t s) {
     // several queries share the device, but a round of one may be most of the work
-    const uint32_t share = 2048 / Q.nq > 256 ? 2048 / Q.nq : 256;
+    const uint32_t share = 1024 / Q.nq > 128 ? 1024 / Q.nq : 128;
     const uint32_t x = push_groups(Q.max_n);
     const dim3 grid(x < share ? x : share, Q.nq), group(kGroup);
     if (Q.table && bounded) hipLaunchKernelGGL((push_kernel<true, true>), grid, group, 0, s, Q.one, Q.table, round);
@@ -396,7 +445,7 @@ hipError_t launch_pushpull_summary(const PushPullLaunch &L, uint32_t rounds, Pus
 }
 
 hipError_t launch_pull(const PushPullQueries &Q, uint32_t round, hipStream_t s) {
-    const dim3 grid(groups_for(Q.max_n, 4096), Q.nq), group(kGroup);
+    const dim3 grid(groups_for(Q.max_n, 2048), Q.nq), group(kGroup);
     if (Q.table) hipLaunchKernelGGL(pull_kernel<true>, grid, group, 0, s, Q.one, Q.table, round);
     else hipLaunchKernelGGL(pull_kernel<false>, grid, group, 0, s, Q.one, Q.table, round);
     return hipGetLastError();

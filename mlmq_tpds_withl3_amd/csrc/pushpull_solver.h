@@ -16,6 +16,12 @@ constexpr uint32_t kBoundedRounds = 12;
 constexpr uint32_t kFullRounds = 5;
 constexpr uint32_t kMaxRounds = 1024;   // counters per query
 
+// Edges examined and improvements of all rounds by the workgroups of one index.
+struct PushPullWork {
+    uint64_t edges, improved;
+};
+constexpr uint32_t kWorkEntries = 4096;   // most workgroups of a launch
+
 struct PushPullLaunch {
     const uint32_t *col;
     const uint32_t *wgt;
@@ -25,7 +31,7 @@ struct PushPullLaunch {
     uint32_t *mark;          // n: last round that queued the vertex
     uint32_t *front[2];      // n each: the rounds' vertices, by parity
     uint32_t *count;         // kMaxRounds + 1: vertices of each round
-    uint64_t *work;          // edges examined, improvements
+    PushPullWork *work;      // a workgroup's share each (null: not counted)
     uint32_t *bound;         // distance up to which phase 1 settles
     uint32_t n;
     uint32_t reach;          // the bound lies this far beyond the nearest hub
@@ -44,7 +50,7 @@ struct PushPullQueries {
 
 // Outcome of a query, written to host memory.
 struct PushPullSummary {
-    uint64_t work[2];
+    PushPullWork work;
     uint64_t time[3];               // ticks: reset, first round, now
     uint32_t count[kMaxRounds + 1];
 };
@@ -58,7 +64,7 @@ hipError_t launch_bound_counts(const uint32_t *row, const uint32_t *wgt, uint32_
 hipError_t launch_pushpull_reset(const PushPullQueries &Q, hipStream_t s);
 // Workgroups of a push launch of one query, and waves of each.
 uint32_t push_groups(uint32_t n);
-constexpr int kPushWaves = 4;
+constexpr int kPushWaves = 8;
 // Round r expands the vertices of count[r] into those of count[r + 1].
 hipError_t launch_push(const PushPullQueries &Q, uint32_t round, bool bounded, hipStream_t s);
 // count[0 .. rounds], work and times of a single query.

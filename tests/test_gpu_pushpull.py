@@ -3,7 +3,7 @@ the oracle, bit for bit: degrees around the hop block's seven edges and the
 wave's and workgroup's widths, zero, equal and very large weights, separate
 parts, a tail of more rounds than the solver launches blindly, a tail longer
 than it is meant for (the vertex queue answers), and directed graphs (never
-taken).  It reports four waves per workgroup.  Tolerance: none, distances are
+taken).  It reports eight waves per workgroup.  Tolerance: none, distances are
 whole numbers."""
 import sys
 
@@ -60,7 +60,7 @@ def check(solver, graph, sources, taken, **params):
         ref, _, _ = O.dijkstra(row, col, w, int(src))
         bad = np.flatnonzero(solver.dist() != ref)
         assert bad.size == 0, f"source {src}: {bad.size} mismatches, first v={bad[0]}"
-        assert (t["waves"] == 4 * t["work_blocks"]) == taken
+        assert (t["waves"] == 8 * t["work_blocks"]) == taken
         q = solver.queue_counts()
         assert q["writes"] == q["reads"] and sum(q["writes"]) == q["completed"] == t["l2_pushes"]
 
