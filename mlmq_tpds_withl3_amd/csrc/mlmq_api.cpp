@@ -306,7 +306,7 @@ int build_pushpull(mlmq_ctx *c, const int32_t *w) {
     HIP_TRY(c, hipMalloc(&flag, sizeof(uint32_t)));
     hipError_t e = mlmq::launch_fill_u32(flag, 1, 0u, c->stream);
     if (e == hipSuccess)
-        e = mlmq::launch_symmetry_check(c->row, c->col, c->wgt, (uint32_t)c->n, flag, c->stream);
+        e = mlmq::launch_symmetry_check(c->row, c->col, c->wgt, (uint32_t)c->n, (uint64_t)c->m, flag, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(&bad, flag, sizeof(bad), hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     (void)hipFree(flag);

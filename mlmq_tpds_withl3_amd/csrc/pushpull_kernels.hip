@@ -320,13 +320,14 @@ __global__ __launch_bounds__(256) void pushpull_reset_kernel(PushPullLaunch one,
     }
 }
 
-__global__ __launch_bounds__(256) void pushpull_summary_kernel(PushPullLaunch L, uint32_t rounds, PushPullSummary *out) {
+__global__ __launch_bounds__(1024) void pushpull_summary_kernel(PushPullLaunch L, uint32_t groups, uint32_t rounds,
+                                                                PushPullSummary *out) {
     for (uint32_t i = threadIdx.x; i <= rounds; i += blockDim.x) out->count[i] = L.count[i];
     __shared__ unsigned long long s_edges, s_improved;
     if (threadIdx.x == 0) s_edges = s_improved = 0;
     __syncthreads();
     uint64_t edges = 0, improved = 0;
-    for (uint32_t i = threadIdx.x; i < kWorkEntries; i += blockDim.x) {
+    for (uint32_t i = threadIdx.x; i < groups; i += blockDim.x) {
         edges += L.work[i].edges;
         improved += L.work[i].improved;
     }
@@ -338,31 +339,49 @@ __global__ __launch_bounds__(256) void pushpull_summary_kernel(PushPullLaunch L,
     if (threadIdx.x == 0) out->time[2] = wall_clock64();
 }
 
+// A workgroup checks kSymEdges consecutive edges, whoever's they are: with a
+// wave per vertex the largest hub of RMAT-22 took 0.3 s.
+constexpr uint32_t kSymEdges = 4096;
 __global__ __launch_bounds__(256) void symmetry_kernel(const uint32_t *row, const uint32_t *col, const uint32_t *wgt,
                                                        uint32_t n, uint32_t *asymmetric) {
-    // a wave per vertex, an edge per lane
-    const uint32_t waves = gridDim.x * blockDim.x / kWave;
-    for (uint32_t u = (blockIdx.x * blockDim.x + threadIdx.x) / kWave; u < n; u += waves) {
-        const uint32_t lo = row[u], hi = row[u + 1];
-        bool bad = false;
-        for (uint32_t e = lo + lane_id(); e < hi; e += kWave) {
-            const uint32_t v = col[e], w = wgt[e];
-            uint32_t a = row[v], b = row[v + 1];
-            bool found = false;
-            if (b - a > kInlineEdges) {
-                while (a < b) {   // first entry >= (w, u)
-                    const uint32_t m = a + (b - a) / 2, mw = wgt[m];
-                    if (mw < w || (mw == w && col[m] < u)) a = m + 1;
-                    else b = m;
-                }
-                found = a < row[v + 1] && wgt[a] == w && col[a] == u;
-            } else {
-                for (; a < b; ++a) found = found || (wgt[a] == w && col[a] == u);
-            }
-            bad = bad || !found;
+    const uint64_t first = (uint64_t)blockIdx.x * kSymEdges;
+    const uint32_t m = row[n], end = (uint32_t)min((uint64_t)m, first + kSymEdges);
+    // the vertices of the first and the last edge: the last with row[u] <= e
+    uint32_t range[2];
+    for (uint32_t i = 0; i < 2; ++i) {
+        const uint32_t e = i ? end - 1u : (uint32_t)first;
+        uint32_t lo = 0, hi = n;
+        while (hi - lo > 1) {
+            const uint32_t mid = lo + (hi - lo) / 2;
+            if (row[mid] <= e) lo = mid;
+            else hi = mid;
         }
-        if (ballot(bad) && lane_id() == 0) *asymmetric = 1;
+        range[i] = lo;
     }
+    bool bad = false;
+    for (uint32_t e = (uint32_t)first + threadIdx.x; e < end; e += blockDim.x) {
+        uint32_t u = range[0], hi = range[1] + 1u;
+        while (hi - u > 1) {
+            const uint32_t mid = u + (hi - u) / 2;
+            if (row[mid] <= e) u = mid;
+            else hi = mid;
+        }
+        const uint32_t v = col[e], w = wgt[e], top = row[v + 1];
+        uint32_t a = row[v], b = top;
+        bool found = false;
+        if (b - a > kInlineEdges) {
+            while (a < b) {   // first entry >= (w, u)
+                const uint32_t mid = a + (b - a) / 2, mw = wgt[mid];
+                if (mw < w || (mw == w && col[mid] < u)) a = mid + 1;
+                else b = mid;
+            }
+            found = a < top && wgt[a] == w && col[a] == u;
+        } else {
+            for (; a < b; ++a) found = found || (wgt[a] == w && col[a] == u);
+        }
+        bad = bad || !found;
+    }
+    if (ballot(bad) && lane_id() == 0) *asymmetric = 1;
 }
 
 __global__ __launch_bounds__(256) void bound_count_kernel(const uint32_t *row, const uint32_t *wgt, uint32_t n,
@@ -395,10 +414,11 @@ uint32_t groups_for(uint64_t items, uint32_t most) {
 
 }  // namespace
 
-hipError_t launch_symmetry_check(const uint32_t *row, const uint32_t *col, const uint32_t *wgt, uint32_t n,
+hipError_t launch_symmetry_check(const uint32_t *row, const uint32_t *col, const uint32_t *wgt, uint32_t n, uint64_t m,
                                  uint32_t *asymmetric, hipStream_t s) {
-    hipLaunchKernelGGL(symmetry_kernel, dim3(groups_for((uint64_t)n * kWave, 16384)), dim3(256), 0, s, row, col, wgt,
-                       n, asymmetric);
+    if (m == 0) return hipSuccess;
+    hipLaunchKernelGGL(symmetry_kernel, dim3((uint32_t)((m + kSymEdges - 1) / kSymEdges)), dim3(256), 0, s, row, col,
+                       wgt, n, asymmetric);
     return hipGetLastError();
 }
 
@@ -440,7 +460,9 @@ hipError_t launch_push(const PushPullQueries &Q, uint32_t round, bool bounded, h
 }
 
 hipError_t launch_pushpull_summary(const PushPullLaunch &L, uint32_t rounds, PushPullSummary *out, hipStream_t s) {
-    hipLaunchKernelGGL(pushpull_summary_kernel, dim3(1), dim3(256), 0, s, L, rounds, out);
+    const uint32_t pushes = push_groups(L.n), pulls = groups_for(L.n, 2048);
+    const uint32_t groups = pushes > pulls ? pushes : pulls;   // entries in use
+    hipLaunchKernelGGL(pushpull_summary_kernel, dim3(1), dim3(1024), 0, s, L, groups, rounds, out);
     return hipGetLastError();
 }
 

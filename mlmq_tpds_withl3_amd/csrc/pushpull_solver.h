@@ -20,7 +20,7 @@ constexpr uint32_t kMaxRounds = 1024;   // counters per query
 struct PushPullWork {
     uint64_t edges, improved;
 };
-constexpr uint32_t kWorkEntries = 4096;   // most workgroups of a launch
+constexpr uint32_t kWorkEntries = 2048;   // most workgroups of a launch
 
 struct PushPullLaunch {
     const uint32_t *col;
@@ -57,7 +57,7 @@ struct PushPullSummary {
 
 // *asymmetric = 1 if some edge (u, v, w) has no edge (v, u, w).  Rows of more
 // than kInlineEdges edges are sorted by (weight, destination).
-hipError_t launch_symmetry_check(const uint32_t *row, const uint32_t *col, const uint32_t *wgt, uint32_t n,
+hipError_t launch_symmetry_check(const uint32_t *row, const uint32_t *col, const uint32_t *wgt, uint32_t n, uint64_t m,
                                  uint32_t *asymmetric, hipStream_t s);
 hipError_t launch_bound_counts(const uint32_t *row, const uint32_t *wgt, uint32_t n, uint32_t reach, uint4 *blocks,
                                hipStream_t s);
