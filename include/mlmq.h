@@ -143,11 +143,11 @@ typedef struct mlmq_params {
 /* Per-solve statistics (all counts summed over wavefronts). */
 typedef struct mlmq_timing {
     double   solve_ms;        /* host steady clock around the persistent launch */
-    double   device_ms;       /* HIP events around the persistent launch */
+    double   device_ms;       /* device time of the solve, without the reset */
     double   reset_ms;        /* per-query reset (device fill + seed) */
     double   query_wall_ms;   /* reset + solve + nothing else (copy-out is separate) */
-    int32_t  work_blocks;     /* workgroups launched */
-    int32_t  waves;           /* persistent wavefronts launched */
+    int32_t  work_blocks;     /* workgroups launched (push-pull solver: per round) */
+    int32_t  waves;           /* wavefronts of these */
     int64_t  bucket_capacity; /* ring slots per bucket used */
     uint64_t l2_pushes;       /* records reserved in L2 (incl. the seed) */
     uint64_t l2_pops;         /* records taken from L2 */
@@ -155,7 +155,8 @@ typedef struct mlmq_timing {
     uint64_t atomics;         /* atomicMin issued: edges examined less those skipped by the
                                  heavy loop's cached pre-check or as a record's back edge
                                  (the edge to the vertex whose expansion created it) */
-    uint64_t improvements;    /* atomicMin that lowered a distance (= records pushed) */
+    uint64_t improvements;    /* atomicMin that lowered a distance (= records pushed);
+                                 region solver: expanded vertices */
     uint64_t stale;           /* popped records skipped as stale */
     uint64_t batches;         /* processed record batches */
     uint64_t idle_polls;      /* idle iterations of all waves */
@@ -175,7 +176,7 @@ typedef struct mlmq_timing {
 /* Statistics of one mlmq_solve_batch call. */
 typedef struct mlmq_batch_timing {
     double   solve_ms;        /* host steady clock around the launch (row reset + batch kernel) */
-    double   device_ms;       /* HIP events around the launch */
+    double   device_ms;       /* device time of the launch with its row reset */
     double   query_ms_p50;    /* per-query time inside the launch (device wall clock), median */
     double   query_ms_p99;
     double   query_ms_max;
@@ -229,8 +230,18 @@ int mlmq_attach_device_csr(mlmq_ctx *ctx, int32_t n, int64_t m,
 int mlmq_graph_stats(mlmq_ctx *ctx, mlmq_graph_info *info);
 int mlmq_graph_size(const mlmq_ctx *ctx, int32_t *n, int64_t *m);
 
-/* One query: reset, seed `src`, run the persistent solver to termination.
- * `params` may be NULL (defaults); `timing` may be NULL. */
+/* One query: reset, seed `src`, run the solver to termination.
+ * `params` may be NULL (defaults); `timing` may be NULL.
+ *
+ * Three solvers answer it, all with the same distances.  In the default queue
+ * mode a road-like graph (degrees up to 64, mean up to 8, weights below 2^20 - 1,
+ * few edges between pieces of 1024 vertices) is solved by the region solver, and
+ * an undirected graph of strongly varying degree loaded through mlmq_load_csr /
+ * mlmq_load_gr by the push-pull solver; neither depends on delta, the buckets or
+ * the other queue settings.  Parameters that ask for a part of the vertex queue
+ * (l1_blocks, hub_split, defer_heavy, strict_window, l1_donate, profile, a
+ * bucket_capacity; on road-like graphs also light_split) select it, and it
+ * serves every other graph. */
 int mlmq_solve(mlmq_ctx *ctx, int32_t src, const mlmq_params *params, mlmq_timing *timing);
 /* Ring slots (8 bytes each) of the static device workspace that
  * mlmq_solve_noalloc uses: buckets x bucket_capacity may not exceed it. */
@@ -257,7 +268,10 @@ int mlmq_solve_noalloc(mlmq_ctx *ctx, int32_t src, const mlmq_params *params, in
  * after another, SSSP/main.cu:213-307).  Each workgroup of
  * params->batch_waves waves owns a private queue partition and serves queries
  * taken from a global counter; params->work_blocks workgroups are in flight
- * (0 = one per CU, at most nq).  Results stay on the device until copied
+ * (0 = one per CU, at most nq).  With work_blocks 0 and settings for which
+ * mlmq_solve takes the region solver, that solver runs the batch in one launch,
+ * a few queries in flight at a time (not 200 queries or more on a graph of more
+ * than about 390,000 vertices, for which the queue is faster).  Results stay on the device until copied
  * with mlmq_copy_batch_dist. */
 int mlmq_solve_batch(mlmq_ctx *ctx, const int32_t *sources, int32_t nq,
                      const mlmq_params *params, mlmq_batch_timing *timing);

@@ -28,9 +28,14 @@
  *     width wait for a later launch.  Lanes run concurrently on the device,
  *     so requests that arrive while others run are admitted as lanes and
  *     bytes free up (continuous batching).
- *   - Each request runs on `workgroups` workgroups of `waves` wave64 that
- *     share its queue partition; distances are exact (the same per vertex as
- *     a CPU Dijkstra), whatever else runs beside it.
+ *   - In a launch lane, requests that mlmq_solve would give to the region or
+ *     the push-pull solver run on it, those of all such graphs in the same
+ *     launches (hub_split, a bucket_capacity, on road-like graphs light_split,
+ *     and slots too small for these solvers' state keep a request on the vertex
+ *     queue, as does live serving).  There each request runs on `workgroups`
+ *     workgroups of `waves` wave64 that share its queue partition.  Distances
+ *     are exact (the same per vertex as a CPU Dijkstra), whatever else runs
+ *     beside it.
  *   - Latency = completion of the request's launch on the device (HIP event)
  *     minus its arrival time; queue time = launch time minus arrival.
  *   - Verification: with config.verify, a request whose (graph, source) has an

@@ -696,6 +696,20 @@ bool wants_pushpull(const mlmq_ctx *c, const mlmq_params &p) {
            !p.defer_heavy && !p.strict_window && p.l1_donate == 0 && p.bucket_capacity == 0;
 }
 
+// A batch of nq queries by the region solver: where mlmq_solve takes it, but not
+// for many queries on a large graph.  There the vertex queue has every CU busy
+// with a query of its own, and with its settings tuned is faster.  Batches of
+// 256, ms by the regions / the queue tuned / the queue with defaults: 100k 3.6 /
+// 3.9 / 7.7, 264k 9.1 / 9.5 / 21.9, 450k 15.0 / 13.2 / -, 600k 20.3 / 17.9 / 28.2,
+// 1.07M 36.3 / 24 / 49.3, 2.5M 88.9 / 66.6 / 115.5; of 192: 450k 11.3 / 12.5 / -;
+// of 128: 1.07M 18.3 / 27.0 / 43.2, 2.5M 45.0 / 61.8 / 100.7.  (By sizes alone: a
+// rule on the settings too would keep a tuner that starts at the defaults from
+// ever seeing the queue.)
+bool wants_batch_regions(const mlmq_ctx *c, uint32_t nq, const mlmq_params &p) {
+    if (!wants_regions(c, p) || p.work_blocks != 0 || nq > mlmq::kRegionQueries) return false;
+    return c->regions.regions < 384 || nq < 200;
+}
+
 // Per-query state and ring of the region solver for nq queries on a grid of
 // at most `grid` workgroups.
 int ensure_region_space(mlmq_ctx *c, uint32_t nq, uint32_t grid) {
@@ -1383,7 +1397,7 @@ int mlmq_solve_batch(mlmq_ctx *c, const int32_t *sources, int32_t nq, const mlmq
 
     // A chosen number of workgroups, one query each, is the vertex queue's.
     // (kRegionQueries: a record's query field.)
-    if (wants_regions(c, p) && p.work_blocks == 0 && nq <= (int32_t)mlmq::kRegionQueries) {
+    if (wants_batch_regions(c, (uint32_t)nq, p)) {
         const int rrc = batch_regions(c, nq, p, timing);
         if (rrc != MLMQ_E_QUEUE_OVERFLOW && rrc != MLMQ_E_NOMEM) return rrc;
     }

@@ -162,3 +162,18 @@ def test_stopped_solve_leaves_a_clean_solver(solver):
         assert e.value.code == -7
         solver.solve(3, timeout_s=TIMEOUT)
         assert np.array_equal(solver.dist(), O.dijkstra(row, col, w, 3)[0])
+
+
+@pytest.mark.parametrize("nq", [199, 200])
+def test_large_batches(solver, nq):
+    """Around the size from which a batch on a large graph goes to the vertex
+    queue (200 queries, 384 regions)."""
+    say(f"{nq} queries on 400k vertices")
+    g = HostGraph.knn(400_000, 3, seed=3, weight_scale=1e5, morton=True)
+    row, col, w = (x.copy() for x in g.arrays())
+    g.close()
+    solver.load_csr(row, col, w)
+    src = np.random.default_rng(nq).integers(0, 400_000, nq).astype(np.int32)
+    solver.solve_batch(src, timeout_s=TIMEOUT)
+    for i in (0, nq // 2, nq - 1):
+        assert np.array_equal(solver.batch_dist(i), O.dijkstra(row, col, w, int(src[i]))[0]), i
