@@ -84,7 +84,24 @@ struct Lane {
     uint64_t *ring = nullptr;
     uint64_t ring_slots = 0;
     bool ring_dirty = true;
+    // push-pull state of requests whose slot has no room for it (allocated with
+    // the first of them; pp_off: without it)
+    uint8_t *pp = nullptr;
+    bool pp_off = false;
+    std::vector<uint8_t *> part;   // state of each request, beside the distance row
 };
+
+// With so many requests of other lanes in flight a launch goes to the vertex
+// queue: each CU then has requests of its own, as in a large batch, and the
+// launches share the device evenly.  Poisson arrivals over road 264k (50 %), road
+// 6.26M (30 %) and RMAT-20 (20 %), nothing tuned, by the queue alone / this way:
+// 1200 queries/s p50 73 / 5.6 ms, p99 111 / 34 ms; 1700 queries/s p50 88 / 92,
+// p99 133 / 126; 2000 offered 1717 / 1832 served.  (By the other solvers alone
+// 1380 of 2000; switching at 96 instead: p99 592 ms at 1500.)
+constexpr uint64_t kCrowd = 32;
+
+// Most bytes of a lane's push-pull states: about 20 requests on RMAT-20.
+constexpr uint64_t kLanePush = 256u << 20;
 
 constexpr size_t kTabBytes = sizeof(mlmq::RegionQuery) + sizeof(mlmq::PushPullLaunch) + sizeof(mlmq::ServeOutcome);
 static_assert(sizeof(mlmq::RegionQuery) % 8 == 0 && sizeof(mlmq::PushPullLaunch) % 8 == 0, "packed one after another");
@@ -345,21 +362,25 @@ int add_graph_ctx(mlmq_server *s, mlmq_ctx *ctx, const mlmq_serve_graph_params *
     return MLMQ_OK;
 }
 
+uint64_t push_bytes(const GraphEntry &g) {
+    return round_up(sizeof(uint32_t) * (3ull * (uint64_t)g.v.n + mlmq::kMaxRounds + 2));
+}
+
 // Which solver serves a request of g whose slot is `slot_bytes` long: as for
-// single queries, and the solver's state must fit the queue partition of the
-// slot, which it takes the place of.  A burst of 17 road-264k, 8 road-1M and 7
-// RMAT-18 requests in one launch: device 43 ms all by the vertex queue, 7.2 ms
-// this way (of it 0.7 ms push-pull, all of a launch's queries in the same
-// rounds, and 6.4 ms regions, all of its queries in the same ring).
-Engine engine_of(const GraphEntry &g, uint64_t slot_bytes) {
+// single queries.  Its state takes the place of the slot's queue partition; a
+// push-pull query that does not fit there may use `spare` bytes beside it.  A
+// burst of 17 road-264k, 8 road-1M and 7 RMAT-18 requests in one launch: device
+// 43 ms all by the vertex queue, 3.4 ms this way (of it 0.7 ms push-pull, all of
+// a launch's queries in the same rounds, and 2.6 ms regions, all of its queries
+// in the same ring).
+Engine engine_of(const GraphEntry &g, uint64_t slot_bytes, uint64_t spare) {
     if (g.p.hub_split || g.p.bucket_capacity) return Engine::kQueue;
     const uint64_t room = slot_bytes - g.row_bytes - g.ctl_bytes;
     if (g.v.regions.regions) {
         const uint64_t words = (uint64_t)g.v.regions.inbox_slots + 1 + g.v.regions.regions;
         return !g.p.light_split && sizeof(uint32_t) * words <= room ? Engine::kRegions : Engine::kQueue;
     }
-    const uint64_t words = 3ull * (uint64_t)g.v.n + mlmq::kMaxRounds + 2;
-    return g.v.pp_reach && sizeof(uint32_t) * words <= room ? Engine::kPushPull : Engine::kQueue;
+    return g.v.pp_reach && push_bytes(g) <= std::max(room, spare) ? Engine::kPushPull : Engine::kQueue;
 }
 
 // A push-pull query whose state lies in `part`.
@@ -969,7 +990,8 @@ int mlmq_server_destroy(mlmq_server *s) {
         if (l.h_reqs) (void)hipHostFree(l.h_reqs);
         if (l.h_tab) (void)hipHostFree(l.h_tab);
         for (void *p : {(void *)l.d_reqs, (void *)l.d_tab, (void *)l.ctl, (void *)l.times,
-                        (void *)l.progress, (void *)l.counts, (void *)l.ring})
+                        (void *)l.progress, (void *)l.counts, (void *)l.ring,
+                        (void *)l.pp})
             if (p) (void)hipFree(p);
         if (l.s) (void)hipStreamDestroy(l.s);
     }
@@ -1167,11 +1189,28 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
         // The solver of each request.
         uint64_t tasks = 0;
         uint32_t nqueue = 0, nregion = 0, npush = 0;
+        const uint64_t push_room = std::min<uint64_t>(kLanePush, s->cfg.hbm_budget / 64);
+        uint64_t push_used = 0;
+        const bool crowded = inflight >= kCrowd;
         l.engines.resize(nb);
+        l.part.resize(nb);
         for (uint32_t i = 0; i < nb; ++i) {
             const GraphEntry &g = s->graphs[reqs[l.ids[i]].graph];
             Engine &e = l.engines[i];
-            e = queue_only[l.ids[i]] ? Engine::kQueue : engine_of(g, l.slots[i].bytes);
+            e = crowded || queue_only[l.ids[i]] ? Engine::kQueue
+                                                : engine_of(g, l.slots[i].bytes, l.pp_off ? 0 : push_room - push_used);
+            l.part[i] = s->arena.base + l.slots[i].off + g.row_bytes + g.ctl_bytes;
+            if (e == Engine::kPushPull && push_bytes(g) > l.slots[i].bytes - g.row_bytes - g.ctl_bytes) {
+                if (!l.pp && hipMalloc((void **)&l.pp, push_room) != hipSuccess) {
+                    (void)hipGetLastError();
+                    l.pp = nullptr;
+                    l.pp_off = true;
+                    e = Engine::kQueue;
+                } else {
+                    l.part[i] = l.pp + push_used;
+                    push_used += push_bytes(g);
+                }
+            }
             if (e == Engine::kRegions) {
                 const uint64_t more = tasks + g.v.regions.regions;
                 if (2 * (more + region_groups) > kLaneRing) e = Engine::kQueue;
@@ -1182,8 +1221,9 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
             nqueue += e == Engine::kQueue;
         }
         const uint32_t relaxers = mlmq::region_relaxers(nregion ? tasks / nregion : 0, nregion, (uint32_t)s->cus);
+        const int per_cu = std::max(1, relaxers == mlmq::kMany ? many : few);
         const uint32_t region_grid =
-            (uint32_t)std::min<uint64_t>({(uint64_t)std::max(relaxers == mlmq::kMany ? many : few, 1) * s->cus, region_groups, tasks});
+            (uint32_t)std::min<uint64_t>({(uint64_t)per_cu * s->cus, region_groups, tasks});
         if (nregion && lane_ring(l, tasks, region_grid) != hipSuccess) {
             (void)hipGetLastError();
             for (Engine &e : l.engines)
@@ -1227,8 +1267,8 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
             L.cap_log2 = l.caps[i];
             L.dist = (uint32_t *)b;
             L.ctl = (uint32_t *)(b + g.row_bytes);
-            uint8_t *part = b + g.row_bytes + g.ctl_bytes;
-            L.slots = (uint64_t *)part;
+            uint8_t *part = l.part[i];
+            L.slots = (uint64_t *)(b + g.row_bytes + g.ctl_bytes);
             const uint32_t *expect = nullptr;
             if (s->cfg.verify) {
                 auto it = g.expected.find(reqs[id].src);
