@@ -61,6 +61,13 @@ def traffic_key(workload, queue, delta, args, work_blocks):
     return json.dumps({k: cfg[k] for k in TRAFFIC_KEYS}, sort_keys=True)
 
 
+def solver_kernel(timing):
+    """Kernel of the solver that answered a query, by the waves of its
+    workgroups (one, or six or ten, or eight)."""
+    per = timing["waves"] // max(1, timing["work_blocks"])
+    return {1: "sssp_persistent_kernel", 8: "push_kernel"}.get(per, "region_solver_kernel")
+
+
 def load_traffic(path, key):
     try:
         tj = json.load(open(path))
@@ -101,7 +108,7 @@ def traffic_update(args):
     if line is None:
         raise SystemExit(f"no bench line in {line_path}")
     key = line["roofline"]["traffic_key"]
-    kern = "sssp_persistent_kernel"
+    kern = line["roofline"]["kernel"]
     fetch, nf = _counter_means(fdir, "FETCH_SIZE", kern)
     write, nw = _counter_means(wdir, "WRITE_SIZE", kern)
     cfetch, _ = _counter_means(cfdir, "FETCH_SIZE", "copy_u32_kernel")
@@ -409,7 +416,7 @@ def main():
             "frac": round(achieved / HBM_PEAK_GBS, 8),
             "traffic": traffic,
             "traffic_key": tkey,
-            "kernel": "sssp_persistent_kernel",
+            "kernel": solver_kernel(last),
             "bytes_per_launch": b_alg,
         },
         "cpu_baseline": {
