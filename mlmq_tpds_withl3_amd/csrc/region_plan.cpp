@@ -86,11 +86,13 @@ bool region_plan(uint32_t n, const uint32_t *row, const uint32_t *col, RegionPla
     // three quarters full.
     std::fill(reg.begin(), reg.end(), kNone);
     plan->first.assign(1, 0);
+    constexpr uint32_t kAhead = 16;
     std::vector<uint32_t> rim;
     size_t rim_head = 0;
     uint32_t next = 0, placed = 0, r = 0;
     auto size = [&]() { return placed - plan->first.back(); };
     auto put = [&](uint32_t v) {
+        __builtin_prefetch(&row[v]);
         reg[v] = r;
         plan->order[placed++] = v;
     };
@@ -115,6 +117,12 @@ bool region_plan(uint32_t n, const uint32_t *row, const uint32_t *col, RegionPla
         uint32_t head = placed;
         put(seed);
         for (; head < placed; ++head) {
+            // (what the next vertices need: the ids are scattered over memory)
+            if (head + kAhead < placed) __builtin_prefetch(&col[row[plan->order[head + kAhead]]]);
+            if (head + kAhead / 2 < placed) {
+                const uint32_t x = plan->order[head + kAhead / 2];
+                for (uint32_t e = row[x]; e < row[x + 1]; ++e) __builtin_prefetch(&reg[col[e]], 1);
+            }
             const uint32_t u = plan->order[head];
             for (uint32_t e = row[u]; e < row[u + 1]; ++e) {
                 const uint32_t v = col[e];
