@@ -68,7 +68,10 @@ typedef struct mlmq_params {
     uint32_t delta;           /* bucket width; reference BENCH_DELTA, default 200000 */
     int32_t  work_blocks;     /* persistent workgroups of one wave64 each; 0 = automatic
                                  (blocks_per_cu x CUs if blocks_per_cu > 0, else n / 25000
-                                 clamped to [128, 512]); mlmq_solve_batch: workgroups of
+                                 clamped to [128, 512]); region and push-pull solvers (see
+                                 mlmq_solve): below the number of CUs at most so many of their
+                                 larger workgroups, so that the other CUs stay free, from there
+                                 on as many as they need; mlmq_solve_batch: workgroups of
                                  batch_waves waves, one query each (0 = as many as the device
                                  holds at once, at most the number of queries) */
     int32_t  blocks_per_cu;   /* used when work_blocks == 0 */
@@ -240,8 +243,8 @@ int mlmq_graph_size(const mlmq_ctx *ctx, int32_t *n, int64_t *m);
  * mlmq_load_gr by the push-pull solver; neither depends on delta, the buckets or
  * the other queue settings.  Parameters that ask for a part of the vertex queue
  * (l1_blocks, hub_split, defer_heavy, strict_window, l1_donate, profile, a
- * bucket_capacity; on road-like graphs also light_split) select it, and it
- * serves every other graph. */
+ * bucket_capacity; on road-like graphs also light_split, or fewer work_blocks
+ * than a 32nd of the pieces) select it, and it serves every other graph. */
 int mlmq_solve(mlmq_ctx *ctx, int32_t src, const mlmq_params *params, mlmq_timing *timing);
 /* Ring slots (8 bytes each) of the static device workspace that
  * mlmq_solve_noalloc uses: buckets x bucket_capacity may not exceed it. */

@@ -680,13 +680,29 @@ struct QueryClock {
     }
 };
 
+// Most workgroups of a query on the other solvers (0: as many as they need).
+// Fewer than one per CU leave the other CUs to the caller's other work; from
+// one per CU on, none is left free.
+uint32_t group_limit(const mlmq_ctx *c, const mlmq_params &p) {
+    return p.work_blocks > 0 && p.work_blocks < c->cus ? (uint32_t)p.work_blocks : 0u;
+}
+
+// Least workgroups with which the region solver takes a graph: one per 32
+// regions.  With fewer, regions wait in the ring and are expanded from distances
+// far from final.  Device ms by the regions / the queue with defaults / tuned, at
+// so many workgroups: 1046 regions 16: 12.5 / 14.3 / 10.3, 32: 4.9 / 7.5 / 5.3,
+// 64: 1.6 / 6.5 / 3.3; 6116 regions 64: 36 / 24 / 16, 128: 12.2 / 18.9 / 8.5,
+// 192: 5.8 / 21.5 / 6.6; 261 regions 4: 8.6 / 19.5 / 21.5.
+constexpr uint32_t kRegionsPerGroup = 32;
+
 // The region solver answers the default queue mode on a cut graph.  Settings
 // that ask for a part of the vertex queue (its kernel variants, its profile,
 // a ring capacity) get the vertex queue.
 bool wants_regions(const mlmq_ctx *c, const mlmq_params &p) {
+    const uint32_t limit = group_limit(c, p);
     return c->regions.regions != 0 && p.queue_mode == MLMQ_QUEUE_L1SLF_L2DQ && !p.profile && !p.l1_blocks &&
            !p.hub_split && !p.light_split && !p.defer_heavy && !p.strict_window && p.l1_donate == 0 &&
-           p.bucket_capacity == 0;
+           p.bucket_capacity == 0 && (limit == 0 || limit >= c->regions.regions / kRegionsPerGroup);
 }
 
 // The push-pull solver answers the same calls on the graphs it is for; the
@@ -747,15 +763,15 @@ int ensure_region_space(mlmq_ctx *c, uint32_t nq, uint32_t grid) {
 }
 
 // Workgroups of a region solve of nq queries: one per region and query, at
-// least `at_least`, at most what the device holds.
-int region_grid(mlmq_ctx *c, uint32_t nq, uint64_t at_least, uint32_t *relaxers, uint32_t *grid) {
+// most `at_most` (0: no limit) and what the device holds.
+int region_grid(mlmq_ctx *c, uint32_t nq, uint64_t at_most, uint32_t *relaxers, uint32_t *grid) {
     int occ = 0;
     const uint64_t tasks = (uint64_t)nq * c->regions.regions;
     *relaxers = mlmq::region_relaxers(c->regions.regions, nq, (uint32_t)c->cus);
     HIP_TRY(c, mlmq::region_occupancy(*relaxers, &occ));
     if (occ < 1) return fail(c, MLMQ_E_HIP, "region solver cannot be resident");
     const uint64_t most = std::min<uint64_t>((uint64_t)occ * c->cus, mlmq::kRegionGroups);
-    *grid = (uint32_t)std::min(most, std::max(tasks, at_least));
+    *grid = (uint32_t)std::min({most, tasks, at_most ? at_most : most});
     return MLMQ_OK;
 }
 
@@ -895,7 +911,7 @@ int run_regions(mlmq_ctx *c, uint32_t nq, int32_t src, const uint32_t *sources, 
 // One query, distances into the context's row.
 int solve_regions(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *timing) {
     uint32_t relaxers = 0, grid = 0;
-    int rc = region_grid(c, 1, (uint64_t)p.work_blocks, &relaxers, &grid);
+    int rc = region_grid(c, 1, group_limit(c, p), &relaxers, &grid);
     if (rc == MLMQ_OK) rc = ensure_region_space(c, 1, grid);
     if (rc) return rc;
     QueryClock t;
@@ -927,6 +943,7 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
     mlmq::PushPullQueries Q{};
     Q.nq = 1;
     Q.max_n = (uint32_t)n;
+    Q.most_groups = group_limit(c, p);
     mlmq::PushPullLaunch &L = Q.one;
     L.src = (uint32_t)src;
     L.col = c->col;
@@ -982,7 +999,7 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
     c->last_window = (uint32_t)p.bucket_window;
     c->last_cap_log2 = ceil_log2(n);
     if (timing) {
-        fill_timing(c, ctl.data(), t, (int)mlmq::push_groups(L.n), c->last_cap_log2, 0, timing);
+        fill_timing(c, ctl.data(), t, (int)mlmq::push_groups(Q), c->last_cap_log2, 0, timing);
         timing->waves = mlmq::kPushWaves * timing->work_blocks;
     }
     return MLMQ_OK;

@@ -416,6 +416,10 @@ uint32_t groups_for(uint64_t items, uint32_t most) {
     return (uint32_t)(g < 1 ? 1 : g > most ? most : g);
 }
 
+uint32_t limited(const PushPullQueries &Q, uint32_t groups) {
+    return Q.most_groups && Q.most_groups < groups ? Q.most_groups : groups;
+}
+
 }  // namespace
 
 hipError_t launch_symmetry_check(const uint32_t *row, const uint32_t *col, const uint32_t *wgt, uint32_t n, uint64_t m,
@@ -446,16 +450,20 @@ hipError_t launch_pushpull_reset(const PushPullQueries &Q, hipStream_t s) {
 // for them (us, RMAT-18 / 20 / 22: 2048 of 256 358 / 626 / 1119, 1024 of 512
 // 304 / 537 / 1089, 512 of 512 280 / 557 / 1114, 512 of 1024 314 / 559 / 1131).
 // A graph of few vertices never fills two per CU.
-uint32_t push_groups(uint32_t n) {
+static uint32_t groups_of_push(uint32_t n) {
     const uint32_t most = n / 1024 < 512 ? 512 : n / 1024 < 1024 ? n / 1024 : 1024;
     return groups_for((uint64_t)n * 8, most);
 }
 
-hipError_t launch_push(const PushPullQueries &Q, uint32_t round, bool bounded, hipStream_t s) {
+uint32_t push_groups(const PushPullQueries &Q) {
     // several queries share the device, but a round of one may be most of the work
     const uint32_t share = 1024 / Q.nq > 128 ? 1024 / Q.nq : 128;
-    const uint32_t x = push_groups(Q.max_n);
-    const dim3 grid(x < share ? x : share, Q.nq), group(kGroup);
+    const uint32_t x = limited(Q, groups_of_push(Q.max_n));
+    return x < share ? x : share;
+}
+
+hipError_t launch_push(const PushPullQueries &Q, uint32_t round, bool bounded, hipStream_t s) {
+    const dim3 grid(push_groups(Q), Q.nq), group(kGroup);
     if (Q.table && bounded) hipLaunchKernelGGL((push_kernel<true, true>), grid, group, 0, s, Q.one, Q.table, round);
     else if (Q.table) hipLaunchKernelGGL((push_kernel<true, false>), grid, group, 0, s, Q.one, Q.table, round);
     else if (bounded) hipLaunchKernelGGL((push_kernel<false, true>), grid, group, 0, s, Q.one, Q.table, round);
@@ -464,14 +472,14 @@ hipError_t launch_push(const PushPullQueries &Q, uint32_t round, bool bounded, h
 }
 
 hipError_t launch_pushpull_summary(const PushPullLaunch &L, uint32_t rounds, PushPullSummary *out, hipStream_t s) {
-    const uint32_t pushes = push_groups(L.n), pulls = groups_for(L.n, 2048);
+    const uint32_t pushes = groups_of_push(L.n), pulls = groups_for(L.n, 2048);
     const uint32_t groups = pushes > pulls ? pushes : pulls;   // entries in use
     hipLaunchKernelGGL(pushpull_summary_kernel, dim3(1), dim3(1024), 0, s, L, groups, rounds, out);
     return hipGetLastError();
 }
 
 hipError_t launch_pull(const PushPullQueries &Q, uint32_t round, hipStream_t s) {
-    const dim3 grid(groups_for(Q.max_n, 2048), Q.nq), group(kGroup);
+    const dim3 grid(limited(Q, groups_for(Q.max_n, 2048)), Q.nq), group(kGroup);
     if (Q.table) hipLaunchKernelGGL(pull_kernel<true>, grid, group, 0, s, Q.one, Q.table, round);
     else hipLaunchKernelGGL(pull_kernel<false>, grid, group, 0, s, Q.one, Q.table, round);
     return hipGetLastError();

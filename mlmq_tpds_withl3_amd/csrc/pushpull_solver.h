@@ -46,6 +46,7 @@ struct PushPullQueries {
     const PushPullLaunch *table;   // nq entries in device memory (null: `one`)
     uint32_t nq;
     uint32_t max_n;                // most vertices of a query
+    uint32_t most_groups;          // workgroups of a push or pull (0: no limit)
 };
 
 // Outcome of a query, written to host memory.
@@ -62,8 +63,8 @@ hipError_t launch_symmetry_check(const uint32_t *row, const uint32_t *col, const
 hipError_t launch_bound_counts(const uint32_t *row, const uint32_t *wgt, uint32_t n, uint32_t reach, uint4 *blocks,
                                hipStream_t s);
 hipError_t launch_pushpull_reset(const PushPullQueries &Q, hipStream_t s);
-// Workgroups of a push launch of one query, and waves of each.
-uint32_t push_groups(uint32_t n);
+// Workgroups of a push launch of each query, and waves of each.
+uint32_t push_groups(const PushPullQueries &Q);
 constexpr int kPushWaves = 8;
 // Round r expands the vertices of count[r] into those of count[r + 1].
 hipError_t launch_push(const PushPullQueries &Q, uint32_t round, bool bounded, hipStream_t s);

@@ -1,0 +1,79 @@
+"""Which solver answers a single query, and on how many workgroups: a chosen
+number of workgroups below the number of CUs (256) bounds the region and the
+push-pull solver too, from there on they take what they need; with fewer
+workgroups than a 32nd of a graph's regions the vertex queue answers.  The
+timing tells the solver by the waves of a workgroup: one (vertex queue), six or
+ten (regions), eight (push-pull).  Every row is compared with the oracle, bit
+for bit."""
+import sys
+
+import numpy as np
+import pytest
+
+from mlmq_tpds_withl3_amd import HostGraph, Solver
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+TIMEOUT = 20.0
+CUS = 256
+
+
+def say(msg):
+    print(f"[gpu-solver-choice] {msg}", flush=True)
+    sys.stdout.flush()
+
+
+def arrays(g):
+    out = tuple(x.copy() for x in g.arrays())
+    g.close()
+    return out
+
+
+@pytest.fixture(scope="module")
+def loaded():
+    """A road-like graph of 70 regions and a power-law graph, resident."""
+    graphs = {"road": arrays(HostGraph.knn(70_001, 3, seed=4, weight_scale=1e5)),
+              "power": arrays(HostGraph.rmat(13, 16, seed=9, wmin=1, wmax=1000))}
+    out = {}
+    for name, g in graphs.items():
+        s = Solver(0)
+        s.load_csr(*g)
+        out[name] = (s, g)
+    yield out
+    for s, _ in out.values():
+        s.close()
+
+
+def solve(loaded, name, src, **params):
+    s, g = loaded[name]
+    t = s.solve(src, timeout_s=TIMEOUT, **params)
+    assert np.array_equal(s.dist(), O.dijkstra(*g, src)[0])
+    return t["work_blocks"], t["waves"] // t["work_blocks"]
+
+
+@pytest.mark.parametrize("blocks", [2, 3, 64, CUS - 1])
+def test_chosen_workgroups_bound_the_regions(loaded, blocks):
+    say(f"regions on {blocks} workgroups")
+    free, _ = solve(loaded, "road", 11)
+    used, waves = solve(loaded, "road", 11, work_blocks=blocks)
+    assert waves in (6, 10) and used == min(blocks, free)
+
+
+def test_few_workgroups_for_many_regions(loaded):
+    say("one workgroup for 70 regions: the vertex queue")
+    assert solve(loaded, "road", 11, work_blocks=1) == (1, 1)
+
+
+@pytest.mark.parametrize("blocks", [1, 7, 64, CUS - 1])
+def test_chosen_workgroups_bound_the_push_pull_rounds(loaded, blocks):
+    say(f"push-pull on {blocks} workgroups")
+    free, _ = solve(loaded, "power", 5)
+    assert solve(loaded, "power", 5, work_blocks=blocks) == (min(blocks, free), 8)
+
+
+@pytest.mark.parametrize("name", ["road", "power"])
+def test_one_workgroup_per_cu_is_no_bound(loaded, name):
+    say(f"{name}: one workgroup per CU or more")
+    free = solve(loaded, name, 3)
+    assert solve(loaded, name, 3, work_blocks=CUS) == free
+    assert solve(loaded, name, 3, work_blocks=2 * CUS) == free
