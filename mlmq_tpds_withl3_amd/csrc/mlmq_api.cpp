@@ -81,7 +81,7 @@ struct mlmq_ctx {
     uint64_t *r_ring = nullptr;
     uint64_t r_ring_slots = 0;
     bool r_ring_dirty = true;
-    uint32_t *h_ctl = nullptr;   // pinned: control block as copied out
+    uint32_t *h_ctl = nullptr;   // pinned: outcome of a region or push-pull solve
     mlmq::RowStage stage;        // rows on their way to the host
     // push-pull solver: the graph's reach and hub degree (reach 0: not for
     // this graph), and
@@ -136,7 +136,10 @@ int fail(mlmq_ctx *c, int code, const std::string &msg) {
     return code;
 }
 
+// (the runtime keeps the error until it is asked for: the next launch would
+// report it)
 int hip_fail(mlmq_ctx *c, hipError_t e, const char *what) {
+    (void)hipGetLastError();
     return fail(c, e == hipErrorOutOfMemory ? MLMQ_E_NOMEM : MLMQ_E_HIP,
                 std::string(what) + ": " + hipGetErrorString(e));
 }
@@ -167,8 +170,8 @@ void free_batch(mlmq_ctx *c) {
     c->b_slots_dirty = true;
 }
 
-void free_regions(mlmq_ctx *c) {
-    mlmq::region_free(&c->regions);
+// Per-query state of the region solver; the graph's cut stays.
+void free_region_space(mlmq_ctx *c) {
     for (void *p : {(void *)c->r_inbox, (void *)c->r_act, (void *)c->r_progress, (void *)c->r_counts, (void *)c->r_ring})
         if (p) (void)hipFree(p);
     c->r_inbox = c->r_act = nullptr;
@@ -180,17 +183,19 @@ void free_regions(mlmq_ctx *c) {
     c->r_ring_dirty = true;
 }
 
-void free_pushpull(mlmq_ctx *c) {
+// Per-query state of the push-pull solver.
+void free_pushpull_space(mlmq_ctx *c) {
     for (void *p : {(void *)c->pp_mark, (void *)c->pp_front, (void *)c->pp_count})
         if (p) (void)hipFree(p);
     c->pp_mark = c->pp_front = c->pp_count = nullptr;
-    c->pp_reach = 0;
 }
 
 void free_graph(mlmq_ctx *c) {
     free_batch(c);
-    free_regions(c);
-    free_pushpull(c);
+    free_region_space(c);
+    mlmq::region_free(&c->regions);
+    free_pushpull_space(c);
+    c->pp_reach = 0;
     if (c->owns_graph) {
         (void)hipFree(c->row);
         (void)hipFree(c->col);
@@ -303,8 +308,13 @@ int build_pushpull(mlmq_ctx *c, const int32_t *w) {
     const mlmq_graph_info &gi = c->info;
     if (!c->sorted || c->regions.regions || c->m < 4ll * c->n || gi.dev_nnz < 2.0f * gi.avg_nnz) return MLMQ_OK;
     uint32_t *flag = nullptr, bad = 0;
-    HIP_TRY(c, hipMalloc(&flag, sizeof(uint32_t)));
-    hipError_t e = mlmq::launch_fill_u32(flag, 1, 0u, c->stream);
+    hipError_t e = hipMalloc(&flag, sizeof(uint32_t));
+    if (e == hipErrorOutOfMemory) {   // the vertex queue serves the graph
+        (void)hipGetLastError();
+        return MLMQ_OK;
+    }
+    HIP_TRY(c, e);
+    e = mlmq::launch_fill_u32(flag, 1, 0u, c->stream);
     if (e == hipSuccess)
         e = mlmq::launch_symmetry_check(c->row, c->col, c->wgt, (uint32_t)c->n, (uint64_t)c->m, flag, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(&bad, flag, sizeof(bad), hipMemcpyDeviceToHost, c->stream);
@@ -460,15 +470,20 @@ int ensure_dist(mlmq_ctx *c) {
     return MLMQ_OK;
 }
 
-// The control block and its host copies.
+// The control block and its host copy.
 int ensure_ctl(mlmq_ctx *c) {
     if (!c->ctl) {
         HIP_TRY(c, hipMalloc(&c->ctl, sizeof(uint32_t) * mlmq::kCtlWords));
         c->ctl_host.assign(mlmq::kCtlWords, 0);
     }
+    return MLMQ_OK;
+}
+
+// Where the region and the push-pull solver write their outcome.
+int ensure_outcome(mlmq_ctx *c) {
     if (!c->h_ctl)
         HIP_TRY(c, hipHostMalloc((void **)&c->h_ctl, sizeof(uint32_t) * mlmq::kCtlWords, hipHostMallocDefault));
-    return MLMQ_OK;
+    return ensure_ctl(c);
 }
 
 int ensure_queue(mlmq_ctx *c, uint32_t nbuckets, uint32_t cap_log2) {
@@ -759,7 +774,7 @@ int ensure_region_space(mlmq_ctx *c, uint32_t nq, uint32_t grid) {
         HIP_TRY(c, mlmq::launch_fill_u64(c->r_ring, c->r_ring_slots, mlmq::kEmpty, c->stream));
         c->r_ring_dirty = false;
     }
-    return ensure_ctl(c);
+    return ensure_outcome(c);
 }
 
 // Workgroups of a region solve of nq queries: one per region and query, at
@@ -932,7 +947,7 @@ int solve_regions(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *t
 // MLMQ_E_QUEUE_OVERFLOW: more rounds than it is meant for.
 int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *timing) {
     const size_t n = (size_t)c->n;
-    int rc = ensure_ctl(c);
+    int rc = ensure_outcome(c);
     if (rc) return rc;
     if (!c->pp_mark) HIP_TRY(c, hipMalloc(&c->pp_mark, sizeof(uint32_t) * n));
     if (!c->pp_front) HIP_TRY(c, hipMalloc(&c->pp_front, sizeof(uint32_t) * 2 * n));
@@ -1003,6 +1018,16 @@ int solve_pushpull(mlmq_ctx *c, int32_t src, const mlmq_params &p, mlmq_timing *
         timing->waves = mlmq::kPushWaves * timing->work_blocks;
     }
     return MLMQ_OK;
+}
+
+// A solver leaves a call to the vertex queue: too much for what it is meant
+// for, or no memory.  Then what it did get is given back, for the queue's rings.
+bool gave_up(mlmq_ctx *c, int rc) {
+    if (rc == MLMQ_E_NOMEM) {
+        free_region_space(c);
+        free_pushpull_space(c);
+    }
+    return rc == MLMQ_E_NOMEM || rc == MLMQ_E_QUEUE_OVERFLOW;
 }
 
 // Statistics of a batch from its device counters and the queries' clock ticks.
@@ -1271,10 +1296,10 @@ int mlmq_solve(mlmq_ctx *c, int32_t src, const mlmq_params *params, mlmq_timing 
     c->solved = false;
     if (wants_regions(c, q.p)) {
         rc = solve_regions(c, src, q.p, timing);
-        if (rc != MLMQ_E_QUEUE_OVERFLOW) return rc;
+        if (!gave_up(c, rc)) return rc;
     } else if (wants_pushpull(c, q.p)) {
         rc = solve_pushpull(c, src, q.p, timing);
-        if (rc != MLMQ_E_QUEUE_OVERFLOW) return rc;
+        if (!gave_up(c, rc)) return rc;
     }
 
     const uint32_t nb = (uint32_t)q.p.buckets;
@@ -1416,7 +1441,7 @@ int mlmq_solve_batch(mlmq_ctx *c, const int32_t *sources, int32_t nq, const mlmq
     // (kRegionQueries: a record's query field.)
     if (wants_batch_regions(c, (uint32_t)nq, p)) {
         const int rrc = batch_regions(c, nq, p, timing);
-        if (rrc != MLMQ_E_QUEUE_OVERFLOW && rrc != MLMQ_E_NOMEM) return rrc;
+        if (!gave_up(c, rrc)) return rrc;
     }
 
     const double timeout_s = p.timeout_s > 0 ? p.timeout_s : 60.0;

@@ -182,7 +182,10 @@ int fail(mlmq_server *s, int code, const std::string &msg) {
     return code;
 }
 
+// (the runtime keeps the error until it is asked for: the next launch would
+// report it)
 int hip_fail(mlmq_server *s, hipError_t e, const char *what) {
+    (void)hipGetLastError();
     return fail(s, e == hipErrorOutOfMemory ? MLMQ_E_NOMEM : MLMQ_E_HIP,
                 std::string(what) + ": " + hipGetErrorString(e));
 }
@@ -967,6 +970,7 @@ int mlmq_server_create(int device, const mlmq_server_config *cfg, mlmq_server **
     }
     if (e != hipSuccess) {
         const int rc = e == hipErrorOutOfMemory ? MLMQ_E_NOMEM : MLMQ_E_HIP;
+        (void)hipGetLastError();
         mlmq_server_destroy(s);
         return rc;
     }
