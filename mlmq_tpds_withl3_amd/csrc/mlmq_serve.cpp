@@ -75,7 +75,8 @@ struct Lane {
     std::vector<uint32_t> caps;   // ring capacity (log2) each request ran with
     std::vector<Engine> engines;
     // of the region and push-pull solvers: their query tables and the outcomes
-    // (h_tab: pinned), control block and query times, ring
+    // (h_tab: pinned, behind them the region solver's summary), control block and
+    // query times, ring
     uint8_t *h_tab = nullptr, *d_tab = nullptr;
     uint32_t *ctl = nullptr;
     uint64_t *times = nullptr;
@@ -84,6 +85,7 @@ struct Lane {
     uint64_t *ring = nullptr;
     uint64_t ring_slots = 0;
     bool ring_dirty = true;
+    mlmq::RegionSummary *summary = nullptr;
     // push-pull state of requests whose slot has no room for it (allocated with
     // the first of them; pp_off: without it)
     uint8_t *pp = nullptr;
@@ -961,7 +963,8 @@ int mlmq_server_create(int device, const mlmq_server_config *cfg, mlmq_server **
         if (e == hipSuccess) e = hipHostMalloc((void **)&l.h_reqs, tb, hipHostMallocDefault);
         if (e == hipSuccess) e = hipMalloc((void **)&l.d_reqs, tb);
         const size_t side = kTabBytes * (size_t)c.max_batch;
-        if (e == hipSuccess) e = hipHostMalloc((void **)&l.h_tab, side, hipHostMallocDefault);
+        if (e == hipSuccess) e = hipHostMalloc((void **)&l.h_tab, side + sizeof(mlmq::RegionSummary), hipHostMallocDefault);
+        if (e == hipSuccess) l.summary = (mlmq::RegionSummary *)(l.h_tab + side);
         if (e == hipSuccess) e = hipMalloc((void **)&l.d_tab, side);
         if (e == hipSuccess) e = hipMalloc((void **)&l.ctl, sizeof(uint32_t) * mlmq::kCtlWords);
         if (e == hipSuccess) e = hipMalloc((void **)&l.progress, sizeof(mlmq::RegionProgress) * (size_t)c.max_batch);
@@ -1329,6 +1332,9 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
             R.ring = l.ring;
             R.ring_mask = (uint32_t)(l.ring_slots - 1);
             R.ctl = l.ctl;
+            l.summary->error = mlmq::kErrInternal;
+            l.summary->over = 0;
+            R.summary = l.summary;
             R.qtime = l.times;
             R.timeout_ticks = timeout_ticks;
             if (nregion > 1) R.table = (const mlmq::RegionQuery *)l.d_tab;
@@ -1361,7 +1367,7 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
         HIP_TRY(s, hipEventElapsedTime(&done_ms, s->ev_ref, l.ev_solve));
         std::vector<int32_t> rerun;   // overflowed requests, in launch order
         std::vector<mlmq::RowCopy> rows;
-        bool ring_used = false, ring_clean = true;
+        bool ring_used = false;
         for (size_t i = 0; i < l.ids.size(); ++i) {
             const int32_t id = l.ids[i];
             const int32_t gi = reqs[id].graph;
@@ -1373,10 +1379,7 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
             mlmq_serve_result &r = results[id];
             const int st = device_status(status);
             const bool queue = l.engines[i] == Engine::kQueue;
-            if (l.engines[i] == Engine::kRegions) {
-                ring_used = true;
-                ring_clean &= st == MLMQ_OK;
-            }
+            ring_used |= l.engines[i] == Engine::kRegions;
             if (st == MLMQ_E_QUEUE_OVERFLOW && (!queue || g.cap_log2 < 30)) {
                 // Run again: by the vertex queue, or with larger partitions
                 // (the graph's grow once per launch).
@@ -1407,7 +1410,9 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
             give_back(s, gi, sl);
             ++finished;
         }
-        if (ring_used && ring_clean) l.ring_dirty = false;
+        // (a launch that ended by an error leaves records, also where all its
+        // requests were over)
+        if (ring_used && l.summary->error == mlmq::kErrNone && l.summary->over) l.ring_dirty = false;
         // (no slot is handed out again before the next launch)
         const hipError_t copied = s->stage.copy(rows.data(), rows.size(), l.s);
         for (auto it = rerun.rbegin(); it != rerun.rend(); ++it) {

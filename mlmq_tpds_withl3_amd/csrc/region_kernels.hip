@@ -65,6 +65,11 @@
 // Whoever ends the last query publishes one exit record per workgroup of the
 // grid, for the ticket each of them takes last.
 //
+// Errors: a workgroup that sees the error word set or its deadline passed writes
+// its region's distances out and ends.  A region that is left this way with work
+// keeps its credit outstanding, so a query that was over by then has all of its
+// distances in the row, and no other one ends any more: qtime tells which.
+//
 // Measured, device us of one query, vertex queue / here: 2,052 vertices 190 / 41,
 // 264k 1250 / 430, 1.06M 4500 / 800-1000, 6.26M 5850 / 1850; 64 queries on 264k
 // 14100 / 2600.  Bound: hops one after another (about 0.25 us each inside a
@@ -500,10 +505,11 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
     dirty = seed != 0;
     for (uint32_t turn = 0;; ++turn) {
         if ((turn & 31u) == 0) {
-            if (uniform(ld_relaxed(a.ctl + kErrOff))) return;
+            // (after an error too the distances go out: this query may be over)
+            if (uniform(ld_relaxed(a.ctl + kErrOff))) break;
             if (wall_clock64() > deadline) {
                 region_raise(a, kErrTimeout);
-                return;
+                break;
             }
         }
         st.polls += lane == 0 ? 1u : 0u;
@@ -576,7 +582,7 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
         if (read_lane(was, 0) & kWork) return_credit(a, query, act, regions, st);   // a sender's credit covers the news
         else if (lane == 0) (void)fetch_or(act + region, kCounted);
     }
-    // the solve is over
+    // the query or the solve is over
     if (dirty)
         for (uint32_t i = lane; i < h.nv; i += kWave) {
             const uint32_t x = sh_ld(S.dist + local_id(i));

@@ -951,8 +951,9 @@ __global__ __launch_bounds__(kWaves * 64) void sssp_serve_kernel(ServeRequest *r
     }
 }
 
-// A region solve is sound when every credit was returned and taken; a
-// push-pull query is done when its last round left nothing.
+// A region solve is sound when every credit was returned and taken; where it
+// ended by an error, the queries that were over before it are done.  A push-pull
+// query is done when its last round left nothing.
 __global__ __launch_bounds__(256) void serve_outcome_kernel(ServeRequest *reqs, uint32_t nreq, const ServeOutcome *out) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nreq) return;
@@ -965,6 +966,7 @@ __global__ __launch_bounds__(256) void serve_outcome_kernel(ServeRequest *reqs, 
         e = o.ctl[kErrOff];
         const uint32_t tail = o.ctl[kTailOff];
         if (e == kErrNone && (o.ctl[kExitOff] != 1u || tail != o.ctl[kTakenOff] || tail != o.ctl[kDoneOff])) e = kErrInternal;
+        else if (e != kErrNone && o.time[1] != 0) e = kErrNone;
     }
     reqs[i].status = e;
     reqs[i].t_start = o.time[0];
