@@ -272,11 +272,11 @@ int validate_csr(mlmq_ctx *c, int32_t n, int64_t m, const int64_t *row, const in
 }
 
 // The cut into regions (region_graph.h), where the graph has one.  A packed
-// edge holds weights below 2^(32 - kWeightShift).  `col`: the destinations
+// edge holds weights below kNoWeight.  `col`: the destinations
 // on the host, or null to copy them from the device.
 int build_regions(mlmq_ctx *c, const std::vector<uint32_t> &row, const uint32_t *col) {
     const uint32_t n = (uint32_t)c->n;
-    if ((double)c->info.max_weight >= (double)(1u << (32 - mlmq::kWeightShift)) || c->m > 8ll * c->n ||
+    if ((double)c->info.max_weight >= (double)mlmq::kNoWeight || c->m > 8ll * c->n ||
         (uint32_t)c->info.max_nnz > mlmq::kRegionMaxDegree)
         return MLMQ_OK;
     std::vector<uint32_t> copy;

@@ -24,8 +24,8 @@
 // distance per slot) and one activity word per region beside the distance row.
 //
 // A graph is cut when the cut pays: few edges between regions (see
-// region_plan), every weight below 2^(32 - kWeightShift), and every region
-// within the limits below.
+// region_plan), every weight below kNoWeight, and every region within the limits
+// below.
 #pragma once
 
 #include <stdint.h>
@@ -40,6 +40,7 @@ constexpr uint32_t kRegionVerts = 1u << kRegionIdBits;
 constexpr uint32_t kBlocks = kRegionVerts / 64;
 constexpr uint32_t kWeightShift = 2 + kRegionIdBits;
 constexpr uint32_t kOffsetMask = (1u << kWeightShift) - 4u;
+constexpr uint32_t kNoWeight = ~0u >> kWeightShift;   // of an absent edge
 constexpr uint32_t kRegionExits = 384;     // exits and inbox slots of a region:
 constexpr uint32_t kRegionInbox = 384;     // 6 per lane of the wave that handles them
 constexpr uint32_t kRegionMaxDegree = 64;

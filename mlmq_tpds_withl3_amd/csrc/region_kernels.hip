@@ -246,7 +246,7 @@ __device__ __forceinline__ void run_relaxer(RegionLds &S, const RegionHdr &h, co
         last[i] = i * kStep + thread < h.nv ? start[i] : 0u;
 #pragma unroll
         for (uint32_t k = 0; k < kLaneEdges; ++k) {
-            if (edge[i][k] >> kWeightShift != ~0u >> kWeightShift) degrees += 1u << 8 * i;
+            if (edge[i][k] >> kWeightShift != kNoWeight) degrees += 1u << 8 * i;
         }
     }
     __syncthreads();
@@ -826,7 +826,7 @@ __global__ __launch_bounds__(256) void region_image_kernel(const uint32_t *row, 
         atomicMax(&most[p / kWave], inside);
         // absent edges: to the vertex itself, which they cannot lower
         for (uint32_t k = inside; k < kLaneEdges; ++k)
-            img[k * kRegionVerts + p] = own | ~0u << kWeightShift;
+            img[k * kRegionVerts + p] = own | kNoWeight << kWeightShift;
     }
     __syncthreads();
     if (threadIdx.x < kBlocks) img[kImageMost + threadIdx.x] = most[threadIdx.x];

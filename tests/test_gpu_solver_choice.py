@@ -77,3 +77,22 @@ def test_one_workgroup_per_cu_is_no_bound(loaded, name):
     free = solve(loaded, name, 3)
     assert solve(loaded, name, 3, work_blocks=CUS) == free
     assert solve(loaded, name, 3, work_blocks=2 * CUS) == free
+
+
+@pytest.mark.parametrize("top,waves", [((1 << 20) - 2, 10), ((1 << 20) - 1, 1)])
+def test_weight_of_the_absent_edge(top, waves):
+    """The region solver's packed edges keep one weight for edges that are not
+    there: a graph with that weight is not cut, and every examined edge counts."""
+    say(f"weights of {top}")
+    n = 1500
+    a = np.arange(n - 1)
+    src, dst = np.concatenate([a, a + 1]), np.concatenate([a + 1, a])
+    order = np.lexsort((dst, src))
+    row = np.concatenate([[0], np.cumsum(np.bincount(src, minlength=n))]).astype(np.int64)
+    g = (row, dst[order].astype(np.int32), np.full(len(order), top, dtype=np.int32))
+    with Solver(0) as s:
+        s.load_csr(*g)
+        t = s.solve(700, timeout_s=TIMEOUT)
+        dist, work, _ = O.dijkstra(*g, 700)
+        assert np.array_equal(s.dist(), dist)
+        assert t["waves"] == waves * t["work_blocks"] and t["relaxations"] >= work
