@@ -96,7 +96,7 @@ typedef struct mlmq_params {
     int32_t  batch_waves;     /* mlmq_solve_batch: waves per query (workgroup size), 4, 8 or 16;
                                  default 8 */
     int32_t  use_graph;       /* mlmq_solve_batch: replay the launch as a captured hipGraph
-                                 (default 1) */
+                                 (default 1; the region solver's two launches are not captured) */
     int32_t  hub_split;       /* 1: a popped hub (> 2048 out-edges) keeps its first 1024-edge
                                  chunk and sends the rest to L2 as chunk records that other
                                  waves relax (with light_split: the heavy-phase part only);
@@ -185,10 +185,10 @@ typedef struct mlmq_batch_timing {
     double   query_ms_max;
     double   query_ms_mean;
     int32_t  queries;
-    int32_t  work_blocks;     /* workgroups = queries in flight */
-    int32_t  waves_per_query;
-    int32_t  graph_replay;    /* 1 if the launch was a hipGraph replay */
-    int64_t  bucket_capacity;
+    int32_t  work_blocks;     /* queries in flight at once (vertex queue: its workgroups) */
+    int32_t  waves_per_query; /* of these, each (region solver: its waves shared among them) */
+    int32_t  graph_replay;    /* 1 if the launch was a hipGraph replay (vertex queue) */
+    int64_t  bucket_capacity; /* ring slots per bucket (region solver: of its one ring) */
     uint64_t relaxations;
     uint64_t improvements;
     uint64_t l2_pushes;

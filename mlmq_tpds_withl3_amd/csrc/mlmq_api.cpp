@@ -1058,7 +1058,8 @@ void fill_batch_timing(mlmq_ctx *c, const uint32_t *h, const std::vector<uint64_
     timing->idle_polls = st[mlmq::kStatIdle];
 }
 
-// A batch by the region solver: every query of it in flight at once.
+// A batch by the region solver: one launch, region_admit queries of it in flight
+// at a time.
 int batch_regions(mlmq_ctx *c, int32_t nq, const mlmq_params &p, mlmq_batch_timing *timing) {
     uint32_t relaxers = 0, grid = 0;
     int rc = region_grid(c, (uint32_t)nq, 0, &relaxers, &grid);
@@ -1074,7 +1075,8 @@ int batch_regions(mlmq_ctx *c, int32_t nq, const mlmq_params &p, mlmq_batch_timi
     HIP_TRY(c, hipMemcpy(qt.data(), c->b_qtime, sizeof(uint64_t) * qt.size(), hipMemcpyDeviceToHost));
     // (the launch counts its row reset, as the vertex queue's does)
     fill_batch_timing(c, c->ctl_host.data(), qt, nq, ms_since(t.q0, t.s1), t.device_ms + ms_since(t.q0, t.q1), p, timing);
-    timing->work_blocks = nq;
+    timing->work_blocks = (int32_t)mlmq::region_admit(c->regions.regions, (uint32_t)nq, grid);
+    timing->waves_per_query = std::max(1, mlmq::region_waves(relaxers) * (int32_t)grid / timing->work_blocks);
     timing->bucket_capacity = (int64_t)c->r_ring_slots;
     if (!p.batch_stats)
         timing->relaxations = timing->improvements = timing->stale = timing->batches = timing->idle_polls = 0;

@@ -96,3 +96,22 @@ def test_weight_of_the_absent_edge(top, waves):
         dist, work, _ = O.dijkstra(*g, 700)
         assert np.array_equal(s.dist(), dist)
         assert t["waves"] == waves * t["work_blocks"] and t["relaxations"] >= work
+
+
+@pytest.mark.parametrize("nq", [3, 64])
+def test_batch_reports_its_queries_in_flight(loaded, nq):
+    """A batch on the region solver admits a few queries at a time (70 regions
+    each: about a thirtieth of its at most 1024 or, for few queries, 512
+    workgroups, all of them where these are more than the queries)."""
+    say(f"batch of {nq}: queries in flight")
+    s, g = loaded["road"]
+    src = np.random.default_rng(nq).integers(0, 70_001, nq).astype(np.int32)
+    t = s.solve_batch(src, timeout_s=TIMEOUT)
+    for i in (0, nq // 2, nq - 1):
+        assert np.array_equal(s.batch_dist(i), O.dijkstra(*g, int(src[i]))[0])
+    assert t["graph_replay"] == 0
+    in_flight = int(1024 * 0.27 / 70 ** 0.5) if nq == 64 else 3
+    assert t["work_blocks"] == in_flight
+    # 1024 workgroups of six waves, or three times 70 of ten
+    waves = 6 * 1024 if nq == 64 else 10 * 210
+    assert t["waves_per_query"] == waves // in_flight
