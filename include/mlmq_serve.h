@@ -76,6 +76,10 @@ extern "C" {
 #define MLMQ_SERVE_LANES 0     /* mlmq_server_run: launches of waiting requests on launch lanes */
 #define MLMQ_SERVE_LIVE  1     /* mlmq_server_run: the persistent launch of live serving */
 
+#define MLMQ_SOLVER_QUEUE     0
+#define MLMQ_SOLVER_REGIONS   1
+#define MLMQ_SOLVER_PUSH_PULL 2
+
 typedef struct mlmq_server mlmq_server;
 
 typedef struct mlmq_server_config {
@@ -137,7 +141,7 @@ typedef struct mlmq_serve_result {
     int32_t  launch;          /* launch sequence number */
     int32_t  batch_size;      /* requests in that launch */
     int32_t  retries;         /* overflow reruns of this request */
-    int32_t  reserved;
+    int32_t  solver;          /* that answered: MLMQ_SOLVER_QUEUE, _REGIONS or _PUSH_PULL */
 } mlmq_serve_result;
 
 typedef struct mlmq_serve_stats {

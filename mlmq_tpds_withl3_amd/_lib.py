@@ -23,6 +23,7 @@ ERRORS = {
 }
 MLMQ_E_PENDING = -11
 SERVE_MODES = {"lanes": 0, "live": 1}
+SERVE_SOLVERS = ("queue", "regions", "push-pull")   # mlmq_serve_result.solver
 QUEUE_MODES = {"L1SLF_L2DQ": 19, "L1N_L2DQ": 1, "L1V_L2DQ": 0}
 NOALLOC_RING_SLOTS = 1 << 23   # MLMQ_NOALLOC_RING_SLOTS
 
@@ -181,7 +182,7 @@ class ServeResult(ctypes.Structure):
         ("device_ms", ctypes.c_double), ("status", ctypes.c_int32),
         ("mismatches", ctypes.c_int32), ("launch", ctypes.c_int32),
         ("batch_size", ctypes.c_int32), ("retries", ctypes.c_int32),
-        ("reserved", ctypes.c_int32),
+        ("solver", ctypes.c_int32),
     ]
 
 

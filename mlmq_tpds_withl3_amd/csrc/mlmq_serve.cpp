@@ -54,7 +54,9 @@ struct GraphEntry {
 };
 
 // Solver of a request in a launch lane.
-enum class Engine : uint8_t { kQueue, kRegions, kPushPull };
+enum class Engine : uint8_t {
+    kQueue = MLMQ_SOLVER_QUEUE, kRegions = MLMQ_SOLVER_REGIONS, kPushPull = MLMQ_SOLVER_PUSH_PULL
+};
 
 // Most ring slots of a lane's region solver (8 MiB); requests that would need
 // more of them in one launch go to the vertex queue.
@@ -1397,6 +1399,7 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
                 continue;
             }
             r.status = st;
+            r.solver = (int32_t)l.engines[i];
             r.retries = retries[id];
             r.latency_ms = (double)done_ms - 1000.0 * reqs[id].arrival_s;
             r.device_ms = te > ts ? (double)(te - ts) / (double)s->wall_khz : 0.0;

@@ -19,7 +19,7 @@ from ._lib import (MLMQ_E_PENDING, MLMQError, SERVE_MODES, ServeGraphParams, Ser
 
 STATUS = {0: "ok", -4: "nomem", -6: "overflow", -7: "timeout", -8: "internal", -10: "rejected"}
 RESULT_FIELDS = ("latency_ms", "queue_ms", "device_ms", "status", "mismatches", "launch", "batch_size",
-                 "retries")
+                 "retries", "solver")
 
 
 def _check(rc: int, h) -> None:
@@ -129,7 +129,7 @@ class Server:
         _check(self._L.mlmq_server_run(self._h, reqs, n, res, ctypes.byref(st)), self._h)
         dt = np.dtype([("latency_ms", "f8"), ("queue_ms", "f8"), ("device_ms", "f8"),
                        ("status", "i4"), ("mismatches", "i4"), ("launch", "i4"),
-                       ("batch_size", "i4"), ("retries", "i4"), ("reserved", "i4")])
+                       ("batch_size", "i4"), ("retries", "i4"), ("solver", "i4")])
         rec = np.frombuffer(bytes(res), dtype=dt, count=n).copy() if n else np.zeros(0, dt)
         return rec, st.as_dict()
 
