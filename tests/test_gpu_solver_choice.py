@@ -3,7 +3,8 @@ number of workgroups below the number of CUs (256) bounds the region and the
 push-pull solver too, from there on they take what they need; with fewer
 workgroups than a 32nd of a graph's regions the vertex queue answers.  The
 timing tells the solver by the waves of a workgroup: one (vertex queue), six or
-ten (regions), eight (push-pull).  Every row is compared with the oracle, bit
+ten (regions), eight (push-pull).  Also the limits of a region (384 exits and
+384 inbox slots), the largest packed weight, and what a solver counts.  Every row is compared with the oracle, bit
 for bit."""
 import sys
 
@@ -115,3 +116,44 @@ def test_batch_reports_its_queries_in_flight(loaded, nq):
     # 1024 workgroups of six waves, or three times 70 of ten
     waves = 6 * 1024 if nq == 64 else 10 * 210
     assert t["waves_per_query"] == waves // in_flight
+
+
+def block_with_exits(exits, entries):
+    """Consecutive blocks of 1024 vertices, each a chain, of which the first has
+    exactly so many edges out of it and into it."""
+    n = 40 * 1024
+    a = np.arange(n - 1)
+    a = a[(a + 1) % 1024 != 0]
+    far = np.arange(2048, n, 61)
+    src = np.concatenate([a, a + 1, a, np.arange(exits) % 1024, far[:entries]])
+    dst = np.concatenate([a + 1, a, a + 1, far[:exits], np.arange(entries) % 1024])
+    w = np.random.default_rng(exits + entries).integers(1, 1000, len(src))
+    order = np.lexsort((dst, src))
+    row = np.concatenate([[0], np.cumsum(np.bincount(src, minlength=n))]).astype(np.int64)
+    return row, dst[order].astype(np.int32), w[order].astype(np.int32)
+
+
+@pytest.mark.parametrize("exits,entries,waves", [(384, 384, 10), (385, 10, 1), (10, 385, 1)])
+def test_limits_of_a_region(exits, entries, waves):
+    say(f"a region of {exits} exits and {entries} inbox slots")
+    g = block_with_exits(exits, entries)
+    with Solver(0) as s:
+        s.load_csr(*g)
+        for src in (0, 700, 5000):
+            t = s.solve(src, timeout_s=TIMEOUT)
+            assert np.array_equal(s.dist(), O.dijkstra(*g, src)[0])
+            assert t["waves"] == waves * t["work_blocks"]
+
+
+def test_push_pull_counts(loaded):
+    """Every reached vertex but the source is lowered and queued at least once,
+    each over an edge that is examined."""
+    say("push-pull counts")
+    s, g = loaded["power"]
+    for src in (0, 5, 77):
+        t = s.solve(src, timeout_s=TIMEOUT)
+        dist = s.dist()
+        reached = int((dist < 0x7FFFFFFF).sum())
+        assert reached > 1000 and t["waves"] == 8 * t["work_blocks"]
+        assert t["improvements"] >= reached - 1 and t["relaxations"] >= t["improvements"]
+        assert t["l2_pushes"] >= reached
