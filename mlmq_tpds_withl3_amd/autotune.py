@@ -26,6 +26,27 @@ def default_delta(row, w) -> int:
     return max(1, int(8 * float(w.mean()))) if len(w) else 1
 
 
+# What chooses a solver for a single query, or bounds it: the region and the
+# push-pull solver do not depend on any other setting.
+_CHOOSING = ("queue", "queue_mode", "work_blocks", "blocks_per_cu", "light_split", "hub_split", "l1_blocks",
+             "defer_heavy", "strict_window", "l1_donate", "profile", "bucket_capacity")
+
+
+def _choosing(params: dict) -> tuple:
+    return tuple(sorted((k, v) for k, v in params.items() if k in _CHOOSING))
+
+
+def _by_queue(timing: dict) -> bool:
+    """Whether the vertex queue answered: its workgroups are of one wave."""
+    return timing.get("waves", 1) == timing.get("work_blocks", 1)
+
+
+def _solvers(results):
+    """Solvers of served requests (0: the vertex queue)."""
+    names = results.dtype.names if hasattr(results, "dtype") else results
+    return results["solver"] if "solver" in names else np.zeros(1)
+
+
 def tune_single(solver, src, deltas, grid=None, repeats: int = 2, confirm: int = 7,
                 log=None) -> dict:
     """Grid search for single queries from `src` (one source or a list of
@@ -36,7 +57,9 @@ def tune_single(solver, src, deltas, grid=None, repeats: int = 2, confirm: int =
     child-block touches off at the four best after that.  Each
     point is the best device time of `repeats` solves per source; the four
     best are then timed `confirm` times more and the lowest median wins (a
-    best-of-two is often a lucky draw).  Returns the best point, its median
+    best-of-two is often a lucky draw).  Points that the region or the
+    push-pull solver would answer like one already measured are left out: the
+    queue's settings mean nothing to them.  Returns the best point, its median
     and the whole table.  Tune on other sources than the one a benchmark
     then times, so the point is not fitted to the measured query."""
     from .solver import default_params
@@ -49,11 +72,16 @@ def tune_single(solver, src, deltas, grid=None, repeats: int = 2, confirm: int =
                 for pop, mr, lb in ((32, 32, 8), (32, 32, 32), (32, 16, 16), (32, 8, 8), (32, 4, 4),
                                     (64, 8, 8))]
     table = []
+    elsewhere = set()   # choosing settings with which another solver answered
 
     def measure(params):
+        if _choosing(params) in elsewhere:
+            return
         p = default_params(timeout_s=30.0, **params)
-        ms = float(np.mean([min(solver.solve(s, p)["device_ms"] for _ in range(repeats))
-                            for s in sources]))
+        runs = [[solver.solve(s, p) for _ in range(repeats)] for s in sources]
+        if not any(_by_queue(t) for r in runs for t in r):
+            elsewhere.add(_choosing(params))
+        ms = float(np.mean([min(t["device_ms"] for t in r) for r in runs]))
         table.append((params, ms))
         if log:
             log(f"tune single: {params} -> {ms:.3f} ms")
@@ -98,7 +126,13 @@ def tune_serving(server, gid: int, sources, base: dict | None = None, burst: int
     burst does not see.  So each candidate also serves `lone` requests one at
     a time, and a candidate whose median lone latency exceeds the starting
     point's by more than `lone_slack` is not taken (None: throughput only);
-    the starting point (`base`) should be the single-query tuned parameters."""
+    the starting point (`base`) should be the single-query tuned parameters.
+
+    In launch lanes the region and the push-pull solver answer bursts and lone
+    requests alike, whatever the settings; these are for what crowded lanes
+    leave to the vertex queue.  There every candidate is scored with the bucket
+    capacity given that the queue takes by itself, which selects it, and by
+    throughput alone."""
     rng = np.random.default_rng(7)
     src = np.asarray(sources, dtype=np.int32)[rng.integers(0, len(sources), size=burst)]
     arrival = np.zeros(burst)
@@ -117,8 +151,15 @@ def tune_serving(server, gid: int, sources, base: dict | None = None, burst: int
             lat.append(float(res["latency_ms"][0]))
         return float(np.median(lat))
 
+    only_queue = {}
+    server.set_graph_params(gid, **cur)
+    first = server.run(np.zeros(1), gsel[:1], src[:1])[0]
+    if np.any(_solvers(first)):
+        only_queue["bucket_capacity"] = max(8192, server.sizes[gid][0] // 32)
+        lone_slack = None
+
     def score(params):
-        server.set_graph_params(gid, **params)
+        server.set_graph_params(gid, **params, **only_queue)
         best = 0.0
         for _ in range(repeats):
             res, st = server.run(arrival, gsel, src)
@@ -160,7 +201,9 @@ def tune_serving(server, gid: int, sources, base: dict | None = None, burst: int
 def tune_batch(solver, sources, base: dict | None = None, log=None) -> dict:
     """Tune a batched launch (``Solver.solve_batch``) over the same sources:
     scored by batch wall time (the best of two timed launches after one
-    untimed one)."""
+    untimed one).  Where the region solver answers the batch (its launch is no
+    captured graph) the settings mean nothing, and the starting point is
+    returned."""
     from ._lib import MLMQError
     from .solver import default_params
 
@@ -171,11 +214,15 @@ def tune_batch(solver, sources, base: dict | None = None, log=None) -> dict:
     # it, and the shape coordinates below move with the stale-check mode
     cur.setdefault("stale_check", 1)
 
+    by_regions = False
+
     def score(params):
+        nonlocal by_regions
         p = default_params(timeout_s=60.0, **params)
         best = float("inf")
         try:
-            solver.solve_batch(sources, p)
+            t = solver.solve_batch(sources, p)
+            by_regions = p.use_graph != 0 and t.get("graph_replay", 1) == 0
             for _ in range(2):
                 t0 = time.perf_counter()
                 solver.solve_batch(sources, p)
@@ -186,6 +233,8 @@ def tune_batch(solver, sources, base: dict | None = None, log=None) -> dict:
 
     best_t = score(cur)
     trail = [(dict(cur), best_t)]
+    if by_regions:
+        return {"params": cur, "batch_s": best_t, "trail": trail}
     # Shape first, then the child-block touches and the stale-check mode
     # (with the whole device busy the touches can cost more memory-side
     # bandwidth than they save), then delta, the bucket count and the queue
