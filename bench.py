@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Single-query SSSP benchmark of the MI355X MLMQ solver.
 
-A step is one exact single-source query (reset + persistent solve) on the
+A step is one exact single-source query (reset + solve) on the
 resident graph.  Default workload: the 6,262,104-vertex road-like graph
 (seeded 3-NN points in the unit square, symmetrised, Morton-ordered, weights
 = scaled Euclidean length with the longest edge at 100,000), source = the
@@ -9,9 +9,9 @@ vertex nearest the centroid, delta 200000, queue L1SLF_L2DQ.
 
 Prints ONE JSON line (rank 0).  value = GTEPS over the timed steps
 (E_r * steps / wall seconds, E_r = out-degree sum of reachable vertices);
-ms_per_step = wall ms per step.  "roofline" prices the persistent kernel's
-algorithmic bytes B = 16 V_r + 12 E_r per query against its HIP-event
-duration and the 8 TB/s HBM peak.  "cpu_baseline" is the CPU oracle
+ms_per_step = wall ms per step.  "roofline" prices the algorithmic bytes
+B = 16 V_r + 12 E_r of a query against its device time and the 8 TB/s HBM
+peak.  "cpu_baseline" is the CPU oracle
 (single-thread binary-heap Dijkstra) on the same graph and source.
 """
 import argparse
@@ -46,26 +46,33 @@ def cpu_model():
 # ---- HBM traffic of the timed point (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE) ----
 
 TRAFFIC_KEYS = ("workload", "queue", "delta", "buckets", "bucket_window", "l2_batch", "min_read",
-                "l1_pop", "l1_donate", "light_split", "stale_check", "prefetch", "work_blocks")
+                "l1_pop", "l1_donate", "light_split", "stale_check", "prefetch", "work_blocks", "kernel")
 
 
-def traffic_key(workload, queue, delta, args, work_blocks):
-    """Canonical text of every setting that changes the persistent kernel's
-    memory traffic: a traffic figure is attached to a bench line only when it
-    was measured at exactly this point."""
+def traffic_key(workload, queue, delta, args, work_blocks, kernel):
+    """Canonical text of every setting that changes a query's memory traffic,
+    and the kernel that answered: a traffic figure is attached to a bench line
+    only when it was measured at exactly this point."""
     cfg = {"workload": workload, "queue": queue, "delta": int(delta), "buckets": args.buckets,
            "bucket_window": args.window, "l2_batch": args.l2_batch, "min_read": args.min_read,
            "l1_pop": args.l1_pop, "l1_donate": args.l1_donate, "light_split": args.light_split,
            "stale_check": args.stale_check, "prefetch": args.prefetch,
-           "work_blocks": int(work_blocks)}
+           "work_blocks": int(work_blocks), "kernel": kernel}
     return json.dumps({k: cfg[k] for k in TRAFFIC_KEYS}, sort_keys=True)
 
 
-def solver_kernel(timing):
-    """Kernel of the solver that answered a query, by the waves of its
-    workgroups (one, or six or ten, or eight)."""
+# Per solver: the kernel a bench line names, and the kernels of a query, of
+# which the last is launched once per query.
+SOLVERS = {"queue": ("sssp_persistent_kernel", ("sssp_persistent_kernel",)),
+           "regions": ("region_solver_kernel", ("region_solver_kernel",)),
+           "push-pull": ("push_kernel", ("push_kernel", "pull_kernel"))}
+
+
+def solver_of(timing):
+    """Solver that answered a query, by the waves of its workgroups (one, or six
+    or ten, or eight)."""
     per = timing["waves"] // max(1, timing["work_blocks"])
-    return {1: "sssp_persistent_kernel", 8: "push_kernel"}.get(per, "region_solver_kernel")
+    return {1: "queue", 8: "push-pull"}.get(per, "regions")
 
 
 def load_traffic(path, key):
@@ -77,26 +84,29 @@ def load_traffic(path, key):
     return entry["bytes_per_launch"] if entry else None
 
 
-def _counter_means(d, counter, kernel):
-    """Mean over dispatches of `kernel` of `counter` (summed per dispatch) in
-    the rocprofv3 counter_collection CSVs under directory d."""
+def _counter_means(d, counter, kernels):
+    """Sum of `counter` over the dispatches of `kernels` in the rocprofv3
+    counter_collection CSVs under directory d, per dispatch of the last of
+    them, and the number of these."""
     import csv
     import glob
-    per = {}
+    total, dispatches = 0.0, set()
     files = glob.glob(os.path.join(d, "**", "*counter_collection.csv"), recursive=True)
     for f in files:
         for r in csv.DictReader(open(f)):
-            if r.get("Counter_Name") != counter or kernel not in r.get("Kernel_Name", ""):
+            name = r.get("Kernel_Name", "")
+            if r.get("Counter_Name") != counter or not any(k in name for k in kernels):
                 continue
-            k = (f, r.get("Dispatch_Id") or r.get("Correlation_Id"))
-            per[k] = per.get(k, 0.0) + float(r["Counter_Value"])
-    if not per:
-        raise SystemExit(f"no {counter} rows of {kernel} under {d}")
-    return sum(per.values()) / len(per), len(per)
+            total += float(r["Counter_Value"])
+            if kernels[-1] in name:
+                dispatches.add((f, r.get("Dispatch_Id") or r.get("Correlation_Id")))
+    if not dispatches:
+        raise SystemExit(f"no {counter} rows of {kernels[-1]} under {d}")
+    return total / len(dispatches), len(dispatches)
 
 
 def traffic_update(args):
-    """Bytes per launch of the persistent kernel from two counter runs of the
+    """Bytes per query of the kernels that answer it from two counter runs of the
     bench, each scaled by what the same counter reads for a plain copy kernel
     of known size, stored under the bench line's traffic key."""
     line_path, fdir, wdir, cfdir, cwdir = args.traffic_update
@@ -108,11 +118,11 @@ def traffic_update(args):
     if line is None:
         raise SystemExit(f"no bench line in {line_path}")
     key = line["roofline"]["traffic_key"]
-    kern = line["roofline"]["kernel"]
-    fetch, nf = _counter_means(fdir, "FETCH_SIZE", kern)
-    write, nw = _counter_means(wdir, "WRITE_SIZE", kern)
-    cfetch, _ = _counter_means(cfdir, "FETCH_SIZE", "copy_u32_kernel")
-    cwrite, _ = _counter_means(cwdir, "WRITE_SIZE", "copy_u32_kernel")
+    kernels = next(k for name, k in SOLVERS.values() if name == line["roofline"]["kernel"])
+    fetch, nf = _counter_means(fdir, "FETCH_SIZE", kernels)
+    write, nw = _counter_means(wdir, "WRITE_SIZE", kernels)
+    cfetch, _ = _counter_means(cfdir, "FETCH_SIZE", ("copy_u32_kernel",))
+    cwrite, _ = _counter_means(cwdir, "WRITE_SIZE", ("copy_u32_kernel",))
     fscale = args.copy_bytes / 1024.0 / cfetch
     wscale = args.copy_bytes / 1024.0 / cwrite
     fb, wb = fetch * 1024.0 * fscale, write * 1024.0 * wscale
@@ -124,7 +134,7 @@ def traffic_update(args):
                "write_bytes": int(round(wb)), "fetch_kib_raw": fetch, "write_kib_raw": write,
                "dispatches": [nf, nw], "fetch_scale": fscale, "write_scale": wscale,
                "device_ms_of_line": line["device_ms"]["mean"],
-               "note": f"rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE per dispatch of {kern}, scaled "
+               "note": f"rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of {' and '.join(kernels)} per query, scaled "
                        f"by the same counters on a {args.copy_bytes}-byte copy kernel"}
     with open(args.traffic_json, "w") as f:
         json.dump(tj, f, indent=1, sort_keys=True)
@@ -300,9 +310,11 @@ def main():
             runs = sorted(solver.solve(src, make_params(int(d)))["device_ms"] for _ in range(3))
             table[str(int(d))] = round(runs[1], 4)
         return table
-    sweep = sweep_ms(spec["delta_sweep"]) if args.delta_sweep else None
+    # (no other solver than the vertex queue depends on delta)
+    swept = args.delta_sweep and solver_of(solver.solve(src, params)) == "queue"
+    sweep = sweep_ms(spec["delta_sweep"]) if swept else None
     log(f"delta sweep (median of 3, device ms): {sweep}")
-    extended = sweep_ms((2_000_000, 20_000_000)) if args.extended_sweep and args.delta_sweep else None
+    extended = sweep_ms((2_000_000, 20_000_000)) if args.extended_sweep and swept else None
     if extended:
         log(f"outside the configured sweep: {extended}")
     for i in range(args.warmup):
@@ -359,7 +371,8 @@ def main():
     dev_avg_s = statistics.mean(dev_ms) / 1e3
     achieved = b_alg / dev_avg_s / 1e9
     last = timings[-1]
-    tkey = traffic_key(args.workload, args.queue, delta, args, last["work_blocks"])
+    kernel = SOLVERS[solver_of(last)][0]
+    tkey = traffic_key(args.workload, args.queue, delta, args, last["work_blocks"], kernel)
     traffic = load_traffic(args.traffic_json, tkey)
     last = timings[-1]
     out = {
@@ -381,7 +394,7 @@ def main():
             "reachable_vertices": v_r, "reachable_edges": e_r,
             "weight_scale": spec.get("weight_scale_applied"),
             "seed": spec.get("seed"),
-            "queue": args.queue, "delta": delta,
+            "queue": args.queue, "solver": solver_of(last), "delta": delta,
             "delta_sweep_device_ms": sweep,
             "outside_sweep_device_ms": extended,
             "point": "tuned on other sources" if tuned_on else
@@ -416,7 +429,7 @@ def main():
             "frac": round(achieved / HBM_PEAK_GBS, 8),
             "traffic": traffic,
             "traffic_key": tkey,
-            "kernel": solver_kernel(last),
+            "kernel": kernel,
             "bytes_per_launch": b_alg,
         },
         "cpu_baseline": {
