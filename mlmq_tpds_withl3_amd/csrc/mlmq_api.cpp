@@ -15,6 +15,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -257,38 +258,70 @@ void compute_info(mlmq_graph_info *gi, int32_t n, int64_t m, const int64_t *row6
 
 // Shared validation of a host CSR (0-based starts, row[n] = m).
 int validate_csr(mlmq_ctx *c, int32_t n, int64_t m, const int64_t *row, const int32_t *col,
-                 const int32_t *w) {
+                 const int32_t *w, int32_t *max_weight) {
     if (n <= 0 || n >= 0x7FFFFFFF) return fail(c, MLMQ_E_INVALID, "vertex count out of range");
     if (m < 0 || m >= 0x7FFFFFFF) return fail(c, MLMQ_E_INVALID, "edge count out of range");
     if (!row || (m > 0 && (!col || !w))) return fail(c, MLMQ_E_INVALID, "null CSR array");
     if (row[0] != 0 || row[n] != m) return fail(c, MLMQ_E_INVALID, "row[0] != 0 or row[n] != m");
     for (int32_t u = 0; u < n; ++u)
         if (row[u + 1] < row[u]) return fail(c, MLMQ_E_INVALID, "row offsets not monotone");
+    int32_t most = 0;
     for (int64_t e = 0; e < m; ++e) {
         if (col[e] < 0 || col[e] >= n) return fail(c, MLMQ_E_INVALID, "destination out of range");
         if (w[e] < 0) return fail(c, MLMQ_E_INVALID, "negative edge weight");
+        most = std::max(most, w[e]);
     }
+    *max_weight = most;
     return MLMQ_OK;
 }
 
-// The cut into regions (region_graph.h), where the graph has one.  A packed
-// edge holds weights below kNoWeight.  `col`: the destinations
-// on the host, or null to copy them from the device.
-int build_regions(mlmq_ctx *c, const std::vector<uint32_t> &row, const uint32_t *col) {
-    const uint32_t n = (uint32_t)c->n;
-    if ((double)c->info.max_weight >= (double)mlmq::kNoWeight || c->m > 8ll * c->n ||
-        (uint32_t)c->info.max_nnz > mlmq::kRegionMaxDegree)
-        return MLMQ_OK;
-    std::vector<uint32_t> copy;
-    if (!col) {
-        copy.resize((size_t)c->m);
-        if (c->m)
-            HIP_TRY(c, hipMemcpy(copy.data(), c->col, sizeof(uint32_t) * (size_t)c->m, hipMemcpyDeviceToHost));
-        col = copy.data();
+// The cut of a graph, made on a thread of its own beside the rest of the load
+// (it needs the host's CSR alone).  Arrays and this object live until it is done.
+class PlanAhead {
+public:
+    PlanAhead() = default;
+    PlanAhead(const PlanAhead &) = delete;
+    ~PlanAhead() { join(); }
+    void start(uint32_t n, const uint32_t *row, const uint32_t *col) {
+        if (n < kAtOnce) return run(n, row, col);
+        try {
+            thread_ = std::thread([this, n, row, col]() { run(n, row, col); });
+        } catch (const std::system_error &) {
+            run(n, row, col);
+        }
     }
-    mlmq::RegionPlan plan;
-    if (!mlmq::region_plan(n, row.data(), col, &plan)) return MLMQ_OK;
-    const hipError_t e = mlmq::region_build(plan, n, (uint64_t)c->m, c->row, c->col, c->wgt,
+    // Null: the graph is not cut.
+    const mlmq::RegionPlan *get() {
+        join();
+        return good_ ? &plan_ : nullptr;
+    }
+
+private:
+    // (a thread costs 30 us)
+    static constexpr uint32_t kAtOnce = 8192;
+    void run(uint32_t n, const uint32_t *row, const uint32_t *col) noexcept {
+        try {
+            good_ = mlmq::region_plan(n, row, col, &plan_);
+        } catch (const std::bad_alloc &) {
+            good_ = false;
+        }
+    }
+    void join() {
+        if (thread_.joinable()) thread_.join();
+    }
+    std::thread thread_;
+    mlmq::RegionPlan plan_;
+    bool good_ = false;
+};
+
+bool worth_a_plan(int32_t n, int64_t m, double max_weight) {
+    return max_weight < (double)mlmq::kNoWeight && m <= 8ll * n;
+}
+
+// The graph's regions on the device (region_graph.h), from its cut.
+int build_regions(mlmq_ctx *c, const mlmq::RegionPlan *plan) {
+    if (!plan) return MLMQ_OK;
+    const hipError_t e = mlmq::region_build(*plan, (uint32_t)c->n, (uint64_t)c->m, c->row, c->col, c->wgt,
                                             (double)c->info.avg_weight, c->stream, &c->regions);
     // past a limit, or no memory for the cut: the vertex queue serves the graph
     if (e == hipErrorInvalidValue || e == hipErrorOutOfMemory) {
@@ -341,7 +374,7 @@ int build_pushpull(mlmq_ctx *c, const int32_t *w) {
 // table: vertices with more than kSplitDeg out-edges, highest degree first,
 // at most kMaxHubs of them, each with a chunk size that keeps its chunk count
 // below 2^kChunkBits.
-int build_blocks(mlmq_ctx *c, const uint32_t *host_col) {
+int build_blocks(mlmq_ctx *c) {
     HIP_TRY(c, hipMalloc(&c->blocks, 64 * (size_t)c->n));
     // Back-edge slots fit when vertex ids and weights stay below 2^kBackShift
     // (the weight statistic is a float: rounding can only refuse a graph
@@ -379,17 +412,20 @@ int build_blocks(mlmq_ctx *c, const uint32_t *host_col) {
         HIP_TRY(c, hipStreamSynchronize(c->stream));
     }
     if (c->stage.reserve(sizeof(int32_t) * (size_t)c->n) != hipSuccess) (void)hipGetLastError();
-    return build_regions(c, row, host_col);
+    return MLMQ_OK;
 }
 
 int upload(mlmq_ctx *c, int32_t n, int64_t m, const int64_t *row, const int32_t *col,
            const int32_t *w) {
-    int rc = validate_csr(c, n, m, row, col, w);
+    int32_t max_weight = 0;
+    int rc = validate_csr(c, n, m, row, col, w, &max_weight);
     if (rc) return rc;
     HIP_TRY(c, hipSetDevice(c->device));
     free_graph(c);
     std::vector<uint32_t> row32((size_t)n + 1);
     for (int64_t i = 0; i <= n; ++i) row32[i] = (uint32_t)row[i];
+    PlanAhead plan;
+    if (worth_a_plan(n, m, max_weight)) plan.start((uint32_t)n, row32.data(), reinterpret_cast<const uint32_t *>(col));
     const size_t me = (size_t)(m > 0 ? m : 1);
     // The adjacency of every vertex with more than kInlineEdges edges (the
     // ones relaxed through the CSR) is sorted by (weight, destination): the
@@ -440,7 +476,8 @@ int upload(mlmq_ctx *c, int32_t n, int64_t m, const int64_t *row, const int32_t 
     c->m = m;
     compute_info(&c->info, n, m, row, nullptr, w);
     c->sorted = true;
-    rc = build_blocks(c, reinterpret_cast<const uint32_t *>(col));
+    rc = build_blocks(c);
+    if (rc == MLMQ_OK) rc = build_regions(c, plan.get());
     return rc ? rc : build_pushpull(c, w);
 }
 
@@ -1258,7 +1295,15 @@ int mlmq_attach_device_csr(mlmq_ctx *c, int32_t n, int64_t m, const int32_t *row
     c->n = n;
     c->m = m;
     compute_info(&c->info, n, m, nullptr, row.data(), w.data());
-    return build_blocks(c, nullptr);
+    const int rc = build_blocks(c);
+    if (rc || !worth_a_plan(n, m, c->info.max_weight)) return rc;
+    std::vector<uint32_t> col((size_t)m);
+    if (m > 0) HIP_TRY(c, hipMemcpy(col.data(), c->col, sizeof(uint32_t) * (size_t)m, hipMemcpyDeviceToHost));
+    for (const uint32_t v : col)
+        if (v >= (uint32_t)n) return MLMQ_OK;   // (nothing checks the destinations of an attached graph)
+    PlanAhead plan;
+    plan.start((uint32_t)n, row.data(), col.data());
+    return build_regions(c, plan.get());
 }
 
 int mlmq_graph_stats(mlmq_ctx *c, mlmq_graph_info *info) {

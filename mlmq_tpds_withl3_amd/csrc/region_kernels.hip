@@ -767,29 +767,34 @@ __global__ __launch_bounds__(256) void region_where_kernel(const uint32_t *verts
         where[verts[i]] = r << kRegionIdBits | local_id(i - lo);
 }
 
-// Per region: exits.  Each takes an inbox slot of the region it enters:
+// Per region: exits and crossing edges.  Each exit takes an inbox slot of the region it enters:
 // tmp[e] = its number there.
 __global__ __launch_bounds__(256) void region_count_kernel(const uint32_t *row, const uint32_t *col,
                                                            const uint32_t *verts, const uint32_t *where,
                                                            RegionHdr *hdr, uint32_t *tmp) {
-    __shared__ uint32_t nx;
+    __shared__ uint32_t nx, cross;
     RegionHdr &h = hdr[blockIdx.x];
-    if (threadIdx.x == 0) nx = 0;
+    if (threadIdx.x == 0) nx = cross = 0;
     __syncthreads();
-    uint32_t mx = 0;
+    uint32_t mx = 0, mine = 0;
     for (uint32_t i = threadIdx.x; i < h.nv; i += blockDim.x) {
         const uint32_t u = verts[h.first + i], lo = row[u], hi = row[u + 1];
         uint32_t inside = 0;
         for (uint32_t e = lo; e < hi; ++e) {
             const uint32_t r = where[col[e]] >> kRegionIdBits;
+            mine += r != blockIdx.x ? 1u : 0u;
             if (r == blockIdx.x && inside++ < kLaneEdges) continue;
             ++mx;
             tmp[e] = atomicAdd(&hdr[r].nin, 1u);
         }
     }
     atomicAdd(&nx, mx);
+    atomicAdd(&cross, mine);
     __syncthreads();
-    if (threadIdx.x == 0) h.nx = nx;
+    if (threadIdx.x == 0) {
+        h.nx = nx;
+        h.cross = cross;
+    }
 }
 
 __global__ __launch_bounds__(256) void region_image_kernel(const uint32_t *row, const uint32_t *col,
@@ -908,7 +913,7 @@ hipError_t region_build(const RegionPlan &plan, uint32_t n, uint64_t m, const ui
     const uint32_t nr = (uint32_t)plan.first.size() - 1;
     if (nr > (1u << (32 - kRegionIdBits))) return hipErrorInvalidValue;
     std::vector<RegionHdr> hdr(nr);
-    for (uint32_t r = 0; r < nr; ++r) hdr[r] = RegionHdr{plan.first[r], plan.first[r + 1] - plan.first[r], 0, 0, 0, 0, {0, 0}};
+    for (uint32_t r = 0; r < nr; ++r) hdr[r] = RegionHdr{plan.first[r], plan.first[r + 1] - plan.first[r], 0, 0, 0, 0, 0, 0};
     uint32_t *tmp = nullptr, *first = nullptr;
     hipError_t e = hipMalloc(&g->hdr, sizeof(RegionHdr) * nr);
     if (e == hipSuccess) e = hipMalloc(&g->verts, sizeof(uint32_t) * (size_t)n);
@@ -925,9 +930,10 @@ hipError_t region_build(const RegionPlan &plan, uint32_t n, uint64_t m, const ui
     }
     if (e == hipSuccess) e = hipMemcpyAsync(hdr.data(), g->hdr, sizeof(RegionHdr) * nr, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    uint64_t slots = 0, words = 0;
+    uint64_t slots = 0, words = 0, cross = 0;
     if (e == hipSuccess) {
         for (RegionHdr &h : hdr) {
+            cross += h.cross;
             if (h.nx > kRegionExits || h.nin > kRegionInbox) e = hipErrorInvalidValue;
             h.inbox = (uint32_t)slots;
             h.image = (uint32_t)words;
@@ -939,7 +945,7 @@ hipError_t region_build(const RegionPlan &plan, uint32_t n, uint64_t m, const ui
         g->inbox_slots = (uint32_t)slots;
         // eight mean edge weights
         g->width = (uint32_t)std::min(1e9, std::max(1.0, 8.0 * mean_weight));
-        if (words > 0xFFFFFFF0ull) e = hipErrorInvalidValue;
+        if (words > 0xFFFFFFF0ull || (double)cross > kMaxCross * (double)m) e = hipErrorInvalidValue;
     }
     if (e == hipSuccess) e = hipMalloc(&g->image, sizeof(uint32_t) * words);
     if (e == hipSuccess) e = hipMemcpy(g->hdr, hdr.data(), sizeof(RegionHdr) * nr, hipMemcpyHostToDevice);

@@ -89,7 +89,8 @@ inline int region_waves(uint32_t relaxers) { return (int)relaxers + 2; }
 uint32_t region_admit(uint64_t regions, uint32_t nq, uint32_t grid);
 RegionQuery region_query(const RegionGraph &g, uint32_t *dist, uint32_t *inbox, uint32_t *act, uint32_t src);
 // Builds the device side of a cut (temporary device memory: 4 bytes per edge).
-// Returns hipErrorInvalidValue when some region exceeds the limits.
+// Returns hipErrorInvalidValue when some region exceeds the limits or too many
+// edges cross.
 hipError_t region_build(const RegionPlan &plan, uint32_t n, uint64_t m, const uint32_t *row, const uint32_t *col,
                         const uint32_t *wgt, double mean_weight, hipStream_t s, RegionGraph *g);
 void region_free(RegionGraph *g);
