@@ -13,6 +13,7 @@ import pytest
 
 from mlmq_tpds_withl3_amd import HostGraph, Solver
 from oracle import oracle as O
+from test_region_plan import expected
 
 pytestmark = pytest.mark.gpu
 TIMEOUT = 20.0
@@ -157,3 +158,32 @@ def test_push_pull_counts(loaded):
         assert reached > 1000 and t["waves"] == 8 * t["work_blocks"]
         assert t["improvements"] >= reached - 1 and t["relaxations"] >= t["improvements"]
         assert t["l2_pushes"] >= reached
+
+
+@pytest.mark.parametrize("far,waves", [(100, 10), (120, 1)])
+def test_share_of_crossing_edges(far, waves):
+    """One-way chains of 1024 with edges to anywhere: 10.3 and 12.2 % of the edges
+    cross between the grown regions, which have up to 211 exits and slots."""
+    say(f"{far} far edges per chain")
+    n = 12 * 1024
+    rng = np.random.default_rng(1)
+    a = np.arange(n - 1)
+    a = a[(a + 1) % 1024 != 0]
+    tail = np.repeat(np.arange(12), far) * 1024 + rng.integers(0, 1024, 12 * far)
+    src = np.concatenate([a, tail])
+    dst = np.concatenate([a + 1, rng.integers(0, n, 12 * far)])
+    order = np.lexsort((dst, src))
+    row = np.concatenate([[0], np.cumsum(np.bincount(src, minlength=n))]).astype(np.int64)
+    col = dst[order].astype(np.int32)
+    region = np.empty(n, dtype=int)
+    for i, r in enumerate(expected(row, col)):
+        region[r] = i
+    share = (region[np.repeat(np.arange(n), np.diff(row))] != region[col]).mean()
+    assert (share <= 0.12) == (waves == 10)
+    w = rng.integers(1, 1000, len(col)).astype(np.int32)
+    with Solver(0) as s:
+        s.load_csr(row, col, w)
+        for x in (0, 5000, n - 1):
+            t = s.solve(x, timeout_s=TIMEOUT)
+            assert np.array_equal(s.dist(), O.dijkstra(row, col, w, x)[0])
+            assert t["waves"] == waves * t["work_blocks"]
