@@ -1296,14 +1296,14 @@ int mlmq_server_run(mlmq_server *s, const mlmq_serve_request *reqs, int32_t nreq
                 uint32_t *inbox = (uint32_t *)part;
                 h_region[R.nq] = mlmq::region_query(*region_graph, L.dist, inbox, inbox + region_graph->inbox_slots + 1,
                                                     (uint32_t)reqs[id].src);
-                h_out[i] = {l.ctl, nullptr, l.times + 2 * R.nq};
+                h_out[i] = {l.ctl, nullptr, l.times + 2 * R.nq, nregion > 1 ? 1u : 0u};
                 R.longest = std::max({R.longest, region_graph->n, region_graph->inbox_slots});
                 ++R.nq;
             } else {
                 uint64_t *time = l.times + 2 * (nregion + P.nq);
                 const mlmq::PushPullLaunch q = pushpull_query(g, (uint32_t)reqs[id].src, L.dist, part, time);
                 h_push[P.nq++] = q;
-                h_out[i] = {nullptr, q.count + mlmq::kBoundedRounds + kLaneRounds, time};
+                h_out[i] = {nullptr, q.count + mlmq::kBoundedRounds + kLaneRounds, time, 0};
                 P.max_n = std::max(P.max_n, L.n);
             }
             mlmq::serve_request_write(l.h_reqs, i, L, (uint32_t)reqs[id].src, sl.fresh, expect, wg_first, wg);

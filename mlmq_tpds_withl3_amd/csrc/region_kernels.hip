@@ -65,10 +65,13 @@
 // Whoever ends the last query publishes one exit record per workgroup of the
 // grid, for the ticket each of them takes last.
 //
-// Errors: a workgroup that sees the error word set or its deadline passed writes
-// its region's distances out and ends.  A region that is left this way with work
-// keeps its credit outstanding, so a query that was over by then has all of its
-// distances in the row, and no other one ends any more: qtime tells which.
+// Errors: a workgroup that sees the error word set or its deadline passed ends.
+// In a launch over a table of queries it writes its region's distances out
+// first: a region that is left this way with work keeps its credit outstanding,
+// so a query that was over by then has all of its distances in the row, and no
+// other one ends any more (qtime tells which).  Launches on one graph answer all
+// of their queries or none; there the write costs road 6.26M 1.4 % by what the
+// compiler makes of the poller's registers.
 //
 // Measured, device us of one query, vertex queue / here: 2,052 vertices 190 / 41,
 // 264k 1250 / 430, 1.06M 4500 / 800-1000, 6.26M 5850 / 1850; 64 queries on 264k
@@ -471,7 +474,7 @@ __device__ __forceinline__ void return_credit(const RegionArgs &a, uint32_t quer
 }
 
 // Serves the adopted region until it is left or the solve is over.
-template <uint32_t kR, int kG>
+template <bool kTable, uint32_t kR, int kG>
 __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, const RegionHdr &h,
                                            const uint32_t *image, const uint32_t *verts, uint32_t region,
                                            uint32_t query, uint32_t *dist, uint32_t *inbox, uint32_t *act,
@@ -505,11 +508,15 @@ __device__ __forceinline__ void run_poller(const RegionArgs &a, RegionLds &S, co
     dirty = seed != 0;
     for (uint32_t turn = 0;; ++turn) {
         if ((turn & 31u) == 0) {
-            // (after an error too the distances go out: this query may be over)
-            if (uniform(ld_relaxed(a.ctl + kErrOff))) break;
-            if (wall_clock64() > deadline) {
+            bool stop = uniform(ld_relaxed(a.ctl + kErrOff)) != 0;
+            if (!stop && wall_clock64() > deadline) {
                 region_raise(a, kErrTimeout);
-                break;
+                stop = true;
+            }
+            if (stop) {
+                // (this query may be over, and others be asked for)
+                if constexpr (kTable) break;
+                else return;
             }
         }
         st.polls += lane == 0 ? 1u : 0u;
@@ -652,9 +659,9 @@ __global__ __launch_bounds__(kThreads<kR>, kPerSimd<kR>) void region_solver_kern
             run_relaxer<kR>(S, h, image, verts, dist, visited, wave, width, rs);
         } else if (wave == kR) {
             uint32_t *in = inbox + h.inbox;
-            if (h.nin <= 2 * kWave) run_poller<kR, 2>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
-            else if (h.nin <= 4 * kWave) run_poller<kR, 4>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
-            else run_poller<kR, 6>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
+            if (h.nin <= 2 * kWave) run_poller<kTable, kR, 2>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
+            else if (h.nin <= 4 * kWave) run_poller<kTable, kR, 4>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
+            else run_poller<kTable, kR, 6>(a, S, h, image, verts, region, query, dist, in, act, regions, seed, visited, deadline, ms);
             if (lane == 0) {
                 sh_st(&S.over, 1u);
                 lds_order();

@@ -147,6 +147,7 @@ struct ServeOutcome {
     const uint32_t *ctl;      // region solver: control block of its launch
     const uint32_t *rest;     // push-pull solver: vertices its last round left
     const uint64_t *time;     // start and end ticks
+    uint64_t own_end;         // region solver: 1 if this query may be over though the launch failed
 };
 // Fills in status and times of those requests.
 hipError_t launch_serve_outcome(const ServeLaunch &S, const ServeOutcome *out, hipStream_t s);

@@ -966,7 +966,7 @@ __global__ __launch_bounds__(256) void serve_outcome_kernel(ServeRequest *reqs, 
         e = o.ctl[kErrOff];
         const uint32_t tail = o.ctl[kTailOff];
         if (e == kErrNone && (o.ctl[kExitOff] != 1u || tail != o.ctl[kTakenOff] || tail != o.ctl[kDoneOff])) e = kErrInternal;
-        else if (e != kErrNone && o.time[1] != 0) e = kErrNone;
+        else if (e != kErrNone && o.own_end && o.time[1] != 0) e = kErrNone;
     }
     reqs[i].status = e;
     reqs[i].t_start = o.time[0];
