@@ -274,7 +274,7 @@ int mlmq_solve_noalloc(mlmq_ctx *ctx, int32_t src, const mlmq_params *params, in
  * (0 = one per CU, at most nq).  With work_blocks 0 and settings for which
  * mlmq_solve takes the region solver, that solver runs the batch in one launch,
  * a few queries in flight at a time (not 200 queries or more on a graph of more
- * than about 390,000 vertices, for which the queue is faster).  Results stay on the device until copied
+ * than about 390,000 vertices, for which the queue with tuned settings is faster).  Results stay on the device until copied
  * with mlmq_copy_batch_dist. */
 int mlmq_solve_batch(mlmq_ctx *ctx, const int32_t *sources, int32_t nq,
                      const mlmq_params *params, mlmq_batch_timing *timing);

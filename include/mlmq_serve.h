@@ -31,8 +31,9 @@
  *   - In a launch lane, requests that mlmq_solve would give to the region or
  *     the push-pull solver run on it, those of all such graphs in the same
  *     launches (hub_split, a bucket_capacity, on road-like graphs light_split,
- *     and slots too small for these solvers' state keep a request on the vertex
- *     queue, as does live serving).  There each request runs on `workgroups`
+ *     slots too small for these solvers' state, and 32 or more requests of other
+ *     lanes in flight keep a request on the vertex queue, as does live serving;
+ *     mlmq_serve_result.solver says which one answered).  There each request runs on `workgroups`
  *     workgroups of `waves` wave64 that share its queue partition.  Distances
  *     are exact (the same per vertex as a CPU Dijkstra), whatever else runs
  *     beside it.
@@ -88,7 +89,8 @@ typedef struct mlmq_server_config {
     int32_t  max_batch;       /* requests per launch, 1..4096; 0 = 64 */
     int32_t  max_pending;     /* waiting requests before arrivals are rejected; 0 = no limit */
     int32_t  verify;          /* compare results with registered expected rows */
-    double   timeout_s;       /* device watchdog per launch; <= 0 means 60 s */
+    double   timeout_s;       /* device watchdog per launch; <= 0 means 60 s.  Requests that were
+                                 done before it are answered */
     int32_t  spread_waves;    /* a launch of few requests runs them on up to this many waves in
                                  total, as one-wave workgroups (at most 512 per request), when
                                  that is more than the graph's workgroups x waves: a request

@@ -98,10 +98,13 @@ struct Lane {
 // With so many requests of other lanes in flight a launch goes to the vertex
 // queue: each CU then has requests of its own, as in a large batch, and the
 // launches share the device evenly.  Poisson arrivals over road 264k (50 %), road
-// 6.26M (30 %) and RMAT-20 (20 %), nothing tuned, by the queue alone / this way:
-// 1200 queries/s p50 73 / 5.6 ms, p99 111 / 34 ms; 1700 queries/s p50 88 / 92,
-// p99 133 / 126; 2000 offered 1717 / 1832 served.  (By the other solvers alone
-// 1380 of 2000; switching at 96 instead: p99 592 ms at 1500.)
+// 6.26M (30 %) and RMAT-20 (20 %), nothing tuned, three traces of 3 s, by the queue
+// alone / this way, ms: 1000 queries/s p50 77-83 / 3-4, p99 116-129 / 18-33; 1200
+// p50 83-86 / 5-8, p99 123-146 / 59-146; 1500 p50 97-104 / 92-93, p99 144-156 /
+// 142-149; 1700 p50 117-137 / 114-128, p99 175-203 / 185-191; 2000 offered
+// 1695-1714 / 1703-1717 served.  Bursts of 32, 64, 96, 128, 256 over road 264k,
+// road 1.06M and RMAT-18: 49, 55, 55, 62, 116 / 3, 6, 42, 63, 110.  (By the other
+// solvers alone 1380 of 2000; switching at 96 instead: p99 592 ms at 1500.)
 constexpr uint64_t kCrowd = 32;
 
 // Most bytes of a lane's push-pull states: about 20 requests on RMAT-20.

@@ -23,7 +23,7 @@
 // reads out-edges as in-edges.
 //
 // Every round is one launch, and no workgroup waits for another.  A round that
-// finds nothing costs its launch (4 us).
+// finds nothing costs its launch (40 more of them: 63-88 us, RMAT-13 to 20).
 //
 // Measured, device us of one query, vertex queue / here: RMAT-14 400 / 165,
 // RMAT-18 2900 / 330, RMAT-22 11000 / 1130 (0.6 TB/s of scattered line fetches;
